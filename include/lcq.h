@@ -395,6 +395,15 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
                         int clip_sym, float qmin, float qmax, int flags, void* best_max, void* best_min, float* errs,
                         void* stream);
 
+/* The same search in the reference's own rounding sequence (every product rounded to bf16, fp32 group sums rounded, the
+ * squared difference and the mean rounded; auto_clip.py:83-191 with clip_version v1, weight-only), one launch:
+ *  w [R, K], x [T, K] LCQ_BF16; group_size 32, 64 or 128, K % group_size == 0; n_steps <= LCQ_CLIP_MAX_STEPS
+ *  best_max, best_min [R, G] bf16 out; errs [R, G, n_steps] fp32 out: the errors as compared (rounded to bf16). */
+#define LCQ_CLIP_MAX_STEPS 12
+int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, int64_t T, int group_size, int n_grid,
+                          int n_steps, int clip_sym, float qmin, float qmax, int flags, void* best_max, void* best_min,
+                          float* errs, void* stream);
+
 /* The grouped products of AutoClipper.auto_clip_layer, auto_clip.py:141,160: `(x * w).sum(dim=-1)` with
  * x [1, T, G, gs] and w [R, 1, G, gs]:  out[r, g, t] = round(sum_j round(x[t, g*gs + j] * w[r, g*gs + j])) - every
  * product rounded to the tensors' type as the materialised product tensor is, fp32 accumulation, one final rounding

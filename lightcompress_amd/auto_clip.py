@@ -9,12 +9,13 @@ Two search paths:
 
 * the default follows the reference's rounding sequence: every product of ``(x * w)`` rounded to the tensors' type,
   fp32 sums per group, the two sums rounded before they are subtracted, the squared difference rounded, the mean over
-  tokens rounded (``lcq_group_dots``); weights go through the quantizer classes exactly as the reference's
+  tokens rounded.  The common case (v1, weight-only, one bf16 input, groups of 32 / 64 / 128) is one launch that keeps
+  the candidates on the chip (``lcq_clip_search_exact``); everything else runs step by step (``lcq_group_dots``): weights go through the quantizer classes exactly as the reference's
   ``fake_quantize_weight`` / ``fake_quantize_input`` do.  It covers ``clip_version`` v1 and v2, ``w_only`` True and
   False, any group size or per_channel weights, bf16 and fp32, several inputs;
 * ``AutoClipper.fast = True`` selects, where it applies (v1, weight-only, per_group 128, bf16, min/max integer
   quantizer), one bf16 MFMA kernel (``lcq_awq_clip_search``) that contracts the weight *difference* with the tokens
-  and does not reproduce the rounding of the two sums: about 50x faster, same range on > 90 % of the groups.
+  and does not reproduce the rounding of the products and sums: about 15x faster, same range on > 90 % of the groups.
 
 ``clip_version='v2'`` with a per_group quantizer fails in the reference (its static fake quant broadcasts
 [ocb * G, gs] rows against [ocb, 1, G, 1] qparams); here it runs, with the qparams matched to the groups.
@@ -128,7 +129,35 @@ class AutoClipper:
                 raise NotImplementedError('inputs of different token counts: the per-input means are not one mean '
                                           '(use fast = False)')
             return self._search_mfma(wc, torch.cat(xs) if len(xs) > 1 else xs[0], n_grid, n_steps)
+        if self._fused_applies(wc, xs, n_steps):
+            return self._search_fused(wc, xs[0], group_size, n_grid, n_steps)
         return self._search_exact(block_idx, layer_name, wc, xs, group_size, n_grid, n_steps, eps)
+
+    def _fused_applies(self, w, xs, n_steps):
+        """lcq_clip_search_exact: one launch with the same roundings as _search_exact, for bf16 tensors, v1, weight-only,
+        groups of 32 / 64 / 128, one input and the min/max integer quantizer."""
+        wq = self.wquantizer
+        return (self.clip_version == 'v1' and self.w_only and len(xs) == 1 and 0 < n_steps <= 12
+                and wq.granularity == 'per_group' and wq.group_size in (32, 64, 128)
+                and getattr(wq, 'quant_type', 'int-quant') == 'int-quant' and wq.round_zp and wq.calib_algo == 'minmax'
+                and -256 <= float(wq.qmin) < float(wq.qmax) <= 256
+                and w.dtype == torch.bfloat16 and xs[0].dtype == torch.bfloat16
+                and w.data_ptr() % 16 == 0 and xs[0].data_ptr() % 16 == 0)
+
+    def _search_fused(self, wc, x, group_size, n_grid, n_steps):
+        wq = self.wquantizer
+        R, K = wc.shape
+        G = K // group_size
+        best_max = torch.empty((R, G, 1), dtype=torch.bfloat16, device=wc.device)
+        best_min = torch.empty((R, G, 1), dtype=torch.bfloat16, device=wc.device)
+        errs = torch.empty((R, G, n_steps), dtype=torch.float32, device=wc.device)
+        L.check(L.lib().lcq_clip_search_exact(L.ptr(wc), L.ptr(x), L.i64(R), L.i64(K), L.i64(x.shape[0]), L.i32(group_size),
+                                              L.i32(n_grid), L.i32(n_steps), L.i32(1 if self.clip_sym else 0),
+                                              L.f32(float(wq.qmin)), L.f32(float(wq.qmax)), L.i32(L.FLAG_SYM if wq.sym else 0),
+                                              L.ptr(best_max), L.ptr(best_min), L.ptr(errs), L.stream()),
+                'lcq_clip_search_exact')
+        self.last_errs = errs
+        return best_max, best_min
 
     def _search_mfma(self, wc, x, n_grid, n_steps):
         """Equal token counts: the mean of the per-input means is the mean over all tokens."""

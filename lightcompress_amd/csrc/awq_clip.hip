@@ -152,6 +152,200 @@ __global__ __launch_bounds__(256) void clamp_groups_scalar_kernel(const void* __
   }
 }
 
+// The reference's rounding sequence on the matrix pipe (16-bit types).
+//
+//   dot(t, r) = sum_j round(x[t, j] * w[r, j])      every product rounded to the tensors' type, fp32 sums
+//
+// The rounding of every product keeps the contraction itself off the matrix pipe, but not its two halves:
+//   products  v_mfma_f32_32x32x4_2b with ONE non-zero k slot per block is an outer product: block 0 gives x[t, j] w[r, j],
+//             block 1 gives x[t, j+1] w[r, j+1] for 32 tokens x 32 rows (exact in fp32), in the same registers of both blocks;
+//   rounding  one v_cvt_pk per pair (j, j+1): 16 instructions for 2048 products, all the vector pipe has to do;
+//   sums      four rounded pairs of a lane are one A operand of v_mfma_f32_16x16x32 (k = 8 values of a lane); a constant
+//             0 / 1 B operand adds each pair and sends it to a column of its own.
+// Layouts: products leave lane l with row l % 32 and tokens 8 (i / 4) + 4 (l / 32) + i % 4 in register i; the sums leave
+// sum[q][i] = token 8 q + 4 ((l >> 3) & 1) + (l & 3), row 16 ((l >> 2) & 1) + 4 (l >> 4) + i.
+// What bounds it: 64 + 4 x 16 matrix-pipe cycles per 2048 products; the 16 conversions (64 vector cycles) run under the
+// next products.  v_mfma_f32_32x32x1 and v_dot2_f32_bf16 would do the same sums, but neither overlaps with vector
+// instructions on this chip (229 against 128 cycles), and moving a quarter of the sums to the vector pipe made it 13 %
+// slower.  Measured (rows 11008 x 4096 + 11008 x 4096 + 4096 x 11008, 512 tokens, 10 steps): 92.3 -> 25.8 ms, the matrix
+// pipes busy in 78 % of the cycles; the products one after the other in the same registers 31.2, without all
+// conversions ahead of the sums 28.3.
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(4))) short i16x4;
+typedef __attribute__((ext_vector_type(32))) float f32x32;
+
+template <int BF> __device__ __forceinline__ f32x32 outer_products(u32x2 a, u32x2 b) {
+  f32x32 z;
+  #pragma unroll
+  for (int i = 0; i < 32; ++i) z[i] = 0.0f;
+  if constexpr (BF == ROW_F16) return __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), z, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), z, 0, 0, 0);
+}
+template <int BF> __device__ __forceinline__ f32x4 add_pairs(u32x4 pairs, u32x4 ones, f32x4 c) {
+  if constexpr (BF == ROW_F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, pairs), __builtin_bit_cast(f16x8, ones), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pairs), __builtin_bit_cast(bf16x8, ones), c, 0, 0, 0);
+}
+template <int BF> __device__ __forceinline__ uint32_t pack_pair(float a, float b) {
+  if constexpr (BF == ROW_F16) return f16_pack_rne(a, b); else return bf16_pack_rne(a, b);
+}
+// B operand of add_pairs: lane (h = l / 16, n = l % 16) holds k = 8 h + i of column n; pair i / 2 of quarter h goes to column 4 h + i / 2
+template <int BF> __device__ __forceinline__ u32x4 pair_columns(int lane) {
+  const uint32_t one = BF == ROW_F16 ? 0x3c003c00u : 0x3f803f80u;
+  u32x4 b;
+  #pragma unroll
+  for (int d = 0; d < 4; ++d) b[d] = (lane & 15) == 4 * (lane >> 4) + d ? one : 0u;
+  return b;
+}
+
+constexpr int GT = 32;                   // tokens and rows of one wave's tile
+template <int GS> constexpr int gd_pitch() { return GS * 2 + 16; }     // bytes per LDS row (16-byte skew)
+// sum[4] of a tile: a = the tokens' GS columns (lane l: token l % 32), wrow = row l % 32 in LDS.  The products of the next
+// column pair are issued before the current ones are rounded: the empty asm keeps that order (without it the compiler
+// runs the two one after the other in the same registers).
+template <int BF, int GS>
+__device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint32_t mask, u32x4 ones, f32x4* sum) {
+  #pragma unroll
+  for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  u32x4 b = *(const u32x4*)wrow;
+  const auto products = [&](int i) {                        // columns 2 i (block 0) and 2 i + 1 (block 1)
+    const int p = i & 3;
+    if (p == 0 && i > 0) b = *(const u32x4*)(wrow + 4 * i);
+    const u32x4 av = a[i >> 2];
+    const uint32_t w = b[p] & mask;
+    return outer_products<BF>(p < 2 ? u32x2{av[0], av[1]} : u32x2{av[2], av[3]}, (p & 1) ? u32x2{0, w} : u32x2{w, 0});
+  };
+  f32x32 d[2];
+  d[0] = products(0);
+  #pragma unroll
+  for (int i = 0; i < GS / 2; ++i) {
+    f32x32& cur = d[i & 1];
+    if (i + 1 < GS / 2) {
+      d[(i + 1) & 1] = products(i + 1);
+      asm volatile("" : "+v"(d[0]), "+v"(d[1]));
+    }
+    u32x4 pr[4];
+    #pragma unroll
+    for (int q = 0; q < 4; ++q)
+      #pragma unroll
+      for (int k = 0; k < 4; ++k) pr[q][k] = pack_pair<BF>(cur[4 * q + k], cur[16 + 4 * q + k]);
+    asm volatile("" : "+v"(pr[0]), "+v"(pr[1]), "+v"(pr[2]), "+v"(pr[3]));
+    #pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] = add_pairs<BF>(pr[q], ones, sum[q]);
+  }
+}
+
+// The whole search of AutoClipper.auto_clip_layer (v1, weight-only, bf16, groups of GS columns) in one launch: a workgroup
+// owns 32 rows of one group, keeps the original and the n_steps clamped-and-quantized versions of them in LDS, and every
+// wave runs all versions over its 32-token tiles; neither the candidates nor the [R, G, T] products reach memory.
+template <int GS>
+__global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ x,
+                                                             int R, int K, int T, int n_grid, int n_steps, int clip_sym,
+                                                             IntOp<true, true> op, uint16_t* __restrict__ best_max,
+                                                             uint16_t* __restrict__ best_min, float* __restrict__ errs) {
+  constexpr int PITCH_W = gd_pitch<GS>(), TEAM = GS / 8, VERSION = GT * PITCH_W;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* const esum = (float*)(smem + (n_steps + 1) * VERSION);          // [waves][n_steps][32]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int G = K / GS, g = blockIdx.x % G, r0 = (blockIdx.x / G) * GT;
+  const auto shrink = [&](float v, int s) { return rnd<true>(v * (float)(1.0 - (double)s / (double)n_grid)); };
+
+  for (int i = tid; i < waves * n_steps * GT; i += blockDim.x) esum[i] = 0.0f;
+  for (int ch = tid; ch < GT * TEAM; ch += blockDim.x) {                 // one 16-byte chunk per thread (and turn)
+    const int row = ch / TEAM, c = ch % TEAM;
+    u32x4 raw = {0, 0, 0, 0};
+    if (r0 + row < R) raw = *(const u32x4*)(w + (int64_t)(r0 + row) * K + g * GS + c * 8);
+    char* dst = smem + row * PITCH_W + c * 16;
+    *(u32x4*)dst = raw;
+    float v[8], mn = __builtin_inff(), mx = -__builtin_inff();
+    unpack<true>(raw, v);
+    chunk_minmax<IntOp<true, true>>(raw, mn, mx);
+    team_range<TEAM>(mn, mx);
+    const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
+    for (int s = 0; s < n_steps; ++s) {
+      const float hi = shrink(org_max, s), lo = clip_sym ? -hi : shrink(mn, s);
+      const IntRow p = op.make(nan_min(nan_max(mn, lo), hi), nan_min(nan_max(mx, lo), hi));   // range of the clamped group
+      float cv[8], d[8];
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) cv[i] = nan_min(nan_max(v[i], lo), hi);
+      op.template fused_dq<8>(cv, d, p);
+      *(u32x4*)(dst + (s + 1) * VERSION) = pack_rne<true>(d);
+    }
+  }
+  __syncthreads();
+
+  const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
+  const u32x4 ones = pair_columns<ROW_BF16>(lane);
+  const char* wrow = smem + (lane & 31) * PITCH_W;
+  for (int t0 = wave * GT; t0 < T; t0 += waves * GT) {
+    u32x4 a[GS / 8];
+    const bool ok = t0 + (lane & 31) < T;                                // tokens past T: zeros, which add nothing
+    const uint16_t* xr = x + (int64_t)(ok ? t0 + (lane & 31) : 0) * K + g * GS;
+    #pragma unroll
+    for (int c = 0; c < GS / 8; ++c) { a[c] = *(const u32x4*)(xr + 8 * c); if (!ok) a[c] = u32x4{0, 0, 0, 0}; }
+    f32x4 org[4], cur[4];
+    dots_tile<ROW_BF16, GS>(a, wrow, mask, ones, org);
+    #pragma unroll
+    for (int q = 0; q < 4; ++q)
+      #pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        float o0 = org[q][i], o1 = org[q][i + 1];
+        rnd_pair<true>(o0, o1);
+        org[q][i] = o0; org[q][i + 1] = o1;
+      }
+    #pragma unroll 1
+    for (int s = 0; s < n_steps; ++s) {
+      dots_tile<ROW_BF16, GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
+      float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      #pragma unroll
+      for (int q = 0; q < 4; ++q)
+        #pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          float c0 = cur[q][i], c1 = cur[q][i + 1];
+          rnd_pair<true>(c0, c1);
+          c0 -= org[q][i]; c1 -= org[q][i + 1];
+          rnd_pair<true>(c0, c1);
+          c0 *= c0; c1 *= c1;
+          rnd_pair<true>(c0, c1);
+          e[i] += c0; e[i + 1] += c1;
+        }
+      // over the tokens of the tile: lanes that differ in bits 0, 1 and 3
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        e[i] += lane_xor<1>(e[i]);
+        e[i] += lane_xor<2>(e[i]);
+        e[i] += u2f((uint32_t)__builtin_amdgcn_ds_swizzle((int)f2u(e[i]), 0x201F));      // xor 8
+      }
+      if ((lane & 0xb) == 0) {
+        float* es = esum + (wave * n_steps + s) * GT + 16 * ((lane >> 2) & 1) + 4 * (lane >> 4);
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) es[i] += e[i];
+      }
+    }
+  }
+  __syncthreads();
+  // err_mean < min_errs, step by step: the first minimum below 1e9 wins, NaN never does
+  if (tid < GT && r0 + tid < R) {
+    const int row = tid;
+    float mn = __builtin_inff(), mx = -__builtin_inff();
+    for (int c = 0; c < TEAM; ++c) chunk_minmax<IntOp<true, true>>(*(const u32x4*)(smem + row * PITCH_W + c * 16), mn, mx);
+    const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
+    float best = 999817216.0f, bmax = org_max, bmin = mn;                 // bf16(1e9)
+    const int64_t at = (int64_t)(r0 + row) * G + g;
+    for (int s = 0; s < n_steps; ++s) {
+      float e = 0.0f;
+      for (int wv = 0; wv < waves; ++wv) e += esum[(wv * n_steps + s) * GT + row];
+      e = rnd<true>(e * (1.0f / (float)T));                              // torch's mean: the sum times an fp32 factor
+      errs[at * n_steps + s] = e;
+      const float hi = shrink(org_max, s), lo = clip_sym ? -hi : shrink(mn, s);
+      if (e < best) { best = e; bmax = hi; bmin = lo; }
+    }
+    best_max[at] = (uint16_t)(f2u(bmax) >> 16);
+    best_min[at] = (uint16_t)(f2u(bmin) >> 16);
+  }
+}
+
 // out[r, g, t] = round( sum_j round(x[t, g*gs + j] * w[r, g*gs + j]) ): the reference's (x * w).sum(dim=-1) of
 // auto_clip.py:141,160 on x [1, T, G, gs] and w [R, 1, G, gs] - the product tensor is materialised in the tensors'
 // type there (every product rounded), the sum accumulates in fp32 and rounds once.  General in the group size, the
@@ -296,6 +490,33 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
   awq_clip_kernel<<<grid, dim3(512), 0, (hipStream_t)stream>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K,
                                                                (int)T, n_grid, n_steps, clip_sym, op, (uint16_t*)best_max,
                                                                (uint16_t*)best_min, errs);
+  LCQ_CHECK_LAUNCH();
+  return LCQ_OK;
+}
+
+int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, int64_t T, int group_size, int n_grid,
+                          int n_steps, int clip_sym, float qmin, float qmax, int flags, void* best_max, void* best_min,
+                          float* errs, void* stream) {
+  if (!w || !x || !best_max || !best_min || !errs || R <= 0 || K <= 0 || T <= 0) return LCQ_EINVAL;
+  if ((group_size != 32 && group_size != 64 && group_size != 128) || K % group_size != 0) return LCQ_EINVAL;
+  if (K > 0x7fffffff / 2 || R > 0x7fffffff || T > 0x7fffffff) return LCQ_EINVAL;
+  if (n_grid <= 0 || n_steps <= 0 || n_steps > n_grid || n_steps > LCQ_CLIP_MAX_STEPS) return LCQ_EINVAL;
+  if (!(qmax > qmin) || qmax > 256.0f || qmin < -256.0f || (flags & (LCQ_FLAG_STATIC | LCQ_FLAG_NO_ROUND_ZP))) return LCQ_EINVAL;
+  if ((((uintptr_t)w | (uintptr_t)x) % 16) != 0) return LCQ_EALIGN;
+  const auto op = make_op<IntOp<true, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
+  const int64_t grid = ((R + GT - 1) / GT) * (K / group_size);
+  if (grid > 0x7fffffff) return LCQ_EINVAL;
+  // one wave per 32 tokens up to eight (two per SIMD: one wave's conversions run under the other's matrix instructions)
+  const int waves = T > 4 * GT ? 8 : (T > 2 * GT ? 4 : 2);
+  hipStream_t st = (hipStream_t)stream;
+  #define LCQ_CLIP(GS) do { \
+    const size_t lds = (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)waves * n_steps * GT * 4; \
+    static const hipError_t once = hipFuncSetAttribute((const void*)clip_search_kernel<GS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+    if (once != hipSuccess) return LCQ_ELAUNCH; \
+    clip_search_kernel<GS><<<dim3((unsigned)grid), dim3(64 * waves), lds, st>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K, \
+        (int)T, n_grid, n_steps, clip_sym, op, (uint16_t*)best_max, (uint16_t*)best_min, errs); } while (0)
+  if (group_size == 128) LCQ_CLIP(128); else if (group_size == 64) LCQ_CLIP(64); else LCQ_CLIP(32);
+  #undef LCQ_CLIP
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

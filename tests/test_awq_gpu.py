@@ -403,6 +403,31 @@ def test_auto_clip_reference_rounding_sequence(dev, ver, w_only, wspec, clip_sym
         assert_bit_equal(got, want, 'learnable fake quant')
 
 
+@pytest.mark.parametrize('gs,T,bit,sym,clip_sym', [(128, 1, 4, False, False), (128, 33, 4, True, True), (64, 32, 4, False, True),
+                                                   (64, 129, 3, False, False), (32, 65, 8, True, False), (32, 31, 4, False, False),
+                                                   (128, 288, 4, False, False)])
+def test_auto_clip_one_launch_search_at_tile_edges(dev, gs, T, bit, sym, clip_sym):
+    """lcq_clip_search_exact where its 32-token tiles and 2 / 4 / 8 waves begin and end, for every group size it takes.
+    Bar as in test_auto_clip_reference_rounding_sequence: only fp32 additions are in another order."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    R, K = 64, 3 * gs
+    spec = Q.IntSpec(bit, sym, 'per_group', group_size=gs)
+    w = weight_like(R, K, seed=T + gs, dtype=torch.bfloat16)
+    x = (torch.randn(T, K, generator=gen(T)) * torch.exp(0.5 * torch.randn(K, generator=gen(K)))).bfloat16()
+    obmax, obmin, oerrs = A.auto_clip_layer(spec, w, [x.clone()], clip_sym=clip_sym, n_sample_token=T)
+    clipper = AutoClipper(True, IntegerQuantizer(bit, sym, 'per_group', group_size=gs), None, 'v1', clip_sym, False, None)
+    assert clipper._fused_applies(w.to(dev), [x.to(dev)], 10)
+    bmax, bmin = clipper.auto_clip_layer(0, 'fc', w.to(dev), [x.to(dev)], n_sample_token=T)
+    errs, oe = clipper.last_errs.cpu(), oerrs.float()
+    assert errs.shape == oe.shape and bmax.shape == obmax.shape and bmin.dtype == torch.bfloat16
+    assert float((errs == oe).float().mean()) > 0.99
+    assert bool(((errs - oe).abs() <= 2 * 2.0 ** -7 * oe.abs()).all())
+    same = (errs == oe).all(-1, keepdim=True)               # equal errors leave no choice
+    assert torch.equal(bmax.cpu()[same], obmax[same]) and torch.equal(bmin.cpu()[same], obmin[same])
+
+
 def test_auto_clip_run_skips_query_key_and_handles_float8_weights(dev):
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
