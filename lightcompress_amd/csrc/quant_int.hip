@@ -103,6 +103,36 @@ __global__ void qparams_kernel(const void* __restrict__ mn, const void* __restri
   op.store_qp(scales, zeros, i, p);
 }
 
+// 16-bit rows with fp32 parameters per row (calibrated ranges are fp32, quant.py:147-205): torch promotes every operation
+// to fp32 and the caller casts the result back, so this reads 16-bit chunks, computes as fp32 rows do and rounds once.
+// HBM-bound; the rows are not reduced over, so chunks are independent (row = chunk / chunks per row).
+template <int BF>
+__global__ __launch_bounds__(256) void static_promoted_kernel(const u32x4* __restrict__ x, int64_t nchunks, int cpr,
+                                                              const void* __restrict__ scales, const void* __restrict__ zeros,
+                                                              void* __restrict__ dq, void* __restrict__ codes, IntOp<0, true> op) {
+  for (int64_t ch = (int64_t)blockIdx.x * 256 + threadIdx.x; ch < nchunks; ch += (int64_t)gridDim.x * 256) {
+    const u32x4 raw = __builtin_nontemporal_load(x + ch);
+    const IntRow p = op.load(scales, zeros, op.scalar_qp ? 0 : (int64_t)((uint64_t)ch / (uint32_t)cpr));
+    float v[8], q[8];
+    unpack<BF>(raw, v);
+    if (!codes) {
+      op.template fused_dq<4>(v, q, p);
+      op.template fused_dq<4>(v + 4, q + 4, p);
+      __builtin_nontemporal_store(pack_rne<BF>(q), (u32x4*)dq + ch);
+      continue;
+    }
+    op.template codes<4>(v, q, p);
+    op.template codes<4>(v + 4, q + 4, p);
+    store_codes(op, codes, ch * 8, q);
+    store_codes(op, codes, ch * 8 + 4, q + 4);
+    if (dq) {
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = op.deq_raw(q[i], p);
+      __builtin_nontemporal_store(pack_rne<BF>(v), (u32x4*)dq + ch);
+    }
+  }
+}
+
 // dequant, quant.py:709-711, on stored float codes
 template <int BF>
 __global__ __launch_bounds__(256) void dequant_kernel(const void* __restrict__ q, int64_t rows, int64_t cols,
@@ -153,6 +183,125 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
     if (err < best) { best = err; cur_min = xmin; cur_max = xmax; }
   }
   if (lane == 0) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
+}
+
+// The same search with the row in registers, for rounded zero points: TEAM lanes (256: a workgroup) share a row, PER
+// elements each.
+//   * t = x * (1/s) instead of x / s: a quotient within 2 ulp of a half-integer may round to the other neighbour, both
+//     of which are half a step away from x, so the error differs by less than the rounding of its sum;
+//   * |d| ^ norm = d^2 * 2 ^ ((norm - 2) log2 |d|): the square is exact to one rounding and only the fraction of the
+//     exponent goes through v_log / v_exp; x and s are scaled by the power of two that brings the row's largest value
+//     to [1, 2), so |log2| stays small (the whole expression is good to 2-3 ulp) and nothing underflows.  The factor is
+//     common to all steps of a row and positive, so it changes no comparison;
+//   * every term of the error is >= 0 and fp32 sums of such terms never shrink, so a part of the sum above `best` decides a
+//     step: first the error of the two extremes alone (most steps behind the best one lose by what they clip there), then
+//     after every quarter of the elements.  A wave goes on to the next step when all its rows are decided;
+//   * elements past the row's end are zeros: with qmin <= z <= qmax they quantize to themselves and add nothing.
+// What bounds it: ten instructions per element and step, two of them transcendental (about 50 vector cycles).  4096 x 4096
+// bf16 in groups of 128, 80 steps: 1870 us with a re-read per step, IEEE divisions and powf; 497 with the row in
+// registers; 222 with the steps cut short (4096 rows of 4096: 1253, 437, 72).
+template <int BF, int TEAM, int PER>
+__global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restrict__ x, int64_t rows, int cols, int vec, int steps,
+                                                             int grid_n, float norm, IntOp<0, false> op,
+                                                             float* __restrict__ mn_out, float* __restrict__ mx_out) {
+  constexpr int N = Vec<BF>::N;
+  constexpr bool BLOCK = TEAM > 64;
+  __shared__ float shrink[256];                              // p of every step (a double division each)
+  __shared__ float sm[8];
+  for (int i = threadIdx.x; i < steps; i += 256) shrink[i] = (float)(1.0 - (double)i / (double)grid_n);
+  __syncthreads();
+  const int64_t row_ = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TEAM;
+  const int64_t row = row_ < rows ? row_ : rows - 1;         // surplus teams repeat the last row and store nothing
+  const int t = threadIdx.x % TEAM;
+  float v[PER], mn = __builtin_inff(), mx = -__builtin_inff();
+  if (vec) {
+    #pragma unroll
+    for (int c = 0; c < PER / N; ++c) {                      // chunks dealt out round robin: whole lines per instruction
+      const int col = (c * TEAM + t) * N;
+      u32x4 raw = {0, 0, 0, 0};
+      if (col < cols) raw = *(const u32x4*)((const char*)x + (row * cols + col) * (BF ? 2 : 4));
+      unpack<BF>(raw, v + c * N);
+      if (col < cols)
+        #pragma unroll
+        for (int i = 0; i < N; ++i) { mn = nan_min(mn, v[c * N + i]); mx = nan_max(mx, v[c * N + i]); }
+    }
+  } else {
+    #pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int col = i * TEAM + t;
+      v[i] = 0.0f;
+      if (col < cols) { v[i] = load_scalar<BF>(x, row * cols + col); mn = nan_min(mn, v[i]); mx = nan_max(mx, v[i]); }
+    }
+  }
+  if constexpr (BLOCK) block_range(mn, mx, sm);
+  else team_range<TEAM>(mn, mx);
+  const auto row_sum = [&](float e) {                        // the same value in every lane of the row
+    if constexpr (!BLOCK) return team_sum<TEAM>(e);
+    e = team_sum<64>(e);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = e;
+    __syncthreads();
+    return (sm[0] + sm[1]) + (sm[2] + sm[3]);
+  };
+  float cur_min = mn, cur_max = mx;
+  // 2^k with 2^k max|x| in [1, 2); 1 where the range is zero, infinite, NaN or so extreme that the factor would overflow
+  const int e = (int)((f2u(fmaxf(fabsf(mn), fabsf(mx))) >> 23) & 0xff);
+  const bool scalable = e > 1 && e < 253;
+  const float up = scalable ? u2f((uint32_t)(254 - e) << 23) : 1.0f, down = scalable ? u2f((uint32_t)e << 23) : 1.0f;
+  #pragma unroll
+  for (int i = 0; i < PER; ++i) v[i] *= up;
+  const float frac = norm - 2.0f, top = mx * up, bottom = mn * up;
+  float best = __builtin_inff();
+  #pragma unroll 1
+  for (int i = 0; i < steps; ++i) {
+    const float p = shrink[i];
+    const float xmin = p * cur_min, xmax = p * cur_max;
+    const IntRow prm = op.make(xmin, xmax);
+    const float s = prm.s * up, r = prm.r * down;
+    const auto add = [&](float w, float sum) {
+      const float q = __builtin_amdgcn_fmed3f(rintf(w * r), prm.lo, prm.hi);
+      const float d = q * s - w;
+      return __builtin_fmaf(d * d, __builtin_amdgcn_exp2f(frac * __builtin_amdgcn_logf(fabsf(d))), sum);
+    };
+    if (__all(fmaxf(add(top, 0.0f), add(bottom, 0.0f)) > best)) continue;      // (a workgroup's lanes all hold the same two)
+    float err = 0.0f, sum = 0.0f;
+    #pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter) {
+      #pragma unroll
+      for (int j = quarter * (PER / 4); j < (quarter + 1) * (PER / 4); ++j) err = add(v[j], err);
+      sum = row_sum(err);
+      if (quarter < 3 && __all(sum > best)) break;
+    }
+    if (sum < best) { best = sum; cur_min = xmin; cur_max = xmax; }
+  }
+  if (t == 0 && row_ < rows) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
+}
+
+template <int BF>
+int run_mse(const void* x, int64_t rows, int64_t cols, int steps, int grid_n, float norm, const IntOp<0, false>& op,
+            float* min_out, float* max_out, hipStream_t st) {
+  constexpr int N = Vec<BF>::N;
+  const int vec = cols % N == 0 && (uintptr_t)x % 16 == 0;
+  #define LCQ_MSE(T, P) do { const int64_t grid = (rows * T + 255) / 256; if (grid > 0x7fffffff) return LCQ_EINVAL; \
+    mse_range_team_kernel<BF, T, P><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, (int)cols, vec, steps, grid_n, norm, op, min_out, max_out); \
+    return LCQ_OK; } while (0)
+  if (op.round_zp && op.qmin <= 0.0f && op.qmax >= 0.0f && norm > 2.0f && norm <= 4.0f && steps <= 256) {
+    // Many elements per lane amortise the step's row arithmetic, but below 20000 rows such waves are too few to fill the
+    // chip and their 80 steps one after the other are what takes the time: rows of 128 on 16 / 2 lanes take 34 / 68 us at
+    // 4096 rows, 60 / 67 at 16384, 98 / 69 at 32768
+    if (cols <= 32) LCQ_MSE(4, 8);
+    if (cols <= 128 && rows < 20000) LCQ_MSE(16, 8);
+    if (cols <= 64) LCQ_MSE(4, 16);
+    if (cols <= 128) LCQ_MSE(2, 64);
+    if (cols <= 512) LCQ_MSE(16, 32);
+    if (cols <= 4096) LCQ_MSE(64, 64);
+    if (cols <= 16384) LCQ_MSE(256, 64);
+  }
+  #undef LCQ_MSE
+  const int64_t grid = (rows + 3) / 4;
+  if (grid > 0x7fffffff) return LCQ_EINVAL;
+  mse_range_kernel<BF><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out);
+  return LCQ_OK;
 }
 
 // One proximal iteration of the HQQ zero-point solver (optimize_weights_proximal, quant.py:587-609):
@@ -217,6 +366,19 @@ int lcq_quant_int(const void* x, int dtype, int64_t rows, int64_t cols, float qm
   if ((flags & LCQ_FLAG_SCALE_F32) && !(flags & LCQ_FLAG_STATIC)) return LCQ_EINVAL;
   if (!codes) code_dtype = LCQ_CODE_NONE;
   hipStream_t st = (hipStream_t)stream;
+  if (flags & LCQ_FLAG_PROMOTED) {
+    if (dtype != LCQ_BF16 && dtype != LCQ_F16) return LCQ_EDTYPE;
+    if (!(flags & LCQ_FLAG_STATIC) || (flags & (LCQ_FLAG_NO_ROUND_ZP | LCQ_FLAG_SCALE_F32)) || qmax > 256.0f || qmin < -256.0f) return LCQ_EINVAL;
+    if (codes && code_dtype != LCQ_CODE_U8 && code_dtype != LCQ_CODE_I8 && code_dtype != LCQ_CODE_I32) return LCQ_EDTYPE;
+    if (cols % 8 != 0 || cols / 8 > 0x7fffffff || (((uintptr_t)x | (uintptr_t)dq | (uintptr_t)codes) % 16) != 0) return LCQ_EALIGN;
+    const auto op = make_op<IntOp<0, true>>(qmin, qmax, flags, out_scale_factor, code_dtype);
+    const int64_t nchunks = rows * (cols / 8);
+    const int64_t grid = nchunks > (int64_t)262144 * 256 ? 262144 : (nchunks + 255) / 256;
+    if (dtype == LCQ_BF16) static_promoted_kernel<ROW_BF16><<<dim3((unsigned)grid), dim3(256), 0, st>>>((const u32x4*)x, nchunks, (int)(cols / 8), scales, zeros, dq, codes, op);
+    else static_promoted_kernel<ROW_F16><<<dim3((unsigned)grid), dim3(256), 0, st>>>((const u32x4*)x, nchunks, (int)(cols / 8), scales, zeros, dq, codes, op);
+    LCQ_CHECK_LAUNCH();
+    return LCQ_OK;
+  }
   int rc;
   if (dtype == LCQ_F32) rc = run<false>(x, rows, cols, qmin, qmax, flags, out_scale_factor, dq, codes, code_dtype, scales, zeros, st);
   else if (dtype == LCQ_BF16) rc = run<true>(x, rows, cols, qmin, qmax, flags, out_scale_factor, dq, codes, code_dtype, scales, zeros, st);
@@ -232,13 +394,13 @@ int lcq_mse_range(const void* x, int dtype, int64_t rows, int64_t cols, float qm
   if (!x || !min_out || !max_out || rows <= 0 || cols <= 0 || steps <= 0 || grid_n <= 0) return LCQ_EINVAL;
   if (!(qmax > qmin) || (flags & LCQ_FLAG_STATIC)) return LCQ_EINVAL;
   auto op = make_op<IntOp<false, false>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
-  const int64_t grid = (rows + 3) / 4;
-  if (grid > 0x7fffffff) return LCQ_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == LCQ_F32) mse_range_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out);
-  else if (dtype == LCQ_BF16) mse_range_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out);
-  else if (dtype == LCQ_F16) mse_range_kernel<ROW_F16><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out);
+  int rc;
+  if (dtype == LCQ_F32) rc = run_mse<false>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out, st);
+  else if (dtype == LCQ_BF16) rc = run_mse<true>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out, st);
+  else if (dtype == LCQ_F16) rc = run_mse<ROW_F16>(x, rows, cols, steps, grid_n, norm, op, min_out, max_out, st);
   else return LCQ_EDTYPE;
+  if (rc != LCQ_OK) return rc;
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

@@ -147,8 +147,7 @@ class BaseQuantizer(object):
     def get_qparams(self, tensor_range, device):
         """quant.py:544-558 -> (scales, zeros, qmax, qmin)."""
         min_val, max_val = tensor_range[0].contiguous(), tensor_range[1].contiguous()
-        qmin = self.qmin.to(device)
-        qmax = self.qmax.to(device)
+        qmax, qmin = self._dev_bounds(device)
         flags = self._int_flags()
         # 0-dim ranges (per_tensor) meet the 0-dim fp32 (qmax - qmin): torch promotes the result to fp32
         if max_val.dim() == 0 and not self.sym and max_val.dtype != torch.float32:
@@ -573,8 +572,9 @@ class IntegerQuantizer(BaseQuantizer):
 
     # -- one fused launch -----------------------------------------------------
     def _launch(self, rows_t, *, static, scales=None, zeros=None, want_dq=False, want_codes=None,
-                osf=1.0, qmin=None, qmax=None):
-        """Run lcq_quant_int over a reshaped tensor.
+                osf=1.0, qmin=None, qmax=None, cast_back=False):
+        """Run lcq_quant_int over a reshaped tensor.  `cast_back`: the caller casts a promoted dq back to the tensor's
+        type (so it may come rounded already).
 
         Returns (dq | None, codes | None, scales, zeros).  Dynamic mode creates
         scales / zeros of shape [rows, 1] (0-dim for per_tensor).
@@ -585,13 +585,21 @@ class IntegerQuantizer(BaseQuantizer):
         qmax = self._bound(self.qmax if qmax is None else qmax)
         if static:
             # dimensioned qparams of another float type promote the computation like torch would
+            promoted = False
             if scales.dim() > 0 and scales.dtype != t.dtype:
                 common = torch.promote_types(t.dtype, scales.dtype)
-                t = t.to(common)
+                # fp32 parameters of 16-bit rows: computed in fp32 by one kernel where nobody sees the fp32 result
+                promoted = (common == torch.float32 and scales.dtype == common and (cast_back or not want_dq)
+                            and self.round_zp and -256 <= qmin and qmax <= 256 and t.shape[-1] % 8 == 0
+                            and t.data_ptr() % 16 == 0 and want_codes in (None, torch.int32, torch.int8, torch.uint8))
+                if promoted:
+                    flags |= L.FLAG_PROMOTED
+                else:
+                    t = t.to(common)
             # a 0-dim fp32 qparam next to a bf16 tensor (per_tensor, quant.py:544-558) goes in as fp32: torch on a GPU
             # reads a 0-dim tensor operand through a cast to the result type, which the kernel does where the
             # parameter meets the rows, while scales * output_scale_factor is still formed in fp32
-            qp_dtype = t.dtype
+            qp_dtype = torch.float32 if promoted else t.dtype
             if scales.dim() == 0 and scales.dtype == torch.float32 and t.dtype != torch.float32:
                 flags |= L.FLAG_SCALE_F32
                 qp_dtype = torch.float32
@@ -687,7 +695,8 @@ class IntegerQuantizer(BaseQuantizer):
             rargs = {k: args[k] for k in ('lowbound_factor', 'upbound_factor') if k in args} \
                 if self.calib_algo == 'learnable' else {}
             rows_t, scales, zeros, qmax, qmin = self.get_tensor_qparams(t, rargs)
-            dq, _, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_dq=True, qmin=qmin, qmax=qmax)
+            dq, _, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_dq=True, qmin=qmin, qmax=qmax,
+                                       cast_back=True)
             return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
         dq, _, _, _ = self._launch(rows_t, static=False, want_dq=True)
         return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
@@ -696,7 +705,7 @@ class IntegerQuantizer(BaseQuantizer):
         shape, dtype = t.shape, t.dtype
         rows_t = self.reshape_tensor(t)
         dq, _, _, _ = self._launch(rows_t, static=True, scales=args['scales'], zeros=args['zeros'], want_dq=True,
-                                   osf=args.get('output_scale_factor', 1), qmin=args['qmin'], qmax=args['qmax'])
+                                   osf=args.get('output_scale_factor', 1), qmin=args['qmin'], qmax=args['qmax'], cast_back=True)
         return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
 
     def fake_quant_act_static(self, act, args={}):

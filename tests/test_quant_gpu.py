@@ -840,3 +840,50 @@ def test_fp16_output_scale_factor_rounds_twice_like_torch(dev):
     ocodes, ors, orz = Q.int_real_quant_static(spec, x, s, z, spec.qmax, spec.qmin, output_scale_factor=1.7)
     assert_bit_equal(codes, ocodes, 'codes')
     assert_bit_equal(rs, ors, 'returned scales')
+
+
+@pytest.mark.parametrize('rows,cols,dtype,bit,sym', [
+    (3, 31, torch.bfloat16, 4, False), (5, 32, torch.float32, 4, True), (9, 64, torch.float16, 4, False),
+    (7, 100, torch.bfloat16, 8, True), (33, 128, torch.bfloat16, 4, False), (20001, 128, torch.bfloat16, 4, False),
+    (6, 129, torch.float32, 3, False), (5, 512, torch.bfloat16, 4, False), (3, 4096, torch.float16, 8, False),
+    (2, 4104, torch.bfloat16, 8, True), (2, 16384, torch.float32, 4, False), (2, 16392, torch.bfloat16, 4, False)])
+def test_mse_range_at_the_edges_of_its_lane_layouts(dev, rows, cols, dtype, bit, sym):
+    """calib_algo mse for every way a row is dealt out to lanes (2 to 64, a workgroup, the re-reading kernel beyond 16384
+    columns), full and ragged.  The sums of |d|**2.4 are fp32 in another order and through another pow than the CPU's: a
+    relative 1e-6 of the sum (a few ulp per term, at most 16384 terms added pairwise by lanes), so where the range
+    differs, the fp64 error of the chosen range is within 1e-5 of the oracle's choice."""
+    w = weight_like(rows, cols, seed=rows + cols, dtype=dtype, outlier_frac=0.002)
+    spec = Q.IntSpec(bit, sym, 'per_channel')
+    q = _iq(bit, sym, 'per_channel', calib_algo='mse')
+    omn, omx = Q.int_mse_range(spec, w)
+    mn, mx = (t.cpu() for t in q.get_mse_range(w.to(dev)))
+    assert mn.shape == omn.shape and mn.dtype == torch.float32
+    same = (mn == omn) & (mx == omx)
+    assert int((~same).sum()) <= max(1, rows // 1000)
+
+    def err64(lo, hi):
+        s, z, qmax, qmin = Q.int_qparams(spec, lo, hi)
+        return (Q.int_quant_dequant(spec, w.float(), s, z, qmax, qmin) - w.float()).double().abs().pow(2.4).sum(1)
+    assert bool(((err64(mn, mx) - err64(omn, omx)).abs() <= 1e-5 * err64(omn, omx)).all())
+    got = q.fake_quant_weight_dynamic(w.to(dev))             # fp32 parameters on the rows as they are stored
+    s, z, qmax, qmin = Q.int_qparams(spec, mn, mx)
+    assert_bit_equal(got, Q.int_quant_dequant(spec, w.float(), s, z, qmax, qmin).to(dtype), 'fake quant with the mse ranges')
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('bit,sym,shape,g', [(4, False, (64, 512), 128), (8, True, (33, 256), 64), (8, False, (7, 96), 32),
+                                             (4, True, (5, 1000), 0), (8, True, (3, 1001), 0)])
+def test_static_fp32_parameters_of_16_bit_rows(dev, dtype, bit, sym, shape, g):
+    """fp32 [rows, 1] parameters next to a 16-bit tensor: the fp32 arithmetic of torch's promotion, cast back once; with
+    and without the one-kernel form (rows of 1001 do not fill 16-byte chunks)."""
+    w = weight_like(*shape, seed=bit + shape[1], dtype=dtype, outlier_frac=0.01)
+    spec = Q.IntSpec(bit, sym, 'per_group' if g else 'per_channel', group_size=g)
+    q = _iq(bit, sym, 'per_group', group_size=g) if g else _iq(bit, sym, 'per_channel')
+    rows = Q.reshape_rows(spec, w)
+    s = torch.rand(rows.shape[0], 1, generator=gen(7)) * 0.01 + 0.001
+    z = torch.tensor(0.0) if sym else torch.randint(0, 2 ** bit, (rows.shape[0], 1), generator=gen(8)).float()
+    args = {'scales': s.to(dev), 'zeros': z if sym else z.to(dev), 'qmax': q.qmax, 'qmin': q.qmin}
+    assert_bit_equal(q.fake_quant_weight_static(w.to(dev), dict(args)),
+                     Q.int_fake_quant_static(spec, w, s, z, q.qmax, q.qmin), 'fake')
+    codes = q.real_quant_weight_static(w.to(dev), dict(args))[0]
+    assert_bit_equal(codes, Q.int_real_quant_static(spec, w, s, z, q.qmax, q.qmin)[0], 'codes')
