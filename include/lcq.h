@@ -102,7 +102,7 @@ extern "C" {
  *          one wave per row: correct to the bit, not tuned; no LCQ_CODE_CT4 for them)
  *  dq      same shape/type or NULL        -> (q - z) * (s * out_scale_factor)
  *  codes   [rows, cols] of code_dtype or NULL
- *  scales  [rows] (or [1] with SCALAR_QP) of `dtype`: output, input if STATIC
+ *  scales  [rows] (or [1] with SCALAR_QP) of `dtype`: output (NULL: not wanted), input if STATIC
  *  zeros   likewise; may be NULL (zero point 0; never written when SYM)
  * bf16 / fp16 rows round to their type after every arithmetic step like torch does. */
 int lcq_quant_int(const void* x, int dtype, int64_t rows, int64_t cols, float qmin, float qmax, int flags,

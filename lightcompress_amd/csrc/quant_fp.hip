@@ -91,7 +91,7 @@ struct FpOp {
     return finish(load_scalar<BF>(scales, i));
   }
   __device__ __forceinline__ void store_qp(void* scales, void*, int64_t row, const Row& p) const {
-    store_scalar<BF>(scales, row, p.s);
+    if (scales) store_scalar<BF>(scales, row, p.s);
   }
 
   __device__ __forceinline__ uint32_t round_mag(uint32_t m) const {
@@ -415,7 +415,7 @@ extern "C" {
 
 int lcq_quant_fp(const void* x, int dtype, int64_t rows, int64_t cols, int e_bits, int m_bits, float qmax, int flags,
                  void* dq, void* codes, int code_dtype, void* scales, void* stream) {
-  if (!x || rows < 0 || cols <= 0 || !scales) return LCQ_EINVAL;
+  if (!x || rows < 0 || cols <= 0 || (!scales && (flags & LCQ_FLAG_STATIC))) return LCQ_EINVAL;
   if (rows == 0) return LCQ_OK;
   if (e_bits < 2 || e_bits > 5 || m_bits < 1 || m_bits > 10 || !(qmax > 0.0f)) return LCQ_EINVAL;
   if (codes) {

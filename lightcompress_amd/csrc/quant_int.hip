@@ -352,7 +352,7 @@ extern "C" {
 int lcq_quant_int(const void* x, int dtype, int64_t rows, int64_t cols, float qmin, float qmax, int flags,
                   float out_scale_factor, void* dq, void* codes, int code_dtype, void* scales, void* zeros,
                   void* stream) {
-  if (!x || rows < 0 || cols <= 0 || !scales) return LCQ_EINVAL;
+  if (!x || rows < 0 || cols <= 0 || (!scales && (flags & LCQ_FLAG_STATIC))) return LCQ_EINVAL;
   if (rows == 0) return LCQ_OK;
   if (codes && !(code_dtype == LCQ_CODE_U8 || code_dtype == LCQ_CODE_I8 || code_dtype == LCQ_CODE_I32 ||
                  code_dtype == LCQ_CODE_SAME || code_dtype == LCQ_CODE_CT4)) return LCQ_EDTYPE;

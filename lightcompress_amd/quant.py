@@ -572,12 +572,13 @@ class IntegerQuantizer(BaseQuantizer):
 
     # -- one fused launch -----------------------------------------------------
     def _launch(self, rows_t, *, static, scales=None, zeros=None, want_dq=False, want_codes=None,
-                osf=1.0, qmin=None, qmax=None, cast_back=False):
+                osf=1.0, qmin=None, qmax=None, cast_back=False, want_qp=True):
         """Run lcq_quant_int over a reshaped tensor.  `cast_back`: the caller casts a promoted dq back to the tensor's
         type (so it may come rounded already).
 
         Returns (dq | None, codes | None, scales, zeros).  Dynamic mode creates
-        scales / zeros of shape [rows, 1] (0-dim for per_tensor).
+        scales / zeros of shape [rows, 1] (0-dim for per_tensor); with `want_qp` False they stay inside the kernel and
+        come back as None.
         """
         t = rows_t.contiguous()
         flags = self._int_flags()
@@ -618,8 +619,10 @@ class IntegerQuantizer(BaseQuantizer):
                 return self._launch(t, static=True, scales=scales, zeros=zeros, want_dq=want_dq,
                                     want_codes=want_codes, osf=osf)
             rows, cols = _rows_cols(t)
-            scales = torch.empty((rows, 1), dtype=t.dtype, device=t.device)
-            z = None if self.sym else torch.empty((rows, 1), dtype=t.dtype, device=t.device)
+            scales = z = None
+            if want_qp:
+                scales = torch.empty((rows, 1), dtype=t.dtype, device=t.device)
+                z = None if self.sym else torch.empty((rows, 1), dtype=t.dtype, device=t.device)
         dq = torch.empty_like(t) if want_dq else None
         codes, cd = None, L.CODE_NONE
         if want_codes is not None:
@@ -634,7 +637,7 @@ class IntegerQuantizer(BaseQuantizer):
                                       L.f32(qmax), L.i32(flags), L.f32(osf), L.ptr(dq), L.ptr(codes), L.i32(cd),
                                       L.ptr(scales), L.ptr(z), L.stream()), 'lcq_quant_int')
         if not static:
-            zeros = torch.tensor(0.0) if self.sym else z
+            zeros = torch.tensor(0.0) if self.sym and want_qp else z
         return dq, codes, scales, zeros
 
     # -- reference API ----------------------------------------------------------
@@ -698,8 +701,8 @@ class IntegerQuantizer(BaseQuantizer):
             dq, _, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_dq=True, qmin=qmin, qmax=qmax,
                                        cast_back=True)
             return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
-        dq, _, _, _ = self._launch(rows_t, static=False, want_dq=True)
-        return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
+        dq, _, _, _ = self._launch(rows_t, static=False, want_dq=True, want_qp=False)
+        return dq if dq.shape == shape and dq.dtype == dtype else self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
 
     def _fake_static(self, t, args):
         shape, dtype = t.shape, t.dtype
@@ -992,7 +995,8 @@ class FloatQuantizer(BaseQuantizer):
                 'lcq_qparams_int')
         return scales, torch.tensor(0.0), self.qmax.to(device), self.qmin.to(device)
 
-    def _launch(self, rows_t, *, static, scales=None, want_dq=None, want_codes=None):
+    def _launch(self, rows_t, *, static, scales=None, want_dq=None, want_codes=None, want_qp=True):
+        """(dq | None, codes | None, scales); dynamic scales that nobody reads (`want_qp` False) stay in the kernel."""
         t = rows_t.contiguous()
         flags = self._fp_flags()
         if static:
@@ -1011,7 +1015,7 @@ class FloatQuantizer(BaseQuantizer):
                 s, _, _, _ = self.get_qparams(self.get_minmax_range(t), t.device)
                 return self._launch(t, static=True, scales=s, want_dq=want_dq, want_codes=want_codes)
             rows, cols = _rows_cols(t)
-            s = torch.empty((rows, 1), dtype=t.dtype, device=t.device)
+            s = torch.empty((rows, 1), dtype=t.dtype, device=t.device) if want_qp else None
         dq = None
         if want_dq == 'f32':
             dq = torch.empty(t.shape, dtype=torch.float32, device=t.device)
@@ -1114,7 +1118,9 @@ class FloatQuantizer(BaseQuantizer):
             dq = self._emu(rows_t, static_scales, want=('dq',))['dq']
             return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
         if static_scales is None:
-            dq, _, _ = self._launch(rows_t, static=False, want_dq=True)
+            dq, _, _ = self._launch(rows_t, static=False, want_dq=True, want_qp=False)
+            if dq.shape == shape and dq.dtype == dtype:
+                return dq
         else:
             dq, _, _ = self._launch(rows_t, static=True, scales=static_scales, want_dq=True)
         return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
