@@ -98,8 +98,7 @@ extern "C" {
  * (quant / dequant / quant_dequant) and so the bodies of
  * fake_quant_{weight,act}_{dynamic,static} (:718-868) and
  * real_quant_weight_{dynamic,static} (:870-952).
- *  x       [rows, cols] of `dtype` (LCQ_F32 | LCQ_BF16 | LCQ_F16; fp16 rows run through the element-wise kernel,
- *          one wave per row: correct to the bit, not tuned; no LCQ_CODE_CT4 for them)
+ *  x       [rows, cols] of `dtype` (LCQ_F32 | LCQ_BF16 | LCQ_F16)
  *  dq      same shape/type or NULL        -> (q - z) * (s * out_scale_factor)
  *  codes   [rows, cols] of code_dtype or NULL
  *  scales  [rows] (or [1] with SCALAR_QP) of `dtype`: output (NULL: not wanted), input if STATIC

@@ -25,7 +25,7 @@ constexpr int RINT_BIAS_BITS = 0x4B400000;
 // FAST: round_zp and |qmin|,qmax <= 256 (every stock configuration).
 template <int BF_, bool FAST, bool PRESCALE = false, int CD_ = -1>
 struct IntOp {
-  static constexpr int BF = BF_;          // row type: 0 fp32, 1 bf16, 2 fp16 (element-wise forms only: FAST is false)
+  static constexpr int BF = BF_;          // row type: 0 fp32, 1 bf16, 2 fp16
   static constexpr bool HAS_PRESCALE = PRESCALE;
   static constexpr bool HAS_FUSED_DQ = FAST;
   static constexpr bool HAS_CUSTOM_EMIT = false;
@@ -173,23 +173,22 @@ struct IntOp {
   //   fp32: |t - x/s| <= 2^-22 |t|; for |t| <= 1024 that is <= 2^-12, so a product farther than
   //         2^-11 from every half integer rounds like the quotient; beyond 1024 both land outside
   //         the clamp range on the same side (|z| <= 512), and a huge t has d == 0;
-  //   bf16: the quotient is rounded to bf16 first; the product is safe unless its low 16 bits
-  //         are within 8 ulp of the bf16 midpoint pattern 0x8000.
+  //   bf16, fp16: the quotient is rounded to the row type first; the product is safe unless its dropped bits are within
+  //         8 ulp of the midpoint pattern (fp16 quotients below 2^-14 round at other places, but all of them to the integer
+  //         0; those beyond 65504 become infinite or stay on the same side of the clamp range).
   // x / s for a chunk, rounded to the row type
   template <int N>
   __device__ __forceinline__ void quotients(const float* x, float* t, const Row& p) const {
     bool ok = p.fast;
     if constexpr (BF) {
-      // distance of the low 16 bits from the midpoint window, two products per packed 16-bit instruction
-      lcq_u16x2 nearest = {0xffff, 0xffff};
+      MidpointGuard guard;
       #pragma unroll
       for (int i = 0; i < N; i += 2) {
         t[i] = x[i] * p.r;
         t[i + 1] = x[i + 1] * p.r;
-        const uint32_t lows = __builtin_amdgcn_perm(f2u(t[i + 1]), f2u(t[i]), 0x05040100u);
-        nearest = __builtin_elementwise_min(nearest, __builtin_bit_cast(lcq_u16x2, lows) - lcq_u16x2{0x7ff8, 0x7ff8});
+        guard.see<BF>(t[i], t[i + 1]);
       }
-      ok = ok && nearest.x > 0x10 && nearest.y > 0x10;
+      ok = ok && guard.clear();
     } else {
       #pragma unroll
       for (int i = 0; i < N; ++i) {

@@ -28,7 +28,7 @@ struct FpRow {
 
 template <int BF_>
 struct FpOp {
-  static constexpr int BF = BF_;          // row type: 0 fp32, 1 bf16, 2 fp16 (element-wise forms only)
+  static constexpr int BF = BF_;          // row type: 0 fp32, 1 bf16, 2 fp16
   static constexpr bool HAS_PRESCALE = false;
   static constexpr bool HAS_FUSED_DQ = false;
   static constexpr bool HAS_CUSTOM_EMIT = true;
@@ -161,8 +161,8 @@ struct FpOp {
   // bf16 rows hold ties all the time (8 significant bits), so ties-away is produced by the convert
   // itself: t is scaled by 1 + 2^-10 first.  Every tie is a bf16 number, so a bf16 value that is
   // not a tie is at least one bf16 ulp away from the nearest one and the nudge (1/4 ulp at most)
-  // cannot carry it across; an exact tie moves to the far side.  The fma also adds the "+ zeros"
-  // of the reference, which turns -0 into +0.
+  // cannot carry it across; an exact tie moves to the far side.  (fp16 rows: 1 + 2^-13, a quarter of their ulp, likewise.)
+  // The fma also adds the "+ zeros" of the reference, which turns -0 into +0.
   template <int N>
   __device__ __forceinline__ bool emit_fast(const float* x, const Row& p, int64_t cidx, void* dq, void* codes) const {
     if (!hw) return false;
@@ -170,16 +170,18 @@ struct FpOp {
     float t[N];
     bool near = !p.fast, far = false;
     if constexpr (BF) {
-      // distance of the low 16 bits from the midpoint window, two products per packed 16-bit instruction
-      lcq_u16x2 nearest = {0xffff, 0xffff};
+      MidpointGuard guard;
       #pragma unroll
       for (int i = 0; i < N; i += 2) {
         t[i] = x[i] * p.r;
         t[i + 1] = x[i + 1] * p.r;
-        const uint32_t lows = __builtin_amdgcn_perm(f2u(t[i + 1]), f2u(t[i]), 0x05040100u);
-        nearest = __builtin_elementwise_min(nearest, __builtin_bit_cast(lcq_u16x2, lows) - lcq_u16x2{0x7ff8, 0x7ff8});
+        guard.see<BF>(t[i], t[i + 1]);
       }
-      near = near || nearest.x <= 0x10 || nearest.y <= 0x10;
+      near = near || !guard.clear();
+      if (BF == ROW_F16 && hw == 2) {                        // fp16 subnormals are on the e5m2 grid's scale: always divided
+        #pragma unroll
+        for (int i = 0; i < N; ++i) near = near || (fabsf(t[i]) < 6.2e-5f && t[i] != 0.0f);
+      }
     } else {
       #pragma unroll
       for (int i = 0; i < N; ++i) {
@@ -208,7 +210,7 @@ struct FpOp {
     }
     #pragma unroll
     for (int i = 0; i < N; i += 2) rnd_pair<BF>(t[i], t[i + 1]);
-    const float nudge = (BF && !tie_even) ? 1.0009765625f : 1.0f;
+    const float nudge = (BF && !tie_even) ? (BF == ROW_F16 ? 1.0001220703125f : 1.0009765625f) : 1.0f;
     #pragma unroll
     for (int i = 0; i < N; ++i) t[i] = __builtin_fmaf(t[i], nudge, 0.0f);
     uint32_t w[N / 4];
@@ -431,8 +433,8 @@ int lcq_quant_fp(const void* x, int dtype, int64_t rows, int64_t cols, int e_bit
     rc = dispatch_rows(x, rows, cols, dq, codes, scales, (void*)nullptr, make_op<false>(e_bits, m_bits, qmax, flags, code_dtype), false, st);
   else if (dtype == LCQ_BF16)
     rc = dispatch_rows(x, rows, cols, dq, codes, scales, (void*)nullptr, make_op<true>(e_bits, m_bits, qmax, flags, code_dtype), false, st);
-  else if (dtype == LCQ_F16)                               // fp16 rows: the element-wise kernel (correct to the bit, not tuned)
-    rc = dispatch_rows(x, rows, cols, dq, codes, scales, (void*)nullptr, make_op<ROW_F16>(e_bits, m_bits, qmax, flags, code_dtype), true, st);
+  else if (dtype == LCQ_F16)
+    rc = dispatch_rows(x, rows, cols, dq, codes, scales, (void*)nullptr, make_op<ROW_F16>(e_bits, m_bits, qmax, flags, code_dtype), false, st);
   else return LCQ_EDTYPE;
   if (rc != LCQ_OK) return rc;
   LCQ_CHECK_LAUNCH();

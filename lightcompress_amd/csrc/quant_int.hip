@@ -14,8 +14,7 @@
 //   fp32 rows : every step is one IEEE fp32 op (true division, rintf).
 //   bf16 rows : every step is computed in fp32 and rounded to bf16 (RNE)
 //               before the next step, as torch does for bf16 tensors.
-//   fp16 rows : the same with fp16 roundings, through the element-wise kernel and true divisions only (one wave per
-//               row, one element per lane and step: a compatibility path, not a tuned one).
+//   fp16 rows : the same with fp16 roundings (the per-row parameters through true divisions).
 // The per-element division x/s is evaluated as x*(1/s) with an exactness
 // guard: whenever the approximate quotient is close enough to a rounding
 // boundary that the IEEE quotient could round differently, the lane falls
@@ -29,16 +28,10 @@ template <int BF>
 int run(const void* x, int64_t rows, int64_t cols, float qmin, float qmax, int flags, float osf, void* dq,
         void* codes, int code_dtype, void* scales, void* zeros, hipStream_t st) {
   const bool big = (qmax > 256.0f) || (qmin < -256.0f);
-  const bool general = big || (flags & LCQ_FLAG_NO_ROUND_ZP) || BF == ROW_F16;     // fp16 rows: the element-wise kernel
-  if constexpr (BF == ROW_F16) {
-    if (code_dtype == LCQ_CODE_CT4) return LCQ_EDTYPE;      // nibbles come from the vectorised bf16 / fp32 kernels only
-  }
-  if (general)
+  if (big || (flags & LCQ_FLAG_NO_ROUND_ZP))
     return dispatch_rows(x, rows, cols, dq, codes, scales, zeros,
                          make_op<IntOp<BF, false>>(qmin, qmax, flags, osf, code_dtype), true, st);
   // the common storage formats get kernels with the store path fixed at compile time
-  if constexpr (BF == ROW_F16) return LCQ_EDTYPE;            // not reached: `general` above
-  else {
   #define LCQ_RUN(CDV) return dispatch_rows(x, rows, cols, dq, codes, scales, zeros, \
                          make_op<IntOp<BF, true, false, CDV>>(qmin, qmax, flags, osf, code_dtype), false, st)
   switch (code_dtype) {
@@ -49,7 +42,6 @@ int run(const void* x, int64_t rows, int64_t cols, float qmin, float qmax, int f
     default: LCQ_RUN(-1);
   }
   #undef LCQ_RUN
-  }
 }
 
 // get_minmax_range (row-wise), quant.py:141-143
@@ -447,10 +439,10 @@ int lcq_awq_scale_quant(const void* w, int dtype, int64_t R, int64_t K, const vo
     auto op = make_op<IntOp<true, true, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
     op.colscale = colscale; op.wrow_cols = (int)K; op.is_static = 0;
     rc = dispatch_rows(w, rows, cols, out, (void*)nullptr, (void*)nullptr, (void*)nullptr, op, false, st);
-  } else if (dtype == LCQ_F16) {                           // element-wise kernel
-    auto op = make_op<IntOp<ROW_F16, false, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
+  } else if (dtype == LCQ_F16) {
+    auto op = make_op<IntOp<ROW_F16, true, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
     op.colscale = colscale; op.wrow_cols = (int)K; op.is_static = 0;
-    rc = dispatch_rows(w, rows, cols, out, (void*)nullptr, (void*)nullptr, (void*)nullptr, op, true, st);
+    rc = dispatch_rows(w, rows, cols, out, (void*)nullptr, (void*)nullptr, (void*)nullptr, op, false, st);
   } else return LCQ_EDTYPE;
   if (rc != LCQ_OK) return rc;
   LCQ_CHECK_LAUNCH();

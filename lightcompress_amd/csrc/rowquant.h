@@ -26,8 +26,7 @@
 
 namespace lcq {
 
-// BF: the row type.  0 = fp32, 1 = bf16, 2 = fp16 (a bool argument reads as 0 / 1).  The fast kernels exist for fp32
-// and bf16; fp16 rows go through the element-wise kernel (row_scalar_kernel) and the element-wise forms of the ops.
+// BF: the row type.  0 = fp32, 1 = bf16, 2 = fp16 (a bool argument reads as 0 / 1).
 constexpr int ROW_F32 = 0, ROW_BF16 = 1, ROW_F16 = 2;
 template <int BF> struct Vec { static constexpr int N = BF ? 8 : 4; };
 typedef unsigned short lcq_u16x2 __attribute__((ext_vector_type(2)));
@@ -55,6 +54,7 @@ __device__ __forceinline__ uint32_t bf16_pack_rne(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(lcq_f32x2{a, b}, lcq_bf16x2));
 }
 __device__ __forceinline__ uint32_t f16_pack_rne(float a, float b) {
+  asm("" : "+v"(a), "+v"(b));                                // as in rnd: no multiply is folded into the conversion
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(lcq_f32x2{a, b}, lcq_f16x2));
 }
 __device__ __forceinline__ float f16_lo(uint32_t w) { return (float)__builtin_bit_cast(lcq_f16x2, w).x; }
@@ -69,6 +69,20 @@ template <int BF> __device__ __forceinline__ void rnd_pair(float& a, float& b) {
     b = u2f(u & 0xffff0000u);
   }
 }
+
+// How close fp32 values come to the midpoints between neighbouring 16-bit numbers (where an approximate quotient may round
+// the other way): distance of the dropped mantissa bits from a window of 8 ulp around the midpoint pattern, two values per
+// packed 16-bit instruction.  bf16 drops 16 bits; fp16 drops 13 (in its normal range; below 2^-14 the pattern says nothing).
+struct MidpointGuard {
+  lcq_u16x2 nearest = {0xffff, 0xffff};
+  template <int BF> __device__ __forceinline__ void see(float a, float b) {
+    uint32_t lows = __builtin_amdgcn_perm(f2u(b), f2u(a), 0x05040100u);
+    constexpr unsigned short start = BF == ROW_F16 ? 0x0ff8 : 0x7ff8;
+    if constexpr (BF == ROW_F16) lows &= 0x1fff1fffu;
+    nearest = __builtin_elementwise_min(nearest, __builtin_bit_cast(lcq_u16x2, lows) - lcq_u16x2{start, start});
+  }
+  __device__ __forceinline__ bool clear() const { return nearest.x > 0x10 && nearest.y > 0x10; }
+};
 
 template <int BF>
 __device__ __forceinline__ void unpack(const u32x4& raw, float* v) {

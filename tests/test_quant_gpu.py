@@ -887,3 +887,33 @@ def test_static_fp32_parameters_of_16_bit_rows(dev, dtype, bit, sym, shape, g):
                      Q.int_fake_quant_static(spec, w, s, z, q.qmax, q.qmin), 'fake')
     codes = q.real_quant_weight_static(w.to(dev), dict(args))[0]
     assert_bit_equal(codes, Q.int_real_quant_static(spec, w, s, z, q.qmax, q.qmin)[0], 'codes')
+
+
+@pytest.mark.parametrize('kind', ['int8_asym', 'int4_sym', 'e4m3', 'e5m2', 'e4m3_even', 'e5m2_even'])
+def test_every_finite_fp16_value_under_many_scales(dev, kind):
+    """The vectorised fp16 rows (reciprocal quotients with a guard, packed conversions, hardware float8 rounding) on all
+    63488 finite fp16 numbers under 8 row scales each, subnormal quotients and overflowing ones included: bit for bit."""
+    x = torch.arange(0, 65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    x = x[x.isfinite()]
+    g = gen(11)
+    for k in range(8):
+        rows = x[torch.randperm(x.numel(), generator=g)].view(-1, 256)
+        s = (torch.rand(rows.shape[0], 1, generator=g) + 0.5) * 2.0 ** torch.randint(-14, 8, (rows.shape[0], 1), generator=g)
+        s = s.half()
+        if kind.startswith('int'):
+            bit, sym = (8, False) if kind == 'int8_asym' else (4, True)
+            spec = Q.IntSpec(bit, sym, 'per_channel')
+            q = _iq(bit, sym, 'per_channel')
+            z = torch.tensor(0.0) if sym else torch.randint(0, 2 ** bit, (rows.shape[0], 1), generator=g).half()
+            args = {'scales': s.to(dev), 'zeros': z if sym else z.to(dev), 'qmax': q.qmax, 'qmin': q.qmin}
+            want = Q.int_fake_quant_static(spec, rows, s, z, q.qmax, q.qmin)
+            assert_bit_equal(q.fake_quant_weight_static(rows.to(dev), args), want, f'{kind} {k}')
+        else:
+            from lightcompress_amd import FloatQuantizer
+            fmt, tie = kind[:4], 'even' if kind.endswith('even') else 'away'
+            spec = Q.FloatSpec(fmt, 'per_channel', tie=tie)
+            q = FloatQuantizer(fmt, True, 'per_channel', use_qtorch=True, fp_tie=tie)
+            codes = q.quant(rows.to(dev), s.to(dev), None, None, None)
+            assert_bit_equal(codes, Q.float_quant(spec, rows, s.clone(), 0.0), f'{kind} {k} codes')
+            want = Q.float_dequant(Q.float_quant(spec, rows, s.clone(), 0.0), s, 0.0).half()
+            assert_bit_equal(q.fake_quant_weight_static(rows.to(dev), {'scales': s.to(dev)}), want, f'{kind} {k}')
