@@ -51,6 +51,8 @@ extern "C" {
 #define LCQ_CODE_SAME 4      /* codes stored as floats of the input type (what .quant() returns) */
 #define LCQ_CODE_F32 5       /* FloatQuantizer.quant(): fp32 values on the minifloat grid */
 #define LCQ_CODE_FP8 6       /* float8_e4m3fn / float8_e5m2 bytes */
+#define LCQ_CODE_CT8 8       /* lcq_quant_int: the same for 8-bit codes: byte i of word j = code[4j+i] + 128 (codes in -128 .. 127); `codes`
+                                is int32 [rows * cols / 4] */
 #define LCQ_CODE_CT4 7       /* lcq_quant_int: 4-bit codes packed like VllmRealQuantLinear.pack (module_utils.py:929-955):
                                 nibble i of int32 word j of a tensor row = code[8j+i] + 8; needs -8 <= qmin, qmax <= 7
                                 and cols % 8 == 0; `codes` is int32 [rows * cols / 8] */
@@ -77,6 +79,7 @@ extern "C" {
 #define LCQ_FLAG_PROMOTED 16384    /* lcq_quant_int, STATIC only: bf16 / fp16 rows, `scales` / `zeros` hold fp32; the arithmetic is the fp32
                                     one torch's type promotion gives, dq is rounded once to the row type (FAST settings:
                                     rounded zero points, |qmin|, qmax <= 256; cols % 8 == 0, 16-byte aligned) */
+#define LCQ_FLAG_SCALES_F16 32768  /* lcq_quant_int, not STATIC: `scales` is fp16: the row type's scale cast once more (scales.to(float16)) */
 #define LCQ_FLAG_RANGE_F16 8192    /* LCQ_FLAG_RANGE_BF16 for ranges that were fp16 */
 #define LCQ_FLAG_ROWS16 4096       /* lcq_gptq_block: 16 rows per workgroup whatever R is (the default takes 32 from 6144 rows on; same results bit for bit) */
 #define LCQ_FLAG_ROW_QP 512       /* lcq_quant_fp_emu, STATIC only: `scales` holds one value per row */

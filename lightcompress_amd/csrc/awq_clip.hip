@@ -481,11 +481,7 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
   if (n_grid <= 0 || n_steps <= 0 || n_steps > n_grid) return LCQ_EINVAL;
   if (!(qmax > qmin) || qmax > 256.0f || qmin < -256.0f || (flags & (LCQ_FLAG_STATIC | LCQ_FLAG_NO_ROUND_ZP))) return LCQ_EINVAL;
   if ((((uintptr_t)w | (uintptr_t)x) % 16) != 0) return LCQ_EALIGN;
-  IntOp<true, true> op;
-  op.qmin = qmin; op.qmax = qmax; op.qrange = qmax - qmin; op.osf = 1.0f;
-  op.rqmax = (float)(1.0 / (double)qmax); op.rqrange = (float)(1.0 / (double)(qmax - qmin));
-  op.sym = (flags & LCQ_FLAG_SYM) != 0; op.round_zp = 1; op.is_static = 0; op.scalar_qp = 0; op.dq_f32 = 0;
-  op.range_bf16 = 0; op.range_f16 = 0; op.scale_f32 = 0; op.colscale = nullptr; op.wrow_cols = 1; op.code_dtype = LCQ_CODE_NONE;
+  const auto op = make_op<IntOp<true, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
   const dim3 grid((unsigned)((R + ROWS_PER_WG - 1) / ROWS_PER_WG), (unsigned)(K / CG));
   awq_clip_kernel<<<grid, dim3(512), 0, (hipStream_t)stream>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K,
                                                                (int)T, n_grid, n_steps, clip_sym, op, (uint16_t*)best_max,

@@ -34,7 +34,7 @@ struct IntOp {
   using Row = IntRow;
   float qmin, qmax, qrange, osf;
   float rqmax, rqrange;         // 1 / qmax, 1 / qrange (fp32-rounded)
-  int sym, round_zp, is_static, scalar_qp, dq_f32, code_dtype, range_bf16, range_f16, scale_f32;
+  int sym, round_zp, is_static, scalar_qp, dq_f32, code_dtype, range_bf16, range_f16, scale_f32, scales_f16;
   // optional per-column factor applied first (AWQ: W * s), rows of the reshaped tensor tile a
   // weight row of wrow_cols columns
   const void* colscale;
@@ -148,7 +148,10 @@ struct IntOp {
   }
 
   __device__ __forceinline__ void store_qp(void* scales, void* zeros, int64_t row, const Row& p) const {
-    if (scales) store_scalar<BF>(scales, row, p.s);
+    if (scales) {
+      if (scales_f16) ((_Float16*)scales)[row] = (_Float16)p.s;
+      else store_scalar<BF>(scales, row, p.s);
+    }
     if (zeros && !sym) store_scalar<BF>(zeros, row, p.z);
   }
 
@@ -275,6 +278,7 @@ struct IntOp {
     } else {
       #pragma unroll
       for (int j = 0; j < 4; ++j) w |= byte(q[j]) << (8 * j);
+      if ((CD >= 0 ? CD : code_dtype) == LCQ_CODE_CT8) w ^= 0x80808080u;       // + 128 in every byte
     }
     return w;
   }
@@ -293,6 +297,7 @@ Op make_op(float qmin, float qmax, int flags, float osf, int code_dtype) {
   c.range_bf16 = (flags & LCQ_FLAG_RANGE_BF16) != 0;
   c.range_f16 = (flags & LCQ_FLAG_RANGE_F16) != 0;
   c.scale_f32 = (flags & LCQ_FLAG_SCALE_F32) != 0;
+  c.scales_f16 = (flags & LCQ_FLAG_SCALES_F16) != 0;
   c.colscale = nullptr; c.wrow_cols = 1;
   c.code_dtype = code_dtype;
   return c;

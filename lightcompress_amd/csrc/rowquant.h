@@ -169,7 +169,7 @@ __device__ __forceinline__ void store_codes(const Op& op, void* codes, int64_t e
       for (int j = 0; j < 4; ++j) w[j] = f2u(q[i + j]);
       *(u32x4*)(p + i) = w;
     }
-  } else if (cd == LCQ_CODE_U8 || cd == LCQ_CODE_I8 || cd == LCQ_CODE_FP8) {
+  } else if (cd == LCQ_CODE_U8 || cd == LCQ_CODE_I8 || cd == LCQ_CODE_CT8 || cd == LCQ_CODE_FP8) {
     uint8_t* p = (uint8_t*)codes + elem0;
     #pragma unroll
     for (int i = 0; i < N; i += 4) {
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void row_team_kernel(
   constexpr int RPW = LCQ_WAVE / TEAM;                      // rows per wave per batch
   constexpr int N = Vec<Op::BF>::N;
   // one-byte codes of a full grid whose lanes each produce exactly 16 bytes of them
-  constexpr bool STAGED = FULL && !Op::HAS_CUSTOM_EMIT && (Op::CD == LCQ_CODE_U8 || Op::CD == LCQ_CODE_I8) && ITERS * N == 16;
+  constexpr bool STAGED = FULL && !Op::HAS_CUSTOM_EMIT && (Op::CD == LCQ_CODE_U8 || Op::CD == LCQ_CODE_I8 || Op::CD == LCQ_CODE_CT8) && ITERS * N == 16;
   __shared__ uint32_t stage[STAGED ? 4 * RPW * TEAM * 4 : 1];
   const int lane = threadIdx.x & 63;
   const int t = lane & (TEAM - 1);

@@ -28,6 +28,19 @@ def _bf16_weight(module):
                                                  module.block_size).to(torch.bfloat16)
 
 
+def _rtn_quantizer(w_q):
+    """The integer quantizer behind `w_q` if it is RTN's own partial (get_replacement_params), i.e. nothing but
+    wquantizer.real_quant_weight_dynamic(module.weight.data); None for any other callable (GPTQ's static parameters, a
+    subclass' or a caller's own function)."""
+    from .quant import IntegerQuantizer
+    from .rtn import RTN
+    if not isinstance(w_q, partial) or w_q.args or set(w_q.keywords) != {'wquantizer'} \
+            or getattr(w_q.func, '__func__', None) is not RTN.w_q:
+        return None
+    q = w_q.keywords['wquantizer']
+    return q if type(q) is IntegerQuantizer else None
+
+
 def _func_name(fn):
     return fn.func.__name__ if isinstance(fn, partial) else fn.__name__
 
@@ -140,18 +153,18 @@ class _RealQuantLinear(torch.nn.Module):
         raise NotImplementedError
 
     def _describe(self, module, weight, scales, zeros):
-        self.in_features = module.in_features
-        self.out_features = module.out_features
-        self.weight_shape, self.weight_dtype = weight.shape, weight.dtype
-        self.scales_shape, self.scales_dtype = scales.shape, scales.dtype
-        self.zeros_shape = zeros.shape if zeros is not None else None
-        self.zeros_dtype = zeros.dtype if zeros is not None else None
+        # plain values, so straight into __dict__: nn.Module.__setattr__ looks for parameters, modules and buffers first,
+        # 10 us for these eight
+        self.__dict__.update(
+            in_features=module.in_features, out_features=module.out_features,
+            weight_shape=weight.shape, weight_dtype=weight.dtype, scales_shape=scales.shape, scales_dtype=scales.dtype,
+            zeros_shape=zeros.shape if zeros is not None else None, zeros_dtype=zeros.dtype if zeros is not None else None)
 
     def _reg(self, name, value):
         if value is not None:
             self.register_buffer(name, value)
         else:
-            setattr(self, name, None)
+            self.__dict__[name] = None
 
     def __repr__(self):
         """The one-line description the reference prints for its deploy modules (module_utils.py:995-1008)."""
@@ -191,8 +204,13 @@ class VllmRealQuantLinear(_RealQuantLinear):
     def quant_pack(cls, module, w_q, quant_config):
         """module_utils.py:913-927: w_q(module) -> (codes, scales, zeros), packed when need_pack."""
         _bf16_weight(module)
+        need_pack = quant_config['weight'].get('need_pack', False)
+        q = _rtn_quantizer(w_q) if need_pack else None
+        if q is not None and q.bit == quant_config['weight']['bit'] and q._can_pack(module.weight.data):
+            # quantized and packed by one kernel; the codes (int32 for 4 bits: eight times the packed words) stay on the chip
+            return q._pack_dynamic(module.weight.data, torch.float16)
         weight, scales, zeros = w_q(module)
-        if quant_config['weight'].get('need_pack', False):
+        if need_pack:
             weight, scales = cls.pack(weight, scales, quant_config)
         return weight, scales
 

@@ -818,6 +818,29 @@ class IntegerQuantizer(BaseQuantizer):
         codes = self.restore_tensor(codes.view(rows_t.shape), org_w_shape)
         return self._finish_real(codes, scales, zeros, output_scale_factor)
 
+    def _can_pack(self, weight):
+        """May `_pack_dynamic` stand for real_quant_weight_dynamic and a pack?  Symmetric 4- or 8-bit min/max codes of a 2-D
+        weight whose rows fill whole 16-byte chunks (the nibbles / bytes then leave the quantizer's kernel in place)."""
+        lo, hi = (-8, 7) if self.bit == 4 else (-128, 127)
+        cols = self.group_size if self.granularity == 'per_group' else weight.shape[-1]
+        return (self.bit in (4, 8) and self.sym and self.calib_algo == 'minmax' and self.round_zp
+                and self.granularity in ('per_group', 'per_channel') and weight.dim() == 2
+                and weight.shape[1] % 8 == 0 and cols % 8 == 0 and weight.dtype in (torch.bfloat16, torch.float16, torch.float32)
+                and lo <= float(self.qmin) and float(self.qmax) <= hi and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+
+    def _pack_dynamic(self, weight, scales_dtype):
+        """-> (int32 words [R, K * bit / 32], scales [R, -1] in `scales_dtype`: the weight's type or fp16), one launch."""
+        rows_t = self.reshape_tensor(weight)
+        R, K = weight.shape
+        rows, cols = rows_t.shape
+        packed = torch.empty((R, K * self.bit // 32), dtype=torch.int32, device=weight.device)
+        scales = torch.empty((R, rows // R), dtype=scales_dtype, device=weight.device)
+        flags = L.FLAG_SYM | (L.FLAG_SCALES_F16 if scales_dtype != weight.dtype else 0)
+        L.check(L.lib().lcq_quant_int(L.ptr(rows_t), L.dtype_code(weight.dtype), rows, cols, float(self.qmin), float(self.qmax),
+                                      flags, 1.0, None, packed.data_ptr(), L.CODE_CT4 if self.bit == 4 else L.CODE_CT8,
+                                      scales.data_ptr(), None, L.stream()), 'lcq_quant_int')
+        return packed, scales
+
     def real_quant_pack_dynamic(self, weight):
         """Quantize and pack in one pass: what VllmRealQuantLinear.pack(*real_quant_weight_dynamic(w)[:2])
         returns for a symmetric 4-bit quantizer (module_utils.py:929-955 after quant.py:915-952), without

@@ -146,3 +146,25 @@ def test_autoawq_new(dev, dtype):
     cfg['weight']['pack_version'] = 'gemv_pack'
     with pytest.raises(NotImplementedError):
         AutoawqRealQuantLinear.new(Lin(w.to(dev)), w_q, cfg)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('bit,g,R,K', [(4, 128, 64, 512), (8, 128, 33, 256), (4, 32, 7, 96), (8, 64, 31, 128), (4, 0, 5, 264), (8, 0, 3, 1000),
+                                       (4, 4, 3, 64)])
+def test_vllm_new_with_the_rtn_partial_packs_in_one_launch(dev, dtype, bit, g, R, K):
+    """RTN's own w_q lets the container quantize and pack in one kernel (groups of 4 do not fill 16-byte chunks: two
+    launches): words and fp16 scales bit for bit those of the two steps, zero rows included."""
+    from lightcompress_amd.module_utils import VllmRealQuantLinear
+    from lightcompress_amd.rtn import RTN
+    gran = 'per_group' if g else 'per_channel'
+    w = weight_like(R, K, seed=R + K, dtype=dtype)
+    w[1] = 0
+    rtn = RTN({'weight': dict(bit=bit, symmetric=True, granularity=gran, need_pack=True, **({'group_size': g} if g else {}))})
+    m = Lin(w.to(dev))
+    assert rtn.wquantizer._can_pack(m.weight.data) == (g != 4)
+    new = VllmRealQuantLinear.new(m, **rtn.get_replacement_params('vllm_quant'))
+    oc, os_, _ = Q.int_real_quant_dynamic(Q.IntSpec(bit, True, gran, group_size=g), w)
+    op, os16 = pack_ref.pack_ct(oc, os_, bit)
+    assert_bit_equal(new.weight_packed, op, 'weight_packed')
+    assert_bit_equal(new.weight_scale, os16, 'weight_scale')
+    assert new.weight_shape == new.weight_packed.shape and new.in_features == K and new.bias is None
