@@ -206,6 +206,11 @@ int lcq_pack_ct(const void* codes, int code_dtype, int64_t R, int64_t K, int bit
 int lcq_pack_awq(const void* w, int dtype, const void* scales, const int32_t* zeros, int64_t R, int64_t K, int group_size,
                  int32_t* qweight, void* scales_f16_out, int32_t* qzeros, void* stream);
 
+/* real_quant_weight_dynamic (quant.py:915-952; asymmetric, min/max, rounded zero points, |qmin|, qmax <= 256) and gemm_pack of
+ * its scales and zero points in one pass: outputs as lcq_pack_awq; group_size 32, 64 or 128, R % 32 == 0, 16-byte aligned. */
+int lcq_quant_pack_awq(const void* w, int dtype, int64_t R, int64_t K, int group_size, float qmin, float qmax,
+                       int32_t* qweight, void* scales_f16_out, int32_t* qzeros, void* stream);
+
 /* ---- GPTQ --------------------------------------------------------------- */
 
 /* GPTQ.add_batch, gptq.py:253-295:  H <- alpha*H + beta * X^T X  with

@@ -266,11 +266,34 @@ class AutoawqRealQuantLinear(_RealQuantLinear):
     def quant_pack(cls, module, w_q, quant_config):
         """module_utils.py:1080-1095."""
         _bf16_weight(module)
-        _, scales, zeros = w_q(module)
         pack_version = quant_config['weight']['pack_version']
         if pack_version != 'gemm_pack':
             raise NotImplementedError(f'Not support {pack_version}.')
+        fused = cls._gemm_pack_fused(module, _rtn_quantizer(w_q), quant_config)
+        if fused is not None:
+            return fused
+        _, scales, zeros = w_q(module)
         return cls.gemm_pack(module, module.weight.data, scales, zeros, quant_config)
+
+    @classmethod
+    def _gemm_pack_fused(cls, module, q, quant_config):
+        """gemm_pack(module, weight, *w_q(module)[1:], quant_config) in one launch for RTN's own w_q: this layout takes the
+        scales and zero points of the quantizer and not its codes.  None where the kernel does not apply."""
+        w, cfg = module.weight.data, quant_config['weight']
+        if q is None or w.dim() != 2 or cfg['bit'] != 4 or q.sym or q.granularity != 'per_group' or q.calib_algo != 'minmax' \
+                or not q.round_zp or q.group_size != cfg['group_size'] or q.group_size not in (32, 64, 128) \
+                or not -256 <= float(q.qmin) < float(q.qmax) <= 256 or not w.is_contiguous() or w.data_ptr() % 16 \
+                or w.dtype not in (torch.bfloat16, torch.float16, torch.float32) or w.shape[0] % 32 or w.shape[1] % q.group_size:
+            return None
+        R, K = w.shape
+        assert module.in_features == K
+        G = K // q.group_size
+        qweight = torch.empty((K, R // 8), dtype=torch.int32, device=w.device)
+        s16 = torch.empty((G, R), dtype=torch.float16, device=w.device)
+        qzeros = torch.empty((G, R // 8), dtype=torch.int32, device=w.device)
+        L.check(L.lib().lcq_quant_pack_awq(L.ptr(w), L.dtype_code(w.dtype), R, K, q.group_size, float(q.qmin), float(q.qmax),
+                                           L.ptr(qweight), L.ptr(s16), L.ptr(qzeros), L.stream()), 'lcq_quant_pack_awq')
+        return qweight, s16, qzeros
 
     @classmethod
     @torch.no_grad()

@@ -168,3 +168,31 @@ def test_vllm_new_with_the_rtn_partial_packs_in_one_launch(dev, dtype, bit, g, R
     assert_bit_equal(new.weight_packed, op, 'weight_packed')
     assert_bit_equal(new.weight_scale, os16, 'weight_scale')
     assert new.weight_shape == new.weight_packed.shape and new.in_features == K and new.bias is None
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('g,R,K', [(128, 32, 128), (128, 288, 256), (64, 544, 192), (32, 1056, 64), (16, 64, 64)])
+def test_autoawq_new_with_the_rtn_partial(dev, dtype, g, R, K):
+    """Scales, zero points and nibbles in one launch (groups of 16: the two steps), where octets of rows fill workgroups and
+    where they do not; then gemm_pack on given parameters over the same shapes.  Rows whose integers leave 0 .. 15 (the
+    layout does not clamp) and constant rows included."""
+    from lightcompress_amd.module_utils import AutoawqRealQuantLinear
+    from lightcompress_amd.rtn import RTN
+    w = weight_like(R, K, seed=R + g, dtype=dtype, outlier_frac=0.01)
+    w[2] = 0
+    # a constant row has the smallest scale, 1e-5 / 15: its integer 2^-8 / 6.6e-7 = 5.9e3 is finite in every type (0.0625 / 6.6e-7
+    # = 9.4e4 is beyond fp16's 65504, and the conversion of an infinity to an integer is undefined in torch)
+    w[3] = 2.0 ** -8
+    cfg = {'weight': dict(bit=4, symmetric=False, granularity='per_group', group_size=g, pack_version='gemm_pack')}
+    rtn = RTN(cfg)
+    m = Lin(w.to(dev))
+    new = AutoawqRealQuantLinear.new(m, **rtn.get_replacement_params('autoawq_quant'))
+    _, os_, oz = Q.int_real_quant_dynamic(Q.IntSpec(4, False, 'per_group', group_size=g), w)
+    want = pack_ref.gemm_pack(w, os_, oz, g)
+    for got, o, name in zip((new.qweight, new.scales, new.qzeros), want, ('qweight', 'scales', 'qzeros')):
+        assert_bit_equal(got, o, name)
+    s2, z2 = os_ * 0.75, (oz + 1).clamp(max=15)             # other parameters: integers beyond the nibble in many places
+    want = pack_ref.gemm_pack(w, s2, z2, g)
+    got = AutoawqRealQuantLinear.gemm_pack(m, m.weight.data, s2.to(dev), z2.to(dev), cfg)
+    for a, o, name in zip(got, want, ('qweight', 'scales', 'qzeros')):
+        assert_bit_equal(a, o, 'given ' + name)
