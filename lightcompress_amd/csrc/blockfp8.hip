@@ -9,8 +9,7 @@
 //   back:  out = float(y) * s
 // Rounding to float8 is the hardware convert (round to nearest even, what Triton's and torch's casts
 // do); LCQ_FLAG_TIE_AWAY nudges exact ties one ulp outwards first (the add-half-then-truncate model of
-// float_quantize).  x / s is evaluated as x * (1/s) unless the product is within 8 ulp of a float8
-// rounding boundary, where the lane divides.
+// float_quantize).
 #include "rowquant.h"
 
 namespace {
@@ -18,16 +17,33 @@ using namespace lcq;
 
 constexpr int BS = 128;
 
+// x / s for a divisor that many elements share, correctly rounded without the division sequence: with y = RN(1/s) the product
+// q0 = x y is within 2 ulp, one residual step makes it faithful and a second one exact (Markstein, IBM J. R&D 34(1), 1990;
+// the residuals are exact).  Five full-rate instructions; a guarded product needs as many to find out whether it may stay, and
+// values below the minimum normal, where the grid's midpoints are not a bit pattern, went through the division sequence.
+// Scales outside 2^-60 .. 2^60 (an infinite or NaN block, a block of subnormals) divide.
+struct Divisor {
+  float s, y;
+  bool fast;
+  __device__ __forceinline__ explicit Divisor(float s_) : s(s_), fast(s_ > 8.6736174e-19f && s_ < 1.1529215e18f) {
+    const float y0 = __builtin_amdgcn_rcpf(s);
+    y = __builtin_fmaf(__builtin_fmaf(-s, y0, 1.0f), y0, y0);
+  }
+  __device__ __forceinline__ float quotient(float x) const {
+    if (__builtin_expect(!fast, 0)) return x / s;
+    float q = x * y;                                         // (s q - x taken off, not x - s q added: that way -0 / s stays -0)
+    q = __builtin_fmaf(-__builtin_fmaf(s, q, -x), y, q);
+    return __builtin_fmaf(-__builtin_fmaf(s, q, -x), y, q);
+  }
+};
+
 // value handed to the float8 convert.  model = false: x / s itself (Triton / torch cast: one rounding, to
 // nearest even, done by the convert).  model = true: the FloatQuantizer route, "x / s + 0" rounded by the
 // float_quantize model first - add-half-then-truncate on the fp32 mantissa (ties away; tie_even: to even),
 // and below the minimum normal 2^-6 the same on |t| + 2^-6 (whose fp32 addition already rounds once) - so the
 // convert only re-encodes an exact grid value.
-__device__ __forceinline__ float fp8_input(float x, float s, float r, bool fast, bool tie_away, bool model) {
-  float t = x * r;
-  const uint32_t lowm = f2u(t) & 0xfffffu;                  // 20 dropped mantissa bits of e4m3
-  const bool sub = !(fabsf(t) >= 0.015625f);                // below the minimum normal 2^-6: fixed step 2^-9
-  if (__builtin_expect(!fast || sub || (lowm - 0x7fff8u) <= 16u, 0)) t = x / s;
+__device__ __forceinline__ float fp8_input(float x, const Divisor& d, bool tie_away, bool model) {
+  float t = d.quotient(x);
   if (!model) return t;
   t = t + 0.0f;                                             // "+ zeros": -0 becomes +0
   if (fabsf(t) >= 0.015625f) {
@@ -46,44 +62,49 @@ struct BlkArgs {
   int nbn, clamp_range, tie_away;
 };
 
-// one workgroup per 128x128 block: 2048 (bf16) / 4096 (fp32) 16-byte chunks, 8 / 16 per thread in registers
+// One workgroup of 512 per 128x128 block: 2048 (bf16) / 4096 (fp32) 16-byte chunks, 4 / 8 per thread in registers.  HBM-bound
+// beyond a few thousand blocks; at 2112 x 7168 (952 blocks, less than four per CU) the latency of load - reduce - store: 16.7 us
+// with 256 lanes per block and guarded quotients, 11.8 so (7.5 at the rate of a plain stream).
 template <bool BF>
-__global__ __launch_bounds__(256) void block_quant_kernel(BlkArgs a) {
-  constexpr int N = Vec<BF>::N, CPR = BS / N, PER = BS * CPR / 256;
-  __shared__ float sm[4];
+__global__ __launch_bounds__(512) void block_quant_kernel(BlkArgs a) {
+  constexpr int N = Vec<BF>::N, CPR = BS / N, PER = BS * CPR / 512;
+  __shared__ float sm[8];
   const int bm = blockIdx.y, bn = blockIdx.x;
   u32x4 raw[PER];
   bool ok[PER];
   float amax = 0.0f;
   #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int ci = threadIdx.x + k * 256, r = ci / CPR, c = ci % CPR;
+    const int ci = threadIdx.x + k * 512, r = ci / CPR, c = ci % CPR;
     const int64_t row = (int64_t)bm * BS + r, col = (int64_t)bn * BS + c * N;
     ok[k] = row < a.M && col < a.N;
     raw[k] = ok[k] ? __builtin_nontemporal_load((const u32x4*)a.x + (row * a.N + col) / N) : u32x4{0, 0, 0, 0};
+  }
+  #pragma unroll
+  for (int k = 0; k < PER; ++k) {
     float v[N];
     unpack<BF>(raw[k], v);
     #pragma unroll
-    for (int i = 0; i < N; ++i) amax = nan_max(amax, fabsf(v[i]));
+    for (int i = 0; i < N; i += 2) amax = nan_max(nan_max(amax, fabsf(v[i])), fabsf(v[i + 1]));
   }
   amax = team_reduce<64, true>(amax);
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = nan_max(nan_max(sm[0], sm[1]), nan_max(sm[2], sm[3]));
+  #pragma unroll
+  for (int w = 0; w < 8; ++w) amax = nan_max(amax, sm[w]);
   if (a.clamp_range) amax = nan_max(amax, 1e-5f);
   const float s = amax / 448.0f;
-  const float r = __builtin_amdgcn_rcpf(s);
-  const bool fast = (s > 8.6736174e-19f) && (s < 1.1529215e18f);
+  const Divisor div(s);
   if (threadIdx.x == 0) a.scales[(int64_t)bm * a.nbn + bn] = s;
   #pragma unroll
   for (int k = 0; k < PER; ++k) {
     if (!ok[k]) continue;
-    const int ci = threadIdx.x + k * 256, rr = ci / CPR, c = ci % CPR;
+    const int ci = threadIdx.x + k * 512, rr = ci / CPR, c = ci % CPR;
     const int64_t row = (int64_t)bm * BS + rr, col = (int64_t)bn * BS + c * N;
     float v[N];
     unpack<BF>(raw[k], v);
     #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = fp8_input(v[i], s, r, fast, a.tie_away, a.clamp_range);
+    for (int i = 0; i < N; ++i) v[i] = fp8_input(v[i], div, a.tie_away, a.clamp_range);
     uint32_t w[N / 4];
     #pragma unroll
     for (int q = 0; q < N / 4; ++q) {
@@ -115,12 +136,11 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const u32x4* __restrict_
   amax = team_reduce<TEAM, true>(amax);
   if (clamp_range) amax = nan_max(amax, 1e-5f);
   const float s = amax / 448.0f;
-  const float r = __builtin_amdgcn_rcpf(s);
-  const bool fast = (s > 8.6736174e-19f) && (s < 1.1529215e18f);
+  const Divisor div(s);
   if (!okb) return;
   if (t == 0) scales[blk] = s;
   #pragma unroll
-  for (int i = 0; i < N; ++i) v[i] = fp8_input(v[i], s, r, fast, tie_away, clamp_range);
+  for (int i = 0; i < N; ++i) v[i] = fp8_input(v[i], div, tie_away, clamp_range);
   uint32_t w[N / 4];
   #pragma unroll
   for (int q = 0; q < N / 4; ++q) {
@@ -134,28 +154,36 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const u32x4* __restrict_
   else *(uint32_t*)dst = w[0];
 }
 
-// out = float(y) * s[block]; 8 float8 per thread
+// out = float(y) * s[block]: a workgroup takes 8 rows of one block row and 256 * W columns, W float8 per lane and row so that
+// a lane's output is one 16-byte piece next to its neighbours'.  HBM-bound: 2112 x 7168 to fp32 (76 MB) 15.4 us with eight
+// float8 per lane, two half-line stores and a 64-bit division per chunk, 13.3 so.
 template <int OUT>   // LCQ_F32 | LCQ_BF16
 __global__ __launch_bounds__(256) void block_dequant_kernel(const uint8_t* __restrict__ y, const float* __restrict__ scales,
                                                             int64_t M, int64_t N, int nbn, void* __restrict__ out) {
-  const int64_t npr = N / 8, total = M * npr;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < total; c += (int64_t)gridDim.x * 256) {
-    const int64_t row = c / npr, col = (c % npr) * 8;
-    const float s = scales[(row / BS) * nbn + col / BS];
-    const u32x2 w = *(const u32x2*)(y + row * N + col);
-    float v[8];
-    #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[q], false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[q], true);
-      v[4 * q] = lo[0] * s; v[4 * q + 1] = lo[1] * s; v[4 * q + 2] = hi[0] * s; v[4 * q + 3] = hi[1] * s;
+  constexpr int W = OUT == LCQ_BF16 ? 8 : 4;
+  const int64_t col = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W, row0 = (int64_t)blockIdx.y * 8;
+  if (col >= N) return;
+  const float s = scales[(row0 / BS) * nbn + col / BS];
+  uint32_t w[8][W / 4];
+  #pragma unroll
+  for (int r = 0; r < 8; ++r)
+    if (row0 + r < M) {
+      if constexpr (W == 8) { const u32x2 v = *(const u32x2*)(y + (row0 + r) * N + col); w[r][0] = v[0]; w[r][W / 4 - 1] = v[1]; }
+      else w[r][0] = *(const uint32_t*)(y + (row0 + r) * N + col);
     }
-    if constexpr (OUT == LCQ_BF16) {
-      *((u32x4*)out + c) = pack_rne<true>(v);
-    } else {
-      *((u32x4*)out + 2 * c) = u32x4{f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])};
-      *((u32x4*)out + 2 * c + 1) = u32x4{f2u(v[4]), f2u(v[5]), f2u(v[6]), f2u(v[7])};
+  #pragma unroll
+  for (int r = 0; r < 8; ++r)
+    if (row0 + r < M) {
+      float v[W];
+      #pragma unroll
+      for (int q = 0; q < W / 4; ++q) {
+        const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[r][q], false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[r][q], true);
+        v[4 * q] = lo[0] * s; v[4 * q + 1] = lo[1] * s; v[4 * q + 2] = hi[0] * s; v[4 * q + 3] = hi[1] * s;
+      }
+      u32x4* const dst = (u32x4*)((char*)out + ((row0 + r) * N + col) * (OUT == LCQ_BF16 ? 2 : 4));
+      if constexpr (OUT == LCQ_BF16) *dst = pack_rne<true>(v);
+      else *dst = u32x4{f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])};
     }
-  }
 }
 
 }  // namespace
@@ -185,8 +213,8 @@ int lcq_fp8_block_quant(const void* x, int dtype, int64_t M, int64_t N, int bloc
     a.nbn = (int)((N + BS - 1) / BS); a.clamp_range = clamp_range; a.tie_away = tie_away;
     const dim3 grid((unsigned)a.nbn, (unsigned)((M + BS - 1) / BS));
     if (grid.y > 65535) return LCQ_EINVAL;
-    if (dtype == LCQ_BF16) block_quant_kernel<true><<<grid, dim3(256), 0, st>>>(a);
-    else block_quant_kernel<false><<<grid, dim3(256), 0, st>>>(a);
+    if (dtype == LCQ_BF16) block_quant_kernel<true><<<grid, dim3(512), 0, st>>>(a);
+    else block_quant_kernel<false><<<grid, dim3(512), 0, st>>>(a);
   }
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
@@ -196,11 +224,12 @@ int lcq_fp8_block_dequant(const void* y, const float* scales, int64_t M, int64_t
   if (!y || !scales || !out || M <= 0 || N <= 0) return LCQ_EINVAL;
   if (N % 8 != 0 || ((uintptr_t)y % 8) != 0 || ((uintptr_t)out % 16) != 0) return LCQ_EALIGN;
   const int nbn = (int)((N + BS - 1) / BS);
-  int64_t grid = (M * (N / 8) + 255) / 256;
-  if (grid > 262144) grid = 262144;
+  const int64_t per = 256 * (out_dtype == LCQ_BF16 ? 8 : 4);
+  if ((M + 7) / 8 > 0x7fffffff || (N + per - 1) / per > 0x7fffffff) return LCQ_EINVAL;
+  const dim3 grid((unsigned)((N + per - 1) / per), (unsigned)((M + 7) / 8));
   hipStream_t st = (hipStream_t)stream;
-  if (out_dtype == LCQ_BF16) block_dequant_kernel<LCQ_BF16><<<dim3((unsigned)grid), dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
-  else if (out_dtype == LCQ_F32) block_dequant_kernel<LCQ_F32><<<dim3((unsigned)grid), dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
+  if (out_dtype == LCQ_BF16) block_dequant_kernel<LCQ_BF16><<<grid, dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
+  else if (out_dtype == LCQ_F32) block_dequant_kernel<LCQ_F32><<<grid, dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
   else return LCQ_EDTYPE;
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;

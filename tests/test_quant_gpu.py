@@ -917,3 +917,25 @@ def test_every_finite_fp16_value_under_many_scales(dev, kind):
             assert_bit_equal(codes, Q.float_quant(spec, rows, s.clone(), 0.0), f'{kind} {k} codes')
             want = Q.float_dequant(Q.float_quant(spec, rows, s.clone(), 0.0), s, 0.0).half()
             assert_bit_equal(q.fake_quant_weight_static(rows.to(dev), {'scales': s.to(dev)}), want, f'{kind} {k}')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('rows', [1, 128])
+def test_blockwise_fp8_quotients_next_to_rounding_boundaries(dev, dtype, rows):
+    """x / s without the division sequence: values on and one ulp beside the midpoints between float8 numbers (subnormal ones
+    included) times their block's scale, -0, bit for bit; per 128 x 128 block and per activation block."""
+    from lightcompress_amd import kernel as K8
+    g = gen(21 + rows)
+    M, N = 256, 512
+    x = torch.randn(M, N, generator=g) * torch.exp(3 * torch.randn(M, 1, generator=g))
+    f8 = lambda: torch.randint(0, 127, (M, N), generator=g, dtype=torch.uint8).view(torch.float8_e4m3fn).float()
+    blk = x.abs().view(M // rows, rows, N // 128, 128).amax((1, 3)).repeat_interleave(rows, 0).repeat_interleave(128, 1)
+    mid = (f8() + f8()) / 2 * (blk / 448)
+    mid = torch.nextafter(mid, mid + torch.randint(-1, 2, mid.shape, generator=g).float())
+    x = torch.where((torch.rand(M, N, generator=g) < 0.9) & (x.abs() < blk) & (mid < 0.99 * blk), mid, x)
+    x[5, 7] = -0.0
+    x = x.to(dtype).contiguous()
+    y, s = (K8.act_quant if rows == 1 else K8.weight_cast_to_fp8)(x.to(dev))
+    oy, os_ = (Q.triton_act_quant if rows == 1 else Q.triton_weight_cast_to_fp8)(x)
+    assert_bit_equal(s, os_, 'scales')
+    assert_bit_equal(y, oy, 'codes')
