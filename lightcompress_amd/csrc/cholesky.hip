@@ -172,15 +172,17 @@ __global__ __launch_bounds__(256) void build_gather_kernel(const float* __restri
 // Here the 128 columns are 8 panels of 16, and the serial part of a panel runs in ONE wave without barriers:
 //   * waves 0-3 ("update waves") hold the lower triangle in registers, 8x8 per thread, dealt out cyclically (thread
 //     (ty, tx) owns rows ty + 16 ii and columns tx + 16 cc);
-//   * wave 4 (the "panel wave") takes the current 16-column panel from LDS with one or two rows per lane and factors
-//     it in registers: pivot and multipliers travel by v_readlane, 3 instructions per (column, later column) pair;
-//     it leaves the scaled panel in LDS;
-//   * the update waves apply a finished panel first to the next panel's columns, hand those to the panel wave, and
-//     apply it to the rest of their registers while the panel wave is already factoring (a right-looking update
+//   * waves 4, 6 and 7 ("panel waves") take the current 16-column panel from LDS with one row per lane and factor it in
+//     registers: pivot and multipliers travel by v_readlane, 2 instructions per (column, later column) pair; they leave
+//     the scaled panel in LDS;
+//   * the update waves apply a finished panel first to the next panel's columns, hand those to the panel waves, and
+//     apply it to the rest of their registers while those are already factoring (a right-looking update
 //     with look-ahead); two barriers per panel;
 //   * wave 5 inverts the 16x16 diagonal block of the previous panel meanwhile (forward substitution in registers);
 //   * afterwards all 8 waves merge the inverted diagonal blocks pairwise, 16 -> 32 -> 64 -> 128,
 //     [[A,0],[B,C]]^-1 = [[A^-1,0],[-C^-1 B A^-1, C^-1]], from LDS.
+// Bound by the serial chain of one wave's instructions: 28.7 us per block (32.8 with two rows per lane in one panel wave,
+// one LDS read at a time in front of the hand-over and one per matrix instruction in the merges; the same bits).
 // Row (column) r of the block lives at float `lds_slot(r)` of an LDS row.  Thread t of the 16 x 16 update grid owns rows
 // t + 16 ii, ii < 8: the first four sit at 4 t .. 4 t + 3 and the other four at 64 + 4 t .., so both 16-byte pieces of
 // a thread are contiguous with its neighbours' (no bank conflicts for 16-byte accesses), and 16 consecutive rows are 16
@@ -200,39 +202,34 @@ __device__ __forceinline__ float rdlane(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
-// panel P: columns 16 P .. +15, rows 16 P .. 127; lane l owns row 16 P + l and (TWO) row 16 P + 64 + l
-template <bool TWO>
-__device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int lane, bool& bad) {
+// panel P: columns 16 P .. +15, rows 16 P .. 127.  Lanes 0 .. 15 of every panel wave hold the panel's own 16 rows (the multipliers
+// come from there), the other 48 lanes the rows behind them, dealt to as many waves as they need: wave `w` (0, 1, 2) takes rows
+// 16 P + 16 + 48 w ...  One row per lane in up to three waves on SIMDs of their own: two rows per lane in one wave are half as many
+// instructions again on the critical path.  Wave 0 writes the panel's own rows.
+__device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int w, int lane, bool& bad) {
   #pragma clang fp contract(fast)   // a -= l*l as one FMA; nothing here needs op-by-op rounding
-  const int c0 = 16 * P;
-  const int rA = c0 + lane, rB = c0 + 64 + lane;
-  const bool okA = rA < NB, okB = TWO && rB < NB;
-  const int sA = lds_slot(okA ? rA : 0), sB = lds_slot(okB ? rB : 0);
-  float a0[16], a1[16];
+  const int row = 16 * P + lane + (lane < 16 ? 0 : 48 * w);
+  const bool ok = row < NB;
+  const int slot = lds_slot(ok ? row : 0);
+  float a[16];
   #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    a0[k] = okA ? s.Pn[k][sA] : 0.0f;
-    a1[k] = okB ? s.Pn[k][sB] : 0.0f;
-  }
+  for (int k = 0; k < 16; ++k) a[k] = ok ? s.Pn[k][slot] : 0.0f;
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const float piv = rdlane(a0[j], j);
+    const float piv = rdlane(a[j], j);
     bad = bad || !(piv > 0.0f);
     float rinv = __builtin_amdgcn_rsqf(piv);          // 1/sqrt(pivot), one Newton step to full precision
     rinv = rinv * (1.5f - 0.5f * piv * rinv * rinv);
-    a0[j] *= rinv;                                    // the diagonal entry becomes sqrt(pivot); rows above it hold zeros
-    if (TWO) a1[j] *= rinv;
+    a[j] *= rinv;                                     // the diagonal entry becomes sqrt(pivot); rows above it hold zeros
     #pragma unroll
     for (int c = j + 1; c < 16; ++c) {
-      const float m = rdlane(a0[j], c);               // L(16 P + c, 16 P + j)
-      a0[c] -= a0[j] * m;                             // (entries above the diagonal pick up garbage; never read, masked below)
-      if (TWO) a1[c] -= a1[j] * m;
+      const float m = rdlane(a[j], c);                // L(16 P + c, 16 P + j)
+      a[c] -= a[j] * m;                               // (entries above the diagonal pick up garbage; never read, masked below)
     }
   }
-  #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if (okA) s.L[P][k][sA] = (lane >= k) ? a0[k] : 0.0f;
-    if (okB) s.L[P][k][sB] = a1[k];
+  if (ok && (lane >= 16 || w == 0)) {
+    #pragma unroll
+    for (int k = 0; k < 16; ++k) s.L[P][k][slot] = (lane >= k) ? a[k] : 0.0f;
   }
 }
 
@@ -267,7 +264,9 @@ template <int PL, int CC_LO, bool ONE>
 __device__ __forceinline__ void potrf_update(const PotrfLds& s, float (&a)[8][8], int ty, int tx) {
   #pragma clang fp contract(fast)
   if constexpr (CC_LO < 8) {
-    #pragma unroll 2
+    constexpr int UNROLL = ONE ? 16 : 2;
+    // ONE is on the critical path (the panel waves wait for it): all of its LDS reads in flight at once
+    #pragma unroll UNROLL
     for (int k = 0; k < 16; ++k) {
       const f32x4 r0 = *(const f32x4*)(s.L[PL][k] + 4 * ty), r1 = *(const f32x4*)(s.L[PL][k] + 64 + 4 * ty);
       const float lr[8] = {r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]};
@@ -301,8 +300,9 @@ __device__ __forceinline__ void potrf_publish(PotrfLds& s, const float (&a)[8][8
 template <int P>
 __device__ __forceinline__ void potrf_phase(PotrfLds& s, float (&a)[8][8], int wave, int lane, bool upd, int ty, int tx, bool& bad) {
   __syncthreads();                                   // Pn holds panel P; L[P - 1] is complete
-  if (wave == 4) {
-    potrf_panel<(16 * P + 64 < NB)>(s, P, lane, bad);
+  constexpr int BEHIND = NB - 16 * P - 16;           // rows behind the panel's own
+  if (wave == 4 || (BEHIND > 48 && wave == 6) || (BEHIND > 96 && wave == 7)) {
+    potrf_panel(s, P, wave == 4 ? 0 : wave - 5, lane, bad);
   } else if (wave == 5) {
     if constexpr (P > 0) potrf_diag_inv(s, P - 1, lane);
   } else if (upd) {
@@ -338,9 +338,16 @@ __device__ __forceinline__ void potrf_merge(PotrfLds& s, int wave, int lane) {
       #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
       const int rs = lds_slot(o + S + 32 * ti + lm);
-      for (int k = 32 * tj; k < S; k += 2) {             // X11(k, j) = 0 for k < j
-        const int kk = o + k + lk;
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.L[kk >> 4][kk & 15][rs], s.X[kk][o + 32 * tj + lm], acc, 0, 0, 0);
+      for (int k0 = 32 * tj; k0 < S; k0 += 32) {         // X11(k, j) = 0 for k < j
+        float av[16], bv[16];                            // the operands of 16 instructions in flight: the chain waits for LDS once
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int kk = o + k0 + 2 * i + lk;
+          av[i] = s.L[kk >> 4][kk & 15][rs];
+          bv[i] = s.X[kk][o + 32 * tj + lm];
+        }
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], acc, 0, 0, 0);
       }
       #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -351,10 +358,16 @@ __device__ __forceinline__ void potrf_merge(PotrfLds& s, int wave, int lane) {
       potrf_f32x16 acc;
       #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-      for (int k = 0; k < 32 * (ti + 1); k += 2) {       // X22(i, k) = 0 for k > i
-        const int kk = k + lk;
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.X[o + S + 32 * ti + lm][o + S + kk], s.T[(p * S + kk) * S + 32 * tj + lm],
-                                                   acc, 0, 0, 0);
+      for (int k0 = 0; k0 < 32 * (ti + 1); k0 += 32) {   // X22(i, k) = 0 for k > i
+        float av[16], bv[16];
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int kk = k0 + 2 * i + lk;
+          av[i] = s.X[o + S + 32 * ti + lm][o + S + kk];
+          bv[i] = s.T[(p * S + kk) * S + 32 * tj + lm];
+        }
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], acc, 0, 0, 0);
       }
       #pragma unroll
       for (int r = 0; r < 16; ++r)
