@@ -93,6 +93,28 @@ __global__ __launch_bounds__(256) void prepare_w_kernel(const void* __restrict__
     }
   }
 }
+// The same without a permutation, 16 bytes per lane (K in whole chunks, everything aligned): four rows per workgroup.
+template <int DT>
+__global__ __launch_bounds__(256) void prepare_w_vec_kernel(const u32x4* __restrict__ w, long long R, int K,
+                                                            const uint8_t* __restrict__ dead, f32x4* __restrict__ out) {
+  constexpr int N = DT == LCQ_F32 ? 4 : 8;
+  const long long row0 = (long long)blockIdx.x * 4;
+  const int cpr = K / N, n = (R - row0 < 4 ? (int)(R - row0) : 4) * cpr;
+  for (int e = threadIdx.x; e < n; e += 256) {
+    const long long at = row0 * cpr + e;
+    const u32x4 raw = w[at];
+    float v[N];
+    #pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = load_w<DT>(&raw, i);
+    if (dead) {
+      const uint8_t* d = dead + (long long)(e % cpr) * N;
+      #pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = d[i] ? 0.0f : v[i];
+    }
+    #pragma unroll
+    for (int i = 0; i < N; i += 4) out[at * (N / 4) + i / 4] = f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+  }
+}
 // The same with a permutation: a gather inside every row.  From memory that is one 64-byte sector per element; here
 // the workgroup's rows (`rows` of them, as many as fit 64 KB) come in as they lie, 16 bytes per lane, and the gather
 // reads LDS.  The permutation is read once per workgroup and column.
@@ -450,22 +472,27 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(float* __restrict__ Abl
   // blocks behind them; place_diag_kernel puts the inverse where the block was.)
 }
 
-// copy the inverted diagonal blocks into place
+// copy the inverted diagonal blocks into place, eight rows per workgroup
 __global__ __launch_bounds__(256) void place_diag_kernel(float* __restrict__ A, int K, const float* __restrict__ Dinv) {
   const int blk = blockIdx.x, k0 = blk * NB;
   const int nb = min(NB, K - k0);
   const float* D = Dinv + (long long)blk * NB * NB;
-  for (int e = threadIdx.x; e < NB * NB; e += 256) {
-    const int r = e / NB, c = e % NB;
-    if (r < nb && c < nb) A[(long long)(k0 + r) * K + k0 + c] = D[e];
+  for (int e = threadIdx.x; e < 8 * NB; e += 256) {
+    const int r = blockIdx.y * 8 + e / NB, c = e % NB;
+    if (r < nb && c < nb) A[(long long)(k0 + r) * K + k0 + c] = D[r * NB + c];
   }
 }
 
-__global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ Linv, int K, float* __restrict__ U) {
+// U[i][j] = Linv[K-1-i][K-1-j].  With `Dinv` (K in whole blocks) the diagonal blocks come from there.
+__global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ Linv, int K, const float* __restrict__ Dinv,
+                                                      float* __restrict__ U) {
   const int i = blockIdx.y;
   const int j = blockIdx.x * 256 + threadIdx.x;
   if (j >= K) return;
-  U[(long long)i * K + j] = (j >= i) ? Linv[(long long)(K - 1 - i) * K + (K - 1 - j)] : 0.0f;
+  const int a = K - 1 - i, b = K - 1 - j;
+  float v = 0.0f;
+  if (j >= i) v = (Dinv && a / NB == b / NB) ? Dinv[(long long)a * NB + b % NB] : Linv[(long long)a * K + b];
+  U[(long long)i * K + j] = v;
 }
 
 }  // namespace
@@ -498,6 +525,14 @@ int lcq_gptq_prepare_weights(const void* w, int dtype, int64_t R, int64_t K, con
     if (dtype == LCQ_F32) prepare_w_gather_kernel<LCQ_F32><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
     else if (dtype == LCQ_BF16) prepare_w_gather_kernel<LCQ_BF16><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
     else prepare_w_gather_kernel<LCQ_F16><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
+  }
+  else if (!p && K % 8 == 0 && K <= (1 << 28) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 15) == 0 &&
+           (dtype == LCQ_F32 || dtype == LCQ_BF16 || dtype == LCQ_F16)) {
+    const u32x4* src = (const u32x4*)w;
+    f32x4* dst = (f32x4*)out;
+    if (dtype == LCQ_F32) prepare_w_vec_kernel<LCQ_F32><<<dim3((unsigned)grid), dim3(256), 0, st>>>(src, R, (int)K, dead, dst);
+    else if (dtype == LCQ_BF16) prepare_w_vec_kernel<LCQ_BF16><<<dim3((unsigned)grid), dim3(256), 0, st>>>(src, R, (int)K, dead, dst);
+    else prepare_w_vec_kernel<LCQ_F16><<<dim3((unsigned)grid), dim3(256), 0, st>>>(src, R, (int)K, dead, dst);
   }
   else if (dtype == LCQ_F32) prepare_w_kernel<LCQ_F32><<<dim3((unsigned)grid), dim3(256), 0, st>>>(w, R, (int)K, p, dead, out);
   else if (dtype == LCQ_BF16) prepare_w_kernel<LCQ_BF16><<<dim3((unsigned)grid), dim3(256), 0, st>>>(w, R, (int)K, p, dead, out);
@@ -561,15 +596,18 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   // one, but their trailing update is applied only inside the current 512-column super-panel;
   // the rest of the matrix is updated once per super-panel with a 512-deep contraction, which
   // cuts the read-modify-write traffic on the trailing matrix fourfold.
-  constexpr int NBO = 4 * NB;
+  // The last 1024 columns are one super-panel: their rank-128 updates are at most 98 of the 64 x 128 tiles, so each still takes
+  // one tile's time (8 us), while the 512-deep update they replace ran on 10 to 36 of 256 CUs (32 us).
+  constexpr int NBO = 4 * NB, TAIL = 8 * NB;
+  const auto super_end = [&](int o0) { return K - o0 <= TAIL ? K : o0 + NBO; };
   // Long chains: the deep update behind a super-panel is split into the columns of the NEXT super-panel (on the
   // caller's stream, the panels that follow need it) and everything behind those (on the side stream, beside those
   // panels: a few narrow launches that leave the chip to it).  The next deep update touches that region again and
   // waits for it.
   SideLane* lane = (g_lookahead.load() && K >= 8192) ? side_lane(st) : nullptr;
   bool pending = false;
-  for (int o0 = 0; o0 < K; o0 += NBO) {
-    const int o1 = (o0 + NBO < K) ? (o0 + NBO) : K;
+  for (int o0 = 0, o1; o0 < K; o0 = o1) {
+    o1 = super_end(o0);
     for (int k0 = o0; k0 < o1; k0 += NB) {
       const int b = k0 / NB, nb = (K - k0 < NB) ? (K - k0) : NB;
       float* Akk = A + (long long)k0 * K + k0;
@@ -585,7 +623,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
       }
     }
     if (o1 < K && lane) {
-      const int o2 = (o1 + NBO < K) ? (o1 + NBO) : K;
+      const int o2 = super_end(o1);
       const float* P = A + (long long)o1 * K + o0;
       if (pending && hipStreamWaitEvent(st, lane->join, 0) != hipSuccess) return LCQ_ELAUNCH;
       pending = false;
@@ -628,11 +666,13 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
         bt.M[q] = K - k1; bt.N[q] = NB; bt.Kc[q] = NB;
         if (K - k1 > maxM) maxM = K - k1;
       }
-      const dim3 grid(1, (unsigned)((maxM + GT - 1) / GT), (unsigned)np);
-      gemm_f32_batched_kernel<false><<<grid, dim3(256), 0, st>>>(A, K, Dinv, NB, A, K, bt, 1.0f, 0.0f, 0);
+      // every tile's operands in flight at once; 32-row tiles while they all fit the chip beside each other
+      const int tm = nblk <= 16 ? 32 : 64;
+      const dim3 grid(1, (unsigned)((maxM + tm - 1) / tm), (unsigned)np);
+      if (tm == 32) gemm_f32_batched_kernel<false, 32, true><<<grid, dim3(256), 0, st>>>(A, K, Dinv, NB, A, K, bt, 1.0f, 0.0f, 0);
+      else gemm_f32_batched_kernel<false, 64, true><<<grid, dim3(256), 0, st>>>(A, K, Dinv, NB, A, K, bt, 1.0f, 0.0f, 0);
     }
-    place_diag_kernel<<<dim3((unsigned)nblk), dim3(256), 0, st>>>(A, K, Dinv);
-    scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, U);
+    scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, Dinv, U);
     if (status)
       (void)hipMemcpyAsync(status, &sc->status, sizeof(int), hipMemcpyDeviceToDevice, st);
     LCQ_CHECK_LAUNCH();
@@ -640,7 +680,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   }
 
   // triangular inverse: inverted diagonal blocks, then pairwise merges
-  place_diag_kernel<<<dim3((unsigned)nblk), dim3(256), 0, st>>>(A, K, Dinv);
+  place_diag_kernel<<<dim3((unsigned)nblk, NB / 8), dim3(256), 0, st>>>(A, K, Dinv);
   int nseg = nblk;
   int seg_start[512], seg_size[512];
   if (nblk > 512) return LCQ_EINVAL;
@@ -684,7 +724,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
     nseg = w;
   }
 
-  scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, U);
+  scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, nullptr, U);
   if (status)
     (void)hipMemcpyAsync(status, &sc->status, sizeof(int), hipMemcpyDeviceToDevice, st);
   LCQ_CHECK_LAUNCH();

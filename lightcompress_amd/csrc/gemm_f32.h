@@ -523,16 +523,16 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmProblem g, float alph
   gemm_tile<B_T, TM, DEEP>(g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, g.Kc, alpha, beta, flags, m0, n0, sA, sB);
 }
 
-template <bool B_T>
+template <bool B_T, int TM = GT, bool DEEP = false>
 __global__ __launch_bounds__(256) void gemm_f32_batched_kernel(const float* A, int lda, const float* B, int ldb, float* C,
                                                                int ldc, GemmBatch bt, float alpha, float beta, int flags) {
-  __shared__ float sA[GT * GPA];
+  __shared__ float sA[TM * GPA];
   __shared__ float sB[B_T ? GT * GPA : GK * GPB];
   const int z = blockIdx.z;
-  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * GT;
   if (m0 >= bt.M[z] || n0 >= bt.N[z]) return;
-  gemm_tile<B_T>(A + bt.offA[z], lda, B + bt.offB[z], ldb, C + bt.offC[z], ldc, bt.M[z], bt.N[z], bt.Kc[z], alpha, beta,
-                 flags, m0, n0, sA, sB);
+  gemm_tile<B_T, TM, DEEP>(A + bt.offA[z], lda, B + bt.offB[z], ldb, C + bt.offC[z], ldc, bt.M[z], bt.N[z], bt.Kc[z], alpha, beta,
+                           flags, m0, n0, sA, sB);
 }
 
 template <bool B_T>

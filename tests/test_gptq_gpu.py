@@ -293,6 +293,63 @@ def test_block_factor_against_fp64(dev, K, actorder, dead):
                                          L.ptr(ws), L.i64(nbytes), L.ptr(status), L.stream()) != 0
 
 
+@pytest.mark.parametrize('K', [896, 1024, 1040, 1152, 1536, 1664, 2176])
+def test_chain_around_the_last_super_panel(dev, K):
+    """The last 1024 columns are one super-panel: sizes with one super-panel, a 512-column one in front of a short, a whole
+    and a nearly whole last one, and a partly filled last block.  U^T U (H + damp I) = I in fp64, and P = M U_bb with
+    M = U^-1 of the same device result (both are fp32 chains of the same blocks: 2e-5 of the largest entry, the bar of the
+    tests against the fp64 chain)."""
+    from lightcompress_amd import _lib as L
+    x = torch.randn(3 * K, K, generator=gen(6100 + K), dtype=torch.float64)
+    H = (x.t() @ x / K).float()
+    nbytes = L.lib().lcq_chol_inv_upper_workspace_bytes(K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    status = torch.ones(1, dtype=torch.int32, device=dev)
+    out = {}
+    for name in ('lcq_chol_inv_upper', 'lcq_chol_block_factor')[:2 if K % 128 == 0 else 1]:
+        Hd = torch.triu(H).to(dev).contiguous()
+        res = torch.empty(K, K, device=dev)
+        L.check(getattr(L.lib(), name)(L.ptr(Hd), K, None, 0.01, None, 0, L.ptr(res), L.ptr(ws), nbytes, L.ptr(status),
+                                       L.stream()), name)
+        assert int(status.item()) == 0
+        out[name] = res.cpu().double()
+        assert torch.equal(torch.triu(out[name]), out[name])
+    U = out['lcq_chol_inv_upper']
+    Hp = H.double() + 0.01 * torch.mean(torch.diag(H).double()) * torch.eye(K, dtype=torch.float64)
+    assert float((U.t() @ U @ Hp - torch.eye(K, dtype=torch.float64)).abs().max()) < 1e-4     # 5e-6 measured up to K = 4096
+    if K % 128 == 0:
+        Uo = torch.linalg.cholesky(torch.linalg.inv(Hp), upper=True)
+        M = torch.linalg.solve_triangular(Uo, torch.eye(K, dtype=torch.float64), upper=True)
+        P = torch.zeros_like(Uo)
+        for b in range(0, K, 128):
+            P[b:b + 128, b:b + 128] = Uo[b:b + 128, b:b + 128]
+            P[:b, b:b + 128] = M[:b, b:b + 128] @ Uo[b:b + 128, b:b + 128]
+        assert float((out['lcq_chol_block_factor'] - P).abs().max()) <= 2e-5 * float(P.abs().max())
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('R,K', [(1, 8), (3, 16), (5, 1000), (7, 1001), (64, 4), (33, 2056)])
+def test_prepare_weights_without_a_permutation(dev, dtype, R, K):
+    """fp32 copy with dead columns zeroed: 16 bytes per lane where rows and pointers allow it, element by element
+    elsewhere (K not in whole chunks, a weight or an output that starts off a 16-byte boundary)."""
+    from lightcompress_amd import _lib as L
+    for woff, ooff in ((0, 0), (1, 0), (0, 1)):
+        w = torch.randn(R * K + 1, generator=gen(R + K)).to(dtype).to(dev)[woff:woff + R * K].view(R, K)
+        w.view(-1)[0] = float('inf')
+        w.view(-1)[R * K - 1] = float('nan')
+        dead = torch.rand(K, generator=gen(K)).to(dev) < 0.3
+        for d in (None, dead):
+            want = w.float()
+            if d is not None:
+                want[:, d] = 0.0
+            out = torch.full((R * K + 2,), 7.0, device=dev)
+            got = out[ooff:ooff + R * K].view(R, K)
+            L.check(L.lib().lcq_gptq_prepare_weights(L.ptr(w), L.dtype_code(dtype), R, K, None,
+                                                     None if d is None else d.data_ptr(), L.ptr(got), L.stream()), 'prepare')
+            assert torch.equal(got.nan_to_num(nan=123.0), want.nan_to_num(nan=123.0))
+            assert float(out[R * K + 1]) == 7.0
+
+
 def test_cholesky_reports_indefinite_matrix(dev):
     from lightcompress_amd import _lib as L
     K = 128
