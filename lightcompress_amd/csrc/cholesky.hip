@@ -203,8 +203,9 @@ __global__ __launch_bounds__(256) void build_gather_kernel(const float* __restri
 //   * wave 5 inverts the 16x16 diagonal block of the previous panel meanwhile (forward substitution in registers);
 //   * afterwards all 8 waves merge the inverted diagonal blocks pairwise, 16 -> 32 -> 64 -> 128,
 //     [[A,0],[B,C]]^-1 = [[A^-1,0],[-C^-1 B A^-1, C^-1]], from LDS.
-// Bound by the serial chain of one wave's instructions: 28.7 us per block (32.8 with two rows per lane in one panel wave,
-// one LDS read at a time in front of the hand-over and one per matrix instruction in the merges; the same bits).
+// Bound by the serial chain of one wave's instructions: 26.4 us per block (32.8 with two rows per lane in one panel wave,
+// one LDS read at a time in front of the hand-over and one per matrix instruction in the merges; 28.7 with a condition around
+// every load of the block; the same bits).
 // Row (column) r of the block lives at float `lds_slot(r)` of an LDS row.  Thread t of the 16 x 16 update grid owns rows
 // t + 16 ii, ii < 8: the first four sit at 4 t .. 4 t + 3 and the other four at 64 + 4 t .., so both 16-byte pieces of
 // a thread are contiguous with its neighbours' (no bank conflicts for 16-byte accesses), and 16 consecutive rows are 16
@@ -433,16 +434,34 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(float* __restrict__ Abl
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ty = (tid >> 4) & 15, tx = tid & 15;
   const bool upd = tid < 256;
-  for (int e = tid; e < NB * LP / 4; e += 512) ((f32x4*)&s.X[0][0])[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float a[8][8];
   if (upd) {
-    #pragma unroll
-    for (int ii = 0; ii < 8; ++ii)
+    // a whole block: plain loads (all in flight), the diagonal 16 x 16 squares masked afterwards; a load under a condition of its
+    // own costs five instructions more and a branch
+    if (nb == NB) {
+      const float* p = Ablk + (long long)ty * lda + tx;
       #pragma unroll
-      for (int cc = 0; cc < 8; ++cc) {
-        const int r = ty + 16 * ii, c = tx + 16 * cc;
-        a[ii][cc] = (r < nb && c <= r) ? Ablk[(long long)r * lda + c] : ((r == c) ? 1.0f : 0.0f);   // pad with identity
+      for (int ii = 0; ii < 8; ++ii)
+        #pragma unroll
+        for (int cc = 0; cc <= ii; ++cc) a[ii][cc] = p[(long long)16 * ii * lda + 16 * cc];
+      #pragma unroll
+      for (int ii = 0; ii < 8; ++ii) {
+        a[ii][ii] = tx <= ty ? a[ii][ii] : 0.0f;
+        #pragma unroll
+        for (int cc = ii + 1; cc < 8; ++cc) a[ii][cc] = 0.0f;
       }
+    } else {
+      #pragma unroll
+      for (int ii = 0; ii < 8; ++ii)
+        #pragma unroll
+        for (int cc = 0; cc < 8; ++cc) {
+          const int r = ty + 16 * ii, c = tx + 16 * cc;
+          a[ii][cc] = (r < nb && c <= r) ? Ablk[(long long)r * lda + c] : ((r == c) ? 1.0f : 0.0f);   // pad with identity
+        }
+    }
+  }
+  for (int e = tid; e < NB * LP / 4; e += 512) ((f32x4*)&s.X[0][0])[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (upd) {
     potrf_publish<0>(s, a, ty, tx);
   }
   bool bad = false;
