@@ -147,6 +147,22 @@ __global__ __launch_bounds__(256) void dequant_kernel(const void* __restrict__ q
 //   err < best  ->  best = err, cur_min = xmin, cur_max = xmax
 // cur_min / cur_max start as the row's min / max and - as in the reference, whose best_min_val / best_max_val
 // alias the range tensors - are the values the NEXT step shrinks.  All arithmetic in fp32 (tensor.float()).
+
+// err of one row, a wave per row: IEEE quotients and powf, lane l adds columns l, l + 64, ... in order.  This sum defines
+// which step wins; every path below takes the decisions it takes.
+template <int BF>
+__device__ __forceinline__ float mse_row_error(const void* __restrict__ x, int64_t row, int64_t cols, const IntRow& prm, float norm,
+                                               const IntOp<0, false>& op, int lane) {
+  float err = 0.0f;
+  #pragma unroll 1
+  for (int64_t j = lane; j < cols; j += 64) {
+    const float v = load_scalar<BF>(x, row * cols + j);
+    const float d = fabsf(op.deq(op.code(v, prm), prm) - v);
+    err += __builtin_powf(d, norm);
+  }
+  return team_sum<64>(err);
+}
+
 // One wave per row; the row is re-read from L1/L2 on every step.
 template <int BF>
 __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__ x, int64_t rows, int64_t cols, int steps,
@@ -165,47 +181,49 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
   for (int i = 0; i < steps; ++i) {
     const float p = (float)(1.0 - (double)i / (double)grid_n);
     const float xmin = p * cur_min, xmax = p * cur_max;
-    const IntRow prm = op.make(xmin, xmax);
-    float err = 0.0f;
-    for (int64_t j = lane; j < cols; j += 64) {
-      const float v = load_scalar<BF>(x, row * cols + j);
-      const float d = fabsf(op.deq(op.code(v, prm), prm) - v);
-      err += __builtin_powf(d, norm);
-    }
-    err = team_sum<64>(err);
+    const float err = mse_row_error<BF>(x, row, cols, op.make(xmin, xmax), norm, op, lane);
     if (err < best) { best = err; cur_min = xmin; cur_max = xmax; }
   }
   if (lane == 0) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
 }
 
 // The same search with the row in registers, for rounded zero points: TEAM lanes (256: a workgroup) share a row, PER
-// elements each.
+// elements each.  A step's error is first estimated:
 //   * t = x * (1/s) instead of x / s: a quotient within 2 ulp of a half-integer may round to the other neighbour, both
-//     of which are half a step away from x, so the error differs by less than the rounding of its sum;
+//     of which are half a step away from x;
 //   * |d| ^ norm = d^2 * 2 ^ ((norm - 2) log2 |d|): the square is exact to one rounding and only the fraction of the
 //     exponent goes through v_log / v_exp; x and s are scaled by the power of two that brings the row's largest value
-//     to [1, 2), so |log2| stays small (the whole expression is good to 2-3 ulp) and nothing underflows.  The factor is
-//     common to all steps of a row and positive, so it changes no comparison;
-//   * every term of the error is >= 0 and fp32 sums of such terms never shrink, so a part of the sum above `best` decides a
-//     step: first the error of the two extremes alone (most steps behind the best one lose by what they clip there), then
-//     after every quarter of the elements.  A wave goes on to the next step when all its rows are decided;
+//     to [1, 2), so |log2| stays small and nothing underflows.  The factor is common to all steps of a row and positive,
+//     so it changes no comparison;
+//   * every term is >= 0 and fp32 sums of such terms never shrink, so a part of the estimate that is far enough above the
+//     best one decides a step: first the error of the two extremes alone (most steps behind the best one lose by what they
+//     clip there), then after every quarter of the elements.  A wave goes on to the next step when all its rows are decided;
 //   * elements past the row's end are zeros: with qmin <= z <= qmax they quantize to themselves and add nothing.
+// The estimate and mse_row_error differ by a relative delta at most (mse_margin below).  Where `margin` cannot tell the two
+// steps apart, the wave evaluates mse_row_error for both of them, so the range is always the one mse_range_kernel finds: an
+// estimate that decides ties by itself picked another range for one group in 16000.  A step with the scale and zero point of
+// the best one (a clamped scale) has its error and is not better.  Rows whose largest value is outside 2^-16 .. 2^16, where
+// powers of the unscaled errors may over- or underflow, and rows with infinities or NaN are always evaluated; so are
+// estimates below SMALL, next to which underflowed terms might count.
 // What bounds it: ten instructions per element and step, two of them transcendental (about 50 vector cycles).  4096 x 4096
-// bf16 in groups of 128, 80 steps: 1870 us with a re-read per step, IEEE divisions and powf; 497 with the row in
-// registers; 222 with the steps cut short (4096 rows of 4096: 1253, 437, 72).
+// bf16 in groups of 128, 4 bits, 80 steps: 1864 us re-reading, 497 with the row in registers, 199 with the steps cut short,
+// 204 with the undecided ones evaluated (4096 rows of 4096: 1268, 437, 366, 380).
+constexpr float MSE_SMALL = 1.1920929e-7f;                   // 2^-23, in units of (largest value of the row, 1 .. 2) ^ norm
 template <int BF, int TEAM, int PER>
 __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restrict__ x, int64_t rows, int cols, int vec, int steps,
-                                                             int grid_n, float norm, IntOp<0, false> op,
+                                                             int grid_n, float norm, float margin, IntOp<0, false> op,
                                                              float* __restrict__ mn_out, float* __restrict__ mx_out) {
   constexpr int N = Vec<BF>::N;
   constexpr bool BLOCK = TEAM > 64;
+  constexpr int SUB = BLOCK ? 64 : TEAM;                     // lanes of a wave that share a row
   __shared__ float shrink[256];                              // p of every step (a double division each)
   __shared__ float sm[8];
   for (int i = threadIdx.x; i < steps; i += 256) shrink[i] = (float)(1.0 - (double)i / (double)grid_n);
   __syncthreads();
   const int64_t row_ = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TEAM;
-  const int64_t row = row_ < rows ? row_ : rows - 1;         // surplus teams repeat the last row and store nothing
-  const int t = threadIdx.x % TEAM;
+  const bool live = row_ < rows;
+  const int64_t row = live ? row_ : rows - 1;                // surplus teams repeat the last row and store nothing
+  const int t = threadIdx.x % TEAM, lane = threadIdx.x & 63;
   float v[PER], mn = __builtin_inff(), mx = -__builtin_inff();
   if (vec) {
     #pragma unroll
@@ -237,14 +255,18 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
     return (sm[0] + sm[1]) + (sm[2] + sm[3]);
   };
   float cur_min = mn, cur_max = mx;
-  // 2^k with 2^k max|x| in [1, 2); 1 where the range is zero, infinite, NaN or so extreme that the factor would overflow
-  const int e = (int)((f2u(fmaxf(fabsf(mn), fabsf(mx))) >> 23) & 0xff);
-  const bool scalable = e > 1 && e < 253;
-  const float up = scalable ? u2f((uint32_t)(254 - e) << 23) : 1.0f, down = scalable ? u2f((uint32_t)e << 23) : 1.0f;
+  // 2^k with 2^k max|x| in [1, 2)
+  const float big = fmaxf(fabsf(mn), fabsf(mx));
+  const bool regular = mn == mn && mx == mx && big >= 1.52587890625e-5f && big <= 65536.0f;
+  const int e = regular ? (int)(f2u(big) >> 23) : 127;
+  const float up = u2f((uint32_t)(254 - e) << 23), down = u2f((uint32_t)e << 23);
   #pragma unroll
   for (int i = 0; i < PER; ++i) v[i] *= up;
   const float frac = norm - 2.0f, top = mx * up, bottom = mn * up;
-  float best = __builtin_inff();
+  // an estimate above `hi` cannot beat the best step, one below `lo` does
+  float hi = live ? __builtin_inff() : -1.0f, lo = regular ? __builtin_inff() : -__builtin_inff();
+  float best = __builtin_inff(), best_s = -1.0f, best_z = 0.0f;        // mse_row_error of the best step (if `have`), its parameters
+  bool have = true;                                          // before the first step: infinity
   #pragma unroll 1
   for (int i = 0; i < steps; ++i) {
     const float p = shrink[i];
@@ -253,21 +275,55 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
     const float s = prm.s * up, r = prm.r * down;
     const auto add = [&](float w, float sum) {
       const float q = __builtin_amdgcn_fmed3f(rintf(w * r), prm.lo, prm.hi);
-      const float d = q * s - w;
+      const float d = q * s - w;                             // (both operations rounded, as in deq)
       return __builtin_fmaf(d * d, __builtin_amdgcn_exp2f(frac * __builtin_amdgcn_logf(fabsf(d))), sum);
     };
-    if (__all(fmaxf(add(top, 0.0f), add(bottom, 0.0f)) > best)) continue;      // (a workgroup's lanes all hold the same two)
+    if (__all(fmaxf(add(top, 0.0f), add(bottom, 0.0f)) > hi)) continue;        // (a workgroup's lanes all hold the same two)
     float err = 0.0f, sum = 0.0f;
     #pragma unroll
     for (int quarter = 0; quarter < 4; ++quarter) {
       #pragma unroll
       for (int j = quarter * (PER / 4); j < (quarter + 1) * (PER / 4); ++j) err = add(v[j], err);
       sum = row_sum(err);
-      if (quarter < 3 && __all(sum > best)) break;
+      if (quarter < 3 && __all(sum > hi)) break;
     }
-    if (sum < best) { best = sum; cur_min = xmin; cur_max = xmax; }
+    bool better = sum < lo;
+    const bool close = live && !better && !(sum > hi) && !(prm.s == best_s && prm.z == best_z);
+    float exact = 0.0f;
+    for (uint64_t need = __ballot(close && lane % SUB == 0); need; need &= need - 1) {
+      const int src = __builtin_ctzll(need);
+      const auto of = [&](float f) { return u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(f), src)); };
+      const int64_t r_ = BLOCK ? (int64_t)blockIdx.x : ((int64_t)blockIdx.x * 256 + (threadIdx.x & ~63) + src) / TEAM;
+      const float en = mse_row_error<BF>(x, r_, cols, op.make(of(xmin), of(xmax)), norm, op, lane);
+      float eb = of(best);
+      if (!__builtin_amdgcn_readlane((int)have, src)) eb = mse_row_error<BF>(x, r_, cols, op.make(of(cur_min), of(cur_max)), norm, op, lane);
+      if (lane / SUB == src / SUB) { exact = en; best = eb; have = true; }
+    }
+    if (close) better = exact < best;
+    if (better) {
+      cur_min = xmin; cur_max = xmax;
+      best_s = prm.s; best_z = prm.z;
+      have = close;
+      if (close) best = exact;
+      if (regular) {
+        hi = live ? fmaxf(sum * (1.0f + margin), MSE_SMALL) : -1.0f;
+        lo = sum >= MSE_SMALL ? sum * (1.0f - margin) : -__builtin_inff();
+      }
+    }
   }
-  if (t == 0 && row_ < rows) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
+  if (t == 0 && live) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
+}
+
+// Two estimates that differ by more than this tell which of the two errors is larger.  delta bounds the relative difference
+// between an estimate and mse_row_error:
+//   powers   v_log is good to an ulp of |log2 d| < 32 (2^-19), times norm - 2; d^2, v_exp and powf to an ulp each;
+//   ties     where x * (1/s) and x / s round to different integers, |x/s| is within |x/s| 2^-22 of a half-integer and both
+//            errors are s / 2 to (levels + 1) 2^-19.5, levels = qmax - qmin >= |x/s| - 1/2; norm times that for the power;
+//   sums     of non-negative terms: 2^-24 for every addition a term goes through, in either order.
+// (1 + delta) / (1 - delta) on either side: 2.5 delta.
+float mse_margin(int64_t cols, int per, float levels, float norm) {
+  const float delta = (norm - 1.0f) * 1.9073486e-6f + 5e-7f + norm * (levels + 1.0f) * 1.35e-6f + (float)(cols / 64 + per + 16) * 6e-8f;
+  return 2.5f * delta;
 }
 
 template <int BF>
@@ -276,9 +332,10 @@ int run_mse(const void* x, int64_t rows, int64_t cols, int steps, int grid_n, fl
   constexpr int N = Vec<BF>::N;
   const int vec = cols % N == 0 && (uintptr_t)x % 16 == 0;
   #define LCQ_MSE(T, P) do { const int64_t grid = (rows * T + 255) / 256; if (grid > 0x7fffffff) return LCQ_EINVAL; \
-    mse_range_team_kernel<BF, T, P><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, (int)cols, vec, steps, grid_n, norm, op, min_out, max_out); \
+    mse_range_team_kernel<BF, T, P><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, (int)cols, vec, steps, grid_n, norm, \
+        mse_margin(cols, P, op.qrange, norm), op, min_out, max_out); \
     return LCQ_OK; } while (0)
-  if (op.round_zp && op.qmin <= 0.0f && op.qmax >= 0.0f && norm > 2.0f && norm <= 4.0f && steps <= 256) {
+  if (op.round_zp && op.qmin <= 0.0f && op.qmax >= 0.0f && op.qrange <= 512.0f && norm > 2.0f && norm <= 4.0f && steps <= 256) {
     // Many elements per lane amortise the step's row arithmetic, but below 20000 rows such waves are too few to fill the
     // chip and their 80 steps one after the other are what takes the time: rows of 128 on 16 / 2 lanes take 34 / 68 us at
     // 4096 rows, 60 / 67 at 16384, 98 / 69 at 32768

@@ -870,6 +870,32 @@ def test_mse_range_at_the_edges_of_its_lane_layouts(dev, rows, cols, dtype, bit,
     assert_bit_equal(got, Q.int_quant_dequant(spec, w.float(), s, z, qmax, qmin).to(dtype), 'fake quant with the mse ranges')
 
 
+@pytest.mark.parametrize('rows,cols,dtype,bit,sym,seed', [
+    (32768, 128, torch.bfloat16, 4, True, 0), (32768, 128, torch.float32, 4, True, 11), (32768, 64, torch.float16, 2, False, 1),
+    (8192, 32, torch.bfloat16, 2, False, 9), (16001, 128, torch.float16, 4, True, 0), (4096, 512, torch.float16, 2, False, 0),
+    (1500, 4096, torch.bfloat16, 4, False, 0), (300, 4104, torch.bfloat16, 8, False, 0), (515, 100, torch.float32, 8, False, 0)])
+def test_mse_range_is_the_one_of_the_re_reading_kernel(dev, rows, cols, dtype, bit, sym, seed):
+    """The kernels that hold a row in registers decide every step as the re-reading kernel does, near-ties included (the
+    first four matrices hold rows where an estimate of the error that is off by 1e-6 decides otherwise).  That kernel takes
+    rows beyond 16384 columns, so the same rows padded with zeros show its decisions: a zero quantizes to itself (no
+    error), and every row has both signs (same range).  Rows of few distinct values, of extreme sizes, with an infinity or
+    a NaN, and zeros."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    w = torch.randn(rows, cols, generator=g, device=dev) * 0.02
+    w = torch.round(w * 200) / 200
+    w[:, 0], w[:, 1] = w[:, 0].abs(), -w[:, 1].abs()
+    w[:64] *= torch.exp2(torch.arange(-40, 24, device=dev).float())[:, None]
+    w[-4, 3], w[-3, 5], w[-2, 7] = float('nan'), float('inf'), -float('inf')
+    w[-1] = 0
+    w = w.to(dtype)
+    q = _iq(bit, sym, 'per_channel', calib_algo='mse')
+    wide = torch.zeros(rows, 16392, dtype=dtype, device=dev)
+    wide[:, :cols] = w
+    want = q.get_mse_range(wide)
+    for got, o, name in zip(q.get_mse_range(w), want, ('min', 'max')):
+        assert_bit_equal(got, o.cpu(), name)
+
+
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize('bit,sym,shape,g', [(4, False, (64, 512), 128), (8, True, (33, 256), 64), (8, False, (7, 96), 32),
                                              (4, True, (5, 1000), 0), (8, True, (3, 1001), 0)])
