@@ -819,13 +819,16 @@ class IntegerQuantizer(BaseQuantizer):
         return self._finish_real(codes, scales, zeros, output_scale_factor)
 
     def _can_pack(self, weight):
-        """May `_pack_dynamic` stand for real_quant_weight_dynamic and a pack?  Symmetric 4- or 8-bit min/max codes of a 2-D
-        weight whose rows fill whole 16-byte chunks (the nibbles / bytes then leave the quantizer's kernel in place)."""
+        """May `_pack_dynamic` stand for real_quant_weight_dynamic and a pack?"""
+        return self.granularity in ('per_group', 'per_channel') and self._packs_in_place(weight)
+
+    def _packs_in_place(self, weight):
+        """Symmetric 4- or 8-bit min/max codes of a 2-D weight whose rows fill whole 16-byte chunks: the nibbles / bytes can
+        leave the quantizer's kernel where a pack of its codes would put them."""
         lo, hi = (-8, 7) if self.bit == 4 else (-128, 127)
         cols = self.group_size if self.granularity == 'per_group' else weight.shape[-1]
         return (self.bit in (4, 8) and self.sym and self.calib_algo == 'minmax' and self.round_zp
-                and self.granularity in ('per_group', 'per_channel') and weight.dim() == 2
-                and weight.shape[1] % 8 == 0 and cols % 8 == 0 and weight.dtype in (torch.bfloat16, torch.float16, torch.float32)
+                and weight.dim() == 2 and weight.shape[1] % 8 == 0 and cols % 8 == 0 and weight.dtype in (torch.bfloat16, torch.float16, torch.float32)
                 and lo <= float(self.qmin) and float(self.qmax) <= hi and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
     def _pack_dynamic(self, weight, scales_dtype):
@@ -842,20 +845,32 @@ class IntegerQuantizer(BaseQuantizer):
         return packed, scales
 
     def real_quant_pack_dynamic(self, weight):
-        """Quantize and pack in one pass: what VllmRealQuantLinear.pack(*real_quant_weight_dynamic(w)[:2])
-        returns for a symmetric 4-bit quantizer (module_utils.py:929-955 after quant.py:915-952), without
-        the int32 codes ever reaching HBM -> (int32 [R, K/8], scales [R, -1], None)."""
+        """Quantize and pack in one call: what VllmRealQuantLinear.pack(*real_quant_weight_dynamic(w)[:2]) returns for a
+        symmetric 4-bit quantizer (module_utils.py:929-955 after quant.py:915-952), the scales in their own type
+        -> (int32 [R, K/8], scales [R, -1], None).  Min/max ranges of rows that fill whole 16-byte chunks take one launch and
+        the int32 codes never reach HBM; everything else (calibrated ranges, short groups) is quantized, then packed."""
         if self.bit != 4 or not self.sym or weight.dim() != 2 or weight.shape[1] % 8 != 0:
             raise NotImplementedError('fused quantize+pack: symmetric 4-bit, 2-D weight, in_features % 8 == 0')
-        rows_t = self.reshape_tensor(weight)
-        _, packed, scales, _ = self._launch(rows_t, static=False, want_codes='ct4')
-        qparams_shape = 1 if self.granularity == 'per_tensor' else (weight.shape[0], -1)
-        return packed.view(weight.shape[0], weight.shape[1] // 8), scales.view(qparams_shape), None
+        weight = weight.contiguous()
+        if self._can_pack(weight):
+            return (*self._pack_dynamic(weight, weight.dtype), None)
+        if self.granularity == 'per_tensor' and self._packs_in_place(weight):
+            _, packed, scales, _ = self._launch(weight, static=False, want_codes='ct4')
+            return packed.view(weight.shape[0], weight.shape[1] // 8), scales.view(1), None
+        codes, scales, _ = self.real_quant_weight_dynamic(weight)
+        cd = {torch.int32: L.CODE_I32, torch.int8: L.CODE_I8, torch.uint8: L.CODE_U8}[codes.dtype]
+        packed = torch.empty((weight.shape[0], weight.shape[1] // 8), dtype=torch.int32, device=weight.device)
+        L.check(L.lib().lcq_pack_ct(L.ptr(codes.contiguous()), cd, weight.shape[0], weight.shape[1], 4, L.ptr(packed),
+                                    L.stream()), 'lcq_pack_ct')
+        return packed, scales, None
 
     def real_quant_pack_dynamic_experts(self, weights):
-        """real_quant_pack_dynamic of every matrix in `weights` with one launch -> list of (packed, scales, None)."""
+        """real_quant_pack_dynamic of every matrix in `weights` with one launch -> list of (packed, scales, None).  (hqq stops
+        on the mean error of its matrix: one after the other.)"""
         if self.granularity not in ('per_channel', 'per_group'):
             raise NotImplementedError('experts are stacked along the rows: per_channel / per_group only')
+        if self.calib_algo == 'hqq':
+            return [self.real_quant_pack_dynamic(w) for w in weights]
         E, (R, K) = len(weights), weights[0].shape
         packed, scales, _ = self.real_quant_pack_dynamic(experts_as_rows(weights))
         ps, ss = packed.view(E, R, -1), scales.view(E, R, -1)

@@ -171,6 +171,38 @@ def test_vllm_new_with_the_rtn_partial_packs_in_one_launch(dev, dtype, bit, g, R
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('gran,kw,R,K,layout', [
+    ('per_group', dict(group_size=64, calib_algo='mse'), 32, 256, 'plain'), ('per_channel', dict(calib_algo='hqq'), 24, 264, 'plain'),
+    ('per_group', dict(group_size=4), 8, 64, 'plain'), ('per_group', dict(group_size=12), 5, 96, 'plain'),
+    ('per_channel', dict(round_zp=False), 9, 128, 'plain'), ('per_group', dict(group_size=32), 7, 128, 'offset'),
+    ('per_group', dict(group_size=32), 64, 32, 'transposed'), ('per_tensor', {}, 6, 40, 'plain'), ('per_group', dict(group_size=128), 9, 256, 'plain')])
+def test_quantize_and_pack_is_the_two_steps(dev, dtype, gran, kw, R, K, layout):
+    """real_quant_pack_dynamic (and the container's quant_pack_fused) for ranges, groups and layouts with and without a kernel
+    that packs: words and scales of real_quant_weight_dynamic followed by a pack, bit for bit; experts like their own call."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.module_utils import VllmRealQuantLinear
+    w = weight_like(R, K, seed=R + K, dtype=dtype, outlier_frac=0.02).to(dev)
+    if layout == 'offset':                                   # two bytes (fp32: four) off the 16-byte boundary
+        w = torch.cat([w.flatten()[:1], w.flatten()])[1:].view(R, K)
+    elif layout == 'transposed':
+        w = w.T.contiguous().T
+    q = IntegerQuantizer(4, True, gran, **kw)
+    cfg = {'weight': dict(bit=4)}
+    codes, scales, _ = q.real_quant_weight_dynamic(w)
+    words, s16 = VllmRealQuantLinear.pack(codes, scales, cfg)
+    got, gs, _ = q.real_quant_pack_dynamic(w)
+    assert_bit_equal(got, words, 'words')
+    assert_bit_equal(gs, scales, 'scales')
+    got, gs = VllmRealQuantLinear.quant_pack_fused(w, q, cfg)
+    assert_bit_equal(got, words, 'quant_pack_fused words')
+    assert_bit_equal(gs, s16, 'quant_pack_fused scales')
+    if gran != 'per_tensor':
+        for (a, b, _), e in zip(q.real_quant_pack_dynamic_experts([w, 2 * w]), (w, 2 * w)):
+            one = q.real_quant_pack_dynamic(e)
+            assert torch.equal(a, one[0]) and torch.equal(b, one[1])
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize('g,R,K', [(128, 32, 128), (128, 288, 256), (64, 544, 192), (32, 1056, 64), (16, 64, 64)])
 def test_autoawq_new_with_the_rtn_partial(dev, dtype, g, R, K):
     """Scales, zero points and nibbles in one launch (groups of 16: the two steps), where octets of rows fill workgroups and
