@@ -51,11 +51,12 @@ extern "C" {
 #define LCQ_CODE_SAME 4      /* codes stored as floats of the input type (what .quant() returns) */
 #define LCQ_CODE_F32 5       /* FloatQuantizer.quant(): fp32 values on the minifloat grid */
 #define LCQ_CODE_FP8 6       /* float8_e4m3fn / float8_e5m2 bytes */
-#define LCQ_CODE_CT8 8       /* lcq_quant_int: the same for 8-bit codes: byte i of word j = code[4j+i] + 128 (codes in -128 .. 127); `codes`
-                                is int32 [rows * cols / 4] */
 #define LCQ_CODE_CT4 7       /* lcq_quant_int: 4-bit codes packed like VllmRealQuantLinear.pack (module_utils.py:929-955):
                                 nibble i of int32 word j of a tensor row = code[8j+i] + 8; needs -8 <= qmin, qmax <= 7
-                                and cols % 8 == 0; `codes` is int32 [rows * cols / 8] */
+                                and cols % 8 == 0, x and dq 16-byte aligned, rounded zero points; `codes` is int32
+                                [rows * cols / 8] */
+#define LCQ_CODE_CT8 8       /* lcq_quant_int: the same for 8-bit codes: byte i of word j = code[4j+i] + 128; needs -128 <= qmin,
+                                qmax <= 127 and cols % 4 == 0; `codes` is int32 [rows * cols / 4], any alignment */
 
 /* flags */
 #define LCQ_FLAG_SYM 1            /* symmetric: zero point is 0 */

@@ -412,7 +412,7 @@ int lcq_quant_int(const void* x, int dtype, int64_t rows, int64_t cols, float qm
     if (qmin < -8.0f || qmax > 7.0f || (flags & LCQ_FLAG_NO_ROUND_ZP) || cols % 8 != 0) return LCQ_EINVAL;
     if ((((uintptr_t)x | (uintptr_t)dq) % 16) != 0 || ((uintptr_t)codes % 4) != 0) return LCQ_EALIGN;
   }
-  if (codes && code_dtype == LCQ_CODE_CT8 && (qmin < -128.0f || qmax > 127.0f)) return LCQ_EINVAL;
+  if (codes && code_dtype == LCQ_CODE_CT8 && (qmin < -128.0f || qmax > 127.0f || cols % 4 != 0)) return LCQ_EINVAL;
   if ((flags & LCQ_FLAG_SCALES_F16) && (flags & LCQ_FLAG_STATIC)) return LCQ_EINVAL;
   if ((flags & LCQ_FLAG_SCALAR_QP) && !(flags & LCQ_FLAG_STATIC)) return LCQ_EINVAL;
   if ((flags & LCQ_FLAG_SCALE_F32) && !(flags & LCQ_FLAG_STATIC)) return LCQ_EINVAL;

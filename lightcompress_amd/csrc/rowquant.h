@@ -192,6 +192,7 @@ __device__ __forceinline__ void store_code1(const Op& op, void* codes, int64_t e
   if (cd == LCQ_CODE_I32) ((int32_t*)codes)[e] = (int32_t)q;
   else if (cd == LCQ_CODE_F32) ((float*)codes)[e] = q;
   else if (cd == LCQ_CODE_U8 || cd == LCQ_CODE_I8 || cd == LCQ_CODE_FP8) ((uint8_t*)codes)[e] = (uint8_t)op.byte(q);
+  else if (cd == LCQ_CODE_CT8) ((uint8_t*)codes)[e] = (uint8_t)(op.byte(q) ^ 0x80u);
   else if (cd == LCQ_CODE_SAME) store_scalar<Op::BF>(codes, e, q);
 }
 

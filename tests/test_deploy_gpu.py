@@ -203,6 +203,30 @@ def test_quantize_and_pack_is_the_two_steps(dev, dtype, gran, kw, R, K, layout):
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('rows,cols,x_off,c_off,flags', [(5, 16, 0, 0, 0), (5, 12, 0, 0, 0), (3, 4, 0, 0, 0), (7, 64, 1, 0, 0),
+                                                         (7, 64, 0, 4, 0), (6, 32, 0, 0, 2), (4, 13, 0, 0, 0)])
+def test_packed_bytes_for_every_form_the_entry_point_takes(dev, dtype, rows, cols, x_off, c_off, flags):
+    """LCQ_CODE_CT8 where rows fill 16-byte chunks and where they do not, off the 16-byte boundary and with round_zp=False
+    (flag 2): the signed codes plus 128 in every byte; a row that ends inside a word is refused."""
+    import lightcompress_amd._lib as L
+    x = weight_like(rows + 1, cols, seed=rows + cols, dtype=dtype).to(dev).flatten()[x_off:x_off + rows * cols]
+    scales = torch.empty(rows, dtype=dtype, device=dev)
+
+    def run(code, out):
+        return L.lib().lcq_quant_int(x.data_ptr(), L.dtype_code(dtype), rows, cols, -128.0, 127.0, L.FLAG_SYM | flags, 1.0, None,
+                                     out.data_ptr(), code, scales.data_ptr(), None, L.stream())
+    buf = torch.full((rows * cols + 16,), 0x5a, dtype=torch.uint8, device=dev)
+    out = buf[c_off:c_off + rows * cols]
+    if cols % 4:
+        assert run(L.CODE_CT8, out) == -1
+        return
+    signed = torch.empty(rows * cols, dtype=torch.int8, device=dev)
+    assert run(L.CODE_CT8, out) == 0 and run(L.CODE_I8, signed) == 0
+    assert torch.equal(out.int(), signed.int() + 128)
+    assert bool((buf[:c_off] == 0x5a).all()) and bool((buf[c_off + rows * cols:] == 0x5a).all())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize('g,R,K', [(128, 32, 128), (128, 288, 256), (64, 544, 192), (32, 1056, 64), (16, 64, 64)])
 def test_autoawq_new_with_the_rtn_partial(dev, dtype, g, R, K):
     """Scales, zero points and nibbles in one launch (groups of 16: the two steps), where octets of rows fill workgroups and
