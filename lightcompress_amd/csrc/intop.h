@@ -62,10 +62,11 @@ struct IntOp {
     p.r = __builtin_amdgcn_rcpf(s);      // 1 ulp: inside the error the exactness guards of x * r allow for
     const float a = fabsf(s);
     p.fast = (a > 8.6736174e-19f) && (a < 1.1529215e18f) && (fabsf(z) <= 512.0f);   // s in 2^-60 .. 2^60
-    // caller-given zero points need not be integers; a row whose scale is infinite or NaN (an infinite or NaN weight)
-    // takes the element-wise form too, which hands NaN codes on like torch.clamp does
-    p.zint = (z == rintf(z)) && (fabsf(z) <= 512.0f) && (a < __builtin_inff());
     p.sdq = rnd<BF>(s * osf);
+    // caller-given zero points need not be integers; a row whose scale is infinite or NaN (an infinite or NaN weight), zero
+    // (0 / 0; the clamp range of an fp16 row may come to that) or negative takes the element-wise form too, which hands
+    // NaN codes on like torch.clamp does and leaves the sign of a product that is zero alone
+    p.zint = (z == rintf(z)) && (fabsf(z) <= 512.0f) && (a < __builtin_inff()) && (p.sdq > 0.0f);
     p.lo = qmin - z; p.hi = qmax - z;                       // exact: small integers
     p.clo = RINT_BIAS_BITS + (int)p.lo; p.chi = RINT_BIAS_BITS + (int)p.hi;
     p.nib0 = (uint32_t)(RINT_BIAS_BITS - ((int)z + 8)) * 0x11111111u;

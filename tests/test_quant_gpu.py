@@ -915,6 +915,26 @@ def test_static_fp32_parameters_of_16_bit_rows(dev, dtype, bit, sym, shape, g):
     assert_bit_equal(codes, Q.int_real_quant_static(spec, w, s, z, q.qmax, q.qmin)[0], 'codes')
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('cols', [256, 3072, 33])
+def test_zero_and_negative_scales_under_given_parameters(dev, dtype, cols):
+    """0 / 0 is NaN and torch.clamp hands it on; (q - z) * s keeps the sign of a zero product.  Zero, negative and ordinary
+    scales side by side, per row and as one scalar, bit for bit (NaN at the same places)."""
+    w = weight_like(6, cols, seed=cols, dtype=dtype, std=0.5)
+    w[:, ::5] = 0
+    for bit, sym in ((8, False), (4, True)):
+        for gran, s in (('per_channel', torch.tensor([[0.02], [0.0], [-0.02], [0.05], [-0.0], [1e-6]])), ('per_tensor', torch.tensor(0.0)),
+                        ('per_tensor', torch.tensor(-0.04))):
+            spec, q = Q.IntSpec(bit, sym, gran), _iq(bit, sym, gran)
+            s = s.to(dtype) if gran == 'per_channel' else s
+            z = torch.tensor(0.0) if sym else torch.full_like(s, 100.0)
+            args = {'scales': s.to(dev), 'zeros': z if sym else z.to(dev), 'qmax': q.qmax, 'qmin': q.qmin}
+            want = Q.int_fake_quant_static(spec, w, s, z, q.qmax, q.qmin)
+            got = q.fake_quant_weight_static(w.to(dev), dict(args)).cpu()
+            assert torch.equal(got.isnan(), want.isnan())
+            assert_bit_equal(got.masked_fill(got.isnan(), 1), want.masked_fill(want.isnan(), 1), f'{bit} {sym} {gran}')
+
+
 @pytest.mark.parametrize('kind', ['int8_asym', 'int4_sym', 'e4m3', 'e5m2', 'e4m3_even', 'e5m2_even'])
 def test_every_finite_fp16_value_under_many_scales(dev, kind):
     """The vectorised fp16 rows (reciprocal quotients with a guard, packed conversions, hardware float8 rounding) on all
