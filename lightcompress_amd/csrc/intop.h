@@ -209,13 +209,27 @@ struct IntOp {
     for (int i = 0; i < N; i += 2) rnd_pair<BF>(t[i], t[i + 1]);
   }
 
+  // Does this chunk take the element-wise form?  med3 turns a NaN into a bound, torch.clamp hands it on.  A NaN in a row
+  // that gave the parameters itself leaves no finite scale, so only given parameters look at the elements.
+  template <int N>
+  __device__ __forceinline__ bool general(const float* x, const Row& p) const {
+    bool g = !p.zint;
+    if (is_static) {
+      float m = nan_max(x[0], x[1]);
+      #pragma unroll
+      for (int i = 2; i < N; i += 2) m = nan_max(nan_max(m, x[i]), x[i + 1]);
+      g = g || m != m;
+    }
+    return g;
+  }
+
   template <int N>
   __device__ __forceinline__ void codes(const float* x, float* q, const Row& p) const {
     if constexpr (!FAST) {
       #pragma unroll
       for (int i = 0; i < N; ++i) q[i] = code(x[i], p);
     } else {
-      if (__builtin_expect(!p.zint, 0)) {
+      if (__builtin_expect(general<N>(x, p), 0)) {
         #pragma unroll
         for (int i = 0; i < N; ++i) q[i] = code(x[i], p);
         return;
@@ -251,7 +265,7 @@ struct IntOp {
   // that (q - z) gives.  The products are left unrounded: the caller rounds to the row type while packing.
   template <int N>
   __device__ __forceinline__ void fused_dq(const float* x, float* d, const Row& p) const {
-    if (__builtin_expect(!p.zint, 0)) {
+    if (__builtin_expect(general<N>(x, p), 0)) {
       #pragma unroll
       for (int i = 0; i < N; ++i) d[i] = deq_raw(code(x[i], p), p);
       return;

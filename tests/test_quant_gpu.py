@@ -935,6 +935,36 @@ def test_zero_and_negative_scales_under_given_parameters(dev, dtype, cols):
             assert_bit_equal(got.masked_fill(got.isnan(), 1), want.masked_fill(want.isnan(), 1), f'{bit} {sym} {gran}')
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('cols', [256, 3072, 33])
+@pytest.mark.parametrize('qp', ['row', 'row_f32', 'scalar'])
+def test_nan_under_given_parameters_is_handed_on(dev, dtype, cols, qp):
+    """torch.clamp keeps a NaN, so a NaN element comes out as NaN under static parameters
+    while its neighbours and the infinities are quantized: fake quantization of weights and activations, float codes."""
+    w = weight_like(9, cols, seed=cols, dtype=dtype, std=0.5)
+    w[0, 5], w[3, cols - 1], w[4, 0], w[4, 8], w[5, 2], w[6, 3] = (float('nan'),) * 4 + (float('inf'), -float('inf'))
+    gran = 'per_tensor' if qp == 'scalar' else 'per_channel'
+    for bit, sym in ((8, False), (4, True)):
+        spec, q = Q.IntSpec(bit, sym, gran), _iq(bit, sym, gran)
+        s = torch.tensor(0.03) if qp == 'scalar' else (torch.rand(9, 1, generator=gen(3)) * 0.02 + 0.01)
+        if qp != 'scalar':
+            s[7] = 0
+        if qp == 'row':
+            s = s.to(dtype)
+        z = torch.tensor(0.0) if sym else torch.full_like(s, 100.0)
+        args = {'scales': s.to(dev), 'zeros': z if sym else z.to(dev), 'qmax': q.qmax, 'qmin': q.qmin}
+        want = Q.int_fake_quant_static(spec, w, s, z, q.qmax, q.qmin)
+        got = [q.fake_quant_weight_static(w.to(dev), dict(args)).cpu(),
+               q.fake_quant_act_static(w.to(dev)[None], dict(args))[0].cpu()]
+        if qp != 'row_f32':
+            codes = q.quant(w.to(dev), s.to(dev), args['zeros'], q.qmax, q.qmin).cpu()
+            got.append(((codes - z) * s).to(dtype) if qp == 'row' else None)
+        for g in got:
+            if g is not None:
+                assert torch.equal(g.isnan(), want.isnan()) and bool(want.isnan().any())
+                assert_bit_equal(g.nan_to_num(9.0, 1e3, -1e3), want.nan_to_num(9.0, 1e3, -1e3), f'{bit} {sym}')
+
+
 @pytest.mark.parametrize('kind', ['int8_asym', 'int4_sym', 'e4m3', 'e5m2', 'e4m3_even', 'e5m2_even'])
 def test_every_finite_fp16_value_under_many_scales(dev, kind):
     """The vectorised fp16 rows (reciprocal quotients with a guard, packed conversions, hardware float8 rounding) on all
