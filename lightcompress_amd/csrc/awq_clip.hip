@@ -236,6 +236,37 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
   }
 }
 
+// One row of A in add_pairs holds two weight rows (lanes m and m + 16), kept apart by the zeros of B, and 0 * infinity is NaN:
+// an infinite or NaN product (an infinite or NaN weight, a product beyond the largest bf16 number) turns the sums of its
+// partner row 16 rows away into NaN as well.  So a lane with a sum that is not finite adds its products up again one by one:
+// x: the group's columns of token 0, w: the tile's rows in LDS.  Off the path of finite tiles, which pay for the test alone.
+template <int GS>
+__device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __restrict__ x, int64_t K, int t0, int T, const char* w,
+                                                              int lane, f32x4* sum) {
+  float m = 0.0f;
+  #pragma unroll
+  for (int q = 0; q < 4; ++q)
+    #pragma unroll
+    for (int i = 0; i < 4; i += 2) m = nan_max(nan_max(m, fabsf(sum[q][i])), fabsf(sum[q][i + 1]));
+  if (__builtin_expect(m < __builtin_inff(), 1)) return;
+  const char* wr = w + (16 * ((lane >> 2) & 1) + 4 * (lane >> 4)) * gd_pitch<GS>();
+  const int tok = t0 + 4 * ((lane >> 3) & 1) + (lane & 3);
+  #pragma unroll
+  for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  #pragma unroll 1
+  for (int j = 0; j < GS; ++j) {
+    float wv[4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) wv[i] = u2f((uint32_t)*(const uint16_t*)(wr + i * gd_pitch<GS>() + 2 * j) << 16);
+    #pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float xv = tok + 8 * q < T ? u2f((uint32_t)x[(int64_t)(tok + 8 * q) * K + j] << 16) : 0.0f;
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) sum[q][i] += rnd<true>(xv * wv[i]);
+    }
+  }
+}
+
 // The whole search of AutoClipper.auto_clip_layer (v1, weight-only, bf16, groups of GS columns) in one launch: a workgroup
 // owns 32 rows of one group, keeps the original and the n_steps clamped-and-quantized versions of them in LDS, and every
 // wave runs all versions over its 32-token tiles; neither the candidates nor the [R, G, T] products reach memory.
@@ -286,6 +317,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
     for (int c = 0; c < GS / 8; ++c) { a[c] = *(const u32x4*)(xr + 8 * c); if (!ok) a[c] = u32x4{0, 0, 0, 0}; }
     f32x4 org[4], cur[4];
     dots_tile<ROW_BF16, GS>(a, wrow, mask, ones, org);
+    redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem, lane, org);
     #pragma unroll
     for (int q = 0; q < 4; ++q)
       #pragma unroll
@@ -297,6 +329,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
     #pragma unroll 1
     for (int s = 0; s < n_steps; ++s) {
       dots_tile<ROW_BF16, GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
+      redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem + (s + 1) * VERSION, lane, cur);
       float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       #pragma unroll
       for (int q = 0; q < 4; ++q)

@@ -428,6 +428,38 @@ def test_auto_clip_one_launch_search_at_tile_edges(dev, gs, T, bit, sym, clip_sy
     assert torch.equal(bmax.cpu()[same], obmax[same]) and torch.equal(bmin.cpu()[same], obmin[same])
 
 
+@pytest.mark.parametrize('gs,clip_sym', [(128, False), (64, True), (32, False)])
+def test_auto_clip_one_launch_search_keeps_rows_apart(dev, gs, clip_sym):
+    """An infinite or NaN weight, and a finite one whose products overflow, spoil their own row of their group only: every
+    other range is the one of the step-by-step path (as far as the errors tell the steps apart, see above), and the spoilt
+    rows keep their whole range there and here."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    R, K, T = 128, 4 * gs, 40
+    w = weight_like(R, K, seed=gs, dtype=torch.bfloat16)
+    x = (torch.randn(T, K, generator=gen(gs)) * torch.exp(0.5 * torch.randn(K, generator=gen(K)))).bfloat16()
+    w[3, 5], w[52, gs + 7], w[71, 2 * gs] = float('inf'), float('nan'), -float('inf')
+    w[9, 3 * gs + 1], x[33, 3 * gs + 1] = 2e35, 3e3          # both finite, the product is not
+    clipper = AutoClipper(True, IntegerQuantizer(4, False, 'per_group', group_size=gs), None, 'v1', clip_sym, False, None)
+    w, x = w.to(dev), x.to(dev)
+    assert clipper._fused_applies(w, [x], 10)
+    bmax, bmin = clipper.auto_clip_layer(0, 'fc', w, [x.clone()], n_sample_token=T)
+    errs = clipper.last_errs
+    omax, omin = clipper._search_exact(0, 'fc', w, [x], gs, 20, 10, 0.0)
+    oe = clipper.last_errs
+    spoilt = torch.zeros(R, 4, dtype=torch.bool, device=dev)
+    spoilt[3, 0] = spoilt[52, 1] = spoilt[71, 2] = spoilt[9, 3] = True
+    assert bool(oe[~spoilt].isfinite().all()) and not bool(oe[spoilt].isfinite().any())
+    assert not bool(errs[spoilt].isfinite().any())
+    assert bool(((errs - oe).abs() <= 2 * 2.0 ** -7 * oe)[~spoilt].all())
+    same = ((errs == oe).all(-1) | spoilt)
+    assert float(same.float().mean()) > 0.95
+    for got, want in ((bmax, omax), (bmin, omin)):
+        got, want = got[..., 0][same], want[..., 0][same]
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~got.isnan()], want[~want.isnan()])
+
+
 def test_auto_clip_run_skips_query_key_and_handles_float8_weights(dev):
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
