@@ -72,7 +72,7 @@ __global__ __launch_bounds__(512, 1) void awq_clip_kernel(const uint16_t* __rest
 
   if (npass == 1) { load_tokens(0); __syncthreads(); }
 
-  float best = 999817216.0f;                                // bf16(1e9), min_errs = ones_like * 1e9
+  float best = 998244352.0f;                                // bf16(1e9), min_errs = ones_like * 1e9
   float bmax = org_max, bmin = org_min;
   for (int s = 0; s < n_steps; ++s) {
     const float fs = (float)(1.0 - (double)s / (double)n_grid);
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
     float mn = __builtin_inff(), mx = -__builtin_inff();
     for (int c = 0; c < TEAM; ++c) chunk_minmax<IntOp<true, true>>(*(const u32x4*)(smem + row * PITCH_W + c * 16), mn, mx);
     const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
-    float best = 999817216.0f, bmax = org_max, bmin = mn;                 // bf16(1e9)
+    float best = 998244352.0f, bmax = org_max, bmin = mn;                 // bf16(1e9)
     const int64_t at = (int64_t)(r0 + row) * G + g;
     for (int s = 0; s < n_steps; ++s) {
       float e = 0.0f;

@@ -460,6 +460,26 @@ def test_auto_clip_one_launch_search_keeps_rows_apart(dev, gs, clip_sym):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~got.isnan()], want[~want.isnan()])
 
 
+@pytest.mark.parametrize('gs,fast', [(32, False), (128, False), (128, True)])
+def test_auto_clip_error_equal_to_the_starting_value_does_not_win(dev, gs, fast):
+    """min_errs starts as ones * 1e9 in the tensors' type, 998244352 in bf16, and a step wins below it only.  One token picks
+    column 0, so a row's error is the square of one difference: these two weights give 1048576000 and 998244352."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    w = torch.zeros(64, gs)
+    w[0, 0], w[0, 1] = 32384, 1007616
+    x = torch.zeros(1, gs)
+    x[0, 0] = 1
+    w, x = w.bfloat16(), x.bfloat16()
+    obmax, _, oerrs = A.auto_clip_layer(Q.IntSpec(4, False, 'per_group', group_size=gs), w, [x.clone()], max_shrink=0.1, n_sample_token=1)
+    assert oerrs.float()[0].flatten().tolist() == [1048576000.0, 998244352.0] and float(obmax[0, 0]) == 1007616
+    clipper = AutoClipper(True, IntegerQuantizer(4, False, 'per_group', group_size=gs), None, 'v1', False, False, None)
+    clipper.fast = fast
+    bmax, _ = clipper.auto_clip_layer(0, 'fc', w.to(dev), [x.to(dev)], max_shrink=0.1, n_sample_token=1)
+    assert clipper.last_errs[0].bfloat16().flatten().tolist() == [1048576000.0, 998244352.0]     # (the fast search compares this too)
+    assert float(bmax[0, 0]) == 1007616
+
+
 def test_auto_clip_run_skips_query_key_and_handles_float8_weights(dev):
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
