@@ -129,15 +129,16 @@ class AutoClipper:
                 raise NotImplementedError('inputs of different token counts: the per-input means are not one mean '
                                           '(use fast = False)')
             return self._search_mfma(wc, torch.cat(xs) if len(xs) > 1 else xs[0], n_grid, n_steps)
-        if self._fused_applies(wc, xs, n_steps):
+        if self._fused_applies(wc, xs, n_steps, n_grid):
             return self._search_fused(wc, xs[0], group_size, n_grid, n_steps)
         return self._search_exact(block_idx, layer_name, wc, xs, group_size, n_grid, n_steps, eps)
 
-    def _fused_applies(self, w, xs, n_steps):
+    def _fused_applies(self, w, xs, n_steps, n_grid=20):
         """lcq_clip_search_exact: one launch with the same roundings as _search_exact, for bf16 tensors, v1, weight-only,
-        groups of 32 / 64 / 128, one input and the min/max integer quantizer."""
+        groups of 32 / 64 / 128, one input, the min/max integer quantizer and whole steps that do not shrink past zero."""
         wq = self.wquantizer
-        return (self.clip_version == 'v1' and self.w_only and len(xs) == 1 and 0 < n_steps <= 12
+        return (self.clip_version == 'v1' and self.w_only and len(xs) == 1
+                and 0 < n_steps <= min(12, n_grid) and n_grid == int(n_grid)
                 and wq.granularity == 'per_group' and wq.group_size in (32, 64, 128)
                 and getattr(wq, 'quant_type', 'int-quant') == 'int-quant' and wq.round_zp and wq.calib_algo == 'minmax'
                 and -256 <= float(wq.qmin) < float(wq.qmax) <= 256

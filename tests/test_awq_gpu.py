@@ -480,6 +480,25 @@ def test_auto_clip_error_equal_to_the_starting_value_does_not_win(dev, gs, fast)
     assert float(bmax[0, 0]) == 1007616
 
 
+@pytest.mark.parametrize('n_grid,max_shrink', [(10, 1.2), (10, 1.0), (8.5, 0.9)])
+def test_auto_clip_grids_the_one_launch_search_does_not_take(dev, n_grid, max_shrink):
+    """Shrinking past zero and grids that are no whole number: the step-by-step path, as before the other one existed."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    w = weight_like(64, 256, seed=5, dtype=torch.bfloat16)
+    x = torch.randn(24, 256, generator=gen(6)).bfloat16()
+    spec = Q.IntSpec(4, True, 'per_group', group_size=128)
+    obmax, obmin, oerrs = A.auto_clip_layer(spec, w, [x.clone()], clip_sym=True, n_grid=n_grid, max_shrink=max_shrink, n_sample_token=24)
+    clipper = AutoClipper(True, IntegerQuantizer(4, True, 'per_group', group_size=128), None, 'v1', True, False, None)
+    bmax, bmin = clipper.auto_clip_layer(0, 'fc', w.to(dev), [x.to(dev)], n_grid=n_grid, max_shrink=max_shrink, n_sample_token=24)
+    errs, oe = clipper.last_errs.cpu(), oerrs.float()
+    assert errs.shape == oe.shape and bool(((errs - oe).abs() <= 2 * 2.0 ** -7 * oe.abs()).all())
+    same = (errs == oe).all(-1, keepdim=True)
+    assert float(same.float().mean()) > 0.9
+    assert torch.equal(bmax.cpu()[same], obmax[same]) and torch.equal(bmin.cpu()[same], obmin[same])
+
+
 def test_auto_clip_run_skips_query_key_and_handles_float8_weights(dev):
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
