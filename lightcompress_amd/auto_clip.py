@@ -27,7 +27,7 @@ import torch
 
 from . import _lib as L
 from .kernel import weight_cast_to_bf16, weight_cast_to_fp8
-from .quant import _scaled
+from .quant import IntegerQuantizer, _scaled
 
 
 class AutoClipper:
@@ -135,13 +135,14 @@ class AutoClipper:
 
     def _fused_applies(self, w, xs, n_steps, n_grid=20):
         """lcq_clip_search_exact: one launch with the same roundings as _search_exact, for bf16 tensors, v1, weight-only,
-        groups of 32 / 64 / 128, one input, the min/max integer quantizer and whole steps that do not shrink past zero."""
+        groups of 32 / 64 / 128, one input, the min/max integer quantizer and whole steps that do not shrink past zero.  A
+        subclass of the quantizer, or of this class with its own fake_quantize_weight, is asked step by step."""
         wq = self.wquantizer
         return (self.clip_version == 'v1' and self.w_only and len(xs) == 1
                 and 0 < n_steps <= min(12, n_grid) and n_grid == int(n_grid)
+                and type(wq) is IntegerQuantizer and getattr(self.fake_quantize_weight, '__func__', None) is AutoClipper.fake_quantize_weight
                 and wq.granularity == 'per_group' and wq.group_size in (32, 64, 128)
-                and getattr(wq, 'quant_type', 'int-quant') == 'int-quant' and wq.round_zp and wq.calib_algo == 'minmax'
-                and -256 <= float(wq.qmin) < float(wq.qmax) <= 256
+                and wq.round_zp and wq.calib_algo == 'minmax' and -256 <= float(wq.qmin) < float(wq.qmax) <= 256
                 and w.dtype == torch.bfloat16 and xs[0].dtype == torch.bfloat16
                 and w.data_ptr() % 16 == 0 and xs[0].data_ptr() % 16 == 0)
 

@@ -100,3 +100,22 @@ def test_rtn_picks_the_quantizers_like_set_quant_config():
     rtn = RTN(cfg)
     assert rtn.act_static and cfg['act']['calib_algo'] == 'static_minmax' and not rtn.w_only
     assert rtn.auto_clipper.clip_version == 'v1' and rtn.aquantizer.calib_algo == 'static_minmax'
+
+
+def test_clip_search_asks_overridden_quantization_step_by_step():
+    """The one-launch clip search stands for IntegerQuantizer and AutoClipper.fake_quantize_weight themselves only."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+
+    class OwnQuantizer(IntegerQuantizer):
+        def fake_quant_weight_dynamic(self, weight, args={}):
+            return weight.round()
+
+    class OwnClipper(AutoClipper):
+        def fake_quantize_weight(self, w, min_val, max_val, org_min_val, org_max_val):
+            return w.round()
+    w, x = torch.zeros(64, 128, dtype=torch.bfloat16), torch.zeros(4, 128, dtype=torch.bfloat16)
+    for cls, quantizer, takes in ((AutoClipper, IntegerQuantizer, True), (AutoClipper, OwnQuantizer, False),
+                                  (OwnClipper, IntegerQuantizer, False)):
+        clipper = cls(True, quantizer(4, False, 'per_group', group_size=128), None, 'v1', False, False, None)
+        assert clipper._fused_applies(w, [x], 10) == takes
