@@ -283,8 +283,8 @@ class AutoClipper:
             R, G = max_val.shape[:2]
             w3 = w.view(R, G, -1)
             tensor_range = self.wquantizer.get_learnable_range(w3, low_factor, up_factor)
-            scales, zeros, qmax, qmin = self.wquantizer.get_qparams(tensor_range, w.device)
-            args = {'scales': scales, 'zeros': zeros, 'qmax': qmax, 'qmin': qmin}
+            scales, zeros = self.wquantizer.get_qparams(tensor_range, w.device)[:2]
+            args = {'scales': scales, 'zeros': zeros, 'qmax': self.wquantizer.qmax, 'qmin': self.wquantizer.qmin}
             q_w = self.wquantizer.fake_quant_weight_static(w3, args).view(w.shape)
         else:
             raise Exception('Not support other clip version')

@@ -145,9 +145,12 @@ class BaseQuantizer(object):
         return (L.FLAG_SYM if self.sym else 0) | (0 if self.round_zp else L.FLAG_NO_ROUND_ZP)
 
     def get_qparams(self, tensor_range, device):
-        """quant.py:544-558 -> (scales, zeros, qmax, qmin)."""
+        """quant.py:544-558 -> (scales, zeros, qmax, qmin); the bounds are the caller's own tensors."""
+        scales, zeros = self._qparams(tensor_range)
+        return scales, zeros, self.qmax.to(device), self.qmin.to(device)
+
+    def _qparams(self, tensor_range):
         min_val, max_val = tensor_range[0].contiguous(), tensor_range[1].contiguous()
-        qmax, qmin = self._dev_bounds(device)
         flags = self._int_flags()
         # 0-dim ranges (per_tensor) meet the 0-dim fp32 (qmax - qmin): torch promotes the result to fp32
         if max_val.dim() == 0 and not self.sym and max_val.dtype != torch.float32:
@@ -159,7 +162,7 @@ class BaseQuantizer(object):
                                         L.i64(max_val.numel()), L.f32(self.qmin), L.f32(self.qmax),
                                         L.i32(flags), L.ptr(scales),
                                         L.ptr(None if self.sym else zeros), L.stream()), 'lcq_qparams_int')
-        return scales, zeros, qmax, qmin
+        return scales, zeros
 
     # -- static activation calibration (quant.py:105-124, 223-262, 523-585) -------------------
     def reshape_batch_tensors(self, act_tensors):
@@ -446,7 +449,7 @@ class BaseQuantizer(object):
         tensor = self.reshape_tensor(tensor.float())
         tensor_range = self.get_minmax_range(tensor)
         scales, zeros, qmax, qmin = self.get_qparams(tensor_range, tensor.device)
-        best_scales, best_zeros = self.optimize_weights_proximal(tensor, scales, zeros, qmax, qmin)
+        best_scales, best_zeros = self.optimize_weights_proximal(tensor, scales, zeros, self.qmax, self.qmin)
         return tensor, best_scales, best_zeros, qmax, qmin
 
     # -- views (quant.py:611-657); torch view ops only ----------------------
@@ -615,7 +618,7 @@ class IntegerQuantizer(BaseQuantizer):
         else:
             if self.granularity == 'per_tensor':
                 lo, hi = self.get_minmax_range(t)
-                scales, zeros, _, _ = self.get_qparams((lo, hi), t.device)
+                scales, zeros = self._qparams((lo, hi))
                 return self._launch(t, static=True, scales=scales, zeros=zeros, want_dq=want_dq,
                                     want_codes=want_codes, osf=osf)
             rows, cols = _rows_cols(t)
@@ -647,11 +650,9 @@ class IntegerQuantizer(BaseQuantizer):
             return self.get_hqq_qparams(tensor, args)
         tensor = self.reshape_tensor(tensor)
         if self.calib_algo != 'minmax':
-            scales, zeros, qmax, qmin = self.get_qparams(self.get_tensor_range(tensor, args), tensor.device)
-            return tensor, scales, zeros, qmax, qmin
+            return (tensor, *self.get_qparams(self.get_tensor_range(tensor, args), tensor.device))
         if self.granularity == 'per_tensor':
-            scales, zeros, qmax, qmin = self.get_qparams(self.get_minmax_range(tensor), tensor.device)
-            return tensor, scales, zeros, qmax, qmin
+            return (tensor, *self.get_qparams(self.get_minmax_range(tensor), tensor.device))
         _, _, scales, zeros = self._launch(tensor, static=False)
         if tensor.dim() != 2:
             scales = scales.view(*tensor.shape[:-1], 1)
@@ -691,15 +692,22 @@ class IntegerQuantizer(BaseQuantizer):
                                    osf=output_scale_factor, qmin=qmin, qmax=qmax)
         return dq.view(tensor.shape)
 
+    def _calibrated_qparams(self, tensor, args={}):
+        """get_tensor_qparams without the bounds: the launches take them as numbers, and reading them back from the device
+        would wait for it."""
+        if self.calib_algo == 'hqq':
+            return self.get_hqq_qparams(tensor, args)[:3]
+        rows_t = self.reshape_tensor(tensor)
+        return (rows_t, *self._qparams(self.get_tensor_range(rows_t, args)))
+
     def _fake_dynamic(self, t, args={}):
         shape, dtype = t.shape, t.dtype
         rows_t = self.reshape_tensor(t)
         if self.calib_algo != 'minmax':                  # calibrated ranges, then the static path (quant.py:853-860)
             rargs = {k: args[k] for k in ('lowbound_factor', 'upbound_factor') if k in args} \
                 if self.calib_algo == 'learnable' else {}
-            rows_t, scales, zeros, qmax, qmin = self.get_tensor_qparams(t, rargs)
-            dq, _, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_dq=True, qmin=qmin, qmax=qmax,
-                                       cast_back=True)
+            rows_t, scales, zeros = self._calibrated_qparams(t, rargs)
+            dq, _, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_dq=True, cast_back=True)
             return self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
         dq, _, _, _ = self._launch(rows_t, static=False, want_dq=True, want_qp=False)
         return dq if dq.shape == shape and dq.dtype == dtype else self.restore_tensor(dq.view(rows_t.shape), shape).to(dtype)
@@ -810,9 +818,8 @@ class IntegerQuantizer(BaseQuantizer):
         output_scale_factor = args.pop('output_scale_factor', 1) if 'output_scale_factor' in args else 1
         rows_t = self.reshape_tensor(weight)
         if self.calib_algo != 'minmax':
-            rows_t, scales, zeros, qmax, qmin = self.get_tensor_qparams(weight)
-            _, codes, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_codes=self._code_dtype(),
-                                          qmin=qmin, qmax=qmax)
+            rows_t, scales, zeros = self._calibrated_qparams(weight)
+            _, codes, _, _ = self._launch(rows_t, static=True, scales=scales, zeros=zeros, want_codes=self._code_dtype())
         else:
             _, codes, scales, zeros = self._launch(rows_t, static=False, want_codes=self._code_dtype())
         codes = self.restore_tensor(codes.view(rows_t.shape), org_w_shape)
@@ -1314,11 +1321,15 @@ class Weight48IntegerQuantizer(BaseQuantizer):
         return (mn, mx)
 
     def get_qparams(self, tensor_range, device, bit):
+        q = self._stage[bit]
+        return (*self._stage_qparams(tensor_range, bit), q.qmax.to(device), q.qmin.to(device))
+
+    def _stage_qparams(self, tensor_range, bit):
         cfg = self.bit_settings[bit]
-        scales, zeros, qmax, qmin = self._stage[bit].get_qparams(tensor_range, device)
+        scales, zeros = self._stage[bit]._qparams(tensor_range)
         if 'scales_bit' in cfg:                                   # a clamp of [rows, 1] parameters
             scales = scales.clamp(cfg['scales_qmin'], cfg['scales_qmax'])
-        return scales, zeros, qmax, qmin
+        return scales, zeros
 
     def quant(self, tensor, scales, zeros, qmax, qmin):
         return self._stage[4].quant(tensor, scales, zeros, qmax, qmin)
@@ -1333,13 +1344,13 @@ class Weight48IntegerQuantizer(BaseQuantizer):
         org_shape16, org_dtype16 = weight.shape, weight.dtype
         # 16 -> 8 bit
         weight = self.reshape_tensor(weight, bit=8)
-        scales816, zeros816, qmax816, qmin816 = self.get_qparams(self.get_tensor_range(weight), weight.device, bit=8)
-        weight = self.quant(weight, scales816, zeros816, qmax816, qmin816)
+        scales816, zeros816 = self._stage_qparams(self.get_tensor_range(weight), bit=8)
+        weight = self.quant(weight, scales816, zeros816, self._stage[8].qmax, self._stage[8].qmin)
         # 8 -> 4 bit
         org_shape8, org_dtype8 = weight.shape, weight.dtype
         weight = self.reshape_tensor(weight, bit=4)
-        scales48, zeros48, qmax48, qmin48 = self.get_qparams(self.get_tensor_range(weight), weight.device, bit=4)
-        weight = self.quant(weight, scales48, zeros48, qmax48, qmin48)
+        scales48, zeros48 = self._stage_qparams(self.get_tensor_range(weight), bit=4)
+        weight = self.quant(weight, scales48, zeros48, self._stage[4].qmax, self._stage[4].qmin)
         # 4 -> 8 -> 16 bit
         weight = self.restore_tensor(self.dequant(weight, scales48, zeros48), org_shape8).to(org_dtype8)
         weight = self.restore_tensor(self.dequant(weight, scales816, zeros816), org_shape16).to(org_dtype16)

@@ -132,16 +132,16 @@ class RTN(ScaleFolding):
 
     @torch.no_grad()
     def register_act_qparams(self, layers_dict, act_tensors):
-        """base_blockwise_quantization.py:590-611 on one GPU (no all-reduce of the scales)."""
+        """base_blockwise_quantization.py:590-611 on one GPU (no all-reduce of the scales); every layer gets its own buffers."""
         scales_list, zeros_list, qmin_list, qmax_list = self.aquantizer.get_batch_tensors_qparams(act_tensors)
         for i, (scales, zeros, qmin, qmax) in enumerate(zip(scales_list, zeros_list, qmin_list, qmax_list)):
             for layer in layers_dict.values():
                 if not is_linear_like(layer):
                     continue
-                layer.register_buffer(f'buf_act_scales_{i}', scales.cuda())
-                layer.register_buffer(f'buf_act_zeros_{i}', zeros.cuda())
-                layer.register_buffer(f'buf_act_qmin_{i}', qmin.cuda())
-                layer.register_buffer(f'buf_act_qmax_{i}', qmax.cuda())
+                layer.register_buffer(f'buf_act_scales_{i}', scales.to('cuda', copy=True))
+                layer.register_buffer(f'buf_act_zeros_{i}', zeros.to('cuda', copy=True))
+                layer.register_buffer(f'buf_act_qmin_{i}', qmin.to('cuda', copy=True))
+                layer.register_buffer(f'buf_act_qmax_{i}', qmax.to('cuda', copy=True))
 
     # -- rtn.py:14-29 -----------------------------------------------------------------------------------------
     @torch.no_grad()
