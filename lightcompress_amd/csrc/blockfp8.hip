@@ -154,25 +154,29 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const u32x4* __restrict_
   else *(uint32_t*)dst = w[0];
 }
 
-// out = float(y) * s[block]: a workgroup takes 8 rows of one block row and 256 * W columns, W float8 per lane and row so that
-// a lane's output is one 16-byte piece next to its neighbours'.  HBM-bound: 2112 x 7168 to fp32 (76 MB) 15.4 us with eight
-// float8 per lane, two half-line stores and a 64-bit division per chunk, 13.3 so.
+// out = float(y) * s[block]: a lane takes W float8 of each of two rows of one block row, so that its output is one 16-byte piece
+// next to its neighbours'; the lanes are numbered along the pieces of a row pair, then down, so none is idle whatever the width
+// (a workgroup per 256 pieces of a row left most of it idle on narrow matrices).  HBM-bound: 2112 x 7168 to fp32 (76 MB) 14.4 us
+// with eight float8 per lane, two half-line stores and a 64-bit division per chunk, 12.3 so (one, four and eight rows: 12.4, 12.3,
+// 12.5); 131072 x 128 to bf16 8.6 (8.7, 8.8, 8.9).
+constexpr int DQ_ROWS = 2;
 template <int OUT>   // LCQ_F32 | LCQ_BF16
 __global__ __launch_bounds__(256) void block_dequant_kernel(const uint8_t* __restrict__ y, const float* __restrict__ scales,
-                                                            int64_t M, int64_t N, int nbn, void* __restrict__ out) {
+                                                            int64_t M, int64_t N, int nbn, uint32_t pieces, void* __restrict__ out) {
   constexpr int W = OUT == LCQ_BF16 ? 8 : 4;
-  const int64_t col = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W, row0 = (int64_t)blockIdx.y * 8;
-  if (col >= N) return;
+  const uint32_t lane = blockIdx.x * 256u + threadIdx.x, group = lane / pieces;
+  const int64_t col = (int64_t)(lane - group * pieces) * W, row0 = (int64_t)group * DQ_ROWS;
+  if (row0 >= M) return;
   const float s = scales[(row0 / BS) * nbn + col / BS];
-  uint32_t w[8][W / 4];
+  uint32_t w[DQ_ROWS][W / 4];
   #pragma unroll
-  for (int r = 0; r < 8; ++r)
+  for (int r = 0; r < DQ_ROWS; ++r)
     if (row0 + r < M) {
       if constexpr (W == 8) { const u32x2 v = *(const u32x2*)(y + (row0 + r) * N + col); w[r][0] = v[0]; w[r][W / 4 - 1] = v[1]; }
       else w[r][0] = *(const uint32_t*)(y + (row0 + r) * N + col);
     }
   #pragma unroll
-  for (int r = 0; r < 8; ++r)
+  for (int r = 0; r < DQ_ROWS; ++r)
     if (row0 + r < M) {
       float v[W];
       #pragma unroll
@@ -224,13 +228,20 @@ int lcq_fp8_block_dequant(const void* y, const float* scales, int64_t M, int64_t
   if (!y || !scales || !out || M <= 0 || N <= 0) return LCQ_EINVAL;
   if (N % 8 != 0 || ((uintptr_t)y % 8) != 0 || ((uintptr_t)out % 16) != 0) return LCQ_EALIGN;
   const int nbn = (int)((N + BS - 1) / BS);
-  const int64_t per = 256 * (out_dtype == LCQ_BF16 ? 8 : 4);
-  if ((M + 7) / 8 > 0x7fffffff || (N + per - 1) / per > 0x7fffffff) return LCQ_EINVAL;
-  const dim3 grid((unsigned)((N + per - 1) / per), (unsigned)((M + 7) / 8));
+  if (out_dtype != LCQ_BF16 && out_dtype != LCQ_F32) return LCQ_EDTYPE;
+  const int64_t pieces = N / (out_dtype == LCQ_BF16 ? 8 : 4);
   hipStream_t st = (hipStream_t)stream;
-  if (out_dtype == LCQ_BF16) block_dequant_kernel<LCQ_BF16><<<grid, dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
-  else if (out_dtype == LCQ_F32) block_dequant_kernel<LCQ_F32><<<grid, dim3(256), 0, st>>>((const uint8_t*)y, scales, M, N, nbn, out);
-  else return LCQ_EDTYPE;
+  // lanes are numbered in 32 bits: whole block rows per launch (one, but for matrices of more than 3e10 elements)
+  const int64_t most = (int64_t)0xffffff00 / (pieces * (BS / DQ_ROWS)) * BS;
+  if (most == 0) return LCQ_EINVAL;
+  for (int64_t m0 = 0; m0 < M; m0 += most) {
+    const int64_t m = M - m0 < most ? M - m0 : most;
+    const dim3 grid((unsigned)((pieces * ((m + DQ_ROWS - 1) / DQ_ROWS) + 255) / 256));
+    const uint8_t* src = (const uint8_t*)y + m0 * N;
+    const float* sc = scales + m0 / BS * nbn;
+    if (out_dtype == LCQ_BF16) block_dequant_kernel<LCQ_BF16><<<grid, dim3(256), 0, st>>>(src, sc, m, N, nbn, (uint32_t)pieces, (uint16_t*)out + m0 * N);
+    else block_dequant_kernel<LCQ_F32><<<grid, dim3(256), 0, st>>>(src, sc, m, N, nbn, (uint32_t)pieces, (float*)out + m0 * N);
+  }
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

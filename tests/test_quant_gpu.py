@@ -996,6 +996,19 @@ def test_every_finite_fp16_value_under_many_scales(dev, kind):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('M,N', [(1, 8), (9, 24), (129, 128), (2049, 264), (7, 1032), (300, 2056), (524296, 8)])
+def test_blockwise_dequant_of_narrow_wide_and_tall_matrices(dev, dtype, M, N):
+    """Rows shorter and longer than a workgroup, odd heights, very many rows: every element is its float8 number times its
+    block's scale."""
+    from lightcompress_amd.kernel import _block_dequant
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    y = torch.randint(0, 127, (M, N), generator=g, device=dev, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    s = torch.rand((M + 127) // 128, (N + 127) // 128, generator=g, device=dev) + 0.5
+    want = (y.float() * s.repeat_interleave(128, 0)[:M].repeat_interleave(128, 1)[:, :N]).to(dtype)
+    assert torch.equal(_block_dequant(y, s, dtype), want)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize('rows', [1, 128])
 def test_blockwise_fp8_quotients_next_to_rounding_boundaries(dev, dtype, rows):
     """x / s without the division sequence: values on and one ulp beside the midpoints between float8 numbers (subnormal ones
