@@ -210,11 +210,12 @@ struct IntOp {
   }
 
   // Does this chunk take the element-wise form?  med3 turns a NaN into a bound, torch.clamp hands it on.  A NaN in a row
-  // that gave the parameters itself leaves no finite scale, so only given parameters look at the elements.
-  template <int N>
+  // that gave the parameters itself leaves no finite scale, so only given parameters look at the elements: GIVEN 1, not: 0;
+  // 2: asked at run time.  (The rolled loop of long rows has one of each: the question costs it 8 %.)
+  template <int N, int GIVEN>
   __device__ __forceinline__ bool general(const float* x, const Row& p) const {
     bool g = !p.zint;
-    if (is_static) {
+    if (GIVEN == 1 || (GIVEN == 2 && is_static)) {
       float m = nan_max(x[0], x[1]);
       #pragma unroll
       for (int i = 2; i < N; i += 2) m = nan_max(nan_max(m, x[i]), x[i + 1]);
@@ -223,13 +224,13 @@ struct IntOp {
     return g;
   }
 
-  template <int N>
+  template <int N, int GIVEN = 2>
   __device__ __forceinline__ void codes(const float* x, float* q, const Row& p) const {
     if constexpr (!FAST) {
       #pragma unroll
       for (int i = 0; i < N; ++i) q[i] = code(x[i], p);
     } else {
-      if (__builtin_expect(general<N>(x, p), 0)) {
+      if (__builtin_expect(general<N, GIVEN>(x, p), 0)) {
         #pragma unroll
         for (int i = 0; i < N; ++i) q[i] = code(x[i], p);
         return;
@@ -263,9 +264,9 @@ struct IntOp {
   // clamp(rint(t), qmin - z, qmax - z) * s when z is a small integer (all terms exact); the "+ 0" of the
   // fused multiply-add (one rounding, that of the product) turns the -0 that rint(-0.3) leaves into the +0
   // that (q - z) gives.  The products are left unrounded: the caller rounds to the row type while packing.
-  template <int N>
+  template <int N, int GIVEN = 2>
   __device__ __forceinline__ void fused_dq(const float* x, float* d, const Row& p) const {
-    if (__builtin_expect(general<N>(x, p), 0)) {
+    if (__builtin_expect(general<N, GIVEN>(x, p), 0)) {
       #pragma unroll
       for (int i = 0; i < N; ++i) d[i] = deq_raw(code(x[i], p), p);
       return;

@@ -23,6 +23,7 @@
 #pragma once
 #include "common.h"
 #include "lcq_internal.h"
+#include <type_traits>
 
 namespace lcq {
 
@@ -197,7 +198,7 @@ __device__ __forceinline__ void store_code1(const Op& op, void* codes, int64_t e
 }
 
 // codes + dq of one chunk, generic form: op.codes -> storage, op.deq_raw -> storage
-template <class Op>
+template <class Op, int GIVEN = 2>
 __device__ __forceinline__ void emit_chunk_generic(const Op& op, const typename Op::Row& p, const float* v_in, int64_t cidx,
                                                    void* dq, void* codes) {
   constexpr int BF = Op::BF;
@@ -211,7 +212,8 @@ __device__ __forceinline__ void emit_chunk_generic(const Op& op, const typename 
       return;
     }
   }
-  op.template codes<N>(v, q, p);
+  if constexpr (Op::HAS_CUSTOM_EMIT) op.template codes<N>(v, q, p);
+  else op.template codes<N, GIVEN>(v, q, p);
   if (codes) store_codes(op, codes, cidx * N, q);
   if (dq) {
     #pragma unroll
@@ -232,7 +234,8 @@ __device__ __forceinline__ void emit_chunk_generic(const Op& op, const typename 
 // Returns false when the op's fast path declined the chunk (HAS_CUSTOM_EMIT only): the caller
 // then runs emit_chunk_slow on it, from ONE rolled loop, so the long generic code exists once per
 // kernel instead of once per unrolled chunk (and stays out of the instruction cache).
-template <class Op>
+// GIVEN: whether the parameters were given (0 / 1, 2: see op.is_static); the integer op asks.
+template <class Op, int GIVEN = 2>
 __device__ __forceinline__ bool emit_chunk(const Op& op, const typename Op::Row& p, const u32x4& r, int64_t cidx,
                                            void* dq, void* codes) {
   constexpr int BF = Op::BF;
@@ -245,13 +248,13 @@ __device__ __forceinline__ bool emit_chunk(const Op& op, const typename Op::Row&
     if constexpr (Op::HAS_FUSED_DQ) {
       if (!codes) {                                          // fake quant: no detour through the codes
         if (dq) {
-          op.template fused_dq<N>(v, q, p);
+          op.template fused_dq<N, GIVEN>(v, q, p);
           __builtin_nontemporal_store(pack_rne<BF>(q), (u32x4*)dq + cidx);
         }
         return true;
       }
     }
-    emit_chunk_generic(op, p, v, cidx, dq, codes);
+    emit_chunk_generic<Op, GIVEN>(op, p, v, cidx, dq, codes);
     return true;
   }
 }
@@ -446,10 +449,21 @@ __global__ __launch_bounds__(256) void row_block_kernel(
     const int ch = threadIdx.x + k * 256;
     if (ch < nchunks) redo = !emit_chunk(op, p, raw[k], row * nchunks + ch, dq, codes) || redo;
   }
-  for (int ch = threadIdx.x + CACHE * 256; ch < nchunks; ch += 256) {
-    u32x4 r = xr[ch];
-    if constexpr (Op::HAS_PRESCALE) r = op.prescale(r, row, ch, nchunks);
-    redo = !emit_chunk(op, p, r, row * nchunks + ch, dq, codes) || redo;
+  if constexpr (Op::HAS_CUSTOM_EMIT) {
+    for (int ch = threadIdx.x + CACHE * 256; ch < nchunks; ch += 256) {
+      u32x4 r = xr[ch];
+      if constexpr (Op::HAS_PRESCALE) r = op.prescale(r, row, ch, nchunks);
+      redo = !emit_chunk(op, p, r, row * nchunks + ch, dq, codes) || redo;
+    }
+  } else {
+    const auto rest = [&](auto given) {
+      for (int ch = threadIdx.x + CACHE * 256; ch < nchunks; ch += 256) {
+        u32x4 r = xr[ch];
+        if constexpr (Op::HAS_PRESCALE) r = op.prescale(r, row, ch, nchunks);
+        emit_chunk<Op, decltype(given)::value>(op, p, r, row * nchunks + ch, dq, codes);
+      }
+    };
+    if (op.is_static) rest(std::integral_constant<int, 1>()); else rest(std::integral_constant<int, 0>());
   }
   if constexpr (Op::HAS_CUSTOM_EMIT) {
     if (__builtin_expect(redo, 0)) {
