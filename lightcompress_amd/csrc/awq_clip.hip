@@ -540,8 +540,8 @@ int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, in
   hipStream_t st = (hipStream_t)stream;
   #define LCQ_CLIP(GS) do { \
     const size_t lds = (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)waves * n_steps * GT * 4; \
-    static const hipError_t once = hipFuncSetAttribute((const void*)clip_search_kernel<GS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-    if (once != hipSuccess) return LCQ_ELAUNCH; \
+    /* on every call, for it belongs to the current device; the same value always, for another thread may set it too */ \
+    if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)clip_search_kernel<GS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return LCQ_ELAUNCH; \
     clip_search_kernel<GS><<<dim3((unsigned)grid), dim3(64 * waves), lds, st>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K, \
         (int)T, n_grid, n_steps, clip_sym, op, (uint16_t*)best_max, (uint16_t*)best_min, errs); } while (0)
   if (group_size == 128) LCQ_CLIP(128); else if (group_size == 64) LCQ_CLIP(64); else LCQ_CLIP(32);

@@ -499,6 +499,22 @@ def test_auto_clip_grids_the_one_launch_search_does_not_take(dev, n_grid, max_sh
     assert torch.equal(bmax.cpu()[same], obmax[same]) and torch.equal(bmin.cpu()[same], obmin[same])
 
 
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason='two GPUs')
+def test_auto_clip_one_launch_search_on_a_second_device(dev):
+    """The kernel asks for more LDS than a launch gets by itself; that request is per device."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    w = weight_like(64, 256, seed=1, dtype=torch.bfloat16)
+    x = torch.randn(16, 256, generator=gen(2)).bfloat16()
+    out = []
+    for d in ('cuda:0', 'cuda:1'):
+        with torch.cuda.device(d):
+            clipper = AutoClipper(True, IntegerQuantizer(4, False, 'per_group', group_size=128), None, 'v1', False, False, None)
+            out.append([t.cpu() for t in clipper.auto_clip_layer(0, 'fc', w.to(d), [x.to(d)], n_sample_token=16)])
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 def test_auto_clip_run_skips_query_key_and_handles_float8_weights(dev):
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
