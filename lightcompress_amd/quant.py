@@ -146,8 +146,10 @@ class BaseQuantizer(object):
 
     def get_qparams(self, tensor_range, device):
         """quant.py:544-558 -> (scales, zeros, qmax, qmin); the bounds are the caller's own tensors."""
-        scales, zeros = self._qparams(tensor_range)
-        return scales, zeros, self.qmax.to(device), self.qmin.to(device)
+        return (*self._qparams(tensor_range), *self._own_bounds(device))
+
+    def _own_bounds(self, device):
+        return self.qmax.to(device), self.qmin.to(device)
 
     def _qparams(self, tensor_range):
         min_val, max_val = tensor_range[0].contiguous(), tensor_range[1].contiguous()
@@ -561,6 +563,10 @@ class IntegerQuantizer(BaseQuantizer):
         if key not in self._bounds_dev:
             self._bounds_dev[key] = (self.qmax.to(device), self.qmin.to(device))
         return self._bounds_dev[key]
+
+    def _own_bounds(self, device):
+        """Copies of those, made on the device (no transfer from the host, which a stream capture would not take)."""
+        return tuple(b.clone() for b in self._dev_bounds(device))
 
     def _bound(self, v):
         """Python float of a qmin/qmax argument without a device sync for our own tensors."""
@@ -1321,8 +1327,7 @@ class Weight48IntegerQuantizer(BaseQuantizer):
         return (mn, mx)
 
     def get_qparams(self, tensor_range, device, bit):
-        q = self._stage[bit]
-        return (*self._stage_qparams(tensor_range, bit), q.qmax.to(device), q.qmin.to(device))
+        return (*self._stage_qparams(tensor_range, bit), *self._stage[bit]._own_bounds(device))
 
     def _stage_qparams(self, tensor_range, bit):
         cfg = self.bit_settings[bit]

@@ -1028,3 +1028,24 @@ def test_blockwise_fp8_quotients_next_to_rounding_boundaries(dev, dtype, rows):
     oy, os_ = (Q.triton_act_quant if rows == 1 else Q.triton_weight_cast_to_fp8)(x)
     assert_bit_equal(s, os_, 'scales')
     assert_bit_equal(y, oy, 'codes')
+
+
+@pytest.mark.parametrize('kw', [dict(granularity='per_tensor'), dict(granularity='per_channel', calib_algo='mse')])
+def test_parameters_of_a_tensor_in_a_captured_graph(dev, kw):
+    """get_tensor_qparams and fake quantization record no transfer from the host: replays on new contents give the eager
+    results."""
+    from lightcompress_amd import IntegerQuantizer
+    q = IntegerQuantizer(8, False, **kw)
+    w = torch.randn(64, 128, generator=gen(1)).bfloat16().to(dev)
+    q.get_tensor_qparams(w), q.fake_quant_weight_dynamic(w)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        qp = q.get_tensor_qparams(w)
+        fake = q.fake_quant_weight_dynamic(w)
+    for i in range(3):
+        w.copy_(torch.randn(64, 128, generator=gen(2 + i)))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = q.get_tensor_qparams(w)
+        assert torch.equal(fake, q.fake_quant_weight_dynamic(w))
+        assert all(torch.equal(a, b) for a, b in zip(qp[1:], want[1:])) and float(qp[3]) == 255
