@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void clamp_groups_scalar_kernel(const void* __
   }
 }
 
-// The reference's rounding sequence on the matrix pipe (16-bit types).
+// The reference's rounding sequence on the matrix pipe (bf16).
 //
 //   dot(t, r) = sum_j round(x[t, j] * w[r, j])      every product rounded to the tensors' type, fp32 sums
 //
@@ -170,32 +170,23 @@ __global__ __launch_bounds__(256) void clamp_groups_scalar_kernel(const void* __
 // slower.  Measured (rows 11008 x 4096 + 11008 x 4096 + 4096 x 11008, 512 tokens, 10 steps): 92.3 -> 25.8 ms, the matrix
 // pipes busy in 78 % of the cycles; the products one after the other in the same registers 31.2, without all
 // conversions ahead of the sums 28.3.
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(4))) short i16x4;
 typedef __attribute__((ext_vector_type(32))) float f32x32;
 
-template <int BF> __device__ __forceinline__ f32x32 outer_products(u32x2 a, u32x2 b) {
+__device__ __forceinline__ f32x32 outer_products(u32x2 a, u32x2 b) {
   f32x32 z;
   #pragma unroll
   for (int i = 0; i < 32; ++i) z[i] = 0.0f;
-  if constexpr (BF == ROW_F16) return __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), z, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), z, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), z, 0, 0, 0);
 }
-template <int BF> __device__ __forceinline__ f32x4 add_pairs(u32x4 pairs, u32x4 ones, f32x4 c) {
-  if constexpr (BF == ROW_F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, pairs), __builtin_bit_cast(f16x8, ones), c, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pairs), __builtin_bit_cast(bf16x8, ones), c, 0, 0, 0);
-}
-template <int BF> __device__ __forceinline__ uint32_t pack_pair(float a, float b) {
-  if constexpr (BF == ROW_F16) return f16_pack_rne(a, b); else return bf16_pack_rne(a, b);
+__device__ __forceinline__ f32x4 add_pairs(u32x4 pairs, u32x4 ones, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pairs), __builtin_bit_cast(bf16x8, ones), c, 0, 0, 0);
 }
 // B operand of add_pairs: lane (h = l / 16, n = l % 16) holds k = 8 h + i of column n; pair i / 2 of quarter h goes to column 4 h + i / 2
-template <int BF> __device__ __forceinline__ u32x4 pair_columns(int lane) {
-  const uint32_t one = BF == ROW_F16 ? 0x3c003c00u : 0x3f803f80u;
+__device__ __forceinline__ u32x4 pair_columns(int lane) {
   u32x4 b;
   #pragma unroll
-  for (int d = 0; d < 4; ++d) b[d] = (lane & 15) == 4 * (lane >> 4) + d ? one : 0u;
+  for (int d = 0; d < 4; ++d) b[d] = (lane & 15) == 4 * (lane >> 4) + d ? 0x3f803f80u : 0u;
   return b;
 }
 
@@ -204,7 +195,7 @@ template <int GS> constexpr int gd_pitch() { return GS * 2 + 16; }     // bytes 
 // sum[4] of a tile: a = the tokens' GS columns (lane l: token l % 32), wrow = row l % 32 in LDS.  The products of the next
 // column pair are issued before the current ones are rounded: the empty asm keeps that order (without it the compiler
 // runs the two one after the other in the same registers).
-template <int BF, int GS>
+template <int GS>
 __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint32_t mask, u32x4 ones, f32x4* sum) {
   #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -214,7 +205,7 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
     if (p == 0 && i > 0) b = *(const u32x4*)(wrow + 4 * i);
     const u32x4 av = a[i >> 2];
     const uint32_t w = b[p] & mask;
-    return outer_products<BF>(p < 2 ? u32x2{av[0], av[1]} : u32x2{av[2], av[3]}, (p & 1) ? u32x2{0, w} : u32x2{w, 0});
+    return outer_products(p < 2 ? u32x2{av[0], av[1]} : u32x2{av[2], av[3]}, (p & 1) ? u32x2{0, w} : u32x2{w, 0});
   };
   f32x32 d[2];
   d[0] = products(0);
@@ -229,10 +220,10 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
     #pragma unroll
     for (int q = 0; q < 4; ++q)
       #pragma unroll
-      for (int k = 0; k < 4; ++k) pr[q][k] = pack_pair<BF>(cur[4 * q + k], cur[16 + 4 * q + k]);
+      for (int k = 0; k < 4; ++k) pr[q][k] = bf16_pack_rne(cur[4 * q + k], cur[16 + 4 * q + k]);
     asm volatile("" : "+v"(pr[0]), "+v"(pr[1]), "+v"(pr[2]), "+v"(pr[3]));
     #pragma unroll
-    for (int q = 0; q < 4; ++q) sum[q] = add_pairs<BF>(pr[q], ones, sum[q]);
+    for (int q = 0; q < 4; ++q) sum[q] = add_pairs(pr[q], ones, sum[q]);
   }
 }
 
@@ -307,7 +298,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
   __syncthreads();
 
   const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
-  const u32x4 ones = pair_columns<ROW_BF16>(lane);
+  const u32x4 ones = pair_columns(lane);
   const char* wrow = smem + (lane & 31) * PITCH_W;
   for (int t0 = wave * GT; t0 < T; t0 += waves * GT) {
     u32x4 a[GS / 8];
@@ -316,7 +307,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
     #pragma unroll
     for (int c = 0; c < GS / 8; ++c) { a[c] = *(const u32x4*)(xr + 8 * c); if (!ok) a[c] = u32x4{0, 0, 0, 0}; }
     f32x4 org[4], cur[4];
-    dots_tile<ROW_BF16, GS>(a, wrow, mask, ones, org);
+    dots_tile<GS>(a, wrow, mask, ones, org);
     redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem, lane, org);
     #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -328,7 +319,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
       }
     #pragma unroll 1
     for (int s = 0; s < n_steps; ++s) {
-      dots_tile<ROW_BF16, GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
+      dots_tile<GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
       redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem + (s + 1) * VERSION, lane, cur);
       float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       #pragma unroll

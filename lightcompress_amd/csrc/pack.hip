@@ -240,8 +240,8 @@ bool awq_team_applies(const void* w, int64_t R, int64_t K, int gs, const void* s
 }
 template <int WDT, bool DYN>
 void launch_awq_team(const void* w, const void* scales, const int32_t* zeros, int64_t R, int64_t K, int gs, float qmin, float qmax,
-                            int flags, int32_t* qweight, void* s16, int32_t* qzeros, hipStream_t st) {
-  const auto op = lcq::make_op<lcq::IntOp<WDT, true>>(qmin, qmax, flags, 1.0f, LCQ_CODE_NONE);
+                     int32_t* qweight, void* s16, int32_t* qzeros, hipStream_t st) {
+  const auto op = lcq::make_op<lcq::IntOp<WDT, true>>(qmin, qmax, 0, 1.0f, LCQ_CODE_NONE);
   const int64_t octs = 512 / (gs / 8);
   const dim3 grid((unsigned)(K / gs), (unsigned)((R / 8 + octs - 1) / octs));        // neighbouring workgroups read the same rows
   #define LCQ_AWQ(GS) pack_awq_team_kernel<WDT, GS, DYN><<<grid, dim3(512), 0, st>>>(w, scales, zeros, R, K, op, (uint32_t*)qweight, (_Float16*)s16, (uint32_t*)qzeros)
@@ -276,9 +276,9 @@ int lcq_quant_pack_awq(const void* w, int dtype, int64_t R, int64_t K, int group
   if (!awq_team_applies(w, R, K, group_size, scales_f16_out) || R % 32 != 0) return LCQ_EINVAL;
   if (!(qmax > qmin) || qmax > 256.0f || qmin < -256.0f) return LCQ_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == LCQ_F32) launch_awq_team<LCQ_F32, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, 0, qweight, scales_f16_out, qzeros, st);
-  else if (dtype == LCQ_BF16) launch_awq_team<LCQ_BF16, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, 0, qweight, scales_f16_out, qzeros, st);
-  else if (dtype == LCQ_F16) launch_awq_team<LCQ_F16, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, 0, qweight, scales_f16_out, qzeros, st);
+  if (dtype == LCQ_F32) launch_awq_team<LCQ_F32, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, qweight, scales_f16_out, qzeros, st);
+  else if (dtype == LCQ_BF16) launch_awq_team<LCQ_BF16, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, qweight, scales_f16_out, qzeros, st);
+  else if (dtype == LCQ_F16) launch_awq_team<LCQ_F16, true>(w, nullptr, nullptr, R, K, group_size, qmin, qmax, qweight, scales_f16_out, qzeros, st);
   else return LCQ_EDTYPE;
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
@@ -290,9 +290,9 @@ int lcq_pack_awq(const void* w, int dtype, const void* scales, const int32_t* ze
   if (R <= 0 || K <= 0 || group_size <= 0 || K % group_size != 0 || R % 32 != 0) return LCQ_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   if (awq_team_applies(w, R, K, group_size, scales_f16_out)) {
-    if (dtype == LCQ_F32) launch_awq_team<LCQ_F32, false>(w, scales, zeros, R, K, group_size, 0, 15, 0, qweight, scales_f16_out, qzeros, st);
-    else if (dtype == LCQ_BF16) launch_awq_team<LCQ_BF16, false>(w, scales, zeros, R, K, group_size, 0, 15, 0, qweight, scales_f16_out, qzeros, st);
-    else if (dtype == LCQ_F16) launch_awq_team<LCQ_F16, false>(w, scales, zeros, R, K, group_size, 0, 15, 0, qweight, scales_f16_out, qzeros, st);
+    if (dtype == LCQ_F32) launch_awq_team<LCQ_F32, false>(w, scales, zeros, R, K, group_size, 0, 15, qweight, scales_f16_out, qzeros, st);
+    else if (dtype == LCQ_BF16) launch_awq_team<LCQ_BF16, false>(w, scales, zeros, R, K, group_size, 0, 15, qweight, scales_f16_out, qzeros, st);
+    else if (dtype == LCQ_F16) launch_awq_team<LCQ_F16, false>(w, scales, zeros, R, K, group_size, 0, 15, qweight, scales_f16_out, qzeros, st);
     else return LCQ_EDTYPE;
     LCQ_CHECK_LAUNCH();
     return LCQ_OK;
