@@ -132,7 +132,9 @@ int lcq_qparams_int(const void* min_in, const void* max_in, int dtype, int64_t n
 /* get_mse_range, quant.py:147-205 (calib_algo 'mse'): per row the shrunken range p * (min, max), p = 1 - i / grid_n,
  * i < steps, with the smallest sum_j |quant_dequant(x_j) - x_j| ^ norm; a better step replaces the range the next
  * steps shrink (the reference's aliasing of best_min_val with min_val).  x [rows, cols] of `dtype`, arithmetic and
- * outputs [rows] in fp32 (the reference upcasts with tensor.float()). */
+ * outputs [rows] in fp32 (the reference upcasts with tensor.float()).  Errors are fp32 sums of 64 partial sums, IEEE
+ * quotients and powf; two steps whose errors tie to the last bits may be told apart otherwise by sums in another order
+ * (torch's on the CPU or the GPU), but every kernel behind this entry point decides alike. */
 int lcq_mse_range(const void* x, int dtype, int64_t rows, int64_t cols, float qmin, float qmax, int flags, int steps,
                   int grid_n, float norm, float* min_out, float* max_out, void* stream);
 
@@ -408,7 +410,8 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
 
 /* The same search in the reference's own rounding sequence (every product rounded to bf16, fp32 group sums rounded, the
  * squared difference and the mean rounded; auto_clip.py:83-191 with clip_version v1, weight-only), one launch:
- *  w [R, K], x [T, K] LCQ_BF16; group_size 32, 64 or 128, K % group_size == 0; n_steps <= LCQ_CLIP_MAX_STEPS
+ *  w [R, K], x [T, K] LCQ_BF16; group_size 32, 64 or 128, K % group_size == 0; n_steps <= n_grid, LCQ_CLIP_MAX_STEPS;
+ *  rows do not mix: an infinite or NaN product spoils the errors of its row and group, which keeps its whole range
  *  best_max, best_min [R, G] bf16 out; errs [R, G, n_steps] fp32 out: the errors as compared (rounded to bf16). */
 #define LCQ_CLIP_MAX_STEPS 12
 int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, int64_t T, int group_size, int n_grid,

@@ -10,8 +10,8 @@ Two search paths:
 * the default follows the reference's rounding sequence: every product of ``(x * w)`` rounded to the tensors' type,
   fp32 sums per group, the two sums rounded before they are subtracted, the squared difference rounded, the mean over
   tokens rounded.  The common case (v1, weight-only, one bf16 input, groups of 32 / 64 / 128) is one launch that keeps
-  the candidates on the chip (``lcq_clip_search_exact``); everything else runs step by step (``lcq_group_dots``): weights go through the quantizer classes exactly as the reference's
-  ``fake_quantize_weight`` / ``fake_quantize_input`` do.  It covers ``clip_version`` v1 and v2, ``w_only`` True and
+  the candidates on the chip (``lcq_clip_search_exact``); everything else runs step by step (``lcq_group_dots``): weights
+  go through the quantizer classes exactly as the reference's ``fake_quantize_weight`` / ``fake_quantize_input`` do.  It covers ``clip_version`` v1 and v2, ``w_only`` True and
   False, any group size or per_channel weights, bf16 and fp32, several inputs;
 * ``AutoClipper.fast = True`` selects, where it applies (v1, weight-only, per_group 128, bf16, min/max integer
   quantizer), one bf16 MFMA kernel (``lcq_awq_clip_search``) that contracts the weight *difference* with the tokens

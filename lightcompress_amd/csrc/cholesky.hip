@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256) void build_gather_kernel(const float* __restri
 // Diagonal block: Cholesky factor L11 of a 128x128 block and its inverse, one workgroup of 8 waves.
 // A wave that is alone on its SIMD issues about one instruction per 8 cycles, and a column-by-column sweep with a
 // barrier per column executes ~150 instructions per column in every wave: 70 us per block, none of it arithmetic.
-// Here the 128 columns are 8 panels of 16, and the serial part of a panel runs in ONE wave without barriers:
+// Here the 128 columns are 8 panels of 16, and the serial part of a panel runs without barriers in one to three waves, a row per lane:
 //   * waves 0-3 ("update waves") hold the lower triangle in registers, 8x8 per thread, dealt out cyclically (thread
 //     (ty, tx) owns rows ty + 16 ii and columns tx + 16 cc);
 //   * waves 4, 6 and 7 ("panel waves") take the current 16-column panel from LDS with one row per lane and factor it in

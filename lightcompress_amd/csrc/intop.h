@@ -82,10 +82,11 @@ struct IntOp {
       if (__builtin_expect(((f2u(q) & 0xffffu) - 0x7ff8u) <= 0x10u, 0)) q = a / c;
       return rnd<BF>(q);
     } else {
-      // the correctly rounded quotient without the division sequence: q0 is within an ulp of a / c and rc is the correctly
-      // rounded reciprocal of c (a small integer or a format's maximum, far from the all-ones significand the theorem
-      // excludes), so one residual step rounds correctly (Markstein, IBM J. R&D 34(1), 1990); a >= 1e-5 and the launch
-      // constants keep everything away from the subnormals, an infinite or NaN a is handed on by q0
+      // the correctly rounded quotient without the division sequence: the product with the correctly rounded reciprocal and
+      // one residual step (Markstein, IBM J. R&D 34(1), 1990).  q0 may be 1.5 ulp off (c = 255), which the theorem does not
+      // cover in general; that one step is enough for these constants, which have few significant bits, was checked with
+      // every significand of a for c = 1 .. 512, 2^n - 1 up to 65535 and 57344.  a >= 1e-5 and the constants keep
+      // everything away from the subnormals, an infinite or NaN a is handed on by q0
       const float q0 = a * rc;
       const float q = __builtin_fmaf(__builtin_fmaf(-c, q0, a), rc, q0);
       return rnd<BF>(fabsf(q0) < __builtin_inff() ? q : q0);       // fp16: the quotient, rounded
