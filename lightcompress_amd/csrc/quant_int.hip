@@ -202,16 +202,18 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
 // The estimate and mse_row_error differ by a relative delta at most (mse_margin below).  Where `margin` cannot tell the two
 // steps apart, the wave evaluates mse_row_error for both of them, so the range is always the one mse_range_kernel finds: an
 // estimate that decides ties by itself picked another range for one group in 16000.  A step with the scale and zero point of
-// the best one (a clamped scale) has its error and is not better.  Rows whose largest value is outside 2^-16 .. 2^16, where
-// powers of the unscaled errors may over- or underflow, and rows with infinities or NaN are always evaluated; so are
-// estimates below SMALL, next to which underflowed terms might count.
+// the best one (a clamped scale) has its error and is not better.  Rows whose largest value is below `small` or above
+// `large`, where powers of the unscaled errors may under- or overflow, are always evaluated, and so are estimates below
+// MSE_SMALL, next to which underflowed terms might count: small = 2^(-68 / norm), 2^-28 for 2.4, leaves MSE_SMALL small^norm = 2^-91,
+// 2^21 times the 2^-112 that 2^14 underflowed terms can come to; large = 2^(113 / norm - 1), 2^46 for 2.4, keeps 2^14 terms of at
+// most (2 large)^norm below 2^127.  In a row with an infinity or a NaN the error of every step is NaN: it keeps its range.
 // What bounds it: ten instructions per element and step, two of them transcendental (about 50 vector cycles).  4096 x 4096
 // bf16 in groups of 128, 4 bits, 80 steps: 1864 us re-reading, 497 with the row in registers, 199 with the steps cut short,
 // 204 with the undecided ones evaluated (4096 rows of 4096: 1268, 437, 366, 380).
 constexpr float MSE_SMALL = 1.1920929e-7f;                   // 2^-23, in units of (largest value of the row, 1 .. 2) ^ norm
 template <int BF, int TEAM, int PER>
 __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restrict__ x, int64_t rows, int cols, int vec, int steps,
-                                                             int grid_n, float norm, float margin, IntOp<0, false> op,
+                                                             int grid_n, float norm, float margin, float small, float large, IntOp<0, false> op,
                                                              float* __restrict__ mn_out, float* __restrict__ mx_out) {
   constexpr int N = Vec<BF>::N;
   constexpr bool BLOCK = TEAM > 64;
@@ -221,8 +223,7 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
   for (int i = threadIdx.x; i < steps; i += 256) shrink[i] = (float)(1.0 - (double)i / (double)grid_n);
   __syncthreads();
   const int64_t row_ = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TEAM;
-  const bool live = row_ < rows;
-  const int64_t row = live ? row_ : rows - 1;                // surplus teams repeat the last row and store nothing
+  const int64_t row = row_ < rows ? row_ : rows - 1;         // surplus teams repeat the last row and store nothing
   const int t = threadIdx.x % TEAM, lane = threadIdx.x & 63;
   float v[PER], mn = __builtin_inff(), mx = -__builtin_inff();
   if (vec) {
@@ -257,7 +258,8 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
   float cur_min = mn, cur_max = mx;
   // 2^k with 2^k max|x| in [1, 2)
   const float big = fmaxf(fabsf(mn), fabsf(mx));
-  const bool regular = mn == mn && mx == mx && big >= 1.52587890625e-5f && big <= 65536.0f;
+  const bool live = row_ < rows && mn > -__builtin_inff() && mx < __builtin_inff();       // (NaN: false)
+  const bool regular = live && big >= small && big <= large;
   const int e = regular ? (int)(f2u(big) >> 23) : 127;
   const float up = u2f((uint32_t)(254 - e) << 23), down = u2f((uint32_t)e << 23);
   #pragma unroll
@@ -306,12 +308,12 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
       have = close;
       if (close) best = exact;
       if (regular) {
-        hi = live ? fmaxf(sum * (1.0f + margin), MSE_SMALL) : -1.0f;
+        hi = fmaxf(sum * (1.0f + margin), MSE_SMALL);
         lo = sum >= MSE_SMALL ? sum * (1.0f - margin) : -__builtin_inff();
       }
     }
   }
-  if (t == 0 && live) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
+  if (t == 0 && row_ < rows) { mn_out[row] = cur_min; mx_out[row] = cur_max; }
 }
 
 // Two estimates that differ by more than this tell which of the two errors is larger.  delta bounds the relative difference
@@ -333,7 +335,7 @@ int run_mse(const void* x, int64_t rows, int64_t cols, int steps, int grid_n, fl
   const int vec = cols % N == 0 && (uintptr_t)x % 16 == 0;
   #define LCQ_MSE(T, P) do { const int64_t grid = (rows * T + 255) / 256; if (grid > 0x7fffffff) return LCQ_EINVAL; \
     mse_range_team_kernel<BF, T, P><<<dim3((unsigned)grid), dim3(256), 0, st>>>(x, rows, (int)cols, vec, steps, grid_n, norm, \
-        mse_margin(cols, P, op.qrange, norm), op, min_out, max_out); \
+        mse_margin(cols, P, op.qrange, norm), ldexpf(1.0f, -(int)(68.0f / norm)), ldexpf(1.0f, (int)(113.0f / norm) - 1), op, min_out, max_out); \
     return LCQ_OK; } while (0)
   if (op.round_zp && op.qmin <= 0.0f && op.qmax >= 0.0f && op.qrange <= 512.0f && norm > 2.0f && norm <= 4.0f && steps <= 256) {
     // Many elements per lane amortise the step's row arithmetic, but below 20000 rows such waves are too few to fill the
