@@ -116,6 +116,8 @@ class AutoClipper:
         for i in range(len(inputs)):
             inputs[i] = inputs[i].to(w.device)
             x = inputs[i].view(-1, inputs[i].shape[-1])
+            if x.shape[1] != K:                          # the kernels read K columns per token
+                raise ValueError(f'activations of {x.shape[1]} features in front of {K} in_features')
             if self.padding_mask and self.padding_mask[i].numel() == x.shape[0]:
                 x = x[self.padding_mask[i].flatten().bool()]
             if n_sample_token is None:

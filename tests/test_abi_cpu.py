@@ -119,3 +119,12 @@ def test_clip_search_asks_overridden_quantization_step_by_step():
                                   (OwnClipper, IntegerQuantizer, False)):
         clipper = cls(True, quantizer(4, False, 'per_group', group_size=128), None, 'v1', False, False, None)
         assert clipper._fused_applies(w, [x], 10) == takes
+
+
+def test_clip_search_refuses_activations_of_another_width():
+    """The kernels read in_features columns per token: a narrower tensor is refused before any launch."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    clipper = AutoClipper(True, IntegerQuantizer(4, False, 'per_group', group_size=128), None, 'v1', False, False, None)
+    with pytest.raises(ValueError):
+        clipper.auto_clip_layer(0, 'fc', torch.zeros(64, 256, dtype=torch.bfloat16), [torch.zeros(4, 128, dtype=torch.bfloat16)])
