@@ -229,38 +229,43 @@ def bench_hessian(args, out, x=None):
     nb = x.shape[0]
     H = torch.zeros(K, K, device=dev)
     lib, st = L.lib(), L.stream()
-    # the launch add_batch issues: lcq_hessian_accum_balanced (the tiles of the last round of workgroups cut into token
-    # ranges; the small launch that folds their partial sums into H is part of the timed call)
-    ws_bytes = lib.lcq_hessian_balanced_workspace_bytes(L.i64(K), L.i64(TL))
+    # the launch add_batch issues: lcq_hessian_accum_packed on tokens staged by lcq_hessian_pack (the small launch that folds
+    # the partial sums of cut tiles into H is part of the timed call; the packing is timed by itself)
+    ws_bytes = lib.lcq_hessian_packed_workspace_bytes(L.i64(K), L.i64(TL))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+    packed = []
+    for b in range(0, min(nb, 3 * FOLD) - FOLD + 1, FOLD):
+        packed.append(torch.empty(lib.lcq_hessian_packed_bytes(K, TL) // 2, dtype=torch.bfloat16, device=dev))
+        for j in range(FOLD):
+            L.check(lib.lcq_hessian_pack(L.ptr(x[b + j]), L.BF16, TOK, K, K, j * TOK, L.ptr(packed[-1]), None, st), 'pack')
+    t_pack = timeit(lambda i: L.check(lib.lcq_hessian_pack(L.ptr(x[i % nb]), L.BF16, TOK, K, K, (i % FOLD) * TOK,
+                                                           L.ptr(packed[0]), None, st), 'pack'), 32, 8)
 
     def hess(b):
-        b = (b * FOLD) % (nb - FOLD + 1)
-        L.check(lib.lcq_hessian_accum_balanced(L.ptr(H), L.i64(K), L.ptr(x[b]), L.ptr(x[b]), L.i32(L.BF16), L.i64(TL), L.i64(K),
-                                               L.f32(0.5), L.f32(0.01), L.ptr(ws), L.i64(ws_bytes), st), 'hessian')
-    t_h = timeit(hess, 32, 16)
+        xp = L.ptr(packed[b % len(packed)])
+        L.check(lib.lcq_hessian_accum_packed(L.ptr(H), K, xp, xp, L.BF16, TL, 0.5, 0.01, L.ptr(ws), ws_bytes, st), 'hessian')
+    t_h = timeit(hess, 16, 8)
     # the vendor library on the same operands, for scale: the full product X^T X as one bf16 GEMM through torch
     # (hipBLASLt; bf16 output, no accumulation into H), same token-major layout of both operands
     xl = [x[b * FOLD:(b + 1) * FOLD].reshape(TL, K) for b in range(nb // FOLD)]
     t_lib = timeit(lambda i: torch.matmul(xl[i % len(xl)].t(), xl[i % len(xl)]), 8, 3)
     alg_flops = 2.0 * TL * K * K
-    tiles = sum(K // 128 - 2 * ti for ti in range(K // 256))          # 256x128 tiles that reach the upper triangle
-    exe_flops = 2.0 * TL * tiles * 256 * 128
-    traffic, stale = traffic_bytes('hessian_kernel_K14336_T8192', t_h * 1e6) if FOLD == 4 else (None, None)
+    tiles = sum(K // 256 - ti for ti in range(K // 256))              # 256x256 tiles that reach the upper triangle
+    exe_flops = 2.0 * TL * tiles * 256 * 256
+    traffic, stale = traffic_bytes('hessian_packed_kernel_K14336_T32768', t_h * 1e6) if TL == 32768 else (None, None)
     out['roofline'] = {
-        'kernel': f'hessian_kernel<bf16> K=14336 T={TL} (+ tail_fold_kernel)', 'bound': 'mfma', 'achieved': round(exe_flops / t_h / 1e12, 2),
+        'kernel': f'hessian_packed_kernel<bf16> K=14336 T={TL} (+ packed_fold_kernel)', 'bound': 'mfma', 'achieved': round(exe_flops / t_h / 1e12, 2),
         'peak': 2500.0, 'unit': 'TFLOP/s', 'frac': round(exe_flops / t_h / 2.5e15, 4),
         'traffic': traffic, 'traffic_stale': stale,
-        'launch_us': round(t_h * 1e6, 2), 'flop_executed_per_launch': exe_flops,
+        'launch_us': round(t_h * 1e6, 2), 'pack_us_per_call': round(t_pack * 1e6, 2), 'flop_executed_per_launch': exe_flops,
         'algorithmic_tflops': round(alg_flops / t_h / 1e12, 2), 'frac_algorithmic': round(alg_flops / t_h / 2.5e15, 4),
         'library_gemm': {'what': 'torch.matmul(X.t(), X), bf16, the whole K x K product on the same tokens (hipBLASLt)',
                          'us': round(t_lib * 1e6, 1), 'tflops': round(alg_flops / t_lib / 1e12, 1),
                          'frac': round(alg_flops / t_lib / 2.5e15, 4)},
-        'note': 'achieved / frac count the flops the matrix pipes execute (the 256x128 tiles that reach the upper '
+        'note': 'achieved / frac count the flops the matrix pipes execute (the 256x256 tiles that reach the upper '
                 'triangle of the symmetric H: matrix-pipe utilisation against the 2.4 GHz peak); the algorithmic figure '
-                '2*T*K^2 of the full product X^T X per launch is in algorithmic_tflops / frac_algorithmic.  rocprofv3 '
-                'counters (profiles/) show the pipes busy for 3/4 of the cycles at a shader clock the chip holds near '
-                '1.4 GHz under this kernel'}
+                '2*T*K^2 of the full product X^T X per launch is in algorithmic_tflops / frac_algorithmic.  The chip '
+                'clocks down under random operands (profiles/)'}
 
 
 # ---------------------------------------------------------------------------------------------------------------

@@ -257,6 +257,26 @@ int64_t lcq_hessian_balanced_workspace_bytes(int64_t K, int64_t T);
 int lcq_hessian_accum_balanced(float* H, int64_t K, const void* XA, const void* XB, int dtype, int64_t T, int64_t ldx, float alpha,
                                float beta, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same update from tokens that were staged in the order the matrix pipe reads them (the kernel of choice where several
+ * calls are folded into one launch; hessian.hip describes the layout).
+ * lcq_hessian_packed_bytes(K, T): size of a buffer for T tokens (whole 32-token slabs, K up to a multiple of 256).
+ * lcq_hessian_pack writes tokens x [T, K] (row pitch ldx elements, % 8 == 0; LCQ_BF16 | LCQ_F16 | LCQ_F32, 16-byte aligned;
+ *   K % 8 == 0) to positions at .. at + T of the buffer and zeros behind them to the end of the slab; earlier positions
+ *   stay.  T == 0 only writes the zeros (x may be NULL).  fp32: packed <- bf16(x), packed_lo <- bf16(x - bf16(x)).
+ * lcq_hessian_compare_packed sets *flag = 1 if the tokens differ from positions at .. at + T (never clears it).
+ * lcq_hessian_accum_packed: H <- alpha*H + beta * XA^T XB over positions 0 .. T (T <= 2^26), as lcq_hessian_accum_ab; the
+ *   positions up to the end of the last slab must hold zeros (as lcq_hessian_pack leaves them).  dtype LCQ_BF16 | LCQ_F16;
+ *   workspace of lcq_hessian_packed_workspace_bytes(K, T) (0: none), everything 16-byte aligned.  Reproducible: runs of slabs
+ *   of one tile are summed in a fixed order. */
+int64_t lcq_hessian_packed_bytes(int64_t K, int64_t T);
+int lcq_hessian_pack(const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, void* packed, void* packed_lo,
+                     void* stream);
+int lcq_hessian_compare_packed(const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, const void* packed,
+                               const void* packed_lo, int* flag, void* stream);
+int64_t lcq_hessian_packed_workspace_bytes(int64_t K, int64_t T);
+int lcq_hessian_accum_packed(float* H, int64_t K, const void* XA, const void* XB, int dtype, int64_t T, float alpha, float beta,
+                             void* workspace, int64_t workspace_bytes, void* stream);
+
 /* H_0 <- ((H_0 + H_1) + H_2) + ... and H_s <- 0 for s >= 1, over all K*K entries: the shares of
  * lcq_hessian_accum_sliced back into the one matrix that gptq.py keeps (layers_cache[name]['H']); accumulation may
  * go on afterwards.  H 16-byte aligned, slice_stride % 4 == 0. */

@@ -350,6 +350,292 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(float* __restrict__ H, i
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same update from staged tokens (lcq_hessian_pack -> lcq_hessian_accum_packed)
+//
+// add_batch copies its tokens to a staging buffer anyway, so the copy lays them out as the matrix pipe reads them: one
+// 16-byte piece holds 8 consecutive tokens of one feature, and the 64 pieces of a v_mfma_f32_32x32x16 operand (32 features
+// x 16 tokens, lane l: feature l % 32, tokens 8 (l / 32) .. + 7) are 1 KiB in a row:
+//   piece(token t, feature f) = (((t / 16) * Kp / 32 + f / 32) * 2 + (t / 8) % 2) * 32 + f % 32,   Kp = K up to a multiple of 256.
+// A wave's direct load moves one operand, an operand is one conflict-free ds_read_b128, and neither needs a swizzle or the
+// transposing reads (which move 64 bytes per clock where ds_read_b128 moves 128).
+//
+//  * a workgroup owns a 256 x 256 tile of H, four waves of 128 x 128 (4 x 4 accumulators of 32x32 = all 256 AGPRs), one
+//    wave per SIMD: per 16 tokens 8 operand reads feed 16 matrix instructions.  The 128 x 64 waves of hessian_kernel read
+//    half as much again per product, and their LDS (reads and direct loads together) is busy longer than their matrix pipe;
+//  * operands are double-buffered in registers: while the products of one 16-token step run, the reads of the next are
+//    issued between them, two matrix instructions apart, and every fourth gap takes one direct load (in one burst the
+//    loads of four waves queue up behind each other);
+//  * four LDS stages of 32 tokens, one barrier per slab: at the middle of a slab every wave holds the rest of it in
+//    registers, so its stage is free for the slab four ahead.
+// The chip clocks down under this load (random tokens 1.7 GHz, zeros run 1.3 times as fast), which is what bounds it.
+// Measured on one box (us, without the copy): K = 14336, 32768 tokens 5919 -> 5010 (1.37 PFLOP/s of the tiles computed),
+// K = 4096, 65536 tokens 1064 -> 861, K = 8192, 32768 tokens 2026 -> 1622, K = 2048, 65536 tokens 305 -> 245; against
+// hessian_kernel with the token shares or split rounds it had for the same work.
+typedef const __attribute__((address_space(3))) char* lds_ptr;
+typedef const __attribute__((address_space(3))) s16x8* lds_frag;
+constexpr int PT = 256;                             // tile of H
+constexpr int P_STAGES = 4, P_HALF = BT * PT * 2, P_STAGE = 2 * P_HALF;
+
+// Which part of which tile a workgroup computes.  Tiles [0, full) fill whole rounds of the chip's CUs, one workgroup each.
+// The rest would leave CUs idle for the time of a tile and is cut along the tokens: m[0] tiles into c[0] pieces each, the
+// m[1] tiles behind them into c[1] pieces (packed_plan).  Piece 0 of a tile updates H; the others leave beta * (their X^T X) in
+// scratch tiles, which packed_fold_kernel adds to H in order.  All tiles of a level are cut at the same tokens and the
+// workgroups of an XCD take the same piece of neighbouring tiles, so they read the same slabs of X at the same time (cut
+// into runs that wander over tile boundaries the launch fetches X from beyond L2: 700 against 462 us for K = 4096, T = 32768).
+struct PackedPlan {
+  int full, slabs;
+  int m[2], c[2];
+  float* scratch;                                   // sum of m (c - 1) tiles of PT x PT floats
+};
+__host__ __device__ __forceinline__ int level_blocks(const PackedPlan& p, int l) { return (p.m[l] * p.c[l] + 7) / 8 * 8; }
+
+template <bool IS_BF16, bool EDGE>
+__global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void hessian_packed_kernel(float* __restrict__ H, int K, const uint16_t* __restrict__ XA, const uint16_t* __restrict__ XB, float alpha,
+                           float beta, int nt, PackedPlan plan) {
+  __shared__ __attribute__((aligned(1024))) char lds[P_STAGES * P_STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 1, wc = wave & 1;
+  const int n = plan.slabs;
+  const int64_t slab = (int64_t)nt * PT * BT;                 // elements of 32 tokens
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds;
+  const lds_ptr readA = (lds_ptr)lds + lane * 16 + wr * 4096, readB = (lds_ptr)lds + P_HALF + lane * 16 + wc * 4096;
+
+  int v, s0 = 0, s1 = n;                            // tile, slabs
+  int64_t scratch = -1;
+  {
+    int b = blockIdx.x;
+    if (b < plan.full) {
+      // block b runs on XCD b % 8: every XCD takes a contiguous range of the tile order
+      v = (b & 7) * (plan.full >> 3) + (b >> 3);
+    } else {
+      b -= plan.full;
+      const int l = b >= level_blocks(plan, 0);
+      if (l) b -= level_blocks(plan, 0);
+      const int m = plan.m[l], c = plan.c[l];
+      const int i = (b & 7) * (level_blocks(plan, l) >> 3) + (b >> 3);
+      if (i >= m * c) return;
+      const int piece = i / m, t = i - piece * m;
+      v = plan.full + (l ? plan.m[0] : 0) + t;
+      s0 = (int)((int64_t)piece * n / c);
+      s1 = (int)((int64_t)(piece + 1) * n / c);
+      if (piece > 0) scratch = (l ? (int64_t)plan.m[0] * (plan.c[0] - 1) : 0) + (int64_t)t * (c - 1) + piece - 1;
+    }
+  }
+  int ti, tj;
+  decode_tile<1>(v, nt, nt, ti, tj);
+  const int steps = s1 - s0;
+  const uint16_t* const A0 = XA + (int64_t)s0 * slab;
+  const uint16_t* const B0 = XB + (int64_t)s0 * slab;
+  uint32_t gof[8];                                // this wave's pieces of a slab: operands wave * 4 + p of A, then of B
+  #pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int c = wave * 4 + p;                   // 16-token group c / 8, feature block c % 8
+    gof[p] = ((c >> 3) * (nt * 8) + ti * 8 + (c & 7)) * 1024u + lane * 16;
+    gof[4 + p] = ((c >> 3) * (nt * 8) + tj * 8 + (c & 7)) * 1024u + lane * 16;
+  }
+  const auto gload = [&](const uint16_t* a, const uint16_t* b, uint32_t dst, int p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 ::"s"(dst + (p >> 2) * P_HALF + (p & 3) * 1024), "v"(gof[p]), "s"(p < 4 ? a : b) : "memory");
+  };
+  f32x16 acc[4][4];
+  #pragma unroll
+  for (int i = 0; i < 4; ++i)
+    #pragma unroll
+    for (int j = 0; j < 4; ++j)
+      #pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+  s16x8 fr[2][8];                                 // two sets of operands: A 0..3, B 0..3
+  const auto rd = [&](int set, int f, uint32_t stage, int ks) {
+    fr[set][f] = *(lds_frag)((f < 4 ? readA : readB) + stage + (f & 3) * 1024 + ks * 8192);
+  };
+  constexpr int ORDER[8] = {4, 0, 1, 2, 3, 5, 6, 7};                     // as the products need them
+  constexpr int READ_AT[16] = {0, 1, 2, -1, 3, -1, 4, -1, 5, -1, 6, -1, 7, -1, -1, -1};
+
+  // Slabs 0 .. P_STAGES - 2 and half of the next; past the last slab a load fetches the first one again (its stage is
+  // never read), so that the number of loads in flight is always the same.
+  #pragma unroll
+  for (int s = 0; s < P_STAGES; ++s) {
+    const int64_t at = s < steps ? s * slab : 0;
+    #pragma unroll
+    for (int p = 0; p < (s == P_STAGES - 1 ? 4 : 8); ++p) gload(A0 + at, B0 + at, lds0 + s * P_STAGE + wave * 4096, p);
+  }
+  constexpr int FIRST = (P_STAGES - 1) * 8 - 4, LATER = (P_STAGES - 2) * 8;
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (FIRST & 15) | ((FIRST >> 4) << 14));
+  __syncthreads();
+  #pragma unroll
+  for (int f = 0; f < 8; ++f) rd(0, ORDER[f], 0, 0);
+  int64_t at = P_STAGES - 1 < steps ? (P_STAGES - 1) * slab : 0;
+  uint32_t cur = 0, dst = lds0 + (P_STAGES - 1) * P_STAGE + wave * 4096;
+  __builtin_amdgcn_sched_barrier(0);
+  int s = 0;
+  do {                                            // (a piece has at least one slab)
+    // tokens 0..15 of the slab; meanwhile the reads of tokens 16..31, and the B half of the loads three slabs ahead
+    #pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      acc[m & 3][m >> 2] = mfma<IS_BF16>(fr[0][m & 3], fr[0][4 + (m >> 2)], acc[m & 3][m >> 2]);
+      if (READ_AT[m] >= 0) rd(1, ORDER[READ_AT[m]], cur, 1);
+      if ((m & 3) == 3) gload(A0 + at, B0 + at, dst, 4 + (m >> 2));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // The next slab has landed (the loads of the two behind it may be in flight) and this one is in registers, in every
+    // wave: its stage takes the slab four ahead.
+    __builtin_amdgcn_s_waitcnt(0x0070 | (LATER & 15) | ((LATER >> 4) << 14));
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t nxt = (cur == (P_STAGES - 1) * P_STAGE) ? 0 : cur + P_STAGE;
+    at = s + P_STAGES < steps ? at + slab : 0;
+    dst = lds0 + cur + wave * 4096;
+    #pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      acc[m & 3][m >> 2] = mfma<IS_BF16>(fr[1][m & 3], fr[1][4 + (m >> 2)], acc[m & 3][m >> 2]);
+      if (READ_AT[m] >= 0) rd(0, ORDER[READ_AT[m]], nxt, 0);
+      if ((m & 3) == 3) gload(A0 + at, B0 + at, dst, m >> 2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur = nxt;
+  } while (++s < steps);
+  __builtin_amdgcn_s_waitcnt(0x0070);             // nothing may still be on its way to LDS when the workgroup ends
+
+  // accumulator register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
+  const bool to_scratch = scratch >= 0;
+  const bool rmw = !to_scratch && alpha != 0.0f;
+  const int row = wr * 128 + 4 * (lane >> 5), col = wc * 128 + (lane & 31);
+  char* out = (char*)(to_scratch ? plan.scratch + scratch * (PT * PT) : H + (int64_t)(ti * PT) * K + tj * PT);
+  uint32_t pitch = 4 * (to_scratch ? PT : K);     // bytes
+  const uint32_t at0 = row * pitch + 4 * col;
+  const int rows = EDGE && !to_scratch ? K - (ti * PT + row) : PT, cols = EDGE && !to_scratch ? K - (tj * PT + col) : PT;
+  const auto cell = [&](int i, int j, int r) { return at0 + (i * 32 + 8 * (r >> 2) + (r & 3)) * pitch + j * 128; };
+  const auto inside = [&](int i, int j, int r) { return !EDGE || (i * 32 + 8 * (r >> 2) + (r & 3) < rows && j * 32 < cols); };
+  #pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // (the accumulators stay where they are until their turn: copied out together they would not fit the other registers)
+    asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]));
+    float old[4][16];
+    if (rmw) {
+      #pragma unroll
+      for (int j = 0; j < 4; ++j)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) old[j][r] = *(float*)(out + (inside(i, j, r) ? cell(i, j, r) : 0u));     // (all loads in flight)
+    }
+    #pragma unroll
+    for (int j = 0; j < 4; ++j)
+      #pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float w = beta * acc[i][j][r];
+        if (rmw) w = alpha * old[j][r] + w;
+        if (inside(i, j, r)) *(float*)(out + cell(i, j, r)) = w;
+      }
+  }
+}
+
+// H tile <- ((H tile + piece 1) + piece 2) + ... for the tiles that were cut: grid (tiles, 16), 16 rows per workgroup.
+__global__ __launch_bounds__(256) void packed_fold_kernel(float* __restrict__ H, int K, int nt, PackedPlan plan) {
+  int ti, tj;
+  decode_tile<1>(plan.full + blockIdx.x, nt, nt, ti, tj);
+  const int l = (int)blockIdx.x >= plan.m[0], t = blockIdx.x - (l ? plan.m[0] : 0), pieces = plan.c[l] - 1;
+  const float* const sc = plan.scratch + ((l ? (int64_t)plan.m[0] * (plan.c[0] - 1) : 0) + (int64_t)t * pieces) * (PT * PT);
+  const int c = (threadIdx.x & 63) * 4;
+  if (pieces <= 0 || tj * PT + c >= K) return;
+  #pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int row = blockIdx.y * 16 + (threadIdx.x >> 6) * 4 + k;
+    if (ti * PT + row >= K) return;
+    float* const hp = H + (int64_t)(ti * PT + row) * K + tj * PT + c;     // K % 8 == 0: four columns or none
+    f32x4 h = *(const f32x4*)hp;
+    #pragma unroll 4
+    for (int i = 0; i < pieces; ++i) {
+      const f32x4 w = *(const f32x4*)(sc + (int64_t)i * (PT * PT) + row * PT + c);
+      h[0] += w[0]; h[1] += w[1]; h[2] += w[2]; h[3] += w[3];
+    }
+    *(f32x4*)hp = h;
+  }
+}
+
+// Tokens [0, T) of x to positions [p0, p0 + T) of a packed buffer, zeros behind them up to a multiple of 32; what lies before
+// p0 stays.  A lane turns an 8 x 8 block (8 positions, 8 features), a wave 8 positions x 512 features; the pieces change lanes
+// through LDS so that a store instruction writes whole lines (37 -> 22 us for 2048 x 14336, the time of a plain copy).
+// F32: hi = bf16(x) to `out`, bf16(x - hi) to `lo`.  COMPARE: nothing is written, *flag = 1 if any of the T tokens differs
+// from what the buffer holds.
+template <bool F32, bool COMPARE>
+__global__ __launch_bounds__(256) void pack_tokens_kernel(const void* __restrict__ x, int64_t ldx, int K, int oct, int64_t p0, int64_t T,
+                                                          int64_t rows, u32x4* __restrict__ out, u32x4* __restrict__ lo,
+                                                          int* __restrict__ flag) {
+  __shared__ u32x4 turn[4][64 * 8];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunks = (oct + 63) / 64;
+  const int64_t id = (int64_t)blockIdx.x * 4 + wave, row = id / chunks, q = p0 / 8 + row;      // positions 8 q .. 8 q + 7
+  if (row >= rows) return;
+  const int o0 = (int)(id - row * chunks) * 64, o = o0 + lane;          // features 8 o .. 8 o + 7
+  uint32_t w[8][4], l[8][4];                        // token k: four pairs of features
+  #pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int64_t t = 8 * q + k - p0;
+    const bool ok = t >= 0 && t < T && 8 * o < K;
+    if constexpr (F32) {
+      f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+      if (ok) {
+        const f32x4* const xp = (const f32x4*)((const float*)x + t * ldx + 8 * o);
+        a = __builtin_nontemporal_load(xp);
+        b = __builtin_nontemporal_load(xp + 1);
+      }
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e0 = i < 2 ? a[2 * i] : b[2 * i - 4], e1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+        const float h0 = bf16_round(e0), h1 = bf16_round(e1);
+        w[k][i] = bf16_pack(h0, h1);
+        l[k][i] = bf16_pack(bf16_round(e0 - h0), bf16_round(e1 - h1));
+      }
+    } else {
+      u32x4 a = {0, 0, 0, 0};
+      if (ok) a = __builtin_nontemporal_load((const u32x4*)((const uint16_t*)x + t * ldx + 8 * o));
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) w[k][i] = a[i];
+    }
+  }
+  const int skip = (int)max(p0 - 8 * q, (int64_t)0);                    // positions of the first piece that belong to earlier tokens
+  const int last = (int)min(p0 + T - 8 * q, (int64_t)8);                // positions from here on hold zeros
+  const auto emit = [&](const uint32_t (*v)[4], u32x4* dst) {
+    u32x4* const mine = turn[wave];
+    #pragma unroll
+    for (int f = 0; f < 8; ++f) {
+      u32x4 r;
+      #pragma unroll
+      for (int d = 0; d < 4; ++d)                   // tokens 2 d, 2 d + 1 of feature f
+        r[d] = __builtin_amdgcn_perm(v[2 * d + 1][f >> 1], v[2 * d][f >> 1], (f & 1) ? 0x07060302u : 0x05040100u);
+      mine[lane * 8 + (f ^ (lane & 7))] = r;        // (the exclusive or keeps eight lanes out of each other's banks)
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {                   // lane l: feature l % 8 of octet 8 j + l / 8
+      const int oo = 8 * j + (lane >> 3), f = lane & 7;
+      const u32x4 r = mine[oo * 8 + (f ^ (oo & 7))];
+      const int at = o0 + oo;
+      if (at >= oct) continue;
+      u32x4* const d = dst + (((q >> 1) * (oct >> 2) + (at >> 2)) * 2 + (q & 1)) * 32 + (at & 3) * 8 + f;
+      if constexpr (COMPARE) {
+        const u32x4 have = *d;
+        uint32_t diff = 0;
+        #pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (k >= skip && k < last) diff |= ((r[k >> 1] ^ have[k >> 1]) >> (16 * (k & 1))) & 0xffffu;
+        if (diff != 0) *flag = 1;                   // every writer stores the same value
+      } else if (skip == 0) {
+        __builtin_nontemporal_store(r, d);
+      } else {
+        #pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (k >= skip) ((uint16_t*)d)[k] = (uint16_t)(r[k >> 1] >> (16 * (k & 1)));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  emit(w, out);
+  if constexpr (F32) emit(l, lo);
+}
+
 // H_0 <- ((H_0 + H_1) + H_2) + ..., H_s <- 0 for s >= 1: the token slices of lcq_hessian_accum_sliced back into one matrix,
 // always in this order.
 __global__ __launch_bounds__(256) void gather_slices_kernel(f32x4* __restrict__ H, int64_t n4, int slices, int64_t stride4) {
@@ -535,6 +821,108 @@ static int hessian_launch(float* H, int64_t K, const void* X, const void* XB, in
   #undef LCQ_HESS
   if (ts.parts > 1)
     tail_fold_kernel<TN><<<dim3((unsigned)(8 * ts.rem_x), 8), dim3(256), 0, st>>>(H, (int)K, ntr, ntc, (int)total, ts);
+  LCQ_CHECK_LAUNCH();
+  return LCQ_OK;
+}
+
+// ---- staged tokens ----
+static int64_t packed_width(int64_t K) { return (K + PT - 1) / PT * PT; }
+
+int64_t lcq_hessian_packed_bytes(int64_t K, int64_t T) {
+  if (K <= 0 || K > (1 << 20) || T < 0 || T > 0x7fffffff - 31) return 0;
+  return (T + BT - 1) / BT * BT * packed_width(K) * 2;
+}
+
+static int pack_tokens(bool compare, const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, const void* packed,
+                       const void* packed_lo, int* flag, void* stream) {
+  if (!packed || (T > 0 && !x) || (compare && !flag) || T < 0 || at < 0 || K <= 0 || K % 8 != 0 || K > (1 << 20)) return LCQ_EINVAL;
+  if (ldx < K || ldx % 8 != 0) return LCQ_EINVAL;
+  if (dtype != LCQ_F32 && dtype != LCQ_BF16 && dtype != LCQ_F16) return LCQ_EDTYPE;
+  const bool f32 = dtype == LCQ_F32;
+  if (f32 && !packed_lo) return LCQ_EINVAL;
+  if ((((uintptr_t)x | (uintptr_t)packed | (uintptr_t)packed_lo) % 16) != 0 || ((uintptr_t)flag % 4) != 0) return LCQ_EALIGN;
+  if (at + T > 0x7fffffff - 31) return LCQ_ESIZE;
+  const int oct = (int)(packed_width(K) / 8);
+  // rows of pieces (8 positions) from the first one written to the end of its slab; a comparison stops at the last token
+  const int64_t rows = (compare ? (at + T + 7) / 8 : (at + T + BT - 1) / BT * (BT / 8)) - at / 8;
+  if (rows <= 0 || (compare && T == 0)) return LCQ_OK;
+  const int64_t grid = (rows * ((oct + 63) / 64) + 3) / 4;
+  if (grid > 0x7fffffff) return LCQ_ESIZE;
+  #define LCQ_PACK(F, C) pack_tokens_kernel<F, C><<<dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream>>>( \
+      x, ldx, (int)K, oct, at, T, rows, (u32x4*)packed, (u32x4*)packed_lo, flag)
+  if (f32) { if (compare) LCQ_PACK(true, true); else LCQ_PACK(true, false); }
+  else { if (compare) LCQ_PACK(false, true); else LCQ_PACK(false, false); }
+  #undef LCQ_PACK
+  LCQ_CHECK_LAUNCH();
+  return LCQ_OK;
+}
+
+int lcq_hessian_pack(const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, void* packed, void* packed_lo,
+                     void* stream) {
+  return pack_tokens(false, x, dtype, T, K, ldx, at, packed, packed_lo, nullptr, stream);
+}
+
+int lcq_hessian_compare_packed(const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, const void* packed,
+                               const void* packed_lo, int* flag, void* stream) {
+  return pack_tokens(true, x, dtype, T, K, ldx, at, packed, packed_lo, flag, stream);
+}
+
+// How a launch over T staged tokens is cut (see PackedPlan): of all pairs of levels the one with the shortest estimate, in
+// slabs' time.  A level runs its pieces side by side, n / c slabs; a round of workgroups costs START slabs for its first
+// loads and its epilogue; a scratch tile, written and read once by a chip that does nothing else, a twelfth of a slab.
+static PackedPlan packed_plan(int64_t K, int64_t T) {
+  constexpr double START = 16.0, TILE = 1.0 / 12;
+  const int64_t nt = packed_width(K) / PT, tiles = nt * (nt + 1) / 2;
+  int cus = hessian_slots() / 2 / 8 * 8;
+  if (cus < 8) cus = 8;
+  PackedPlan p{};
+  p.slabs = (int)((T + BT - 1) / BT);
+  p.full = (int)(tiles / cus * cus);
+  const int rest = (int)(tiles - p.full), n = p.slabs;
+  p.c[0] = p.c[1] = 1;
+  if (rest == 0) return p;
+  const auto level = [&](int m, int c) { return (double)((n + c - 1) / c) + START + TILE * m * (c - 1); };
+  double best = 1e30;
+  for (int c0 = 1; c0 <= cus && c0 <= n; ++c0) {
+    const int m0 = rest < cus / c0 ? rest : cus / c0, m1 = rest - m0;
+    const int most = m1 ? cus / m1 : 1;             // (m1 < cus)
+    for (int c1 = 1; c1 <= most && c1 <= n; ++c1) {
+      const double t = level(m0, c0) + (m1 ? level(m1, c1) : 0.0);
+      if (t < best) { best = t; p.m[0] = m0; p.c[0] = c0; p.m[1] = m1; p.c[1] = c1; }
+    }
+  }
+  return p;
+}
+static int64_t packed_scratch_tiles(const PackedPlan& p) {
+  return (int64_t)p.m[0] * (p.c[0] - 1) + (int64_t)p.m[1] * (p.c[1] - 1);
+}
+
+int64_t lcq_hessian_packed_workspace_bytes(int64_t K, int64_t T) {
+  if (K <= 0 || K > (1 << 20) || T <= 0 || T > (1 << 26)) return 0;
+  return packed_scratch_tiles(packed_plan(K, T)) * PT * PT * 4;
+}
+
+int lcq_hessian_accum_packed(float* H, int64_t K, const void* XA, const void* XB, int dtype, int64_t T, float alpha, float beta,
+                             void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!H || !XA || !XB || K <= 0 || K % 8 != 0 || K > (1 << 20) || T <= 0) return LCQ_EINVAL;
+  if (T > (1 << 26)) return LCQ_ESIZE;
+  if (dtype != LCQ_BF16 && dtype != LCQ_F16) return LCQ_EDTYPE;
+  if ((((uintptr_t)XA | (uintptr_t)XB | (uintptr_t)H | (uintptr_t)workspace) % 16) != 0) return LCQ_EALIGN;
+  PackedPlan p = packed_plan(K, T);
+  const int64_t need = packed_scratch_tiles(p) * PT * PT * 4;
+  if (need > 0 && (!workspace || workspace_bytes < need)) return LCQ_EWORKSPACE;
+  p.scratch = (float*)workspace;
+  const int nt = (int)(packed_width(K) / PT);
+  const int64_t grid = (int64_t)p.full + level_blocks(p, 0) + level_blocks(p, 1);
+  hipStream_t st = (hipStream_t)stream;
+  #define LCQ_HESSP(BF, E) hessian_packed_kernel<BF, E><<<dim3((unsigned)grid), dim3(256), 0, st>>>( \
+      H, (int)K, (const uint16_t*)XA, (const uint16_t*)XB, alpha, beta, nt, p)
+  const bool edge = K % PT != 0;
+  if (dtype == LCQ_BF16) { if (edge) LCQ_HESSP(true, true); else LCQ_HESSP(true, false); }
+  else { if (edge) LCQ_HESSP(false, true); else LCQ_HESSP(false, false); }
+  #undef LCQ_HESSP
+  if (need > 0)
+    packed_fold_kernel<<<dim3((unsigned)(p.m[0] + p.m[1]), PT / 16), dim3(256), 0, st>>>(H, (int)K, nt, p);
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

@@ -40,13 +40,13 @@ Differences a caller can observe
     instead of errors to later columns; the same results up to fp32 rounding (closer to fp64 than the reference's
     cholesky / cholesky_inverse / cholesky chain).  process_hessian_and_weights called on its own returns the
     reference's U;
-  * ``special.hessian_defer`` (default 'auto': 16 for K <= 4096, 8 for K <= 8192, else 4) add_batch calls are copied to a staging buffer and
-    folded into one launch, so ``layers_cache[name]['H']`` lags behind ``nsamples`` until
+  * ``special.hessian_defer`` add_batch calls (default 'auto': as many as make 8192 tokens for K <= 1024, 65536 for K <= 4096, 32768 above) are
+    copied to a staging buffer, in the order the matrix pipe reads them (lcq_hessian_pack), and folded into one launch, so ``layers_cache[name]['H']`` lags behind ``nsamples`` until
     ``hessian(name)``, ``hessian_sorting`` or ``process_hessian_and_weights`` settles it
     (``hessian_defer: 1`` updates H on every call);
-  * ``special.hessian_slices`` (default 'auto': 3 at K = 4096, 1 at K = 14336): a launch whose Hessian has too few
-    tiles to fill the chip cuts its tokens into that many shares, each with an accumulator of its own; the same
-    calls settle them into H (a sum in a fixed order; H differs from a single accumulator's by fp32 rounding);
+  * ``special.hessian_slices`` (default 'auto': 8 up to K = 512, else 1): with a number above 1 every launch cuts its tokens into that many
+    shares, each with an accumulator of its own; the same calls settle them into H (a sum in a fixed order; H differs
+    from a single accumulator's by fp32 rounding);
   * per-group qparams of the loop live in two [R, G] tensors instead of a
     Python list of dicts; ``layer.buf_scales`` / ``buf_zeros`` get the same
     [R*G, 1] layout the reference writes;
@@ -98,7 +98,7 @@ class GPTQ:
         # add_batch calls folded into one Hessian launch (1 = one launch per call)
         hd = special_config.get('hessian_defer', 'auto')
         self.hessian_defer = hd if hd == 'auto' else int(hd)
-        # token shares of one Hessian launch, each with an accumulator of its own ('auto': by the number of tiles)
+        # token shares of one Hessian launch, each with an accumulator of its own ('auto': by K)
         hs = special_config.get('hessian_slices', 'auto')
         self.hessian_slices = hs if hs == 'auto' else int(hs)
         # subset_transform starts the Cholesky chains of all Linears of a subset side by side (False: one by one)
@@ -208,11 +208,18 @@ class GPTQ:
         flag = lead.get('share_flag')
         if flag is None:
             flag = lead['share_flag'] = torch.zeros(1, dtype=torch.int32, device=stage.device)
-        es = stage.element_size()
-        off = (lead['stage_fill'] - tokens) * K * es
-        nbytes = tokens * K * es
         lo = lead.get('stage_lo')
         lib, st = L.lib(), L.stream()
+        at = lead['stage_fill'] - tokens
+        if lead['stage_packed']:
+            x = self._token_rows(inp, K)
+            L.check(lib.lcq_hessian_compare_packed(x.data_ptr(), L.dtype_code(x.dtype), tokens, K, K, at, stage.data_ptr(),
+                                                   0 if lo is None else lo.data_ptr(), flag.data_ptr(), st),
+                    'lcq_hessian_compare_packed')
+            return True
+        es = stage.element_size()
+        off = at * K * es
+        nbytes = tokens * K * es
         if lo is not None:                               # fp32 activations: both bf16 halves
             hi_, lo_ = self._halves(inp.reshape((-1, K)).contiguous())
             L.check(lib.lcq_compare_bytes(L.ptr(hi_), ctypes.c_void_p(stage.data_ptr() + off), L.i64(nbytes), L.ptr(flag), st),
@@ -294,16 +301,22 @@ class GPTQ:
         cache['upper_only'] = lead.get('upper_only', False)
         if lead.get('share_flag') is not None:            # what was compared so far concerns this Hessian too
             cache['share_flag'] = lead['share_flag'].clone()
-        for k in ('stage', 'stage_lo', 'stage_fill', 'stage_batches', 'last_stage'):
+        for k in ('stage', 'stage_lo', 'stage_packed', 'stage_fill', 'stage_batches', 'last_stage'):
             cache.pop(k, None)
         if fill > 0:
-            cache['stage'] = torch.empty_like(lead['stage'])
-            cache['stage'][:fill].copy_(lead['stage'][:fill])
-            cache['stage_lo'] = None
-            if lead.get('stage_lo') is not None:
-                cache['stage_lo'] = torch.empty_like(lead['stage_lo'])
-                cache['stage_lo'][:fill].copy_(lead['stage_lo'][:fill])
+            packed = cache['stage_packed'] = lead['stage_packed']
+            rows = -(-fill // 32) * 32 if packed else fill
+            for k in ('stage', 'stage_lo'):
+                cache[k] = None
+                if lead.get(k) is not None:
+                    cache[k] = torch.empty_like(lead[k])
+                    cache[k][:rows].copy_(lead[k][:rows])
             cache['stage_fill'], cache['stage_batches'] = fill, batches
+            if packed:                                    # the rest of the last slab: zeros in place of the call left out
+                lo, K = cache['stage_lo'], cache['columns']
+                L.check(L.lib().lcq_hessian_pack(None, L.F32 if lo is not None else L.dtype_code(cache['stage'].dtype), 0, K, K, fill,
+                                                 cache['stage'].data_ptr(), None if lo is None else lo.data_ptr(), L.stream()),
+                        'lcq_hessian_pack')
 
     def _release_laggards(self, lead_name, lead):
         """Followers that have not seen their leader's latest call yet (it skipped a forward pass, or H is being read
@@ -339,8 +352,8 @@ class GPTQ:
             raise NotImplementedError(f'add_batch takes bf16 / fp16 / fp32 activations; got {inp.dtype}')
         assert tokens % self.chunk_num == 0, \
             f'Error: inp.shape[1] ({tokens}) cannot be evenly divided by chunk_num.'
-        defer = self.hessian_fold(K)
-        if self._follow(name, cache, key, defer > 1 and kind == 'linear', inp, tokens, K):
+        staged = self.hessian_defer == 'auto' or self.hessian_defer > 1
+        if self._follow(name, cache, key, staged and kind == 'linear', inp, tokens, K):
             cache['calls'] += 1
             cache['nsamples'] += tmp
             return                                      # the Linear it follows accumulates
@@ -360,19 +373,36 @@ class GPTQ:
         # apart from H when a follower needs the state before it.  (`calls` counts the calls whose tokens are in
         # the buffer or in H: it moves only once this call's tokens are.)
         stage = cache.get('stage')
-        if defer > 1:
+        if staged:
             if stage is not None and (stage.dtype != sdtype or split != (cache.get('stage_lo') is not None)
                                       or cache['stage_fill'] + tokens > stage.shape[0]):
                 self._flush(cache)
                 if stage.dtype != sdtype or split != (cache.get('stage_lo') is not None) or tokens > stage.shape[0]:
                     stage = None                        # another type, or a call larger than the whole buffer
             if stage is None:
-                stage = torch.empty((defer * tokens, K), dtype=sdtype, device=inp.device)
+                # packed where one accumulator takes it all; the launches with token shares read the tokens as they come
+                packed = cache['stage_packed'] = cache.get('H_shares') is None
+                defer = self.hessian_fold(K, tokens)
+                rows, cols = (-(-defer * tokens // 32) * 32, -(-K // 256) * 256) if packed else (defer * tokens, K)
+                stage = torch.empty((rows, cols), dtype=sdtype, device=inp.device)
                 cache['stage'] = stage
                 cache['stage_lo'] = torch.empty_like(stage) if split else None
                 cache['stage_fill'] = 0
                 cache['stage_batches'] = 0
             f = cache['stage_fill']
+            if cache['stage_packed']:
+                lo = cache['stage_lo']
+                x = inp if key[0] % 16 == 0 and inp.is_contiguous() else self._token_rows(inp, K)
+                rc = L.lib().lcq_hessian_pack(x.data_ptr(), L.dtype_code(x.dtype), tokens, K, K, f, stage.data_ptr(),
+                                              None if lo is None else lo.data_ptr(), L.stream())
+                if rc != 0:
+                    L.check(rc, 'lcq_hessian_pack')
+                cache['stage_fill'] = f + tokens
+                cache['stage_batches'] += tmp
+                cache['last_stage'] = (tokens, tmp)
+                cache['calls'] += 1
+                cache['nsamples'] += tmp
+                return
             nbytes = tokens * K * stage.element_size()
             dst = stage.data_ptr() + f * K * stage.element_size()
             if not split and key[0] % 16 == 0 and nbytes % 16 == 0 and dst % 16 == 0 and inp.is_contiguous():
@@ -397,37 +427,33 @@ class GPTQ:
         cache['nsamples'] += tmp
         self._accumulate(cache, *self._halves(inp.reshape((-1, K)).contiguous()), tmp)
 
-    def hessian_fold(self, K):
-        """add_batch calls folded into one Hessian launch for a Linear with K input features.  'auto': 4 calls of 2048
-        tokens at K = 14336 (1.5 ms per launch; longer launches run at a lower sustained clock and are slower per
-        token), 8 up to K = 8192, 16 up to K = 4096 (the longer the launch, the smaller the share of its ramp and tail,
-        and the more tokens each of its shares gets, see hessian_shares)."""
+    @staticmethod
+    def _token_rows(inp, K):
+        """The tokens of a call as a contiguous [tokens, K] tensor on a 16-byte boundary (the input itself where it is one)."""
+        x = inp
+        if not inp.is_contiguous():
+            x = inp.reshape((-1, K)).contiguous()
+        return x if x.data_ptr() % 16 == 0 else x.clone()
+
+    def hessian_fold(self, K, tokens=2048):
+        """add_batch calls of `tokens` tokens folded into one Hessian launch for a Linear with K input features.  'auto': what
+        makes 65536 tokens for K <= 4096 and 32768 above (half a GB of staged tokens at K = 4096, one at K = 14336), 128 calls
+        at most (so that a few short ones do not ask for such a buffer).  A launch reads and writes H and fills and drains the
+        chip once, whatever its tokens: 861 us for 65536 tokens at K = 4096 against 2 x 462, 5.01 ms for 32768 at K = 14336
+        against 4 x 1.32.  Up to K = 1024 a launch is short (25 us for 8192 tokens) and runs while the host stages the next
+        calls, so it is issued early."""
         if self.hessian_defer == 'auto':
-            return 16 if K <= 4096 else (8 if K <= 8192 else 4)
+            window = 8192 if K <= 1024 else (65536 if K <= 4096 else 32768)
+            return min(max(window // max(tokens, 1), 2), 128)
         return self.hessian_defer
 
     def hessian_shares(self, K):
-        """Token shares of one Hessian launch for K input features (lcq_hessian_accum_sliced).  A launch has one
-        workgroup per 256 x 128 tile that reaches the upper triangle and the chip has 512 workgroup slots: K = 4096
-        gives 272 tiles, one workgroup on most CUs, whose four waves cannot hide their own latencies.  Cutting the
-        tokens of the launch into three shares with an accumulator each puts 816 workgroups on the chip; the
-        accumulators are summed when H is asked for.  'auto' follows what was measured on 128 calls of 2048 tokens
-        (ms, one share -> best count): K=1024 4.4 -> 1.6 (8), 2048 4.6 -> 2.0 (5), 3072 5.0 -> 3.3 (3), 4096 5.8 -> 5.1
-        (3), 6144 11.9 -> 10.6 (2), 8192 18.6 -> 17.6 (2); one share is best at K = 5120, 7168, 11008, 14336 (every
-        share reads and writes its accumulator once per launch)."""
+        """Token shares of one Hessian launch for K input features, each with an accumulator of its own
+        (lcq_hessian_accum_sliced).  'auto': one, whose launch cuts its tiles by itself (lcq_hessian_accum_packed), but eight
+        up to K = 512, where the 256 x 256 tiles of that kernel are three: 35 against 41 us for 16384 tokens."""
         if self.hessian_slices != 'auto':
             return max(1, self.hessian_slices)
-        ntr, ntc = (K + 255) // 256, (K + 127) // 128
-        tiles = sum(max(ntc - 2 * r, 0) for r in range(ntr))
-        if tiles <= 40:
-            return 8
-        if tiles <= 100:
-            return 5
-        if tiles <= 300:
-            return 3
-        if 512 < tiles < 1536 and tiles % 512 < 128:      # a round or two of workgroups and a small rest
-            return 2
-        return 1
+        return 8 if K <= 512 else 1
 
     def _halves(self, x, hi=None, lo=None):
         """(x, None) for 16-bit activations; for fp32 the two bf16 halves hi = bf16(x), lo = bf16(x - hi)."""
@@ -478,12 +504,33 @@ class GPTQ:
         for a, b, al in ((x_lo, x_lo, alpha), (x, x_lo, 1.0), (x_lo, x, 1.0), (x, x, 1.0)):      # small terms first
             launch(a, b, al)
 
+    def _accumulate_packed(self, cache):
+        """_accumulate for the packed staging buffer."""
+        H, hi, lo, T, batches = cache['H'], cache['stage'], cache.get('stage_lo'), cache['stage_fill'], cache['stage_batches']
+        n, K = cache.get('n_in_H', 0), H.shape[0]
+        alpha, beta = n / (n + batches), 2.0 / (n + batches)
+        cache['n_in_H'] = n + batches
+        lib, st = L.lib(), L.stream()
+        if cache.get('hws_key') != ('packed', K, T):               # the workspace goes by the tokens of the launch: kept while they stay
+            nbytes = lib.lcq_hessian_packed_workspace_bytes(K, T)
+            cache['hws'] = torch.empty(nbytes, dtype=torch.uint8, device=H.device) if nbytes > 0 else None
+            cache['hws_key'] = ('packed', K, T)
+        ws = cache['hws']
+        pairs = ((hi, hi, alpha),) if lo is None else ((lo, lo, alpha), (hi, lo, 1.0), (lo, hi, 1.0), (hi, hi, 1.0))
+        for a, b, al in pairs:                           # fp32 activations: small terms first
+            L.check(lib.lcq_hessian_accum_packed(L.ptr(H), K, a.data_ptr(), b.data_ptr(), L.dtype_code(a.dtype), T, al, beta,
+                                                 0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), st),
+                    'lcq_hessian_accum_packed')
+
     def _flush(self, cache):
         """Fold the staged tokens into H."""
         if cache.get('stage_fill', 0) > 0:
             lo = cache.get('stage_lo')
-            self._accumulate(cache, cache['stage'][:cache['stage_fill']], None if lo is None else lo[:cache['stage_fill']],
-                             cache['stage_batches'])
+            if cache['stage_packed']:
+                self._accumulate_packed(cache)
+            else:
+                self._accumulate(cache, cache['stage'][:cache['stage_fill']], None if lo is None else lo[:cache['stage_fill']],
+                                 cache['stage_batches'])
             cache['stage_fill'] = 0
             cache['stage_batches'] = 0
         cache['last_stage'] = (0, 0)                     # the latest call is inside H now
@@ -500,6 +547,8 @@ class GPTQ:
         self._flush(lead)
         lead.pop('stage', None)
         lead.pop('stage_lo', None)
+        lead.pop('hws', None)
+        lead.pop('hws_key', None)
         if lead.get('shares_apart'):                      # the token shares of the launches back into the one H
             sh = lead['H_shares']
             L.check(L.lib().lcq_hessian_gather_slices(L.ptr(sh), L.i64(sh.shape[1]), L.i32(sh.shape[0]), L.i64(sh.stride(0)),

@@ -138,6 +138,66 @@ def test_hessian_with_the_last_round_split(dev, K, T):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize('K,cuts,dtype', [
+    (8, [1], torch.bfloat16), (256, [32], torch.float16), (264, [7, 8, 1, 16, 3], torch.bfloat16), (640, [31, 129, 0, 2], torch.float16),
+    (1000, [77, 500], torch.float32), (1024, [4096], torch.bfloat16), (2304, [333, 1], torch.bfloat16), (4096, [1024], torch.bfloat16),
+    (5888, [64], torch.float16), (6144, [96, 5], torch.bfloat16)])
+def test_hessian_from_packed_tokens(dev, K, cuts, dtype):
+    """lcq_hessian_pack / _compare_packed / _accum_packed: tokens appended call by call land where the layout says (zeros to the
+    end of the slab, earlier tokens untouched), a changed token is seen, and H is the fp64 sum to the rounding of fp32: the
+    products of 16-bit values are exact, so an element errs by at most its T / 16 + 64 additions (matrix instruction by
+    instruction, pieces, alpha * H) of 2^-24 each, of the magnitudes added.  K: edges of the 256-column tiles, one tile, and
+    numbers of tiles that give whole rounds, cut tiles and both."""
+    from lightcompress_amd import _lib as L
+    lib, T = L.lib(), sum(cuts)
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + T)
+    x = torch.randn(T, K, device=dev, generator=g).mul_(torch.exp(torch.randn(K, device=dev, generator=g))).to(dtype)
+    half = torch.bfloat16 if dtype == torch.float32 else dtype
+    Kp, Tp = -(-K // 256) * 256, -(-T // 32) * 32
+    assert lib.lcq_hessian_packed_bytes(K, T) == Kp * Tp * 2
+    bufs = [torch.full((Kp * Tp,), 3.0, dtype=half, device=dev) for _ in range(2 if dtype == torch.float32 else 1)]
+    lo = bufs[1].data_ptr() if len(bufs) > 1 else None
+    at = 0
+    for n in cuts:
+        L.check(lib.lcq_hessian_pack(x[at:at + n].data_ptr() if n else None, L.dtype_code(dtype), n, K, K, at, bufs[0].data_ptr(), lo,
+                                     L.stream()), 'pack')
+        at += n
+    planes = [x] if len(bufs) == 1 else [x.bfloat16(), (x - x.bfloat16().float()).bfloat16()]
+    for p, b in zip(planes, bufs):
+        full = torch.zeros(Tp, Kp, dtype=half, device=dev)
+        full[:T, :K] = p
+        want = full.view(Tp // 16, 2, 8, Kp // 32, 32).permute(0, 3, 1, 4, 2).reshape(-1)
+        assert torch.equal(want.view(torch.int16), b.view(torch.int16))
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+
+    def compare(y, a, n):
+        L.check(lib.lcq_hessian_compare_packed(y[a:a + n].contiguous().data_ptr(), L.dtype_code(dtype), n, K, K, a, bufs[0].data_ptr(),
+                                               lo, flag.data_ptr(), L.stream()), 'compare')
+        return int(flag.item())
+    assert compare(x, 0, T) == 0 and compare(x, T - cuts[-1], cuts[-1]) == 0
+    y = x.clone()
+    y[0, 0] += 1                                                # outside the tokens compared: not seen
+    assert T == cuts[-1] or compare(y, T - cuts[-1], cuts[-1]) == 0
+    assert compare(y, 0, T) == 1
+    H0 = torch.randn(K, K, device=dev, generator=g)
+    H, alpha, beta = H0.clone(), 0.75, 2.0 / T
+    ws = torch.empty(lib.lcq_hessian_packed_workspace_bytes(K, T) + 16, dtype=torch.uint8, device=dev)
+    for i, (a, b) in enumerate([(0, 0)] if len(bufs) == 1 else [(1, 1), (0, 1), (1, 0), (0, 0)]):
+        L.check(lib.lcq_hessian_accum_packed(H.data_ptr(), K, bufs[a].data_ptr(), bufs[b].data_ptr(), L.dtype_code(half), T,
+                                             alpha if i == 0 else 1.0, beta, ws.data_ptr(), ws.numel(), L.stream()), 'accum')
+    xd = sum(p.double() for p in planes)
+    ref = alpha * H0.double() + beta * (xd.t() @ xd)
+    mag = alpha * H0.double().abs() + beta * (xd.abs().t() @ xd.abs())
+    up = torch.triu(torch.ones(K, K, dtype=torch.bool, device=dev))
+    assert bool(((H.double() - ref).abs() <= (T / 16 + 64) * 2.0 ** -24 * mag)[up].all())
+    again = H0.clone()
+    if len(bufs) == 1:
+        L.check(lib.lcq_hessian_accum_packed(again.data_ptr(), K, bufs[0].data_ptr(), bufs[0].data_ptr(), L.dtype_code(half), T, alpha,
+                                             beta, ws.data_ptr(), ws.numel(), L.stream()), 'accum')
+        assert torch.equal(again, H)
+
+
 @pytest.mark.parametrize('slices', [1, 3, 'auto'])
 def test_hessian_shares_through_add_batch_and_reads_in_between(dev, slices):
     """`special.hessian_slices`: whatever the number of accumulators, reading H in the middle of the calibration
