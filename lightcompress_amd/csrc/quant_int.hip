@@ -191,13 +191,17 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
 // elements each.  A step's error is first estimated:
 //   * t = x * (1/s) instead of x / s: a quotient within 2 ulp of a half-integer may round to the other neighbour, both
 //     of which are half a step away from x;
-//   * |d| ^ norm = d^2 * 2 ^ ((norm - 2) log2 |d|): the square is exact to one rounding and only the fraction of the
-//     exponent goes through v_log / v_exp; x and s are scaled by the power of two that brings the row's largest value
-//     to [1, 2), so |log2| stays small and nothing underflows.  The factor is common to all steps of a row and positive,
-//     so it changes no comparison;
+//   * |d| ^ norm = 2 ^ (norm log2 |d|) through v_log / v_exp; x and s are scaled by the power of two that brings the row's
+//     largest value to [1, 2), so |log2| stays small and nothing underflows.  The factor is common to all steps of a row and
+//     positive, so it changes no comparison;
 //   * every term is >= 0 and fp32 sums of such terms never shrink, so a part of the estimate that is far enough above the
 //     best one decides a step: first the error of the two extremes alone (most steps behind the best one lose by what they
 //     clip there), then after every quarter of the elements.  A wave goes on to the next step when all its rows are decided;
+//   * the steps that are left only shrink the range further (it changes when one of them wins).  Quantized values end at
+//     xmax + s / 2 and xmin - s / 2 at the latest (symmetric: at qmax s and qmin s; a zero point is rounded, and clamped
+//     towards the range), which moves towards zero from step to step, so once what the ends alone clip there (less MSE_SLACK
+//     for the roundings of either evaluation, |x| < 2) is more than the best error for all rows of a wave, it is done: after
+//     28 of 80 steps on average.  Not where a later step's scale would be clamped at 1e-5, which widens its range again;
 //   * elements past the row's end are zeros: with qmin <= z <= qmax they quantize to themselves and add nothing.
 // The estimate and mse_row_error differ by a relative delta at most (mse_margin below).  Where `margin` cannot tell the two
 // steps apart, the wave evaluates mse_row_error for both of them, so the range is always the one mse_range_kernel finds: an
@@ -207,10 +211,12 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
 // MSE_SMALL, next to which underflowed terms might count: small = 2^(-68 / norm), 2^-28 for 2.4, leaves MSE_SMALL small^norm = 2^-91,
 // 2^21 times the 2^-112 that 2^14 underflowed terms can come to; large = 2^(113 / norm - 1), 2^46 for 2.4, keeps 2^14 terms of at
 // most (2 large)^norm below 2^127.  In a row with an infinity or a NaN the error of every step is NaN: it keeps its range.
-// What bounds it: ten instructions per element and step, two of them transcendental (about 50 vector cycles).  4096 x 4096
-// bf16 in groups of 128, 4 bits, 80 steps: 1864 us re-reading, 497 with the row in registers, 199 with the steps cut short,
-// 204 with the undecided ones evaluated (4096 rows of 4096: 1268, 437, 366, 380).
+// What bounds it: nine instructions per element and step, two of them transcendental (60 vector cycles for 64 elements), over
+// the 20 steps' worth of elements that the slowest row of a wave needs.  4096 x 4096 bf16 in groups of 128, 80 steps, 4 bits:
+// 1864 us re-reading, 497 with the row in registers, 225 with the steps cut short and near-ties evaluated, 183 with the last
+// steps left out, 179 on four lanes a row; 8 bits 62 -> 19 (4096 rows of 4096: 381 -> 350 and 102 -> 65).
 constexpr float MSE_SMALL = 1.1920929e-7f;                   // 2^-23, in units of (largest value of the row, 1 .. 2) ^ norm
+constexpr float MSE_SLACK = 2e-5f;
 template <int BF, int TEAM, int PER>
 __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restrict__ x, int64_t rows, int cols, int vec, int steps,
                                                              int grid_n, float norm, float margin, float small, float large, IntOp<0, false> op,
@@ -264,7 +270,8 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
   const float up = u2f((uint32_t)(254 - e) << 23), down = u2f((uint32_t)e << 23);
   #pragma unroll
   for (int i = 0; i < PER; ++i) v[i] *= up;
-  const float frac = norm - 2.0f, top = mx * up, bottom = mn * up;
+  const float top = mx * up, bottom = mn * up, last_p = shrink[steps - 1];
+  const auto power = [&](float d) { return __builtin_amdgcn_exp2f(norm * __builtin_amdgcn_logf(fabsf(d))); };
   // an estimate above `hi` cannot beat the best step, one below `lo` does
   float hi = live ? __builtin_inff() : -1.0f, lo = regular ? __builtin_inff() : -__builtin_inff();
   float best = __builtin_inff(), best_s = -1.0f, best_z = 0.0f;        // mse_row_error of the best step (if `have`), its parameters
@@ -278,9 +285,17 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
     const auto add = [&](float w, float sum) {
       const float q = __builtin_amdgcn_fmed3f(rintf(w * r), prm.lo, prm.hi);
       const float d = q * s - w;                             // (both operations rounded, as in deq)
-      return __builtin_fmaf(d * d, __builtin_amdgcn_exp2f(frac * __builtin_amdgcn_logf(fabsf(d))), sum);
+      return sum + power(d);
     };
-    if (__all(fmaxf(add(top, 0.0f), add(bottom, 0.0f)) > hi)) continue;        // (a workgroup's lanes all hold the same two)
+    if (__all(fmaxf(add(top, 0.0f), add(bottom, 0.0f)) > hi)) {                // (a workgroup's lanes all hold the same two)
+      // what this and every later step clip at the ends, from above (see the comment)
+      const float slack = op.sym ? 0.0f : 0.5f * s;
+      const float over = fmaxf(top - ((op.sym ? op.qmax * s : xmax * up) + slack) - MSE_SLACK, 0.0f);
+      const float under = fmaxf((op.sym ? op.qmin * s : xmin * up) - slack - bottom - MSE_SLACK, 0.0f);
+      const float smallest = last_p * (op.sym ? fmaxf(fabsf(cur_min), fabsf(cur_max)) : cur_max - cur_min);
+      if (__all((smallest > 2e-5f && power(over) + power(under) > hi) || hi < 0.0f)) break;
+      continue;
+    }
     float err = 0.0f, sum = 0.0f;
     #pragma unroll
     for (int quarter = 0; quarter < 4; ++quarter) {
@@ -318,13 +333,14 @@ __global__ __launch_bounds__(256) void mse_range_team_kernel(const void* __restr
 
 // Two estimates that differ by more than this tell which of the two errors is larger.  delta bounds the relative difference
 // between an estimate and mse_row_error:
-//   powers   v_log is good to an ulp of |log2 d| < 32 (2^-19), times norm - 2; d^2, v_exp and powf to an ulp each;
+//   powers   v_log is good to an ulp of |log2 d| < 32 (2^-19), times norm, and the product to half an ulp of 128 (2^-18), both
+//            times ln 2; v_exp and powf to an ulp each;
 //   ties     where x * (1/s) and x / s round to different integers, |x/s| is within |x/s| 2^-22 of a half-integer and both
 //            errors are s / 2 to (levels + 1) 2^-19.5, levels = qmax - qmin >= |x/s| - 1/2; norm times that for the power;
 //   sums     of non-negative terms: 2^-24 for every addition a term goes through, in either order.
 // (1 + delta) / (1 - delta) on either side: 2.5 delta.
 float mse_margin(int64_t cols, int per, float levels, float norm) {
-  const float delta = (norm - 1.0f) * 1.9073486e-6f + 5e-7f + norm * (levels + 1.0f) * 1.35e-6f + (float)(cols / 64 + per + 16) * 6e-8f;
+  const float delta = norm * 1.33e-6f + 2.65e-6f + 5e-7f + norm * (levels + 1.0f) * 1.35e-6f + (float)(cols / 64 + per + 16) * 6e-8f;
   return 2.5f * delta;
 }
 
@@ -339,12 +355,12 @@ int run_mse(const void* x, int64_t rows, int64_t cols, int steps, int grid_n, fl
     return LCQ_OK; } while (0)
   if (op.round_zp && op.qmin <= 0.0f && op.qmax >= 0.0f && op.qrange <= 512.0f && norm > 2.0f && norm <= 4.0f && steps <= 256) {
     // Many elements per lane amortise the step's row arithmetic, but below 20000 rows such waves are too few to fill the
-    // chip and their 80 steps one after the other are what takes the time: rows of 128 on 16 / 2 lanes take 34 / 68 us at
-    // 4096 rows, 60 / 67 at 16384, 98 / 69 at 32768
+    // chip and their steps one after the other are what takes the time: bf16 rows of 128 on 16 / 4 / 2 lanes take 26 / 38 /
+    // 38 us at 4096 rows, 42 / 41 / 42 at 16384, - / 54 / 59 at 32768, - / 174 / 181 at 131072 (4 bits, symmetric)
     if (cols <= 32) LCQ_MSE(4, 8);
     if (cols <= 128 && rows < 20000) LCQ_MSE(16, 8);
     if (cols <= 64) LCQ_MSE(4, 16);
-    if (cols <= 128) LCQ_MSE(2, 64);
+    if (cols <= 128) LCQ_MSE(4, 32);
     if (cols <= 512) LCQ_MSE(16, 32);
     if (cols <= 4096) LCQ_MSE(64, 64);
     if (cols <= 16384) LCQ_MSE(256, 64);

@@ -896,6 +896,31 @@ def test_mse_range_is_the_one_of_the_re_reading_kernel(dev, rows, cols, dtype, b
         assert_bit_equal(got, o.cpu(), name)
 
 
+@pytest.mark.parametrize('rows,cols,dtype,bit,sym', [
+    (20000, 128, torch.bfloat16, 4, False), (20000, 100, torch.float32, 8, True), (4096, 128, torch.float16, 8, False),
+    (1024, 32, torch.float32, 2, False), (512, 512, torch.bfloat16, 3, True), (128, 4096, torch.float32, 4, False),
+    (64, 4104, torch.bfloat16, 4, True)])
+def test_mse_range_search_that_ends_early(dev, rows, cols, dtype, bit, sym):
+    """Once the ends of a row alone clip more than the best error, the steps that only shrink the range further are left out;
+    not where one of them would have its scale clamped at 1e-5, which widens its range again.  Rows with outliers (the search
+    ends after a few steps), lopsided rows (zero point at a bound), and rows whose range crosses 1e-5 * levels at the first,
+    a middle or the last step; compared with the re-reading kernel, which runs every step (rows padded with zeros as above)."""
+    g = torch.Generator(device=dev).manual_seed(rows + cols)
+    w = torch.randn(rows, cols, generator=g, device=dev) * 0.02
+    w[:, 0], w[:, 1] = w[:, 0].abs(), -w[:, 1].abs()
+    w[::2, 2] *= 10
+    w[1::4, 0] = 1e-4                                            # nearly one-sided
+    w[1::4, 1:] = -w[1::4, 1:].abs()
+    sizes = torch.logspace(-8, -2, rows // 2, device=dev)        # |w| from below to above the clamp, every step in between
+    w[rows - rows // 2:] *= (sizes / 0.05)[:, None]
+    w = w.to(dtype)
+    q = _iq(bit, sym, 'per_channel', calib_algo='mse')
+    wide = torch.zeros(rows, 16392, dtype=dtype, device=dev)
+    wide[:, :cols] = w
+    for got, o, name in zip(q.get_mse_range(w), q.get_mse_range(wide), ('min', 'max')):
+        assert_bit_equal(got, o.cpu(), name)
+
+
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize('bit,sym,shape,g', [(4, False, (64, 512), 128), (8, True, (33, 256), 64), (8, False, (7, 96), 32),
                                              (4, True, (5, 1000), 0), (8, True, (3, 1001), 0)])
