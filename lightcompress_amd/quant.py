@@ -833,26 +833,35 @@ class IntegerQuantizer(BaseQuantizer):
 
     def _can_pack(self, weight):
         """May `_pack_dynamic` stand for real_quant_weight_dynamic and a pack?"""
-        return self.granularity in ('per_group', 'per_channel') and self._packs_in_place(weight)
+        return self.granularity in ('per_group', 'per_channel') and self._pack_bounds(weight) is not None
 
-    def _packs_in_place(self, weight):
+    def _pack_bounds(self, weight):
         """Symmetric 4- or 8-bit min/max codes of a 2-D weight whose rows fill whole 16-byte chunks: the nibbles / bytes can
-        leave the quantizer's kernel where a pack of its codes would put them."""
+        leave the quantizer's kernel where a pack of its codes would put them.  -> (qmin, qmax) as numbers, or None"""
+        if not (self.bit in (4, 8) and self.sym and self.calib_algo == 'minmax' and self.round_zp and weight.dim() == 2
+                and weight.dtype in (torch.bfloat16, torch.float16, torch.float32)):
+            return None
+        K = weight.shape[1]
+        cols = self.group_size if self.granularity == 'per_group' else K
         lo, hi = (-8, 7) if self.bit == 4 else (-128, 127)
-        cols = self.group_size if self.granularity == 'per_group' else weight.shape[-1]
-        return (self.bit in (4, 8) and self.sym and self.calib_algo == 'minmax' and self.round_zp
-                and weight.dim() == 2 and weight.shape[1] % 8 == 0 and cols % 8 == 0 and weight.dtype in (torch.bfloat16, torch.float16, torch.float32)
-                and lo <= float(self.qmin) and float(self.qmax) <= hi and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+        qmin, qmax = float(self.qmin), float(self.qmax)
+        ok = K % 8 == 0 and cols % 8 == 0 and lo <= qmin and qmax <= hi and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+        return (qmin, qmax) if ok else None
 
-    def _pack_dynamic(self, weight, scales_dtype):
-        """-> (int32 words [R, K * bit / 32], scales [R, -1] in `scales_dtype`: the weight's type or fp16), one launch."""
-        rows_t = self.reshape_tensor(weight)
+    def _pack_dynamic(self, weight, scales_dtype, bounds=None):
+        """-> (int32 words [R, K * bit / 32], scales [R, -1] in `scales_dtype`: the weight's type or fp16), one launch.
+        `bounds`: what _pack_bounds returned, if it has been asked."""
+        bounds = bounds or self._pack_bounds(weight)
         R, K = weight.shape
-        rows, cols = rows_t.shape
+        cols = K
+        if self.granularity == 'per_group' and K >= self.group_size:
+            cols = self.group_size
+            if K % cols != 0:
+                self.reshape_tensor(weight)                  # raises
         packed = torch.empty((R, K * self.bit // 32), dtype=torch.int32, device=weight.device)
-        scales = torch.empty((R, rows // R), dtype=scales_dtype, device=weight.device)
+        scales = torch.empty((R, K // cols), dtype=scales_dtype, device=weight.device)
         flags = L.FLAG_SYM | (L.FLAG_SCALES_F16 if scales_dtype != weight.dtype else 0)
-        L.check(L.lib().lcq_quant_int(L.ptr(rows_t), L.dtype_code(weight.dtype), rows, cols, float(self.qmin), float(self.qmax),
+        L.check(L.lib().lcq_quant_int(L.ptr(weight), L.dtype_code(weight.dtype), R * (K // cols), cols, *bounds,
                                       flags, 1.0, None, packed.data_ptr(), L.CODE_CT4 if self.bit == 4 else L.CODE_CT8,
                                       scales.data_ptr(), None, L.stream()), 'lcq_quant_int')
         return packed, scales
@@ -867,7 +876,7 @@ class IntegerQuantizer(BaseQuantizer):
         weight = weight.contiguous()
         if self._can_pack(weight):
             return (*self._pack_dynamic(weight, weight.dtype), None)
-        if self.granularity == 'per_tensor' and self._packs_in_place(weight):
+        if self.granularity == 'per_tensor' and self._pack_bounds(weight):
             _, packed, scales, _ = self._launch(weight, static=False, want_codes='ct4')
             return packed.view(weight.shape[0], weight.shape[1] // 8), scales.view(1), None
         codes, scales, _ = self.real_quant_weight_dynamic(weight)

@@ -237,6 +237,41 @@ def test_hessian_batched_call_and_fp16(dev):
     assert float((H - ref).abs().max() / ref.abs().max()) < 1e-5
 
 
+@pytest.mark.parametrize('defer', [2, 4, 'auto'])
+@pytest.mark.parametrize('follower_at', [None, 0, 3])
+def test_hessian_calls_like_the_one_before_and_others(dev, defer, follower_at):
+    """add_batch calls that repeat the previous one's form and calls that do not: another number of tokens, a tensor off a
+    16-byte boundary, strided rows, fp32 in between, H read in between, and a second Linear that shares the input for a
+    while or joins late."""
+    K, T = 1024, 40
+    gp = make_gptq(hessian_defer=defer)
+    layers = {n: Layer(torch.zeros(8, K, device=dev)) for n in ('a', 'b')}
+    gp.subset_init({'layers': layers})
+    g = torch.Generator(device=dev).manual_seed(5)
+
+    def tokens(n, dtype=torch.bfloat16):
+        return (torch.randn(1, n, K, device=dev, generator=g)).to(dtype)
+    odd = torch.empty(T * K + 1, dtype=torch.bfloat16, device=dev)[1:].view(1, T, K)
+    odd.copy_(tokens(T))
+    feeds = [tokens(T) for _ in range(5)] + [odd, odd, tokens(7), tokens(7), tokens(T, torch.float32), tokens(T, torch.float32),
+                                             tokens(T), tokens(2 * T)[:, ::2], tokens(T), tokens(1), tokens(T)]
+    seen = {'a': [], 'b': []}
+    for i, x in enumerate(feeds):
+        for n in ('a', 'b'):
+            if n == 'b' and (follower_at is None or i < follower_at or i % 7 == 6):
+                continue
+            gp.add_batch(layers[n], n, x, None)
+            seen[n].append(x)
+        if i == 12:
+            gp.hessian('a')
+    for n in ('a', 'b') if follower_at is not None else ('a',):
+        ref = 2.0 / len(seen[n]) * sum(x[0].double().t() @ x[0].double() for x in seen[n])
+        H = gp.hessian(n)
+        assert gp.layers_cache[n]['nsamples'] == len(seen[n])
+        assert float((H.double() - ref).abs().max() / ref.abs().max()) < 1e-5
+        assert torch.equal(H, H.t())
+
+
 @pytest.mark.parametrize('defer', [1, 3, 4, 'auto'])
 def test_hessian_deferred_launches(dev, defer):
     """Folding several add_batch calls into one launch leaves H and nsamples as per-call updates do,
