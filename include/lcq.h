@@ -432,7 +432,8 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
  * squared difference and the mean rounded; auto_clip.py:83-191 with clip_version v1, weight-only), one launch:
  *  w [R, K], x [T, K] LCQ_BF16; group_size 32, 64 or 128, K % group_size == 0; n_steps <= n_grid, LCQ_CLIP_MAX_STEPS;
  *  rows do not mix: an infinite or NaN product spoils the errors of its row and group, which keeps its whole range
- *  best_max, best_min [R, G] bf16 out; errs [R, G, n_steps] fp32 out: the errors as compared (rounded to bf16). */
+ *  best_max, best_min [R, G] bf16 out; errs [R, G, n_steps] fp32 out: the errors as compared (rounded to bf16), or NULL: the
+ *  same ranges without the errors (up to 512 tokens, steps that cannot win are left out). */
 #define LCQ_CLIP_MAX_STEPS 12
 int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, int64_t T, int group_size, int n_grid,
                           int n_steps, int clip_sym, float qmin, float qmax, int flags, void* best_max, void* best_min,

@@ -41,7 +41,7 @@ class AutoClipper:
         self.weight_clips = {}
         self.w_only = w_only
         self.logit = lambda x: torch.log(x / (1 - x))
-        self.last_errs = None            # [R, G, n_steps] fp32 of the last auto_clip_layer call
+        self.last_errs = None            # [R, G, n_steps] fp32 of the last auto_clip_layer call (None with errors=False)
         self.fast = False                # True: the bf16 MFMA search kernel where it applies (see the module docstring)
         self.fp8_block_size = 128
 
@@ -61,7 +61,10 @@ class AutoClipper:
                     m.register_buffer('buf_lowbound_factor', None)
                 continue
             inputs = [torch.cat(input_feat[n])] if len(input_feat[n]) != 1 else input_feat[n]
-            max_val, min_val = self.auto_clip_layer(block_idx, n, m.weight, inputs, n_sample_token=n_sample_token)
+            # nobody sees the errors of a step here: only what decides is computed (a subclass' own search is called as it is)
+            plain = getattr(self.auto_clip_layer, '__func__', None) is AutoClipper.auto_clip_layer
+            max_val, min_val = self.auto_clip_layer(block_idx, n, m.weight, inputs, n_sample_token=n_sample_token,
+                                                    **({'errors': False} if plain else {}))
             self.apply_clip(block_idx, m, min_val, max_val, n)
             if is_fp8_weight:
                 m.weight.data, m.weight_scale_inv.data = weight_cast_to_fp8(m.weight.data.contiguous(), self.fp8_block_size)
@@ -97,7 +100,9 @@ class AutoClipper:
     # -- auto_clip.py:83-191 -----------------------------------------------------------------------
     @torch.no_grad()
     def auto_clip_layer(self, block_idx, layer_name, w, inputs, n_grid=20, max_shrink=0.5, n_sample_token=512,
-                        eps=0.0):
+                        eps=0.0, errors=True):
+        """`errors`: leave the errors of all steps in `last_errs`; without, the one-launch search skips the steps that its
+        bounds show to lose (the same ranges) and `last_errs` is None."""
         assert w.dim() == 2
         wq = self.wquantizer
         if self.clip_version not in ('v1', 'v2'):
@@ -132,7 +137,7 @@ class AutoClipper:
                                           '(use fast = False)')
             return self._search_mfma(wc, torch.cat(xs) if len(xs) > 1 else xs[0], n_grid, n_steps)
         if self._fused_applies(wc, xs, n_steps, n_grid):
-            return self._search_fused(wc, xs[0], group_size, n_grid, n_steps)
+            return self._search_fused(wc, xs[0], group_size, n_grid, n_steps, errors)
         return self._search_exact(block_idx, layer_name, wc, xs, group_size, n_grid, n_steps, eps)
 
     def _fused_applies(self, w, xs, n_steps, n_grid=20):
@@ -148,13 +153,13 @@ class AutoClipper:
                 and w.dtype == torch.bfloat16 and xs[0].dtype == torch.bfloat16
                 and w.data_ptr() % 16 == 0 and xs[0].data_ptr() % 16 == 0)
 
-    def _search_fused(self, wc, x, group_size, n_grid, n_steps):
+    def _search_fused(self, wc, x, group_size, n_grid, n_steps, errors=True):
         wq = self.wquantizer
         R, K = wc.shape
         G = K // group_size
         best_max = torch.empty((R, G, 1), dtype=torch.bfloat16, device=wc.device)
         best_min = torch.empty((R, G, 1), dtype=torch.bfloat16, device=wc.device)
-        errs = torch.empty((R, G, n_steps), dtype=torch.float32, device=wc.device)
+        errs = torch.empty((R, G, n_steps), dtype=torch.float32, device=wc.device) if errors else None
         L.check(L.lib().lcq_clip_search_exact(L.ptr(wc), L.ptr(x), L.i64(R), L.i64(K), L.i64(x.shape[0]), L.i32(group_size),
                                               L.i32(n_grid), L.i32(n_steps), L.i32(1 if self.clip_sym else 0),
                                               L.f32(float(wq.qmin)), L.f32(float(wq.qmax)), L.i32(L.FLAG_SYM if wq.sym else 0),

@@ -230,9 +230,10 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
 // One row of A in add_pairs holds two weight rows (lanes m and m + 16), kept apart by the zeros of B, and 0 * infinity is NaN:
 // an infinite or NaN product (an infinite or NaN weight, a product beyond the largest bf16 number) turns the sums of its
 // partner row 16 rows away into NaN as well.  So a lane with a sum that is not finite adds its products up again one by one:
-// x: the group's columns of token 0, w: the tile's rows in LDS.  Off the path of finite tiles, which pay for the test alone.
-template <int GS>
-__device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __restrict__ x, int64_t K, int t0, int T, const char* w,
+// x: the group's columns of token 0, w(i): where the weights of the lane's row i lie in LDS.  Off the path of finite tiles,
+// which pay for the test alone.
+template <int GS, class Rows>
+__device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __restrict__ x, int64_t K, int t0, int T, const Rows& w,
                                                               int lane, f32x4* sum) {
   float m = 0.0f;
   #pragma unroll
@@ -240,7 +241,6 @@ __device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __
     #pragma unroll
     for (int i = 0; i < 4; i += 2) m = nan_max(nan_max(m, fabsf(sum[q][i])), fabsf(sum[q][i + 1]));
   if (__builtin_expect(m < __builtin_inff(), 1)) return;
-  const char* wr = w + (16 * ((lane >> 2) & 1) + 4 * (lane >> 4)) * gd_pitch<GS>();
   const int tok = t0 + 4 * ((lane >> 3) & 1) + (lane & 3);
   #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -248,12 +248,86 @@ __device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __
   for (int j = 0; j < GS; ++j) {
     float wv[4];
     #pragma unroll
-    for (int i = 0; i < 4; ++i) wv[i] = u2f((uint32_t)*(const uint16_t*)(wr + i * gd_pitch<GS>() + 2 * j) << 16);
+    for (int i = 0; i < 4; ++i) wv[i] = u2f((uint32_t)*(const uint16_t*)(w(i) + 2 * j) << 16);
     #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float xv = tok + 8 * q < T ? u2f((uint32_t)x[(int64_t)(tok + 8 * q) * K + j] << 16) : 0.0f;
       #pragma unroll
       for (int i = 0; i < 4; ++i) sum[q][i] += rnd<true>(xv * wv[i]);
+    }
+  }
+}
+
+// the columns of one token; a token past T: zeros, which add nothing
+template <int GS>
+__device__ __forceinline__ void load_token(const uint16_t* __restrict__ x, int64_t K, int T, int t, u32x4* a) {
+  const bool ok = t < T;
+  const uint16_t* xr = x + (ok ? t : 0) * K;
+  #pragma unroll
+  for (int c = 0; c < GS / 8; ++c) { a[c] = *(const u32x4*)(xr + 8 * c); if (!ok) a[c] = u32x4{0, 0, 0, 0}; }
+}
+__device__ __forceinline__ void round_sums(f32x4* v) {
+  #pragma unroll
+  for (int q = 0; q < 4; ++q)
+    #pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      float o0 = v[q][i], o1 = v[q][i + 1];
+      rnd_pair<true>(o0, o1);
+      v[q][i] = o0; v[q][i + 1] = o1;
+    }
+}
+// e[i] = the errors of row i of the lane over the tokens of the tile (the same in the eight lanes that share its rows); org rounded
+__device__ __forceinline__ void tile_errors(const f32x4* cur, const f32x4* org, float* e) {
+  #pragma unroll
+  for (int i = 0; i < 4; ++i) e[i] = 0.0f;
+  #pragma unroll
+  for (int q = 0; q < 4; ++q)
+    #pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      float c0 = cur[q][i], c1 = cur[q][i + 1];
+      rnd_pair<true>(c0, c1);
+      c0 -= org[q][i]; c1 -= org[q][i + 1];
+      rnd_pair<true>(c0, c1);
+      c0 *= c0; c1 *= c1;
+      rnd_pair<true>(c0, c1);
+      e[i] += c0; e[i + 1] += c1;
+    }
+  // over the tokens of the tile: lanes that differ in bits 0, 1 and 3
+  #pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    e[i] += lane_xor<1>(e[i]);
+    e[i] += lane_xor<2>(e[i]);
+    e[i] += u2f((uint32_t)__builtin_amdgcn_ds_swizzle((int)f2u(e[i]), 0x201F));      // xor 8
+  }
+}
+
+__device__ __forceinline__ float shrunk(float v, int s, int n_grid) { return rnd<true>(v * (float)(1.0 - (double)s / (double)n_grid)); }
+
+// 32 rows of one group to LDS: version 0 as they are, version s + 1 clamped to the range of step s and fake-quantized.
+template <int GS>
+__device__ __forceinline__ void make_versions(char* smem, const uint16_t* __restrict__ w, int R, int K, int r0, int g, int n_grid, int n_steps,
+                                              int clip_sym, const IntOp<true, true>& op) {
+  constexpr int PITCH_W = gd_pitch<GS>(), TEAM = GS / 8, VERSION = GT * PITCH_W;
+  const int tid = threadIdx.x;
+  for (int ch = tid; ch < GT * TEAM; ch += blockDim.x) {                 // one 16-byte chunk per thread (and turn)
+    const int row = ch / TEAM, c = ch % TEAM;
+    u32x4 raw = {0, 0, 0, 0};
+    if (r0 + row < R) raw = *(const u32x4*)(w + (int64_t)(r0 + row) * K + g * GS + c * 8);
+    char* dst = smem + row * PITCH_W + c * 16;
+    *(u32x4*)dst = raw;
+    float v[8], mn = __builtin_inff(), mx = -__builtin_inff();
+    unpack<true>(raw, v);
+    chunk_minmax<IntOp<true, true>>(raw, mn, mx);
+    team_range<TEAM>(mn, mx);
+    const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
+    for (int s = 0; s < n_steps; ++s) {
+      const float hi = shrunk(org_max, s, n_grid), lo = clip_sym ? -hi : shrunk(mn, s, n_grid);
+      const IntRow p = op.make(nan_min(nan_max(mn, lo), hi), nan_min(nan_max(mx, lo), hi));   // range of the clamped group
+      float cv[8], d[8];
+      #pragma unroll
+      for (int i = 0; i < 8; ++i) cv[i] = nan_min(nan_max(v[i], lo), hi);
+      op.template fused_dq<8>(cv, d, p);
+      *(u32x4*)(dst + (s + 1) * VERSION) = pack_rne<true>(d);
     }
   }
 }
@@ -271,76 +345,29 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
   float* const esum = (float*)(smem + (n_steps + 1) * VERSION);          // [waves][n_steps][32]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
   const int G = K / GS, g = blockIdx.x % G, r0 = (blockIdx.x / G) * GT;
-  const auto shrink = [&](float v, int s) { return rnd<true>(v * (float)(1.0 - (double)s / (double)n_grid)); };
+  const auto shrink = [&](float v, int s) { return shrunk(v, s, n_grid); };
 
   for (int i = tid; i < waves * n_steps * GT; i += blockDim.x) esum[i] = 0.0f;
-  for (int ch = tid; ch < GT * TEAM; ch += blockDim.x) {                 // one 16-byte chunk per thread (and turn)
-    const int row = ch / TEAM, c = ch % TEAM;
-    u32x4 raw = {0, 0, 0, 0};
-    if (r0 + row < R) raw = *(const u32x4*)(w + (int64_t)(r0 + row) * K + g * GS + c * 8);
-    char* dst = smem + row * PITCH_W + c * 16;
-    *(u32x4*)dst = raw;
-    float v[8], mn = __builtin_inff(), mx = -__builtin_inff();
-    unpack<true>(raw, v);
-    chunk_minmax<IntOp<true, true>>(raw, mn, mx);
-    team_range<TEAM>(mn, mx);
-    const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
-    for (int s = 0; s < n_steps; ++s) {
-      const float hi = shrink(org_max, s), lo = clip_sym ? -hi : shrink(mn, s);
-      const IntRow p = op.make(nan_min(nan_max(mn, lo), hi), nan_min(nan_max(mx, lo), hi));   // range of the clamped group
-      float cv[8], d[8];
-      #pragma unroll
-      for (int i = 0; i < 8; ++i) cv[i] = nan_min(nan_max(v[i], lo), hi);
-      op.template fused_dq<8>(cv, d, p);
-      *(u32x4*)(dst + (s + 1) * VERSION) = pack_rne<true>(d);
-    }
-  }
+  make_versions<GS>(smem, w, R, K, r0, g, n_grid, n_steps, clip_sym, op);
   __syncthreads();
 
   const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
   const u32x4 ones = pair_columns(lane);
   const char* wrow = smem + (lane & 31) * PITCH_W;
+  const char* const rows_of_lane = smem + (16 * ((lane >> 2) & 1) + 4 * (lane >> 4)) * PITCH_W;
   for (int t0 = wave * GT; t0 < T; t0 += waves * GT) {
     u32x4 a[GS / 8];
-    const bool ok = t0 + (lane & 31) < T;                                // tokens past T: zeros, which add nothing
-    const uint16_t* xr = x + (int64_t)(ok ? t0 + (lane & 31) : 0) * K + g * GS;
-    #pragma unroll
-    for (int c = 0; c < GS / 8; ++c) { a[c] = *(const u32x4*)(xr + 8 * c); if (!ok) a[c] = u32x4{0, 0, 0, 0}; }
+    load_token<GS>(x + g * GS, K, T, t0 + (lane & 31), a);
     f32x4 org[4], cur[4];
     dots_tile<GS>(a, wrow, mask, ones, org);
-    redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem, lane, org);
-    #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      #pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        float o0 = org[q][i], o1 = org[q][i + 1];
-        rnd_pair<true>(o0, o1);
-        org[q][i] = o0; org[q][i + 1] = o1;
-      }
+    redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, [&](int i) { return rows_of_lane + i * PITCH_W; }, lane, org);
+    round_sums(org);
     #pragma unroll 1
     for (int s = 0; s < n_steps; ++s) {
       dots_tile<GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
-      redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, smem + (s + 1) * VERSION, lane, cur);
-      float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        #pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          float c0 = cur[q][i], c1 = cur[q][i + 1];
-          rnd_pair<true>(c0, c1);
-          c0 -= org[q][i]; c1 -= org[q][i + 1];
-          rnd_pair<true>(c0, c1);
-          c0 *= c0; c1 *= c1;
-          rnd_pair<true>(c0, c1);
-          e[i] += c0; e[i + 1] += c1;
-        }
-      // over the tokens of the tile: lanes that differ in bits 0, 1 and 3
-      #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        e[i] += lane_xor<1>(e[i]);
-        e[i] += lane_xor<2>(e[i]);
-        e[i] += u2f((uint32_t)__builtin_amdgcn_ds_swizzle((int)f2u(e[i]), 0x201F));      // xor 8
-      }
+      redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, [&](int i) { return rows_of_lane + (s + 1) * VERSION + i * PITCH_W; }, lane, cur);
+      float e[4];
+      tile_errors(cur, org, e);
       if ((lane & 0xb) == 0) {
         float* es = esum + (wave * n_steps + s) * GT + 16 * ((lane >> 2) & 1) + 4 * (lane >> 4);
         #pragma unroll
@@ -361,10 +388,247 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
       float e = 0.0f;
       for (int wv = 0; wv < waves; ++wv) e += esum[(wv * n_steps + s) * GT + row];
       e = rnd<true>(e * (1.0f / (float)T));                              // torch's mean: the sum times an fp32 factor
-      errs[at * n_steps + s] = e;
+      if (errs) errs[at * n_steps + s] = e;
       const float hi = shrink(org_max, s), lo = clip_sym ? -hi : shrink(mn, s);
       if (e < best) { best = e; bmax = hi; bmin = lo; }
     }
+    best_max[at] = (uint16_t)(f2u(bmax) >> 16);
+    best_min[at] = (uint16_t)(f2u(bmin) >> 16);
+  }
+}
+
+// The same search without the errors of steps that cannot win (errs == NULL, at most two tiles of tokens per wave).
+//
+// The rounded original sums o_t are computed as above; a step's sums only up to their roundings, as plain matrix products:
+//   a_t = sum_j x w_s - o_t,   |e_t - a_t| <= b_t = u (sum_j |x w_s| + |sum_j x w_s| + |a_t|),   u a little above 2^-9
+// (every product, the sum and the difference are rounded once, each by at most 2^-9 of itself), so with Minkowski's
+// inequality over the tokens  (|a| - |b|)^2 <= sum_t e_t^2 <= (|a| + |b|)^2.  A step whose lower bound is above the smallest
+// upper bound of its row by more than what rounding the squares (2^-9 either way) and the mean (a bf16 step, 2^-7) can make up
+// for neither wins nor ties (MARGIN).  The other steps of rows with more than one of them are evaluated as above, 32 (step,
+// row) pairs to a tile whatever rows and steps they come from, first on half of the tokens: the exact sums of those with the
+// bounds of the rest decide again.  Rows that are not plain (a bound that is not finite, or below SMALL where underflow might
+// count, or near the 1e9 the search starts from) have every step evaluated.
+// Measured (an MLP's Linears as above, 10 steps): 25.8 -> 18.3 ms; 4.3 of 10 steps are evaluated, the matrix pipes are busy in
+// 58 % of the cycles (the making of the versions, estimates and decisions are not overlapped by another workgroup: one fills
+// the LDS).  One step at a time in the estimates and decisions by a single wave: 19.9 ms.
+constexpr float CLIP_U = 2.03e-3f, CLIP_MARGIN = 1.02f, CLIP_SMALL = 1e-25f;
+template <int GS> constexpr size_t clip_pruned_lds(int n_steps, int waves, int rounds) {
+  return (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)rounds * waves * GT * GT * 2 + (size_t)waves * n_steps * GT * 8 +
+         (size_t)(rounds + 1) * n_steps * GT * 8 + (size_t)(n_steps + 1) * GT * 2 + GT * 4 + 16;
+}
+
+template <int GS>
+__global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ x,
+                                                                    int R, int K, int T, int n_grid, int n_steps, int clip_sym,
+                                                                    IntOp<true, true> op, uint16_t* __restrict__ best_max,
+                                                                    uint16_t* __restrict__ best_min) {
+  constexpr int PITCH_W = gd_pitch<GS>(), TEAM = GS / 8, VERSION = GT * PITCH_W;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int rounds = (T + waves * GT - 1) / (waves * GT), pairs = n_steps * GT;
+  const int G = K / GS, g = blockIdx.x % G, r0 = (blockIdx.x / G) * GT;
+  uint16_t* const orgs = (uint16_t*)(smem + (n_steps + 1) * VERSION);    // [tokens][32] bf16
+  float* const part = (float*)(orgs + rounds * waves * GT * GT);         // [waves][pairs] a^2, b^2; later [waves][pairs] exact sums
+  float* const tab = part + waves * pairs * 2;                           // [rounds][pairs] a^2, b^2
+  float* const bounds = tab + rounds * pairs * 2;                        // [pairs] lower, upper
+  uint16_t* const list = (uint16_t*)(bounds + pairs * 2);                // (step, row) = entry / 32, entry % 32
+  uint32_t* const masks = (uint32_t*)(list + pairs + GT);                // steps of a row that may still win; FOUND: the one left does
+  int* const count = (int*)(masks + GT);
+  const uint16_t* const xg = x + g * GS;
+  constexpr uint32_t FOUND = 1u << 31;
+
+  make_versions<GS>(smem, w, R, K, r0, g, n_grid, n_steps, clip_sym, op);
+  __syncthreads();
+
+  const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
+  const u32x4 ones = pair_columns(lane);
+  const int h = lane >> 5, c = lane & 31;
+  const int row4 = 16 * ((lane >> 2) & 1) + 4 * (lane >> 4), tok4 = 4 * ((lane >> 3) & 1) + (lane & 3);    // of the exact sums
+  for (int k = 0; k < rounds; ++k) {
+    const int t0 = (k * waves + wave) * GT;
+    if (t0 < T) {
+      u32x4 a[GS / 8];
+      load_token<GS>(xg, K, T, t0 + c, a);
+      {
+        f32x4 org[4];
+        dots_tile<GS>(a, smem + c * PITCH_W, mask, ones, org);
+        redo_sums_that_are_not_finite<GS>(xg, K, t0, T, [&](int i) { return smem + (row4 + i) * PITCH_W; }, lane, org);
+        round_sums(org);
+        #pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(u32x2*)(orgs + (t0 + 8 * q + tok4) * GT + row4) = u32x2{bf16_pack(org[q][0], org[q][1]), bf16_pack(org[q][2], org[q][3])};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // v_mfma_f32_32x32x16: lane (h, c) supplies token / row c and columns 16 ks + 8 h .. + 7; register r holds token
+      // 8 (r / 4) + 4 h + r % 4 of row c
+      float o[16];
+      #pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = u2f((uint32_t)orgs[(t0 + 8 * (r >> 2) + 4 * h + (r & 3)) * GT + c] << 16);
+      u32x4 ax[GS / 16];
+      #pragma unroll
+      for (int ks = 0; ks < GS / 16; ++ks)
+        #pragma unroll
+        for (int d = 0; d < 4; ++d) ax[ks][d] = h ? a[2 * ks + 1][d] : a[2 * ks][d];
+      // two steps at a time: four independent chains of matrix instructions
+      #pragma unroll 1
+      for (int s = 0; s < n_steps; s += 2) {
+        const char* wr[2];
+        f32x16 sum[2], mag[2];
+        #pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          wr[v] = smem + (min(s + v, n_steps - 1) + 1) * VERSION + c * PITCH_W + 16 * h;
+          #pragma unroll
+          for (int r = 0; r < 16; ++r) { sum[v][r] = 0.0f; mag[v][r] = 0.0f; }
+        }
+        #pragma unroll
+        for (int ks = 0; ks < GS / 16; ++ks) {
+          u32x4 aa;
+          #pragma unroll
+          for (int d = 0; d < 4; ++d) aa[d] = ax[ks][d] & 0x7fff7fffu;
+          #pragma unroll
+          for (int v = 0; v < 2; ++v) {
+            const u32x4 b = *(const u32x4*)(wr[v] + 32 * ks);
+            u32x4 ab;
+            #pragma unroll
+            for (int d = 0; d < 4; ++d) ab[d] = b[d] & 0x7fff7fffu;
+            sum[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ax[ks]), __builtin_bit_cast(bf16x8, b), sum[v], 0, 0, 0);
+            mag[v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, aa), __builtin_bit_cast(bf16x8, ab), mag[v], 0, 0, 0);
+          }
+        }
+        #pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          float a2 = 0.0f, b2 = 0.0f;
+          #pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float d = sum[v][r] - o[r], e = (mag[v][r] + fabsf(sum[v][r])) + fabsf(d);
+            a2 = __builtin_fmaf(d, d, a2);
+            b2 = __builtin_fmaf(e, e, b2);
+          }
+          a2 += __shfl_xor(a2, 32);
+          b2 += __shfl_xor(b2, 32);
+          if (h == 0 && s + v < n_steps) *(f32x2*)(part + 2 * ((wave * n_steps + s + v) * GT + c)) = f32x2{a2, b2 * (CLIP_U * CLIP_U)};
+        }
+      }
+    } else {
+      for (int i = lane; i < pairs; i += 64) *(f32x2*)(part + 2 * (wave * pairs + i)) = f32x2{0.0f, 0.0f};
+    }
+    __syncthreads();
+    for (int i = tid; i < pairs; i += blockDim.x) {
+      float a2 = 0.0f, b2 = 0.0f;
+      for (int v = 0; v < waves; ++v) { a2 += part[2 * (v * pairs + i)]; b2 += part[2 * (v * pairs + i) + 1]; }
+      *(f32x2*)(tab + 2 * (k * pairs + i)) = f32x2{a2, b2};
+    }
+    __syncthreads();
+  }
+
+  // Which steps may still win, with `done` rounds of tokens evaluated: masks and the list of pairs to go on with.
+  const auto decide = [&](int done) {
+    for (int i = tid; i < pairs; i += blockDim.x) {                      // bounds of every pair
+      float a2 = 0.0f, b2 = 0.0f, e = 0.0f;
+      for (int k = done; k < rounds; ++k) { a2 += tab[2 * (k * pairs + i)]; b2 += tab[2 * (k * pairs + i) + 1]; }
+      if (done)
+        for (int v = 0; v < waves; ++v) e += part[v * pairs + i];
+      const float ra = __builtin_amdgcn_sqrtf(a2), rb = __builtin_amdgcn_sqrtf(b2);
+      const float lo = fmaxf(ra * (1.0f - 1e-5f) - rb, 0.0f), hi = (ra + rb) * (1.0f + 1e-5f);
+      *(f32x2*)(bounds + 2 * i) = f32x2{e + lo * lo, e + hi * hi};
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    uint32_t alive = 0;
+    if (lane < GT && r0 + lane < R) {
+      const uint32_t cand = done ? masks[lane] : (1u << n_steps) - 1;
+      if (!(cand & FOUND)) {
+        f32x2 bnd[LCQ_CLIP_MAX_STEPS];
+        #pragma unroll
+        for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s) {
+          bnd[s] = f32x2{0.0f, __builtin_inff()};
+          if (s < n_steps) bnd[s] = *(const f32x2*)(bounds + 2 * (s * GT + lane));
+        }
+        float best = __builtin_inff();
+        bool plain = true;
+        #pragma unroll
+        for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s)
+          if ((cand >> s) & 1) {
+            plain = plain && bnd[s][1] < 1e38f;                          // (NaN: false)
+            best = fminf(best, bnd[s][1]);
+          }
+        plain = plain && best > CLIP_SMALL && best < 9e8f * (float)T;
+        alive = cand;
+        if (plain)
+          #pragma unroll
+          for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s)
+            if (bnd[s][0] > best * CLIP_MARGIN) alive &= ~(1u << s);
+        const bool found = plain && (alive & (alive - 1)) == 0;          // needs no more sums
+        masks[lane] = found ? alive | FOUND : alive;
+        if (found) alive = 0;
+      }
+    }
+    int n = 0;
+    for (int s = 0; s < n_steps; ++s) {
+      const bool on = (alive >> s) & 1;
+      const uint64_t b = __ballot(on);
+      if (on) list[n + __popcll(b & ((1ull << lane) - 1))] = (uint16_t)(s * GT + lane);
+      n += __popcll(b);
+    }
+    if (lane < GT && n + lane < (n + GT - 1) / GT * GT) list[n + lane] = 0;               // (the last tile's surplus lanes)
+    if (lane == 0) *count = n;
+  };
+  decide(0);
+  __syncthreads();
+  for (int i = tid; i < waves * pairs; i += blockDim.x) part[i] = 0.0f;  // from here on: exact sums
+  __syncthreads();
+  for (int k = 0; k < rounds; ++k) {
+    const int t0 = (k * waves + wave) * GT, n = *count;
+    if (t0 < T && n > 0) {
+      u32x4 a[GS / 8];
+      load_token<GS>(xg, K, T, t0 + c, a);
+      #pragma unroll 1
+      for (int p = 0; p < n; p += GT) {
+        const int mine = list[p + c];
+        int entry[4];
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) entry[i] = list[p + row4 + i];
+        const auto where = [&](int e) { return smem + ((e >> 5) + 1) * VERSION + (e & 31) * PITCH_W; };
+        f32x4 org[4], cur[4];
+        dots_tile<GS>(a, where(mine), mask, ones, cur);
+        redo_sums_that_are_not_finite<GS>(xg, K, t0, T, [&](int i) { return where(entry[i]); }, lane, cur);
+        #pragma unroll
+        for (int q = 0; q < 4; ++q)
+          #pragma unroll
+          for (int i = 0; i < 4; ++i) org[q][i] = u2f((uint32_t)orgs[(t0 + 8 * q + tok4) * GT + (entry[i] & 31)] << 16);
+        float e[4];
+        tile_errors(cur, org, e);
+        if ((lane & 0xb) == 0) {
+          #pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (p + row4 + i < n) part[wave * pairs + entry[i]] += e[i];
+        }
+      }
+    }
+    __syncthreads();
+    if (k + 1 < rounds) {
+      decide(k + 1);
+      __syncthreads();
+    }
+  }
+  // err_mean < min_errs over the steps that are left: the first minimum below 1e9 wins, NaN never does
+  if (tid < GT && r0 + tid < R) {
+    const int row = tid;
+    float mn = __builtin_inff(), mx = -__builtin_inff();
+    for (int ch = 0; ch < TEAM; ++ch) chunk_minmax<IntOp<true, true>>(*(const u32x4*)(smem + row * PITCH_W + ch * 16), mn, mx);
+    const float org_max = clip_sym ? nan_max(fabsf(mx), fabsf(mn)) : mx;
+    float best = 998244352.0f, bmax = org_max, bmin = mn;                 // bf16(1e9)
+    const uint32_t alive = masks[row];
+    for (int s = 0; s < n_steps; ++s) {
+      if (!((alive >> s) & 1)) continue;
+      float e = 0.0f;
+      for (int v = 0; v < waves; ++v) e += part[v * pairs + s * GT + row];
+      e = rnd<true>(e * (1.0f / (float)T));                              // torch's mean: the sum times an fp32 factor
+      const float hi = shrunk(org_max, s, n_grid), lo = clip_sym ? -hi : shrunk(mn, s, n_grid);
+      if (e < best || (alive & FOUND)) { best = e; bmax = hi; bmin = lo; }
+    }
+    const int64_t at = (int64_t)(r0 + row) * G + g;
     best_max[at] = (uint16_t)(f2u(bmax) >> 16);
     best_min[at] = (uint16_t)(f2u(bmin) >> 16);
   }
@@ -517,7 +781,7 @@ int lcq_awq_clip_search(const void* w, const void* x, int64_t R, int64_t K, int6
 int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, int64_t T, int group_size, int n_grid,
                           int n_steps, int clip_sym, float qmin, float qmax, int flags, void* best_max, void* best_min,
                           float* errs, void* stream) {
-  if (!w || !x || !best_max || !best_min || !errs || R <= 0 || K <= 0 || T <= 0) return LCQ_EINVAL;
+  if (!w || !x || !best_max || !best_min || R <= 0 || K <= 0 || T <= 0) return LCQ_EINVAL;
   if ((group_size != 32 && group_size != 64 && group_size != 128) || K % group_size != 0) return LCQ_EINVAL;
   if (K > 0x7fffffff / 2 || R > 0x7fffffff || T > 0x7fffffff) return LCQ_EINVAL;
   if (n_grid <= 0 || n_steps <= 0 || n_steps > n_grid || n_steps > LCQ_CLIP_MAX_STEPS) return LCQ_EINVAL;
@@ -529,14 +793,24 @@ int lcq_clip_search_exact(const void* w, const void* x, int64_t R, int64_t K, in
   // one wave per 32 tokens up to eight (two per SIMD: one wave's conversions run under the other's matrix instructions)
   const int waves = T > 4 * GT ? 8 : (T > 2 * GT ? 4 : 2);
   hipStream_t st = (hipStream_t)stream;
-  #define LCQ_CLIP(GS) do { \
-    const size_t lds = (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)waves * n_steps * GT * 4; \
+  const int rounds = (int)((T + waves * GT - 1) / (waves * GT));
+  constexpr size_t LDS = 160 * 1024;
+  #define LCQ_CLIP_LAUNCH(KERNEL, BYTES, ...) do { \
     /* on every call, for it belongs to the current device; the same value always, for another thread may set it too */ \
-    if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)clip_search_kernel<GS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return LCQ_ELAUNCH; \
-    clip_search_kernel<GS><<<dim3((unsigned)grid), dim3(64 * waves), lds, st>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K, \
-        (int)T, n_grid, n_steps, clip_sym, op, (uint16_t*)best_max, (uint16_t*)best_min, errs); } while (0)
+    if (BYTES > 64 * 1024 && hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return LCQ_ELAUNCH; \
+    KERNEL<<<dim3((unsigned)grid), dim3(64 * waves), BYTES, st>>>((const uint16_t*)w, (const uint16_t*)x, (int)R, (int)K, (int)T, n_grid, \
+        n_steps, clip_sym, op, (uint16_t*)best_max, (uint16_t*)best_min __VA_ARGS__); } while (0)
+  // without errors, and with few enough tokens and steps that the original sums and the bounds of all steps fit LDS (T <= 512,
+  // 10 steps at groups of 128): only the steps that may win
+  #define LCQ_CLIP(GS) do { \
+    const size_t pruned = clip_pruned_lds<GS>(n_steps, waves, rounds < 2 ? rounds : 2); \
+    if (!errs && rounds <= 2 && pruned <= LDS) LCQ_CLIP_LAUNCH(clip_search_pruned_kernel<GS>, pruned); \
+    else { \
+      const size_t lds = (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)waves * n_steps * GT * 4; \
+      LCQ_CLIP_LAUNCH(clip_search_kernel<GS>, lds, , errs); } } while (0)
   if (group_size == 128) LCQ_CLIP(128); else if (group_size == 64) LCQ_CLIP(64); else LCQ_CLIP(32);
   #undef LCQ_CLIP
+  #undef LCQ_CLIP_LAUNCH
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

@@ -428,6 +428,38 @@ def test_auto_clip_one_launch_search_at_tile_edges(dev, gs, T, bit, sym, clip_sy
     assert torch.equal(bmax.cpu()[same], obmax[same]) and torch.equal(bmin.cpu()[same], obmin[same])
 
 
+@pytest.mark.parametrize('gs,T,bit,sym,clip_sym,n_steps', [
+    (128, 512, 4, False, False, 10), (128, 480, 4, True, True, 10), (128, 257, 3, False, True, 10), (128, 256, 8, True, False, 10),
+    (64, 512, 4, False, False, 12), (64, 129, 4, True, True, 3), (64, 128, 2, False, False, 10), (32, 65, 4, False, True, 10),
+    (32, 512, 4, True, False, 1), (128, 1, 4, False, False, 10), (128, 513, 4, False, False, 10), (128, 64, 4, False, False, 11)])
+def test_auto_clip_search_without_the_losing_steps(dev, gs, T, bit, sym, clip_sym, n_steps):
+    """With errors=False the steps that a bound shows to lose are not evaluated: the ranges are those of the search that
+    evaluates them all, bit for bit (beyond 512 tokens, or where LDS does not hold the bounds, it IS that search).  Tiles of
+    rows and tokens full and ragged, one and two rounds of tokens; rows of every size from underflow to overflow, of few
+    distinct values (exact ties), of zeros, with an infinity or a NaN; tokens of very different sizes."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    R, K = 192, 3 * gs
+    w = weight_like(R, K, seed=T + gs, dtype=torch.float32, outlier_frac=0.002)
+    w[32:64] = torch.round(w[32:64] * 100) / 100
+    w[64:128] *= torch.exp2(torch.linspace(-100, 110, 64))[:, None]
+    w[128:132] = 0
+    w[133, 1], w[134, 2], w[135, gs + 3] = float('inf'), float('nan'), -float('inf')
+    w[136:140] = w[136:140, :1]
+    w = w.bfloat16().to(dev)
+    x = torch.randn(T, K, generator=gen(T)) * torch.exp(torch.randn(K, generator=gen(K)))
+    x = (x * torch.exp(torch.randn(T, 1, generator=gen(T + 1)))).bfloat16().to(dev)
+    clipper = AutoClipper(True, IntegerQuantizer(bit, sym, 'per_group', group_size=gs), None, 'v1', clip_sym, False, None)
+    kw = dict(n_grid=20, max_shrink=n_steps / 20 + 0.01, n_sample_token=T)
+    want = clipper.auto_clip_layer(0, 'fc', w, [x], **kw)
+    assert clipper.last_errs.shape[-1] == n_steps
+    got = clipper.auto_clip_layer(0, 'fc', w, [x], errors=False, **kw)
+    assert clipper.last_errs is None
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 @pytest.mark.parametrize('gs,clip_sym', [(128, False), (64, True), (32, False)])
 def test_auto_clip_one_launch_search_keeps_rows_apart(dev, gs, clip_sym):
     """An infinite or NaN weight, and a finite one whose products overflow, spoil their own row of their group only: every
