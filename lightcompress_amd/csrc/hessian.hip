@@ -598,6 +598,13 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(const void* __restrict
   const int last = (int)min(p0 + T - 8 * q, (int64_t)8);                // positions from here on hold zeros
   const auto emit = [&](const uint32_t (*v)[4], u32x4* dst) {
     u32x4* const mine = turn[wave];
+    // where lane l's piece j goes: feature l % 8 of octet 8 j + l / 8
+    const auto place = [&](int j) { const int at = o0 + 8 * j + (lane >> 3); return dst + (((q >> 1) * (oct >> 2) + (at >> 2)) * 2 + (q & 1)) * 32 + (at & 3) * 8 + (lane & 7); };
+    u32x4 have[COMPARE ? 8 : 1];
+    if constexpr (COMPARE) {                        // on their way while the tokens come in and change lanes
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) have[j] = o0 + 8 * j + (lane >> 3) < oct ? *place(j) : u32x4{0, 0, 0, 0};
+    }
     #pragma unroll
     for (int f = 0; f < 8; ++f) {
       u32x4 r;
@@ -609,18 +616,16 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(const void* __restrict
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     #pragma unroll
-    for (int j = 0; j < 8; ++j) {                   // lane l: feature l % 8 of octet 8 j + l / 8
-      const int oo = 8 * j + (lane >> 3), f = lane & 7;
-      const u32x4 r = mine[oo * 8 + (f ^ (oo & 7))];
-      const int at = o0 + oo;
-      if (at >= oct) continue;
-      u32x4* const d = dst + (((q >> 1) * (oct >> 2) + (at >> 2)) * 2 + (q & 1)) * 32 + (at & 3) * 8 + f;
+    for (int j = 0; j < 8; ++j) {
+      const int oo = 8 * j + (lane >> 3);
+      const u32x4 r = mine[oo * 8 + ((lane & 7) ^ (oo & 7))];
+      if (o0 + oo >= oct) continue;
+      u32x4* const d = place(j);
       if constexpr (COMPARE) {
-        const u32x4 have = *d;
         uint32_t diff = 0;
         #pragma unroll
         for (int k = 0; k < 8; ++k)
-          if (k >= skip && k < last) diff |= ((r[k >> 1] ^ have[k >> 1]) >> (16 * (k & 1))) & 0xffffu;
+          if (k >= skip && k < last) diff |= ((r[k >> 1] ^ have[j][k >> 1]) >> (16 * (k & 1))) & 0xffffu;
         if (diff != 0) *flag = 1;                   // every writer stores the same value
       } else if (skip == 0) {
         __builtin_nontemporal_store(r, d);
