@@ -24,6 +24,7 @@
 //   scatter        U[i][j] = Linv[K-1-i][K-1-j], j >= i; zeros below the diagonal
 #include <mutex>
 #include "gemm_f32.h"
+#include "gemm_h2.h"
 #include "lcq_internal.h"
 
 namespace lcq {
@@ -516,11 +517,17 @@ __global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ 
 
 }  // namespace
 
+// super-panels of the factorization, and the workspace in front of the packed one
+constexpr int NBO = 4 * NB;
+static int64_t chol_base_bytes(int64_t K, int64_t nblk) {
+  return (K * K * 4 + nblk * NB * NB * 4 + ((K + 255) / 256) * 256 + 256 + 255) / 256 * 256;
+}
+
 extern "C" {
 
 int64_t lcq_chol_inv_upper_workspace_bytes(int64_t K) {
   const int64_t nblk = (K + NB - 1) / NB;
-  return K * K * 4 + nblk * NB * NB * 4 + ((K + 255) / 256) * 256 + 256;
+  return chol_base_bytes(K, nblk) + h2_bytes(K, NBO);
 }
 
 int lcq_set_gemm_split(int on) {
@@ -597,6 +604,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   float* Dinv = A + (long long)K * K;
   uint8_t* dead = (uint8_t*)(Dinv + (long long)nblk * NB * NB);
   PrepScalars* sc = (PrepScalars*)(dead + ((K + 255) / 256) * 256);
+  void* const h2_space = (char*)workspace + chol_base_bytes(K, nblk);     // the current super-panel for the deep updates
 
   diag_prep_kernel<<<dim3(1), dim3(1024), 0, st>>>(H, K, percdamp, dead, sc);
   if (W && R > 0) {
@@ -617,13 +625,18 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   // cuts the read-modify-write traffic on the trailing matrix fourfold.
   // The last 1024 columns are one super-panel: their rank-128 updates are at most 98 of the 64 x 128 tiles, so each still takes
   // one tile's time (8 us), while the 512-deep update they replace ran on 10 to 36 of 256 CUs (32 us).
-  constexpr int NBO = 4 * NB, TAIL = 8 * NB;
+  constexpr int TAIL = 8 * NB;
   const auto super_end = [&](int o0) { return K - o0 <= TAIL ? K : o0 + NBO; };
   // Long chains: the deep update behind a super-panel is split into the columns of the NEXT super-panel (on the
   // caller's stream, the panels that follow need it) and everything behind those (on the side stream, beside those
   // panels: a few narrow launches that leave the chip to it).  The next deep update touches that region again and
   // waits for it.
   SideLane* lane = (g_lookahead.load() && K >= 8192) ? side_lane(st) : nullptr;
+  // The deep updates as fp16 products (gemm_h2.h) from 3072 rows on, 78 of their 256 x 256 tiles (41 against 48 us; 13824 rows:
+  // 343 against 655).
+  const auto deep_pays = [&](const float* P, int o0, int o1, int rows) {
+    return g_gemm_split.load() != 0 && rows >= 3072 && o1 - o0 == NBO && h2_operand(P, K, o1 - o0);
+  };
   bool pending = false;
   for (int o0 = 0, o1; o0 < K; o0 = o1) {
     o1 = super_end(o0);
@@ -646,21 +659,32 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
       const float* P = A + (long long)o1 * K + o0;
       if (pending && hipStreamWaitEvent(st, lane->join, 0) != hipSuccess) return LCQ_ELAUNCH;
       pending = false;
+      const H2Operand panel(h2_space, K - o1, NBO);                                   // (the side stream is done with the last one)
+      const bool deep = deep_pays(P, o0, o1, K - o1);
+      if (deep) h2_pack<false>(P, K, K - o1, o1 - o0, panel, st);
       if (hipEventRecord(lane->fork, st) != hipSuccess) return LCQ_ELAUNCH;           // the panels of this super-panel
-      launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, o2 - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                        GEMM_LOWER_TILES, st);
+      if (deep) h2_multiply<false>(panel, 0, panel, 0, A + (long long)o1 * K + o1, K, K - o1, o2 - o1, o1 - o0, st);
+      else launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, o2 - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
+                             GEMM_LOWER_TILES, st);
       if (o2 < K) {
         const float* P2 = A + (long long)o2 * K + o0;
         if (hipStreamWaitEvent(lane->side, lane->fork, 0) != hipSuccess) return LCQ_ELAUNCH;
-        launch_gemm<true>(GemmProblem{P2, P2, A + (long long)o2 * K + o2, K - o2, K - o2, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                          GEMM_LOWER_TILES, lane->side);
+        if (deep) h2_multiply<true>(panel, o2 - o1, panel, o2 - o1, A + (long long)o2 * K + o2, K, K - o2, K - o2, o1 - o0, lane->side);
+        else launch_gemm<true>(GemmProblem{P2, P2, A + (long long)o2 * K + o2, K - o2, K - o2, o1 - o0, K, K, K}, -1.0f, 1.0f,
+                               GEMM_LOWER_TILES, lane->side);
         if (hipEventRecord(lane->join, lane->side) != hipSuccess) return LCQ_ELAUNCH;
         pending = true;
       }
     } else if (o1 < K) {                                                                          // everything behind it
       const float* P = A + (long long)o1 * K + o0;
-      launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, K - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                        GEMM_LOWER_TILES, st);
+      if (deep_pays(P, o0, o1, K - o1)) {
+        const H2Operand panel(h2_space, K - o1, NBO);
+        h2_pack<false>(P, K, K - o1, o1 - o0, panel, st);
+        h2_multiply<true>(panel, 0, panel, 0, A + (long long)o1 * K + o1, K, K - o1, K - o1, o1 - o0, st);
+      } else {
+        launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, K - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
+                          GEMM_LOWER_TILES, st);
+      }
     }
   }
   if (pending && hipStreamWaitEvent(st, lane->join, 0) != hipSuccess) return LCQ_ELAUNCH;

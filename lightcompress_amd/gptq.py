@@ -948,6 +948,7 @@ class GPTQ:
         B = int(self.blocksize)
         window = 8 * B if B <= 128 else B * max(1, 1024 // B)
         Err = torch.empty((R, window), device=W.device)
+        space = None                                     # the split operands of the deep updates
         lib = L.lib()
         st = L.stream()
         qmin, qmax = L.f32(wq.qmin), L.f32(wq.qmax)
@@ -995,8 +996,11 @@ class GPTQ:
                         L.check(lib.lcq_gptq_trailing(L.ptr(W), C_ptr(err_blk), L.i64(window), L.ptr(Hinv), L.i64(R), L.i64(K),
                                                       L.i64(i1), L.i64(i2), L.i64(i2), L.i64(hi), st), 'lcq_gptq_trailing')
             if hi < K:
-                L.check(lib.lcq_gptq_trailing(L.ptr(W), L.ptr(Err), L.i64(window), L.ptr(Hinv), L.i64(R), L.i64(K),
-                                              L.i64(o0), L.i64(o1), L.i64(hi), L.i64(K), st), 'lcq_gptq_trailing')
+                nbytes = lib.lcq_gptq_trailing_workspace_bytes(R, K, o0, o1, hi, K)
+                if nbytes > (0 if space is None else space.numel()):     # (the first window asks for the most)
+                    space = torch.empty(nbytes, dtype=torch.uint8, device=W.device)
+                L.check(lib.lcq_gptq_trailing_deep(L.ptr(W), L.ptr(Err), window, L.ptr(Hinv), R, K, o0, o1, hi, K, L.ptr(space),
+                                                   0 if space is None else space.numel(), st), 'lcq_gptq_trailing_deep')
 
     # -- qparam bookkeeping (gptq.py:332-409) ---------------------------------------
     @torch.no_grad()

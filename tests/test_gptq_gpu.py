@@ -1147,6 +1147,63 @@ def test_split_gemm_has_fp32_accuracy(dev):
         lib.lcq_set_gemm_split(L.i32(1))
 
 
+@pytest.mark.parametrize('R,Kc,N,kind', [(2560, 1024, 2560, 'plain'), (2305, 256, 2700, 'rows'), (4096, 512, 1537, 'spread'),
+                                         (1000, 1024, 6200, 'spread'), (6144, 320, 1024, 'columns'), (2560, 1024, 2560, 'odd')])
+def test_deep_update_on_fp16_pairs(dev, R, Kc, N, kind):
+    """lcq_gptq_trailing_deep against fp64 and against the three-way bf16 split of lcq_gptq_trailing: hi + lo carries an operand
+    to 2^-24 of itself or 2^-40 of its row's (column's) largest value, the dropped product is another 2^-24, and the sum is
+    rounded 3 Kc / 16 times to 2^-24 of what it holds, so an element is off by at most (3 + 3 Kc / 16 + 2) 2^-24 of
+    |row| . |column| + |W| and 2 Kc 2^-40 of the largest values; in the norm it is no further from fp64 than the split it
+    replaces.  Tiles full and ragged; rows and columns of very different sizes, wide spread inside a row, zeros, denormals, a
+    column with an infinity and a row with a NaN (which spoil themselves only)."""
+    from lightcompress_amd import _lib as L
+    lib = L.lib()
+    g = torch.Generator(device=dev).manual_seed(R + N)
+    K = Kc + N
+    W0 = torch.randn(R, K, device=dev, generator=g)
+    U = torch.randn(Kc, K, device=dev, generator=g)
+    Err = torch.randn(R, Kc, device=dev, generator=g)
+    if kind in ('rows', 'odd'):
+        Err *= torch.exp(6 * torch.randn(R, 1, device=dev, generator=g))
+    if kind in ('columns', 'odd'):
+        U *= torch.exp(6 * torch.randn(1, K, device=dev, generator=g))
+    if kind == 'spread':
+        Err *= torch.exp(2 * torch.randn(R, Kc, device=dev, generator=g))
+        U *= torch.exp(2 * torch.randn(Kc, K, device=dev, generator=g))
+    if kind == 'odd':
+        Err[3], U[:, Kc + 5] = 0, 0
+        Err[4] *= 1e-42
+        U[:, Kc + 6] *= 1e-30
+    nbytes = lib.lcq_gptq_trailing_workspace_bytes(R, K, 0, Kc, Kc, K)
+    assert nbytes > 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+
+    def run(deep, Err, U):
+        W = W0.clone()
+        if deep:
+            L.check(lib.lcq_gptq_trailing_deep(L.ptr(W), L.ptr(Err), Kc, L.ptr(U), R, K, 0, Kc, Kc, K, L.ptr(ws), nbytes, L.stream()), 'deep')
+        else:
+            L.check(lib.lcq_gptq_trailing(L.ptr(W), L.ptr(Err), Kc, L.ptr(U), R, K, 0, Kc, Kc, K, L.stream()), 'trailing')
+        assert torch.equal(W[:, :Kc], W0[:, :Kc])
+        return W[:, Kc:]
+    got, old = run(True, Err, U), run(False, Err, U)
+    A, B, C = Err.double(), U[:, Kc:].double(), W0[:, Kc:].double()
+    ref, mag = C - A @ B, C.abs() + A.abs() @ B.abs()
+    tops = A.abs().amax(1, keepdim=True) * B.abs().amax(0, keepdim=True)
+    bound = (5 + 3 * Kc / 16) * 2.0 ** -24 * mag + 2 * Kc * 2.0 ** -40 * tops + 1e-37
+    assert bool(((got.double() - ref).abs() <= bound).all())
+    size = mag.clamp(min=1e-30)
+    far = {n: float((((x.double() - ref) / size) ** 2).mean().sqrt()) for n, x in (('got', got), ('old', old))}
+    assert far['got'] <= 1.05 * far['old'], far
+    Err2, U2 = Err.clone(), U.clone()
+    Err2[7, 1], U2[2, Kc + 9] = float('nan'), float('inf')
+    bad = run(True, Err2, U2)
+    keep = torch.ones_like(bad, dtype=torch.bool)
+    keep[7], keep[:, 9] = False, False
+    assert torch.equal(bad[keep], got[keep]) and bool(bad[7].isnan().all()) and not bool(bad[:, 9].isfinite().any())
+    assert lib.lcq_gptq_trailing_deep(L.ptr(W0), L.ptr(Err), Kc, L.ptr(U), R, K, 0, Kc, Kc, K, L.ptr(ws), nbytes - 1, L.stream()) == -5
+
+
 @pytest.mark.parametrize('sym', [False, True])
 def test_groups_view_and_ready(dev, sym):
     """`groups` is the reference's list of per-group dicts (gptq.py:358-366, 385-395): entry i holds the [R, 1]
