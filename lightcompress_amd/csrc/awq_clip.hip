@@ -400,18 +400,19 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
 // The same search without the errors of steps that cannot win (errs == NULL, at most two tiles of tokens per wave).
 //
 // The rounded original sums o_t are computed as above; a step's sums only up to their roundings, as plain matrix products:
-//   a_t = sum_j x w_s - o_t,   |e_t - a_t| <= b_t = u (sum_j |x w_s| + |sum_j x w_s| + |a_t|),   u a little above 2^-9
-// (every product, the sum and the difference are rounded once, each by at most 2^-9 of itself), so with Minkowski's
-// inequality over the tokens  (|a| - |b|)^2 <= sum_t e_t^2 <= (|a| + |b|)^2.  A step whose lower bound is above the smallest
-// upper bound of its row by more than what rounding the squares (2^-9 either way) and the mean (a bf16 step, 2^-7) can make up
-// for neither wins nor ties (MARGIN).  The other steps of rows with more than one of them are evaluated as above, 32 (step,
-// row) pairs to a tile whatever rows and steps they come from, first on half of the tokens: the exact sums of those with the
-// bounds of the rest decide again.  Rows that are not plain (a bound that is not finite, or below SMALL where underflow might
-// count, or near the 1e9 the search starts from) have every step evaluated.
-// Measured (an MLP's Linears as above, 10 steps): 25.8 -> 18.3 ms; 4.3 of 10 steps are evaluated, the matrix pipes are busy in
-// 58 % of the cycles (the making of the versions, estimates and decisions are not overlapped by another workgroup: one fills
-// the LDS).  One step at a time in the estimates and decisions by a single wave: 19.9 ms.
-constexpr float CLIP_U = 2.03e-3f, CLIP_MARGIN = 1.02f, CLIP_SMALL = 1e-25f;
+//   a_t = sum_j x w_s - o_t,   |e_t - a_t| <= b_t = u (sum_j |x w_s| + |sum_j x w_s| + |a_t|)
+// (every product, the sum and the difference are rounded once, each by at most 2^-8 / (1 + 2^-8) of itself; CLIP_U adds what these
+// roundings do to each other, 2 u of u, and 2.5e-3 u for the fp32 sums of either side), so
+//   sum_t max(|a_t| - b_t, 0)^2 <= sum_t e_t^2 <= sum_t (|a_t| + b_t)^2.
+// A step whose lower bound is above the smallest upper bound of its row by more than what rounding the squares (2^-8 either way)
+// and the mean (a bf16 step, 2^-7) can make up for neither wins nor ties (CLIP_MARGIN).  The other steps of rows with more than one of
+// them are evaluated as above, 32 (step, row) pairs to a tile whatever rows and steps they come from, first on half of the tokens:
+// the exact sums of those with the bounds of the rest decide again.  Rows that are not plain (a bound that is not finite, or below
+// CLIP_SMALL where underflow might count, or near the 1e9 the search starts from) have every step evaluated.
+// Measured (an MLP's Linears as above, 10 steps): 25.7 -> 21.3 ms; 5.6 of 10 steps are evaluated, the matrix pipes are busy in
+// 60 % of the cycles (the making of the versions, estimates and decisions are not overlapped by another workgroup: one fills
+// the LDS).  One step at a time in the estimates, and decisions by a single wave: 1.6 ms more.
+constexpr float CLIP_U = 3.95e-3f, CLIP_MARGIN = 1.02f, CLIP_SMALL = 1e-25f;
 template <int GS> constexpr size_t clip_pruned_lds(int n_steps, int waves, int rounds) {
   return (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)rounds * waves * GT * GT * 2 + (size_t)waves * n_steps * GT * 8 +
          (size_t)(rounds + 1) * n_steps * GT * 8 + (size_t)(n_steps + 1) * GT * 2 + GT * 4 + 16;
@@ -428,8 +429,8 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
   const int rounds = (T + waves * GT - 1) / (waves * GT), pairs = n_steps * GT;
   const int G = K / GS, g = blockIdx.x % G, r0 = (blockIdx.x / G) * GT;
   uint16_t* const orgs = (uint16_t*)(smem + (n_steps + 1) * VERSION);    // [tokens][32] bf16
-  float* const part = (float*)(orgs + rounds * waves * GT * GT);         // [waves][pairs] a^2, b^2; later [waves][pairs] exact sums
-  float* const tab = part + waves * pairs * 2;                           // [rounds][pairs] a^2, b^2
+  float* const part = (float*)(orgs + rounds * waves * GT * GT);         // [waves][pairs] bounds; later [waves][pairs] exact sums
+  float* const tab = part + waves * pairs * 2;                           // [rounds][pairs] lower, upper
   float* const bounds = tab + rounds * pairs * 2;                        // [pairs] lower, upper
   uint16_t* const list = (uint16_t*)(bounds + pairs * 2);                // (step, row) = entry / 32, entry % 32
   uint32_t* const masks = (uint32_t*)(list + pairs + GT);                // steps of a row that may still win; FOUND: the one left does
@@ -498,16 +499,17 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
         }
         #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          float a2 = 0.0f, b2 = 0.0f;
+          float lo = 0.0f, hi = 0.0f;
           #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const float d = sum[v][r] - o[r], e = (mag[v][r] + fabsf(sum[v][r])) + fabsf(d);
-            a2 = __builtin_fmaf(d, d, a2);
-            b2 = __builtin_fmaf(e, e, b2);
+            const float d = fabsf(sum[v][r] - o[r]), b = CLIP_U * ((mag[v][r] + fabsf(sum[v][r])) + d);
+            const float l = fmaxf(d - b, 0.0f), u = d + b;
+            lo = __builtin_fmaf(l, l, lo);
+            hi = __builtin_fmaf(u, u, hi);
           }
-          a2 += __shfl_xor(a2, 32);
-          b2 += __shfl_xor(b2, 32);
-          if (h == 0 && s + v < n_steps) *(f32x2*)(part + 2 * ((wave * n_steps + s + v) * GT + c)) = f32x2{a2, b2 * (CLIP_U * CLIP_U)};
+          lo += __shfl_xor(lo, 32);
+          hi += __shfl_xor(hi, 32);
+          if (h == 0 && s + v < n_steps) *(f32x2*)(part + 2 * ((wave * n_steps + s + v) * GT + c)) = f32x2{lo, hi};
         }
       }
     } else {
@@ -515,9 +517,9 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
     }
     __syncthreads();
     for (int i = tid; i < pairs; i += blockDim.x) {
-      float a2 = 0.0f, b2 = 0.0f;
-      for (int v = 0; v < waves; ++v) { a2 += part[2 * (v * pairs + i)]; b2 += part[2 * (v * pairs + i) + 1]; }
-      *(f32x2*)(tab + 2 * (k * pairs + i)) = f32x2{a2, b2};
+      float lo = 0.0f, hi = 0.0f;
+      for (int v = 0; v < waves; ++v) { lo += part[2 * (v * pairs + i)]; hi += part[2 * (v * pairs + i) + 1]; }
+      *(f32x2*)(tab + 2 * (k * pairs + i)) = f32x2{lo, hi};
     }
     __syncthreads();
   }
@@ -525,13 +527,14 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
   // Which steps may still win, with `done` rounds of tokens evaluated: masks and the list of pairs to go on with.
   const auto decide = [&](int done) {
     for (int i = tid; i < pairs; i += blockDim.x) {                      // bounds of every pair
-      float a2 = 0.0f, b2 = 0.0f, e = 0.0f;
-      for (int k = done; k < rounds; ++k) { a2 += tab[2 * (k * pairs + i)]; b2 += tab[2 * (k * pairs + i) + 1]; }
-      if (done)
+      float lo = 0.0f, hi = 0.0f;
+      for (int k = done; k < rounds; ++k) { lo += tab[2 * (k * pairs + i)]; hi += tab[2 * (k * pairs + i) + 1]; }
+      if (done) {
+        float e = 0.0f;
         for (int v = 0; v < waves; ++v) e += part[v * pairs + i];
-      const float ra = __builtin_amdgcn_sqrtf(a2), rb = __builtin_amdgcn_sqrtf(b2);
-      const float lo = fmaxf(ra * (1.0f - 1e-5f) - rb, 0.0f), hi = (ra + rb) * (1.0f + 1e-5f);
-      *(f32x2*)(bounds + 2 * i) = f32x2{e + lo * lo, e + hi * hi};
+        lo += e; hi += e;
+      }
+      *(f32x2*)(bounds + 2 * i) = f32x2{lo * (1.0f - 1e-4f), hi * (1.0f + 1e-4f)};              // (their own fp32 sums)
     }
     __syncthreads();
     if (wave != 0) return;

@@ -436,7 +436,8 @@ def test_auto_clip_search_without_the_losing_steps(dev, gs, T, bit, sym, clip_sy
     """With errors=False the steps that a bound shows to lose are not evaluated: the ranges are those of the search that
     evaluates them all, bit for bit (beyond 512 tokens, or where LDS does not hold the bounds, it IS that search).  Tiles of
     rows and tokens full and ragged, one and two rounds of tokens; rows of every size from underflow to overflow, of few
-    distinct values (exact ties), of zeros, with an infinity or a NaN; tokens of very different sizes."""
+    distinct values (exact ties), of zeros, with an infinity or a NaN; tokens of very different sizes, products that round by as
+    much as they can, all the same way."""
     from lightcompress_amd import IntegerQuantizer
     from lightcompress_amd.auto_clip import AutoClipper
     from tests.helpers import weight_like
@@ -447,9 +448,13 @@ def test_auto_clip_search_without_the_losing_steps(dev, gs, T, bit, sym, clip_sy
     w[128:132] = 0
     w[133, 1], w[134, 2], w[135, gs + 3] = float('inf'), float('nan'), -float('inf')
     w[136:140] = w[136:140, :1]
+    w[144:160] = 1.0625 * torch.exp2(torch.randint(-9, -3, (16, K), generator=gen(3)).float())
     w = w.bfloat16().to(dev)
     x = torch.randn(T, K, generator=gen(T)) * torch.exp(torch.randn(K, generator=gen(K)))
-    x = (x * torch.exp(torch.randn(T, 1, generator=gen(T + 1)))).bfloat16().to(dev)
+    x = x * torch.exp(torch.randn(T, 1, generator=gen(T + 1)))
+    if T % 2 == 0:                                           # 1.0625 * 1.0625 lies on a tie: every product rounds by 2^-8 / 1.129
+        x = torch.where(torch.rand(T, 1, generator=gen(7)) < 0.5, 1.0625 * torch.exp2(torch.floor(torch.log2(x.abs() + 1e-9))), x)
+    x = x.bfloat16().to(dev)
     clipper = AutoClipper(True, IntegerQuantizer(bit, sym, 'per_group', group_size=gs), None, 'v1', clip_sym, False, None)
     kw = dict(n_grid=20, max_shrink=n_steps / 20 + 0.01, n_sample_token=T)
     want = clipper.auto_clip_layer(0, 'fc', w, [x], **kw)
