@@ -564,21 +564,21 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(const void* __restrict
                                                           int64_t rows, u32x4* __restrict__ out, u32x4* __restrict__ lo,
                                                           int* __restrict__ flag) {
   __shared__ u32x4 turn[4][64 * 8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunks = (oct + 63) / 64;
-  const int64_t id = (int64_t)blockIdx.x * 4 + wave, row = id / chunks, q = p0 / 8 + row;      // positions 8 q .. 8 q + 7
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), chunks = (oct + 63) / 64;
+  const uint32_t id = blockIdx.x * 4 + wave, row = id / (uint32_t)chunks;
+  const int64_t q = p0 / 8 + row;                   // positions 8 q .. 8 q + 7
   if (row >= rows) return;
-  const int o0 = (int)(id - row * chunks) * 64, o = o0 + lane;          // features 8 o .. 8 o + 7
+  const int o0 = (int)(id - row * (uint32_t)chunks) * 64, o = o0 + lane;          // features 8 o .. 8 o + 7
   uint32_t w[8][4], l[8][4];                        // token k: four pairs of features
-  #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int64_t t = 8 * q + k - p0;
-    const bool ok = t >= 0 && t < T && 8 * o < K;
+  const int64_t first = 8 * q - p0;                 // token of position 8 q (negative: it belongs to an earlier call)
+  constexpr int ES = F32 ? 4 : 2;
+  const char* const xp = (const char*)x + (first * ldx + 8 * o) * ES;
+  const auto load = [&](int k, bool ok) {
     if constexpr (F32) {
       f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
       if (ok) {
-        const f32x4* const xp = (const f32x4*)((const float*)x + t * ldx + 8 * o);
-        a = __builtin_nontemporal_load(xp);
-        b = __builtin_nontemporal_load(xp + 1);
+        a = __builtin_nontemporal_load((const f32x4*)(xp + k * ldx * ES));
+        b = __builtin_nontemporal_load((const f32x4*)(xp + k * ldx * ES) + 1);
       }
       #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -589,17 +589,27 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(const void* __restrict
       }
     } else {
       u32x4 a = {0, 0, 0, 0};
-      if (ok) a = __builtin_nontemporal_load((const u32x4*)((const uint16_t*)x + t * ldx + 8 * o));
+      if (ok) a = __builtin_nontemporal_load((const u32x4*)(xp + k * ldx * ES));
       #pragma unroll
       for (int i = 0; i < 4; ++i) w[k][i] = a[i];
     }
+  };
+  // nearly all waves: eight whole tokens.  (A lone wave issues an instruction every eight cycles: what a small call costs is
+  // counted in them.)
+  if (first >= 0 && first + 8 <= T && 8 * (o0 + 64) <= K) {
+    #pragma unroll
+    for (int k = 0; k < 8; ++k) load(k, true);
+  } else {
+    #pragma unroll
+    for (int k = 0; k < 8; ++k) load(k, first + k >= 0 && first + k < T && 8 * o < K);
   }
   const int skip = (int)max(p0 - 8 * q, (int64_t)0);                    // positions of the first piece that belong to earlier tokens
   const int last = (int)min(p0 + T - 8 * q, (int64_t)8);                // positions from here on hold zeros
   const auto emit = [&](const uint32_t (*v)[4], u32x4* dst) {
     u32x4* const mine = turn[wave];
-    // where lane l's piece j goes: feature l % 8 of octet 8 j + l / 8
-    const auto place = [&](int j) { const int at = o0 + 8 * j + (lane >> 3); return dst + (((q >> 1) * (oct >> 2) + (at >> 2)) * 2 + (q & 1)) * 32 + (at & 3) * 8 + (lane & 7); };
+    // where lane l's piece j goes: feature l % 8 of octet 8 j + l / 8 (o0 is a multiple of 64: two blocks of 32 features per j)
+    u32x4* const place0 = dst + (((q >> 1) * (oct >> 2) + ((o0 + (lane >> 3)) >> 2)) * 2 + (q & 1)) * 32 + ((lane >> 3) & 3) * 8 + (lane & 7);
+    const auto place = [&](int j) { return place0 + j * 128; };
     u32x4 have[COMPARE ? 8 : 1];
     if constexpr (COMPARE) {                        // on their way while the tokens come in and change lanes
       #pragma unroll
@@ -852,7 +862,7 @@ static int pack_tokens(bool compare, const void* x, int dtype, int64_t T, int64_
   const int64_t rows = (compare ? (at + T + 7) / 8 : (at + T + BT - 1) / BT * (BT / 8)) - at / 8;
   if (rows <= 0 || (compare && T == 0)) return LCQ_OK;
   const int64_t grid = (rows * ((oct + 63) / 64) + 3) / 4;
-  if (grid > 0x7fffffff) return LCQ_ESIZE;
+  if (grid > 0x3fffffff) return LCQ_ESIZE;          // (the kernel numbers its waves with 32 bits)
   #define LCQ_PACK(F, C) pack_tokens_kernel<F, C><<<dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream>>>( \
       x, ldx, (int)K, oct, at, T, rows, (u32x4*)packed, (u32x4*)packed_lo, flag)
   if (f32) { if (compare) LCQ_PACK(true, true); else LCQ_PACK(true, false); }
