@@ -1,11 +1,13 @@
 // fp32 products as three fp16 products, for the large launches of the Cholesky chain and of the column loop.
 //
 //   x = hi + lo,  hi = fp16(s x), lo = fp16(s x - hi)       s a power of two per row of A and per column of B
-// carries x to 2^-24 of itself (hi leaves a residual of at most 2^-12 |x|, lo rounds that by 2^-12), as long as x is above
-// 2^-17 of the largest value of its row, and to 2^-40 of that value below; a b = lo hi + hi lo + hi hi, the dropped lo lo being
-// at most 2^-24 of the product.  Three matrix instructions accumulate in fp32 where the three-way bf16 split takes six, so the sum
-// is rounded half as often: against fp64 it is as close as the bf16 split or closer (measured: tests and DESIGN), which is
-// closer than the fp32 pipe.
+// carries x to 2^-23 of itself (hi, 11 bits, leaves a residual of at most 2^-11 |x|, whose last bit lo loses where it has more
+// than 11), as long as x is above 2^-17 of the largest value of its row, and to 2^-40 of that value below; a b = lo hi + hi lo +
+// hi hi, the dropped lo lo being at most 2^-22 of the product.  Three matrix instructions accumulate in fp32 where the three-way
+// bf16 split takes six, so the sum is rounded half as often.  The operands' part does not grow with the depth (some 7e-8 of the
+// norm, the three-way split's is 1e-8), the sum's does: from 512 on the result is closer to fp64 than the three-way split's
+// (below), which is closer than the fp32 pipe's; at 256 a few large products per element (exp(2 N) of a normal N as elements of
+// both) leave 1.6e-7 against 0.8e-7.  Shallower products stay with the three-way split.
 //
 // The operands are split once (h2_pack_kernel), not by every tile that reads them, into the order the matrix pipe reads:
 //   planes[k / 16][hi, lo][row / 32][(k / 8) % 2][row % 32][k % 8]        1 KiB per operand of v_mfma_f32_32x32x16_f16
@@ -252,7 +254,7 @@ inline void h2_pack(const float* src, int64_t ld, int rows, int Kc, const H2Oper
 }
 
 // May a row-major operand [rows, Kc] be packed?  (One given as [Kc, rows] only needs the depth.)
-inline bool h2_depth(int64_t Kc) { return Kc % 64 == 0 && Kc >= 256 && Kc <= H2_MAX_K; }
+inline bool h2_depth(int64_t Kc) { return Kc % 64 == 0 && Kc >= 512 && Kc <= H2_MAX_K; }      // (why 512: at the top)
 inline bool h2_operand(const float* p, int64_t ld, int64_t Kc) { return h2_depth(Kc) && ld % 4 == 0 && (uintptr_t)p % 16 == 0; }
 inline int64_t h2_tiles(int64_t M, int64_t N) { return ((M + H2_T - 1) / H2_T) * ((N + H2_T - 1) / H2_T); }
 

@@ -8,7 +8,11 @@
 // bf16 x bf16 products are exact in fp32, so a bf16-in / fp32-accumulate MFMA
 // GEMM differs from the reference's fp32 SGEMM only in summation order.
 //
-// Shape of the kernel
+// Two kernels.  hessian_packed_kernel reads tokens that were staged in the matrix pipe's own order (pack_tokens_kernel); it is
+// what add_batch uses beyond K = 512, and its comment has the figures.  hessian_kernel below reads a plain [T, K] tensor: the
+// entry points without staging, the token shares of small K, and explicit ones.
+//
+// Shape of hessian_kernel
 //  * a workgroup owns a 256 x TN tile of H, TN = 128: 4 waves (2 x 2), two
 //    workgroups per CU, so one tile's barriers and epilogue overlap the other's
 //    MFMAs.  (The template also covers TN = 256 - 8 waves, one workgroup
@@ -369,7 +373,7 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(float* __restrict__ H, i
 //  * four LDS stages of 32 tokens, one barrier per slab: at the middle of a slab every wave holds the rest of it in
 //    registers, so its stage is free for the slab four ahead.
 // The chip clocks down under this load (random tokens 1.7 GHz, zeros run 1.3 times as fast), which is what bounds it.
-// Measured on one box (us, without the copy): K = 14336, 32768 tokens 5919 -> 5010 (1.37 PFLOP/s of the tiles computed),
+// Measured (us, without the copy): K = 14336, 32768 tokens 5919 -> 5010 (1.37 PFLOP/s of the tiles computed),
 // K = 4096, 65536 tokens 1064 -> 861, K = 8192, 32768 tokens 2026 -> 1622, K = 2048, 65536 tokens 305 -> 245; against
 // hessian_kernel with the token shares or split rounds it had for the same work.
 typedef const __attribute__((address_space(3))) char* lds_ptr;

@@ -1147,12 +1147,12 @@ def test_split_gemm_has_fp32_accuracy(dev):
         lib.lcq_set_gemm_split(L.i32(1))
 
 
-@pytest.mark.parametrize('R,Kc,N,kind', [(2560, 1024, 2560, 'plain'), (2305, 256, 2700, 'rows'), (4096, 512, 1537, 'spread'),
-                                         (1000, 1024, 6200, 'spread'), (6144, 320, 1024, 'columns'), (2560, 1024, 2560, 'odd')])
+@pytest.mark.parametrize('R,Kc,N,kind', [(2560, 1024, 2560, 'plain'), (2305, 512, 2700, 'rows'), (4096, 512, 1537, 'spread'),
+                                         (1000, 1024, 6200, 'spread'), (6144, 576, 1024, 'columns'), (2560, 1024, 2560, 'odd')])
 def test_deep_update_on_fp16_pairs(dev, R, Kc, N, kind):
     """lcq_gptq_trailing_deep against fp64 and against the three-way bf16 split of lcq_gptq_trailing: hi + lo carries an operand
-    to 2^-24 of itself or 2^-40 of its row's (column's) largest value, the dropped product is another 2^-24, and the sum is
-    rounded 3 Kc / 16 times to 2^-24 of what it holds, so an element is off by at most (3 + 3 Kc / 16 + 2) 2^-24 of
+    to 2^-23 of itself or 2^-40 of its row's (column's) largest value, the dropped product is at most 2^-22, and the sum is
+    rounded 3 Kc / 16 times to 2^-24 of what it holds, so an element is off by at most (8 + 3 Kc / 16 + 2) 2^-24 of
     |row| . |column| + |W| and 2 Kc 2^-40 of the largest values; in the norm it is no further from fp64 than the split it
     replaces.  Tiles full and ragged; rows and columns of very different sizes, wide spread inside a row, zeros, denormals, a
     column with an infinity and a row with a NaN (which spoil themselves only)."""
@@ -1190,7 +1190,7 @@ def test_deep_update_on_fp16_pairs(dev, R, Kc, N, kind):
     A, B, C = Err.double(), U[:, Kc:].double(), W0[:, Kc:].double()
     ref, mag = C - A @ B, C.abs() + A.abs() @ B.abs()
     tops = A.abs().amax(1, keepdim=True) * B.abs().amax(0, keepdim=True)
-    bound = (5 + 3 * Kc / 16) * 2.0 ** -24 * mag + 2 * Kc * 2.0 ** -40 * tops + 1e-37
+    bound = (10 + 3 * Kc / 16) * 2.0 ** -24 * mag + 2 * Kc * 2.0 ** -40 * tops + 1e-37
     assert bool(((got.double() - ref).abs() <= bound).all())
     size = mag.clamp(min=1e-30)
     far = {n: float((((x.double() - ref) / size) ** 2).mean().sqrt()) for n, x in (('got', got), ('old', old))}
