@@ -199,10 +199,14 @@ template <int GS>
 __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint32_t mask, u32x4 ones, f32x4* sum) {
   #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  u32x4 b = *(const u32x4*)wrow;
+  u32x4 b = *(const u32x4*)wrow, ahead = *(const u32x4*)(wrow + 16);
   const auto products = [&](int i) {                        // columns 2 i (block 0) and 2 i + 1 (block 1)
     const int p = i & 3;
-    if (p == 0 && i > 0) b = *(const u32x4*)(wrow + 4 * i);
+    if (p == 0 && i > 0) {
+      asm volatile("" : "+v"(ahead));                       // (or the load moves to where it is used: 1 %)
+      b = ahead;
+      if (i + 4 < GS / 2) ahead = *(const u32x4*)(wrow + 4 * (i + 4));
+    }
     const u32x4 av = a[i >> 2];
     const uint32_t w = b[p] & mask;
     return outer_products(p < 2 ? u32x2{av[0], av[1]} : u32x2{av[2], av[3]}, (p & 1) ? u32x2{0, w} : u32x2{w, 0});
@@ -406,12 +410,16 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
 //   sum_t max(|a_t| - b_t, 0)^2 <= sum_t e_t^2 <= sum_t (|a_t| + b_t)^2.
 // A step whose lower bound is above the smallest upper bound of its row by more than what rounding the squares (2^-8 either way)
 // and the mean (a bf16 step, 2^-7) can make up for neither wins nor ties (CLIP_MARGIN).  The other steps of rows with more than one of
-// them are evaluated as above, 32 (step, row) pairs to a tile whatever rows and steps they come from, first on half of the tokens:
-// the exact sums of those with the bounds of the rest decide again.  Rows that are not plain (a bound that is not finite, or below
+// them are evaluated as above, 32 (step, row) pairs to a tile whatever rows and steps they come from: first the most promising step of
+// each row (its exact sum decides again, with nothing of the bounds' slack on its side), then the others on half of the tokens, where
+// exact sums and the bounds of the rest decide once more.  Rows that are not plain (a bound that is not finite, or below
 // CLIP_SMALL where underflow might count, or near the 1e9 the search starts from) have every step evaluated.
-// Measured (an MLP's Linears as above, 10 steps): 25.7 -> 21.3 ms; 5.6 of 10 steps are evaluated, the matrix pipes are busy in
-// 60 % of the cycles (the making of the versions, estimates and decisions are not overlapped by another workgroup: one fills
-// the LDS).  One step at a time in the estimates, and decisions by a single wave: 1.6 ms more.
+// Measured (an MLP's Linears as above, 10 steps): 25.7 -> 17.9 ms; 3.7 of 10 steps are evaluated (5.6 without the
+// first step ahead of the others: 21.0 ms; a second and a third step by itself: 19.2, 20.7, a pass costs its tiles however few rows
+// it still has), the matrix pipes are busy in 58 % of the cycles (the making of the versions, estimates and decisions are not
+// overlapped by another workgroup: one fills the LDS).  One step at a time in the estimates, and decisions by a single wave: 1.6 ms
+// more.  Four waves per SIMD, tokens read as they are used so that 128 registers hold it: 23.0 against 21.0 ms, the conversions of
+// two waves already fill the vector pipe beside the products.
 constexpr float CLIP_U = 3.95e-3f, CLIP_MARGIN = 1.02f, CLIP_SMALL = 1e-25f;
 template <int GS> constexpr size_t clip_pruned_lds(int n_steps, int waves, int rounds) {
   return (size_t)(n_steps + 1) * GT * gd_pitch<GS>() + (size_t)rounds * waves * GT * GT * 2 + (size_t)waves * n_steps * GT * 8 +
@@ -433,10 +441,11 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
   float* const tab = part + waves * pairs * 2;                           // [rounds][pairs] lower, upper
   float* const bounds = tab + rounds * pairs * 2;                        // [pairs] lower, upper
   uint16_t* const list = (uint16_t*)(bounds + pairs * 2);                // (step, row) = entry / 32, entry % 32
-  uint32_t* const masks = (uint32_t*)(list + pairs + GT);                // steps of a row that may still win; FOUND: the one left does
+  uint32_t* const masks = (uint32_t*)(list + pairs + GT);                // steps of a row that may still win, the step evaluated first (from bit LEAD on); FOUND: the one left wins
   int* const count = (int*)(masks + GT);
   const uint16_t* const xg = x + g * GS;
   constexpr uint32_t FOUND = 1u << 31;
+  constexpr int LEAD = 24;
 
   make_versions<GS>(smem, w, R, K, r0, g, n_grid, n_steps, clip_sym, op);
   __syncthreads();
@@ -524,24 +533,24 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
     __syncthreads();
   }
 
-  // Which steps may still win, with `done` rounds of tokens evaluated: masks and the list of pairs to go on with.
-  const auto decide = [&](int done) {
+  // Which steps may still win: masks and the list of pairs to go on with.  Before anything is evaluated (!led) that is the most
+  // promising step of each row; then, with that one evaluated and `done` rounds of tokens of the others, the others.
+  const auto decide = [&](bool led, int done) {
     for (int i = tid; i < pairs; i += blockDim.x) {                      // bounds of every pair
-      float lo = 0.0f, hi = 0.0f;
-      for (int k = done; k < rounds; ++k) { lo += tab[2 * (k * pairs + i)]; hi += tab[2 * (k * pairs + i) + 1]; }
-      if (done) {
-        float e = 0.0f;
+      float e = 0.0f, lo = 0.0f, hi = 0.0f;
+      if (led)
         for (int v = 0; v < waves; ++v) e += part[v * pairs + i];
-        lo += e; hi += e;
-      }
+      if (!led || ((masks[i % GT] >> LEAD) & 31) != (uint32_t)(i / GT))
+        for (int k = done; k < rounds; ++k) { lo += tab[2 * (k * pairs + i)]; hi += tab[2 * (k * pairs + i) + 1]; }
+      lo += e; hi += e;
       *(f32x2*)(bounds + 2 * i) = f32x2{lo * (1.0f - 1e-4f), hi * (1.0f + 1e-4f)};              // (their own fp32 sums)
     }
     __syncthreads();
     if (wave != 0) return;
-    uint32_t alive = 0;
+    uint32_t go = 0;
     if (lane < GT && r0 + lane < R) {
-      const uint32_t cand = done ? masks[lane] : (1u << n_steps) - 1;
-      if (!(cand & FOUND)) {
+      const uint32_t all = (1u << n_steps) - 1, was = led ? masks[lane] : all, cand = was & all;
+      if (!(was & FOUND)) {
         f32x2 bnd[LCQ_CLIP_MAX_STEPS];
         #pragma unroll
         for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s) {
@@ -557,19 +566,27 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
             best = fminf(best, bnd[s][1]);
           }
         plain = plain && best > CLIP_SMALL && best < 9e8f * (float)T;
-        alive = cand;
+        uint32_t alive = cand;
         if (plain)
           #pragma unroll
           for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s)
             if (bnd[s][0] > best * CLIP_MARGIN) alive &= ~(1u << s);
         const bool found = plain && (alive & (alive - 1)) == 0;          // needs no more sums
-        masks[lane] = found ? alive | FOUND : alive;
-        if (found) alive = 0;
+        int lead = (was >> LEAD) & 31;
+        if (!led) {
+          lead = __builtin_ctz(alive);                                   // (the best step is never ruled out: not empty)
+          float least = __builtin_inff();
+          #pragma unroll
+          for (int s = 0; s < LCQ_CLIP_MAX_STEPS; ++s)
+            if ((alive >> s) & 1 && bnd[s][0] + bnd[s][1] < least) { least = bnd[s][0] + bnd[s][1]; lead = s; }
+        }
+        masks[lane] = alive | (uint32_t)lead << LEAD | (found ? FOUND : 0);
+        if (!found) go = led ? alive & ~(1u << lead) : 1u << lead;
       }
     }
     int n = 0;
     for (int s = 0; s < n_steps; ++s) {
-      const bool on = (alive >> s) & 1;
+      const bool on = (go >> s) & 1;
       const uint64_t b = __ballot(on);
       if (on) list[n + __popcll(b & ((1ull << lane) - 1))] = (uint16_t)(s * GT + lane);
       n += __popcll(b);
@@ -577,11 +594,12 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
     if (lane < GT && n + lane < (n + GT - 1) / GT * GT) list[n + lane] = 0;               // (the last tile's surplus lanes)
     if (lane == 0) *count = n;
   };
-  decide(0);
+  decide(false, 0);
   __syncthreads();
   for (int i = tid; i < waves * pairs; i += blockDim.x) part[i] = 0.0f;  // from here on: exact sums
   __syncthreads();
-  for (int k = 0; k < rounds; ++k) {
+  for (int pass = 0; pass < 2 * rounds; ++pass) {                        // all tokens of the first step, then round by round the others
+    const int k = pass < rounds ? pass : pass - rounds;
     const int t0 = (k * waves + wave) * GT, n = *count;
     if (t0 < T && n > 0) {
       u32x4 a[GS / 8];
@@ -610,8 +628,8 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
       }
     }
     __syncthreads();
-    if (k + 1 < rounds) {
-      decide(k + 1);
+    if (pass + 1 >= rounds && pass + 1 < 2 * rounds) {
+      decide(true, pass + 1 - rounds);
       __syncthreads();
     }
   }
