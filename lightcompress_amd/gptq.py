@@ -467,11 +467,12 @@ class GPTQ:
         makes 65536 tokens for K <= 4096 and 32768 above (half a GB of staged tokens at K = 4096, one at K = 14336), 128 calls
         at most (so that a few short ones do not ask for such a buffer).  A launch reads and writes H and fills and drains the
         chip once, whatever its tokens: 861 us for 65536 tokens at K = 4096 against 2 x 462, 5.01 ms for 32768 at K = 14336
-        against 4 x 1.32.  Up to K = 1024 a launch is short (25 us for 8192 tokens) and runs while the host stages the next
-        calls, so it is issued early."""
+        against 4 x 1.32.  Up to K = 1024 a launch is short (25 us for 8192 tokens, and 10 for its fold) and runs while the host
+        stages the next calls, so it is issued early: 8192 tokens, but 16 calls at least, for a call leaves the GPU idle for some
+        3 us while it is issued (16 calls of 2000 tokens, four launches: 770 us for the Linear, one: 692)."""
         if self.hessian_defer == 'auto':
-            window = 8192 if K <= 1024 else (65536 if K <= 4096 else 32768)
-            return min(max(window // max(tokens, 1), 2), 128)
+            window, least = (8192, 16) if K <= 1024 else (65536 if K <= 4096 else 32768, 2)
+            return min(max(window // max(tokens, 1), least), 128)
         return self.hessian_defer
 
     def hessian_shares(self, K):
