@@ -368,8 +368,8 @@ int lcq_gptq_block(float* W, float* tmp, float* Losses, float* Err, int64_t ldEr
 int lcq_gptq_trailing(float* W, const float* Err, int64_t ldErr, const float* U, int64_t R, int64_t K, int64_t k1,
                       int64_t k2, int64_t j1, int64_t j2, void* stream);
 
-/* lcq_gptq_trailing for a whole window: with the workspace of lcq_gptq_trailing_workspace_bytes (16-byte aligned) large updates
- * run as fp16 products on operands split once (512 <= k2 - k1 <= 1024, a multiple of 64; closer to fp64 than the other forms).
+/* lcq_gptq_trailing for a whole window, the same bits: with the workspace of lcq_gptq_trailing_workspace_bytes (16-byte aligned)
+ * large updates (512 <= k2 - k1 <= 1024, a multiple of 64) have their operands split into bf16 planes once and not by every tile.
  * 0 bytes: the call is lcq_gptq_trailing and takes a NULL workspace. */
 int64_t lcq_gptq_trailing_workspace_bytes(int64_t R, int64_t K, int64_t k1, int64_t k2, int64_t j1, int64_t j2);
 int lcq_gptq_trailing_deep(float* W, const float* Err, int64_t ldErr, const float* U, int64_t R, int64_t K, int64_t k1, int64_t k2,

@@ -24,7 +24,7 @@
 //   scatter        U[i][j] = Linv[K-1-i][K-1-j], j >= i; zeros below the diagonal
 #include <mutex>
 #include "gemm_f32.h"
-#include "gemm_h2.h"
+#include "gemm_s3p.h"
 #include "lcq_internal.h"
 
 namespace lcq {
@@ -527,7 +527,7 @@ extern "C" {
 
 int64_t lcq_chol_inv_upper_workspace_bytes(int64_t K) {
   const int64_t nblk = (K + NB - 1) / NB;
-  return chol_base_bytes(K, nblk) + h2_bytes(K, NBO);
+  return chol_base_bytes(K, nblk) + s3p_bytes(K, NBO);
 }
 
 int lcq_set_gemm_split(int on) {
@@ -604,7 +604,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   float* Dinv = A + (long long)K * K;
   uint8_t* dead = (uint8_t*)(Dinv + (long long)nblk * NB * NB);
   PrepScalars* sc = (PrepScalars*)(dead + ((K + 255) / 256) * 256);
-  void* const h2_space = (char*)workspace + chol_base_bytes(K, nblk);     // the current super-panel for the deep updates
+  void* const panel_space = (char*)workspace + chol_base_bytes(K, nblk);     // the current super-panel for the deep updates
 
   diag_prep_kernel<<<dim3(1), dim3(1024), 0, st>>>(H, K, percdamp, dead, sc);
   if (W && R > 0) {
@@ -632,10 +632,18 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   // panels: a few narrow launches that leave the chip to it).  The next deep update touches that region again and
   // waits for it.
   SideLane* lane = (g_lookahead.load() && K >= 8192) ? side_lane(st) : nullptr;
-  // The deep updates as fp16 products (gemm_h2.h) from 3072 rows on, 78 of their 256 x 256 tiles (41 against 48 us; 13824 rows:
-  // 343 against 655).
-  const auto deep_pays = [&](const float* P, int o0, int o1, int rows) {
-    return g_gemm_split.load() != 0 && rows >= 3072 && o1 - o0 == NBO && h2_operand(P, K, o1 - o0);
+  // The update of rows and columns from `from` on by the super-panel [o0, o1).
+  const auto deep_update = [&](int o0, int o1, int from, hipStream_t on) {
+    const float* P = A + (long long)from * K + o0;
+    float* C = A + (long long)from * K + from;
+    const int rows = K - from, n = (rows + S3P_T - 1) / S3P_T;
+    if (g_gemm_split.load() != 0 && o1 - o0 == NBO && s3p_pays(rows, rows, (int64_t)n * (n + 1) / 2) && s3p_operand(P, K, NBO)) {
+      const S3POperand panel(panel_space, rows);    // (all deep updates of a chain are on one stream)
+      s3p_pack<false>(P, K, rows, NBO, panel, on);
+      s3p_multiply<true>(panel, panel, C, K, rows, rows, NBO, on);
+    } else {
+      launch_gemm<true>(GemmProblem{P, P, C, rows, rows, o1 - o0, K, K, K}, -1.0f, 1.0f, GEMM_LOWER_TILES, on);
+    }
   };
   bool pending = false;
   for (int o0 = 0, o1; o0 < K; o0 = o1) {
@@ -659,32 +667,17 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
       const float* P = A + (long long)o1 * K + o0;
       if (pending && hipStreamWaitEvent(st, lane->join, 0) != hipSuccess) return LCQ_ELAUNCH;
       pending = false;
-      const H2Operand panel(h2_space, K - o1, NBO);                                   // (the side stream is done with the last one)
-      const bool deep = deep_pays(P, o0, o1, K - o1);
-      if (deep) h2_pack<false>(P, K, K - o1, o1 - o0, panel, st);
       if (hipEventRecord(lane->fork, st) != hipSuccess) return LCQ_ELAUNCH;           // the panels of this super-panel
-      if (deep) h2_multiply<false>(panel, 0, panel, 0, A + (long long)o1 * K + o1, K, K - o1, o2 - o1, o1 - o0, st);
-      else launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, o2 - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                             GEMM_LOWER_TILES, st);
+      launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, o2 - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
+                        GEMM_LOWER_TILES, st);
       if (o2 < K) {
-        const float* P2 = A + (long long)o2 * K + o0;
         if (hipStreamWaitEvent(lane->side, lane->fork, 0) != hipSuccess) return LCQ_ELAUNCH;
-        if (deep) h2_multiply<true>(panel, o2 - o1, panel, o2 - o1, A + (long long)o2 * K + o2, K, K - o2, K - o2, o1 - o0, lane->side);
-        else launch_gemm<true>(GemmProblem{P2, P2, A + (long long)o2 * K + o2, K - o2, K - o2, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                               GEMM_LOWER_TILES, lane->side);
+        deep_update(o0, o1, o2, lane->side);
         if (hipEventRecord(lane->join, lane->side) != hipSuccess) return LCQ_ELAUNCH;
         pending = true;
       }
     } else if (o1 < K) {                                                                          // everything behind it
-      const float* P = A + (long long)o1 * K + o0;
-      if (deep_pays(P, o0, o1, K - o1)) {
-        const H2Operand panel(h2_space, K - o1, NBO);
-        h2_pack<false>(P, K, K - o1, o1 - o0, panel, st);
-        h2_multiply<true>(panel, 0, panel, 0, A + (long long)o1 * K + o1, K, K - o1, K - o1, o1 - o0, st);
-      } else {
-        launch_gemm<true>(GemmProblem{P, P, A + (long long)o1 * K + o1, K - o1, K - o1, o1 - o0, K, K, K}, -1.0f, 1.0f,
-                          GEMM_LOWER_TILES, st);
-      }
+      deep_update(o0, o1, o1, st);
     }
   }
   if (pending && hipStreamWaitEvent(st, lane->join, 0) != hipSuccess) return LCQ_ELAUNCH;

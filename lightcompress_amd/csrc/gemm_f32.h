@@ -243,8 +243,8 @@ __device__ __forceinline__ void gemm_tile(const float* A, int lda, const float* 
 // partial products of weight >= 2^-16:  lo*hi + hi*lo + mid*mid + mid*hi + hi*mid + hi*hi.  The dropped terms
 // (mid*lo, lo*mid, lo*lo) are below 2^-24 of the product - the rounding of an fp32 multiply - so the result is as
 // accurate as the fp32 pipe's, at 16 / 6 times its rate (v_mfma_f32_32x32x16_bf16 against v_mfma_f32_32x32x2f32).
-// Used for the launches that fill the chip (more than one 128x128 tile per CU) and are not deep enough, or too small, for the
-// fp16 pairs of gemm_h2.h; small launches stay on the fp32 pipe.
+// Used for the launches that fill the chip (more than one 128x128 tile per CU); the deep ones of two rounds and more have their
+// operands split ahead (gemm_s3p.h); small launches stay on the fp32 pipe.
 // LDS: per operand three planes of [128 rows][32 k] bf16 (64-byte rows, 16-byte chunks XOR-swizzled by the row) or, for B given as [k][n], of [32 k][128 n] (row pitch 320 B) read through the transposing
 // ds_read_b64_tr_b16 (a 16-lane group addresses 4 k-rows x 16 columns and receives 4 k-values of one column each).
 typedef __attribute__((ext_vector_type(8))) __bf16 s3_bf16x8;

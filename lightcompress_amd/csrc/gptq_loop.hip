@@ -38,7 +38,7 @@
 #include <type_traits>
 
 #include "gemm_f32.h"
-#include "gemm_h2.h"
+#include "gemm_s3p.h"
 #include "lcq_internal.h"
 
 namespace {
@@ -410,27 +410,26 @@ int lcq_gptq_trailing(float* W, const float* Err, int64_t ldErr, const float* U,
   return LCQ_OK;
 }
 
-// The fp16 products (gemm_h2.h) where the launch has 96 of their 256 x 256 tiles (4096 x 1024 x 1024, 64 tiles: 81 against
-// 72 us; 6144 x 1024, 96 tiles: 76 against 85; 28672 x 3072: 539 against 1015).
+// The operands split once (gemm_s3p.h) where that pays; the same bits either way.
 int64_t lcq_gptq_trailing_workspace_bytes(int64_t R, int64_t K, int64_t k1, int64_t k2, int64_t j1, int64_t j2) {
-  if (R <= 0 || R > 0x7fffffff || K <= 0 || K > (1 << 20) || k1 < 0 || k2 <= k1 || k2 > j1 || j2 > K || j2 <= j1) return 0;
-  if (!g_gemm_split.load(std::memory_order_relaxed) || !h2_depth(k2 - k1) || h2_tiles(R, j2 - j1) < 96) return 0;
-  return h2_bytes(R, k2 - k1) + h2_bytes(j2 - j1, k2 - k1);
+  if (R <= 0 || R > (1 << 24) || K <= 0 || K > (1 << 20) || k1 < 0 || k2 <= k1 || k2 > j1 || j2 > K || j2 <= j1) return 0;
+  if (!g_gemm_split.load(std::memory_order_relaxed) || !s3p_depth(k2 - k1) || !s3p_pays(R, j2 - j1, s3p_tiles(R, j2 - j1))) return 0;
+  return s3p_bytes(R, k2 - k1) + s3p_bytes(j2 - j1, k2 - k1);
 }
 
 int lcq_gptq_trailing_deep(float* W, const float* Err, int64_t ldErr, const float* U, int64_t R, int64_t K, int64_t k1, int64_t k2,
                            int64_t j1, int64_t j2, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = lcq_gptq_trailing_workspace_bytes(R, K, k1, k2, j1, j2);
-  if (need == 0 || !W || !Err || !U || ldErr < k2 - k1 || !h2_operand(Err, ldErr, k2 - k1))
+  if (need == 0 || !W || !Err || !U || ldErr < k2 - k1 || !s3p_operand(Err, ldErr, k2 - k1))
     return lcq_gptq_trailing(W, Err, ldErr, U, R, K, k1, k2, j1, j2, stream);
   if (!workspace || workspace_bytes < need) return LCQ_EWORKSPACE;
   if (((uintptr_t)workspace % 16) != 0) return LCQ_EALIGN;
   const int Kc = (int)(k2 - k1), N = (int)(j2 - j1);
   hipStream_t st = (hipStream_t)stream;
-  const H2Operand a(workspace, R, Kc), b((char*)workspace + h2_bytes(R, Kc), N, Kc);
-  h2_pack<false>(Err, ldErr, (int)R, Kc, a, st);
-  h2_pack<true>(U + k1 * K + j1, K, N, Kc, b, st);
-  h2_multiply<false>(a, 0, b, 0, W + j1, (int)K, (int)R, N, Kc, st);
+  const S3POperand a(workspace, R), b((char*)workspace + s3p_bytes(R, Kc), N);
+  s3p_pack<false>(Err, ldErr, (int)R, Kc, a, st);
+  s3p_pack<true>(U + k1 * K + j1, K, N, Kc, b, st);
+  s3p_multiply<false>(a, b, W + j1, (int)K, (int)R, N, Kc, st);
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }
