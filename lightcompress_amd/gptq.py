@@ -40,8 +40,8 @@ Differences a caller can observe
     instead of errors to later columns; the same results up to fp32 rounding (closer to fp64 than the reference's
     cholesky / cholesky_inverse / cholesky chain).  process_hessian_and_weights called on its own returns the
     reference's U;
-  * ``special.hessian_defer`` add_batch calls (default 'auto': as many as make 8192 tokens for K <= 1024, 65536 for K <= 4096, 32768 above) are
-    copied to a staging buffer, in the order the matrix pipe reads them (lcq_hessian_pack), and folded into one launch, so ``layers_cache[name]['H']`` lags behind ``nsamples`` until
+  * ``special.hessian_defer`` add_batch calls (default 'auto': 16 for K <= 4096, 8 for K <= 8192, else 4) are copied to a staging
+    buffer, in the order the matrix pipe reads them (lcq_hessian_pack), and folded into one launch, so ``layers_cache[name]['H']`` lags behind ``nsamples`` until
     ``hessian(name)``, ``hessian_sorting`` or ``process_hessian_and_weights`` settles it
     (``hessian_defer: 1`` updates H on every call);
   * ``special.hessian_slices`` (default 'auto': 8 up to K = 512, else 1): with a number above 1 every launch cuts its tokens into that many
@@ -407,7 +407,7 @@ class GPTQ:
             if stage is None:
                 # packed where one accumulator takes it all; the launches with token shares read the tokens as they come
                 packed = cache['stage_packed'] = cache.get('H_shares') is None
-                defer = self.hessian_fold(K, tokens)
+                defer = self.hessian_fold(K)
                 rows, cols = (-(-defer * tokens // 32) * 32, -(-K // 256) * 256) if packed else (defer * tokens, K)
                 stage = torch.empty((rows, cols), dtype=sdtype, device=inp.device)
                 cache['stage'] = stage
@@ -462,17 +462,13 @@ class GPTQ:
             x = inp.reshape((-1, K)).contiguous()
         return x if x.data_ptr() % 16 == 0 else x.clone()
 
-    def hessian_fold(self, K, tokens=2048):
-        """add_batch calls of `tokens` tokens folded into one Hessian launch for a Linear with K input features.  'auto': what
-        makes 65536 tokens for K <= 4096 and 32768 above (half a GB of staged tokens at K = 4096, one at K = 14336), 128 calls
-        at most (so that a few short ones do not ask for such a buffer).  A launch reads and writes H and fills and drains the
-        chip once, whatever its tokens: 861 us for 65536 tokens at K = 4096 against 2 x 462, 5.01 ms for 32768 at K = 14336
-        against 4 x 1.32.  Up to K = 1024 a launch is short (25 us for 8192 tokens, and 10 for its fold) and runs while the host
-        stages the next calls, so it is issued early: 8192 tokens, but 16 calls at least, for a call leaves the GPU idle for some
-        3 us while it is issued (16 calls of 2000 tokens, four launches: 770 us for the Linear, one: 692)."""
+    def hessian_fold(self, K):
+        """add_batch calls folded into one Hessian launch for a Linear with K input features.  'auto': 16 calls up to K = 4096, 8
+        up to K = 8192, 4 above, whatever their size: every Linear that is calibrated at a time has a buffer of its own, and the
+        many small ones of a layer of experts see calls of a few hundred tokens (16 calls of 2048 tokens are 268 MB at K = 4096,
+        4 are 235 MB at K = 14336)."""
         if self.hessian_defer == 'auto':
-            window, least = (8192, 16) if K <= 1024 else (65536 if K <= 4096 else 32768, 2)
-            return min(max(window // max(tokens, 1), least), 128)
+            return 16 if K <= 4096 else (8 if K <= 8192 else 4)
         return self.hessian_defer
 
     def hessian_shares(self, K):

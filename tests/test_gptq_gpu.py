@@ -304,6 +304,21 @@ def test_hessian_deferred_launches(dev, defer):
     assert float((H.double() - ref).abs().max() / ref.abs().max()) < 1e-5
 
 
+@pytest.mark.parametrize('K,calls', [(1024, 16), (2048, 16), (4096, 16), (4104, 8), (7168, 8), (8200, 4), (14336, 4)])
+@pytest.mark.parametrize('tokens', [200, 2048])
+def test_staging_buffers_hold_a_number_of_calls(dev, K, calls, tokens):
+    """Every Linear that is calibrated has a staging buffer of its own, and a layer of experts has hundreds: the buffer is for a
+    number of calls whatever their size (whole slabs of 32 tokens, K up to a multiple of 256), and it grows when the calls do."""
+    gp = make_gptq()
+    layer = Layer(torch.zeros(8, K, device=dev))
+    gp.subset_init({'layers': {'l': layer}})
+    cache = gp.layers_cache['l']
+    for n in (tokens // 50, tokens):
+        gp.add_batch(layer, 'l', torch.ones(1, n, K, dtype=torch.bfloat16, device=dev), None)
+        rows = -(-calls * n // 32) * 32
+        assert cache['stage'].shape == (rows, -(-K // 256) * 256)
+
+
 def _chain_inputs(K, seed, dead=()):
     H = G.hessian_closed_form(calib_batches(4, max(64, K // 4), K, seed=seed)).float()
     for j in dead:
@@ -1321,9 +1336,9 @@ def test_indefinite_hessian_raises_unless_the_check_is_off(dev):
 
 @pytest.mark.parametrize('K', [768, 1536, 2304, 3072, 5120, 6144])
 def test_hessian_auto_settings_between_the_tuned_widths(dev, K):
-    """`hessian_defer: auto` / `hessian_slices: auto` are tables tuned at a handful of widths; whatever they pick at
-    the widths in between (folds of 16 / 8 calls, 1 - 8 token shares, with or without the split last round), add_batch
-    over a number of calls that leaves a partly filled staging buffer ends at the closed form."""
+    """Whatever `hessian_defer: auto` picks (16 calls up to K = 4096, 8 up to 8192, 4 above) and however the launch is cut (tiles
+    in pieces, whole rounds, both, several launches), add_batch over a number of calls that fills the staging buffer at least
+    once and leaves it partly filled ends at the closed form."""
     T, nb = 96, 21
     gp = make_gptq()
     layer = Layer(torch.zeros(8, K, device=dev))
