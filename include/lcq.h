@@ -266,8 +266,8 @@ int lcq_hessian_accum_balanced(float* H, int64_t K, const void* XA, const void* 
  * lcq_hessian_compare_packed sets *flag = 1 if the tokens differ from positions at .. at + T (never clears it).
  * lcq_hessian_accum_packed: H <- alpha*H + beta * XA^T XB over positions 0 .. T (T <= 2^26), as lcq_hessian_accum_ab; the
  *   positions up to the end of the last slab must hold zeros (as lcq_hessian_pack leaves them).  dtype LCQ_BF16 | LCQ_F16;
- *   workspace of lcq_hessian_packed_workspace_bytes(K, T) (0: none), everything 16-byte aligned.  Reproducible: runs of slabs
- *   of one tile are summed in a fixed order. */
+ *   workspace of lcq_hessian_packed_workspace_bytes(K, T) (0: none), everything 16-byte aligned.  Reproducible: a tile's tokens are
+ *   summed in runs of at most 16384, and the runs in a fixed order. */
 int64_t lcq_hessian_packed_bytes(int64_t K, int64_t T);
 int lcq_hessian_pack(const void* x, int dtype, int64_t T, int64_t K, int64_t ldx, int64_t at, void* packed, void* packed_lo,
                      void* stream);

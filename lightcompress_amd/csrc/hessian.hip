@@ -373,9 +373,9 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(float* __restrict__ H, i
 //  * four LDS stages of 32 tokens, one barrier per slab: at the middle of a slab every wave holds the rest of it in
 //    registers, so its stage is free for the slab four ahead.
 // The chip clocks down under this load (random tokens 1.7 GHz, zeros run 1.3 times as fast), which is what bounds it.
-// Measured (us, without the copy): K = 14336, 32768 tokens 5919 -> 5010 (1.37 PFLOP/s of the tiles computed),
-// K = 4096, 65536 tokens 1064 -> 861, K = 8192, 32768 tokens 2026 -> 1622, K = 2048, 65536 tokens 305 -> 245; against
-// hessian_kernel with the token shares or split rounds it had for the same work.
+// Measured (us, without the copy): K = 14336, 8192 tokens 1448 -> 1293 (1.33 PFLOP/s of the tiles computed; 1.25 on another box),
+// K = 4096, 32768 tokens 525 -> 477, K = 8192, 16384 tokens 996 -> 901, K = 7168, 16384 tokens 743 -> 660, K = 2048, 32768 tokens
+// 143 -> 136; against hessian_kernel with the token shares or split rounds it had for the same work.
 typedef const __attribute__((address_space(3))) char* lds_ptr;
 typedef const __attribute__((address_space(3))) s16x8* lds_frag;
 constexpr int PT = 256;                             // tile of H
@@ -383,16 +383,19 @@ constexpr int P_STAGES = 4, P_HALF = BT * PT * 2, P_STAGE = 2 * P_HALF;
 
 // Which part of which tile a workgroup computes.  Tiles [0, full) fill whole rounds of the chip's CUs, one workgroup each.
 // The rest would leave CUs idle for the time of a tile and is cut along the tokens: m[0] tiles into c[0] pieces each, the
-// m[1] tiles behind them into c[1] pieces (packed_plan).  Piece 0 of a tile updates H; the others leave beta * (their X^T X) in
-// scratch tiles, which packed_fold_kernel adds to H in order.  All tiles of a level are cut at the same tokens and the
+// m[1] tiles behind them into c[1] pieces (packed_plan).  A tile of one piece updates H; the pieces of a cut one leave their
+// X^T X in scratch tiles, and packed_fold_kernel adds their sum to H: an element of H is rounded once per launch however many
+// pieces there are (each added to H by itself: an error of 2.3e-7 at K = 1024, 262144 tokens, with 25 pieces).  All tiles of a
+// level are cut at the same tokens and the
 // workgroups of an XCD take the same piece of neighbouring tiles, so they read the same slabs of X at the same time (cut
 // into runs that wander over tile boundaries the launch fetches X from beyond L2: 700 against 462 us for K = 4096, T = 32768).
 struct PackedPlan {
   int full, slabs;
   int m[2], c[2];
-  float* scratch;                                   // sum of m (c - 1) tiles of PT x PT floats
+  float* scratch;                                   // m c tiles of PT x PT floats for every level with c > 1
 };
 __host__ __device__ __forceinline__ int level_blocks(const PackedPlan& p, int l) { return (p.m[l] * p.c[l] + 7) / 8 * 8; }
+__host__ __device__ __forceinline__ int64_t level_scratch(const PackedPlan& p, int l) { return p.c[l] > 1 ? (int64_t)p.m[l] * p.c[l] : 0; }
 
 template <bool IS_BF16, bool EDGE>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -425,7 +428,7 @@ void hessian_packed_kernel(float* __restrict__ H, int K, const uint16_t* __restr
       v = plan.full + (l ? plan.m[0] : 0) + t;
       s0 = (int)((int64_t)piece * n / c);
       s1 = (int)((int64_t)(piece + 1) * n / c);
-      if (piece > 0) scratch = (l ? (int64_t)plan.m[0] * (plan.c[0] - 1) : 0) + (int64_t)t * (c - 1) + piece - 1;
+      if (c > 1) scratch = (l ? level_scratch(plan, 0) : 0) + (int64_t)t * c + piece;
     }
   }
   int ti, tj;
@@ -506,6 +509,7 @@ void hessian_packed_kernel(float* __restrict__ H, int K, const uint16_t* __restr
   // accumulator register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
   const bool to_scratch = scratch >= 0;
   const bool rmw = !to_scratch && alpha != 0.0f;
+  const float scale = to_scratch ? 1.0f : beta;
   const int row = wr * 128 + 4 * (lane >> 5), col = wc * 128 + (lane & 31);
   char* out = (char*)(to_scratch ? plan.scratch + scratch * (PT * PT) : H + (int64_t)(ti * PT) * K + tj * PT);
   uint32_t pitch = 4 * (to_scratch ? PT : K);     // bytes
@@ -528,33 +532,38 @@ void hessian_packed_kernel(float* __restrict__ H, int K, const uint16_t* __restr
     for (int j = 0; j < 4; ++j)
       #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float w = beta * acc[i][j][r];
-        if (rmw) w = alpha * old[j][r] + w;
+        float w = acc[i][j][r] * scale;
+        if (rmw) w = __builtin_fmaf(alpha, old[j][r], w);
         if (inside(i, j, r)) *(float*)(out + cell(i, j, r)) = w;
       }
   }
 }
 
-// H tile <- ((H tile + piece 1) + piece 2) + ... for the tiles that were cut: grid (tiles, 16), 16 rows per workgroup.
-__global__ __launch_bounds__(256) void packed_fold_kernel(float* __restrict__ H, int K, int nt, PackedPlan plan) {
+// H tile <- alpha * (H tile) + beta * ((piece 0 + piece 1) + ...) for the tiles that were cut: grid (tiles, 16), 16 rows per
+// workgroup.
+__global__ __launch_bounds__(256) void packed_fold_kernel(float* __restrict__ H, int K, int nt, float alpha, float beta, PackedPlan plan) {
   int ti, tj;
   decode_tile<1>(plan.full + blockIdx.x, nt, nt, ti, tj);
-  const int l = (int)blockIdx.x >= plan.m[0], t = blockIdx.x - (l ? plan.m[0] : 0), pieces = plan.c[l] - 1;
-  const float* const sc = plan.scratch + ((l ? (int64_t)plan.m[0] * (plan.c[0] - 1) : 0) + (int64_t)t * pieces) * (PT * PT);
+  const int l = (int)blockIdx.x >= plan.m[0], t = blockIdx.x - (l ? plan.m[0] : 0), pieces = plan.c[l];
+  const float* const sc = plan.scratch + ((l ? level_scratch(plan, 0) : 0) + (int64_t)t * pieces) * (PT * PT);
   const int c = (threadIdx.x & 63) * 4;
-  if (pieces <= 0 || tj * PT + c >= K) return;
+  if (pieces <= 1 || tj * PT + c >= K) return;
   #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int row = blockIdx.y * 16 + (threadIdx.x >> 6) * 4 + k;
     if (ti * PT + row >= K) return;
     float* const hp = H + (int64_t)(ti * PT + row) * K + tj * PT + c;     // K % 8 == 0: four columns or none
-    f32x4 h = *(const f32x4*)hp;
+    f32x4 h = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (alpha != 0.0f) h = *(const f32x4*)hp;
+    f32x4 sum = *(const f32x4*)(sc + row * PT + c);
     #pragma unroll 4
-    for (int i = 0; i < pieces; ++i) {
+    for (int i = 1; i < pieces; ++i) {
       const f32x4 w = *(const f32x4*)(sc + (int64_t)i * (PT * PT) + row * PT + c);
-      h[0] += w[0]; h[1] += w[1]; h[2] += w[2]; h[3] += w[3];
+      sum[0] += w[0]; sum[1] += w[1]; sum[2] += w[2]; sum[3] += w[3];
     }
-    *(f32x4*)hp = h;
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) sum[e] = __builtin_fmaf(alpha, h[e], beta * sum[e]);
+    *(f32x4*)hp = sum;
   }
 }
 
@@ -886,39 +895,78 @@ int lcq_hessian_compare_packed(const void* x, int dtype, int64_t T, int64_t K, i
   return pack_tokens(true, x, dtype, T, K, ldx, at, packed, packed_lo, flag, stream);
 }
 
-// How a launch over T staged tokens is cut (see PackedPlan): of all pairs of levels the one with the shortest estimate, in
-// slabs' time.  A level runs its pieces side by side, n / c slabs; a round of workgroups costs START slabs for its first
-// loads and its epilogue; a scratch tile, written and read once by a chip that does nothing else, a twelfth of a slab.
-static PackedPlan packed_plan(int64_t K, int64_t T) {
+// Tokens are added up in runs, one accumulator each, whose rounding error grows faster than their length.  A run is at most 16384
+// tokens, and a launch has at least three runs up to K = 4352, two where the tiles are one or two whole rounds and little more (a
+// second launch then costs its start and not much else): the widths at which hessian_kernel has token shares for the same work.
+// On the diagonal H was 4.8e-7 from fp64 with runs of 32768 tokens at K = 8192 (131072 in all) and is 1.4e-7; 3.6e-7 and 1.2e-7 at
+// K = 4096 (262144 in all).
+constexpr int PACKED_RUN = 512;                     // slabs
+static int packed_cus() {
+  const int cus = hessian_slots() / 2 / 8 * 8;
+  return cus < 8 ? 8 : cus;
+}
+static int packed_runs(int64_t K, int n) {
+  const int64_t nt = packed_width(K) / PT, tiles = nt * (nt + 1) / 2, cus = packed_cus();
+  const int by_length = (n + PACKED_RUN - 1) / PACKED_RUN;
+  const int by_width = K <= 4352 ? 3 : tiles >= cus && tiles < 3 * cus && tiles % cus < cus / 4 ? 2 : 1;
+  return by_length > by_width ? by_length : by_width < n ? by_width : n;
+}
+
+// How a launch over n slabs is cut (see PackedPlan): of all pairs of levels with at least `least` pieces the one with the
+// shortest estimate, in slabs' time; slabs = 0 if there is none.  A level runs its pieces side by side, n / c slabs; a round of
+// workgroups costs START slabs for its first loads and its epilogue; a scratch tile, written and read once by a chip that does
+// nothing else, a twelfth of a slab.
+static PackedPlan packed_plan(int64_t K, int n, int least) {
   constexpr double START = 16.0, TILE = 1.0 / 12;
   const int64_t nt = packed_width(K) / PT, tiles = nt * (nt + 1) / 2;
-  int cus = hessian_slots() / 2 / 8 * 8;
-  if (cus < 8) cus = 8;
+  const int cus = packed_cus();
   PackedPlan p{};
-  p.slabs = (int)((T + BT - 1) / BT);
   p.full = (int)(tiles / cus * cus);
-  const int rest = (int)(tiles - p.full), n = p.slabs;
+  const int rest = (int)(tiles - p.full);
   p.c[0] = p.c[1] = 1;
-  if (rest == 0) return p;
-  const auto level = [&](int m, int c) { return (double)((n + c - 1) / c) + START + TILE * m * (c - 1); };
+  if (p.full > 0 && least > 1) return p;
+  if (rest == 0) { p.slabs = n; return p; }
+  const auto level = [&](int m, int c) { return (double)((n + c - 1) / c) + START + (c > 1 ? TILE * m * c : 0.0); };
   double best = 1e30;
-  for (int c0 = 1; c0 <= cus && c0 <= n; ++c0) {
+  for (int c0 = least; c0 <= cus && c0 <= n; ++c0) {
     const int m0 = rest < cus / c0 ? rest : cus / c0, m1 = rest - m0;
-    const int most = m1 ? cus / m1 : 1;             // (m1 < cus)
-    for (int c1 = 1; c1 <= most && c1 <= n; ++c1) {
+    const int most = m1 ? cus / m1 : least;         // (m1 < cus)
+    for (int c1 = least; c1 <= most && c1 <= n; ++c1) {
       const double t = level(m0, c0) + (m1 ? level(m1, c1) : 0.0);
-      if (t < best) { best = t; p.m[0] = m0; p.c[0] = c0; p.m[1] = m1; p.c[1] = c1; }
+      if (t < best) { best = t; p.slabs = n; p.m[0] = m0; p.c[0] = c0; p.m[1] = m1; p.c[1] = c1; }
     }
   }
   return p;
 }
-static int64_t packed_scratch_tiles(const PackedPlan& p) {
-  return (int64_t)p.m[0] * (p.c[0] - 1) + (int64_t)p.m[1] * (p.c[1] - 1);
+static int64_t packed_scratch_tiles(const PackedPlan& p) { return level_scratch(p, 0) + level_scratch(p, 1); }
+
+// T tokens as `count` launches of first.slabs slabs each, the last of last.slabs: as few as have a plan.
+struct PackedSpans {
+  int count;
+  PackedPlan first, last;
+};
+static PackedSpans packed_spans(int64_t K, int64_t T) {
+  const int n = (int)((T + BT - 1) / BT), runs = packed_runs(K, n);
+  PackedSpans s{};
+  for (int want = 1; ; ++want) {                    // (a launch of one run always has a plan)
+    const int each = (n + want - 1) / want, count = (n + each - 1) / each, least = (runs + count - 1) / count;
+    s.first = packed_plan(K, each, least);
+    if (s.first.slabs == 0) continue;
+    const int rest = n - (count - 1) * each;
+    s.last = rest == each ? s.first : packed_plan(K, rest, least < rest ? least : rest);
+    if (s.last.slabs == 0) continue;
+    s.count = count;
+    return s;
+  }
+}
+static int64_t packed_scratch_bytes(const PackedSpans& s) {
+  const int64_t a = packed_scratch_tiles(s.first), b = packed_scratch_tiles(s.last);
+  return (a > b ? a : b) * PT * PT * 4;
 }
 
 int64_t lcq_hessian_packed_workspace_bytes(int64_t K, int64_t T) {
   if (K <= 0 || K > (1 << 20) || T <= 0 || T > (1 << 26)) return 0;
-  return packed_scratch_tiles(packed_plan(K, T)) * PT * PT * 4;
+  return packed_scratch_bytes(packed_spans(K, T));
 }
 
 int lcq_hessian_accum_packed(float* H, int64_t K, const void* XA, const void* XB, int dtype, int64_t T, float alpha, float beta,
@@ -927,21 +975,27 @@ int lcq_hessian_accum_packed(float* H, int64_t K, const void* XA, const void* XB
   if (T > (1 << 26)) return LCQ_ESIZE;
   if (dtype != LCQ_BF16 && dtype != LCQ_F16) return LCQ_EDTYPE;
   if ((((uintptr_t)XA | (uintptr_t)XB | (uintptr_t)H | (uintptr_t)workspace) % 16) != 0) return LCQ_EALIGN;
-  PackedPlan p = packed_plan(K, T);
-  const int64_t need = packed_scratch_tiles(p) * PT * PT * 4;
+  const PackedSpans spans = packed_spans(K, T);
+  const int64_t need = packed_scratch_bytes(spans);
   if (need > 0 && (!workspace || workspace_bytes < need)) return LCQ_EWORKSPACE;
-  p.scratch = (float*)workspace;
   const int nt = (int)(packed_width(K) / PT);
-  const int64_t grid = (int64_t)p.full + level_blocks(p, 0) + level_blocks(p, 1);
-  hipStream_t st = (hipStream_t)stream;
-  #define LCQ_HESSP(BF, E) hessian_packed_kernel<BF, E><<<dim3((unsigned)grid), dim3(256), 0, st>>>( \
-      H, (int)K, (const uint16_t*)XA, (const uint16_t*)XB, alpha, beta, nt, p)
   const bool edge = K % PT != 0;
-  if (dtype == LCQ_BF16) { if (edge) LCQ_HESSP(true, true); else LCQ_HESSP(true, false); }
-  else { if (edge) LCQ_HESSP(false, true); else LCQ_HESSP(false, false); }
-  #undef LCQ_HESSP
-  if (need > 0)
-    packed_fold_kernel<<<dim3((unsigned)(p.m[0] + p.m[1]), PT / 16), dim3(256), 0, st>>>(H, (int)K, nt, p);
+  hipStream_t st = (hipStream_t)stream;
+  for (int i = 0; i < spans.count; ++i) {
+    PackedPlan p = i + 1 < spans.count ? spans.first : spans.last;
+    p.scratch = (float*)workspace;
+    const int64_t at = (int64_t)i * spans.first.slabs * nt * PT * BT;   // elements of the slabs before
+    const uint16_t* const xa = (const uint16_t*)XA + at;
+    const uint16_t* const xb = (const uint16_t*)XB + at;
+    const float al = i == 0 ? alpha : 1.0f;
+    const int64_t grid = (int64_t)p.full + level_blocks(p, 0) + level_blocks(p, 1);
+    #define LCQ_HESSP(BF, E) hessian_packed_kernel<BF, E><<<dim3((unsigned)grid), dim3(256), 0, st>>>(H, (int)K, xa, xb, al, beta, nt, p)
+    if (dtype == LCQ_BF16) { if (edge) LCQ_HESSP(true, true); else LCQ_HESSP(true, false); }
+    else { if (edge) LCQ_HESSP(false, true); else LCQ_HESSP(false, false); }
+    #undef LCQ_HESSP
+    if (packed_scratch_tiles(p) > 0)
+      packed_fold_kernel<<<dim3((unsigned)(p.m[0] + p.m[1]), PT / 16), dim3(256), 0, st>>>(H, (int)K, nt, al, beta, p);
+  }
   LCQ_CHECK_LAUNCH();
   return LCQ_OK;
 }

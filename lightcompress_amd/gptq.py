@@ -466,7 +466,8 @@ class GPTQ:
         """add_batch calls folded into one Hessian launch for a Linear with K input features.  'auto': 16 calls up to K = 4096, 8
         up to K = 8192, 4 above, whatever their size: every Linear that is calibrated at a time has a buffer of its own, and the
         many small ones of a layer of experts see calls of a few hundred tokens (16 calls of 2048 tokens are 268 MB at K = 4096,
-        4 are 235 MB at K = 14336)."""
+        4 are 235 MB at K = 14336).  More calls would save little: a sum runs over at most 16384 tokens before it is added to H
+        (lcq_hessian_accum_packed), so a longer buffer is cut into as many launches."""
         if self.hessian_defer == 'auto':
             return 16 if K <= 4096 else (8 if K <= 8192 else 4)
         return self.hessian_defer

@@ -319,6 +319,31 @@ def test_staging_buffers_hold_a_number_of_calls(dev, K, calls, tokens):
         assert cache['stage'].shape == (rows, -(-K // 256) * 256)
 
 
+@pytest.mark.parametrize('K,nb,T,launches,runs', [(640, 100, 1000, 7, 32), (1024, 128, 2048, 8, 16), (3584, 64, 2048, 4, 3),
+                                                  (4096, 64, 512, 4, 3), (4352, 40, 512, 5, 3), (5888, 32, 256, 4, 2),
+                                                  (8192, 24, 256, 3, 2), (8448, 64, 512, 16, 2)])
+def test_hessian_sums_are_as_short_as_the_launches(dev, K, nb, T, launches, runs):
+    """The rounding error of H on the diagonal, where nothing cancels.  A run of r matrix instructions (16 tokens each) adds up
+    to r in r roundings of what is there, an rms error of sqrt(r / 3) roundings; `launches` x `runs` of them average out to
+    sqrt(r / (3 launches runs)).  H itself is rounded once per launch, at i / launches of its size: sqrt(launches / 3).  Scaling
+    and the sum of the runs: three roundings at most.  A rounding is 2^-24 at most, its rms less than that."""
+    gp = make_gptq()
+    layer = Layer(torch.zeros(8, K, device=dev))
+    gp.subset_init({'layers': {'l': layer}})
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randn(nb, T, K, device=dev, dtype=torch.bfloat16, generator=g)
+    for b in range(nb):
+        gp.add_batch(layer, 'l', x[b:b + 1], None)
+    H = gp.hessian('l')
+    ref = torch.zeros(K, dtype=torch.float64, device=dev)
+    for b in range(nb):
+        ref += x[b].double().square().sum(0)
+    ref *= 2.0 / nb
+    err = float(((torch.diag(H).double() - ref) / ref).square().mean().sqrt())
+    r = nb * T / 16 / (launches * runs)
+    assert err <= 2.0 ** -24 * (r / (3 * launches * runs) + launches / 3 + 3) ** 0.5, err * 2 ** 24
+
+
 def _chain_inputs(K, seed, dead=()):
     H = G.hessian_closed_form(calib_batches(4, max(64, K // 4), K, seed=seed)).float()
     for j in dead:
