@@ -186,6 +186,7 @@ class GPTQ:
             self.layers_cache[n]['H_shares'] = None
             self.layers_cache[n]['leader'] = leader
             self.layers_cache[n]['manual_share'] = True
+            self.layers_cache[n].pop('again', None)
         self.layers_cache[leader]['leader'] = leader
         self.layers_cache[leader]['manual_share'] = True
 
@@ -332,17 +333,21 @@ class GPTQ:
     def add_batch(self, layer, name, inp, out=None):
         # Called once per Linear per calibration batch (896 times for one decoder layer), and where the batches are small the
         # host's time per call is what staging takes.  A call like the one before it (shape, type, room in the same buffer; no
-        # Linear follows this one) goes straight to the launch: 9.5 -> 7.6 us.
+        # Linear follows this one) goes straight to the launch: 9.5 -> 7.6 us.  ('again' describes that call and holds neither
+        # tensor nor address; it goes when the buffer goes.)
         cache = self.layers_cache[name]
         again = cache.get('again')
-        if again is not None:
-            shape, dtype, code, tokens, tmp, stage, lo = again
-            fill = cache.get('stage_fill', 0)
+        stage = cache.get('stage')
+        if again is not None and stage is not None:
+            shape, dtype, code, tokens, tmp = again
+            fill = cache['stage_fill']
             at = inp.data_ptr()
-            if cache.get('stage') is stage and inp.shape == shape and inp.dtype == dtype and fill + tokens <= stage.shape[0] \
+            if inp.shape == shape and inp.dtype == dtype and fill + tokens <= stage.shape[0] \
                     and at % 16 == 0 and inp.is_contiguous() and inp.is_cuda and not cache.get('followers'):
+                lo = cache['stage_lo']
                 K = shape[-1]
-                rc = L.lib().lcq_hessian_pack(at, code, tokens, K, K, fill, stage.data_ptr(), lo, L.stream())
+                rc = L.lib().lcq_hessian_pack(at, code, tokens, K, K, fill, stage.data_ptr(),
+                                              None if lo is None else lo.data_ptr(), L.stream())
                 if rc != 0:
                     L.check(rc, 'lcq_hessian_pack')
                 cache['last_key'] = (at, shape, inp.stride(), dtype)
@@ -428,7 +433,7 @@ class GPTQ:
                 cache['calls'] += 1
                 cache['nsamples'] += tmp
                 if kind == 'linear' and cache.get('leader', name) == name and tokens > 0:
-                    cache['again'] = (shape, inp.dtype, L.dtype_code(inp.dtype), tokens, tmp, stage, None if lo is None else lo.data_ptr())
+                    cache['again'] = (shape, inp.dtype, L.dtype_code(inp.dtype), tokens, tmp)
                 return
             nbytes = tokens * K * stage.element_size()
             dst = stage.data_ptr() + f * K * stage.element_size()
@@ -570,10 +575,8 @@ class GPTQ:
             if cache.get('leader', name) != lead_name:   # `name` itself was a call behind: it owns its Hessian now
                 lead = cache
         self._flush(lead)
-        lead.pop('stage', None)
-        lead.pop('stage_lo', None)
-        lead.pop('hws', None)
-        lead.pop('hws_key', None)
+        for k in ('stage', 'stage_lo', 'again', 'hws', 'hws_key'):
+            lead.pop(k, None)
         if lead.get('shares_apart'):                      # the token shares of the launches back into the one H
             sh = lead['H_shares']
             L.check(L.lib().lcq_hessian_gather_slices(L.ptr(sh), L.i64(sh.shape[1]), L.i32(sh.shape[0]), L.i64(sh.stride(0)),

@@ -344,6 +344,52 @@ def test_hessian_sums_are_as_short_as_the_launches(dev, K, nb, T, launches, runs
     assert err <= 2.0 ** -24 * (r / (3 * launches * runs) + launches / 3 + 3) ** 0.5, err * 2 ** 24
 
 
+@pytest.mark.parametrize('K', [320, 1024])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_staging_buffers_go_when_the_hessian_is_settled(dev, K, dtype):
+    """The tokens are staged until H is read; the chain and the column loop behind that are the memory peak, so the buffers of
+    every Linear are given back before (nothing else holds them), and calibration may go on afterwards."""
+    import weakref
+    gp = make_gptq()
+    layer = Layer(torch.zeros(8, K, device=dev))
+    gp.subset_init({'layers': {'l': layer}})
+    cache = gp.layers_cache['l']
+    xs = [torch.randn(1, 64, K, device=dev, dtype=dtype) for _ in range(6)]
+    for x in xs[:3]:
+        gp.add_batch(layer, 'l', x, None)
+    held = [weakref.ref(cache[k]) for k in ('stage', 'stage_lo') if cache.get(k) is not None]
+    assert len(held) == (2 if dtype == torch.float32 else 1) and all(h() is not None for h in held)
+    gp.hessian('l')
+    assert all(h() is None for h in held)
+    for x in xs[3:]:
+        gp.add_batch(layer, 'l', x, None)
+    H = gp.hessian('l')
+    ref = 2.0 / len(xs) * sum(x[0].double().t() @ x[0].double() for x in xs)
+    assert float((H.double() - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_a_copy_made_between_two_calls_stages_its_own_tokens(dev, dtype):
+    """copy.deepcopy of a GPTQ object in the middle of a calibration: what either of them is fed afterwards stays its own (no
+    address of the other's buffers is kept)."""
+    import copy
+    K = 1024
+    gp = make_gptq()
+    layer = Layer(torch.zeros(8, K, device=dev))
+    gp.subset_init({'layers': {'l': layer}})
+    xs = [torch.randn(1, 48, K, device=dev, dtype=dtype) for _ in range(6)]
+    for x in xs[:2]:
+        gp.add_batch(layer, 'l', x, None)
+    twin = copy.deepcopy(gp)
+    for x in xs[2:4]:
+        gp.add_batch(layer, 'l', x, None)
+    for x in xs[4:]:
+        twin.add_batch(layer, 'l', x, None)
+    for g, mine in ((gp, xs[:4]), (twin, xs[:2] + xs[4:])):
+        ref = 2.0 / 4 * sum(x[0].double().t() @ x[0].double() for x in mine)
+        assert float((g.hessian('l').double() - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
 def _chain_inputs(K, seed, dead=()):
     H = G.hessian_closed_form(calib_batches(4, max(64, K // 4), K, seed=seed)).float()
     for j in dead:
