@@ -21,6 +21,11 @@ from .quant import IntegerQuantizer, weight_cast_to_bf16
 from .rtn import RTN
 
 _CODE = {torch.int32: L.CODE_I32, torch.int8: L.CODE_I8, torch.uint8: L.CODE_U8}
+# torch's register_buffer itself (None where it was already replaced by another when this module was imported)
+_REGISTER = torch.nn.Module.register_buffer
+if getattr(_REGISTER, '__globals__', None) is not vars(_module):
+    _REGISTER = None
+_NAMES = frozenset(('weight', 'weight_packed', 'weight_scale', 'weight_scale_inv', 'input_scale', 'bias', 'qweight', 'scales', 'qzeros'))
 
 
 def _bf16_weight(module):
@@ -168,12 +173,16 @@ class _RealQuantLinear(torch.nn.Module):
             self.__dict__[name] = None
 
     def _buffer(self, name, value):
-        """register_buffer of a module that is being made: nothing to look for under that name.  (A subclass' own
-        register_buffer, and hooks registered for all modules, are called all the same.)"""
-        if type(self).register_buffer is not torch.nn.Module.register_buffer or _module._global_buffer_registration_hooks:
-            self.register_buffer(name, value)
-        else:
+        """register_buffer of a module that is being made.  One of the containers' own names, nothing of that name yet, a plain
+        tensor, and torch's own register_buffer without hooks: then the entry is all that it would make (1.4 us a buffer, a
+        fifth of what a container costs).  Everything else goes through it: a subclass' register_buffer, one put in place of
+        torch.nn.Module's, hooks registered for all modules, names and values that it refuses."""
+        cls = type(self)
+        if cls.register_buffer is _REGISTER and not _module._global_buffer_registration_hooks and name in _NAMES \
+                and (value is None or type(value) is torch.Tensor) and name not in self.__dict__ and not hasattr(cls, name):
             self._buffers[name] = value
+        else:
+            self.register_buffer(name, value)
 
     def __repr__(self):
         """The one-line description the reference prints for its deploy modules (module_utils.py:995-1008)."""

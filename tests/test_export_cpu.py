@@ -3,6 +3,7 @@
 import json
 import types
 
+import pytest
 import torch
 
 from lightcompress_amd import export as E
@@ -101,3 +102,44 @@ def test_container_buffer_names():
     a = AutoawqRealQuantLinear(w, None, s, w.clone())
     assert set(dict(a.named_buffers())) == {'qweight', 'scales', 'qzeros'}
     assert set(AutoawqRealQuantLinear(w, None, s, None).state_dict()) == {'qweight', 'scales'}
+
+
+def test_container_buffers_go_through_a_replaced_register_buffer(monkeypatch):
+    """Buffers are registered through whatever stands in for torch's register_buffer: a replacement of torch.nn.Module's method
+    (contexts that create modules on another device do that), a subclass' own, a hook for all modules; and what it refuses (not
+    a tensor, a name that is taken or has a dot) stays refused."""
+    from lightcompress_amd.module_utils import AutoawqRealQuantLinear, VllmRealQuantLinear
+    w, s = torch.zeros(4, 2, dtype=torch.int32), torch.ones(4, 1, dtype=torch.float16)
+    torchs, seen = torch.nn.Module.register_buffer, []
+
+    def replacement(self, name, tensor, persistent=True):
+        seen.append(name)
+        return torchs(self, name, None if tensor is None else tensor + 1, persistent)
+    with monkeypatch.context() as m:
+        m.setattr(torch.nn.Module, 'register_buffer', replacement)
+        v = VllmRealQuantLinear(w, None, s, None, True, 'weight_scale')
+        a = AutoawqRealQuantLinear(w, torch.zeros(4), s, w)
+    assert seen == ['weight_packed', 'weight_scale', 'input_scale', 'qweight', 'bias', 'scales', 'qzeros']
+    assert int(v.weight_packed.min()) == 1 and float(a.bias.min()) == 1
+
+    class Own(VllmRealQuantLinear):
+        def register_buffer(self, name, tensor, persistent=True):
+            seen.append(name)
+            torchs(self, name, tensor, persistent)
+    del seen[:]
+    Own(w, None, s, None, True, 'weight_scale')
+    assert seen == ['weight_packed', 'weight_scale', 'input_scale']
+    hook = torch.nn.modules.module.register_module_buffer_registration_hook(lambda mod, name, t: seen.append(name))
+    try:
+        del seen[:]
+        VllmRealQuantLinear(w, None, s, None, False, 'weight_scale')
+    finally:
+        hook.remove()
+    assert seen == ['weight', 'weight_scale', 'input_scale']
+
+    class Taken(VllmRealQuantLinear):
+        weight_packed = 3
+    for cls, args in ((Taken, (w, None, s, None, True, 'weight_scale')), (VllmRealQuantLinear, (w, None, s, None, True, 'a.b')),
+                      (VllmRealQuantLinear, ([1, 2], None, s, None, True, 'weight_scale'))):
+        with pytest.raises((KeyError, TypeError)):
+            cls(*args)
