@@ -41,13 +41,21 @@ class AutoClipper:
         self.weight_clips = {}
         self.w_only = w_only
         self.logit = lambda x: torch.log(x / (1 - x))
-        self.last_errs = None            # [R, G, n_steps] fp32 of the last auto_clip_layer call (None with errors=False)
+        self.last_errs = None            # [R, G, n_steps] fp32 of the last auto_clip_layer call (None with errors=False); after `run`: of its last Linear
         self.fast = False                # True: the bf16 MFMA search kernel where it applies (see the module docstring)
         self.fp8_block_size = 128
 
     # -- auto_clip.py:45-81 ----------------------------------------------------------------------
+    @staticmethod
+    def _clipped(name, module):
+        return isinstance(module, torch.nn.Linear) and not any(_ in name for _ in ['q_', 'k_', 'query', 'key', 'Wqkv'])
+
     @torch.no_grad()
     def run(self, block, block_idx, input_feat, n_sample_token):
+        # `last_errs` holds the errors of the last Linear afterwards; nobody sees those of the ones before it, so there only what
+        # decides is computed (a subclass' own search is called as it is, and its own apply_clip may look)
+        own = all(getattr(getattr(self, f), '__func__', None) is getattr(AutoClipper, f) for f in ('auto_clip_layer', 'apply_clip'))
+        last = [n for n, m in block.named_modules() if self._clipped(n, m)][-1:]
         for n, m in block.named_modules():
             if not isinstance(m, torch.nn.Linear):
                 continue
@@ -55,16 +63,14 @@ class AutoClipper:
             if is_fp8_weight:                              # block-wise float8 checkpoint: search on the bf16 weights
                 m.weight.data = weight_cast_to_bf16(m.weight.data.contiguous(), m.weight_scale_inv.data.contiguous(),
                                                     self.fp8_block_size).to(torch.bfloat16)
-            if any(_ in n for _ in ['q_', 'k_', 'query', 'key', 'Wqkv']):
+            if not self._clipped(n, m):
                 if self.clip_version == 'v2':
                     m.register_buffer('buf_upbound_factor', None)
                     m.register_buffer('buf_lowbound_factor', None)
                 continue
             inputs = [torch.cat(input_feat[n])] if len(input_feat[n]) != 1 else input_feat[n]
-            # nobody sees the errors of a step here: only what decides is computed (a subclass' own search is called as it is)
-            plain = getattr(self.auto_clip_layer, '__func__', None) is AutoClipper.auto_clip_layer
             max_val, min_val = self.auto_clip_layer(block_idx, n, m.weight, inputs, n_sample_token=n_sample_token,
-                                                    **({'errors': False} if plain else {}))
+                                                    **({'errors': False} if own and [n] != last else {}))
             self.apply_clip(block_idx, m, min_val, max_val, n)
             if is_fp8_weight:
                 m.weight.data, m.weight_scale_inv.data = weight_cast_to_fp8(m.weight.data.contiguous(), self.fp8_block_size)

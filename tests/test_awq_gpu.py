@@ -465,6 +465,39 @@ def test_auto_clip_search_without_the_losing_steps(dev, gs, T, bit, sym, clip_sy
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize('watched', [False, True])
+def test_auto_clip_run_leaves_the_errors_of_its_last_linear(dev, watched):
+    """`last_errs` after `run` holds the errors of every step of the last Linear that was searched (one that is skipped may come
+    behind it), and an apply_clip of a subclass finds those of the Linear it is called for."""
+    from lightcompress_amd import IntegerQuantizer
+    from lightcompress_amd.auto_clip import AutoClipper
+    from tests.helpers import weight_like
+    K, T = 256, 96
+    names = ('gate_proj', 'o_proj', 'q_proj')
+    blk = torch.nn.ModuleDict({n: torch.nn.Linear(K, 64, bias=False, device=dev, dtype=torch.bfloat16) for n in names})
+    for i, n in enumerate(names):
+        blk[n].weight.data = weight_like(64, K, seed=i, dtype=torch.float32, outlier_frac=0.002).bfloat16().to(dev)
+    feats = {n: [torch.randn(1, T, K, generator=gen(i)).bfloat16().to(dev)] for i, n in enumerate(names)}
+    want, seen = {}, {}
+
+    class Watching(AutoClipper):
+        def apply_clip(self, block_idx, layer, min_val, max_val, layer_name):
+            seen[layer_name] = self.last_errs
+            super().apply_clip(block_idx, layer, min_val, max_val, layer_name)
+
+    def make(cls):
+        return cls(True, IntegerQuantizer(4, False, 'per_group', group_size=128), None, 'v1', False, False, None)
+    for n in names[:2]:
+        clipper = make(AutoClipper)
+        clipper.auto_clip_layer(0, n, blk[n].weight, feats[n], n_sample_token=T)
+        want[n] = clipper.last_errs
+    clipper = make(Watching if watched else AutoClipper)
+    clipper.run(blk, 0, feats, T)
+    assert torch.equal(clipper.last_errs, want['o_proj']) and want['o_proj'].shape == (64, 2, 10)
+    if watched:
+        assert set(seen) == set(want) and all(torch.equal(seen[n], want[n]) for n in want)
+
+
 @pytest.mark.parametrize('gs,clip_sym', [(128, False), (64, True), (32, False)])
 def test_auto_clip_one_launch_search_keeps_rows_apart(dev, gs, clip_sym):
     """An infinite or NaN weight, and a finite one whose products overflow, spoil their own row of their group only: every
