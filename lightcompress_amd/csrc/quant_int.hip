@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void mse_range_kernel(const void* __restrict__
 //     xmax + s / 2 and xmin - s / 2 at the latest (symmetric: at qmax s and qmin s; a zero point is rounded, and clamped
 //     towards the range), which moves towards zero from step to step, so once what the ends alone clip there (less MSE_SLACK
 //     for the roundings of either evaluation, |x| < 2) is more than the best error for all rows of a wave, it is done: after
-//     28 of 80 steps on average.  Not where a later step's scale would be clamped at 1e-5, which widens its range again;
+//     28 of 80 steps on average.  Not where a later step's range would be clamped at 1e-5, which widens it again;
 //   * elements past the row's end are zeros: with qmin <= z <= qmax they quantize to themselves and add nothing.
 // The estimate and mse_row_error differ by a relative delta at most (mse_margin below).  Where `margin` cannot tell the two
 // steps apart, the wave evaluates mse_row_error for both of them, so the range is always the one mse_range_kernel finds: an

@@ -198,17 +198,17 @@ def test_hessian_from_packed_tokens(dev, K, cuts, dtype):
         assert torch.equal(again, H)
 
 
-@pytest.mark.parametrize('slices', [1, 3, 'auto'])
-def test_hessian_shares_through_add_batch_and_reads_in_between(dev, slices):
+@pytest.mark.parametrize('K,slices', [(512, 1), (512, 3), (512, 'auto'), (768, 1), (768, 3), (768, 'auto')])
+def test_hessian_shares_through_add_batch_and_reads_in_between(dev, K, slices):
     """`special.hessian_slices`: whatever the number of accumulators, reading H in the middle of the calibration
     (which sums the shares and clears all but the first) and going on afterwards ends at the closed form."""
-    K, T = 512, 160
+    T = 160
     batches = calib_batches(7, T, K, seed=1400)
     g = make_gptq(hessian_slices=slices, hessian_defer=3)
     layer = Layer(torch.zeros(8, K, device=dev))
     g.layers_cache['l'] = {}
     g.layer_init(layer, 'l')
-    assert (g.layers_cache['l']['H_shares'] is None) == (slices == 1)
+    assert (g.layers_cache['l']['H_shares'] is None) == (slices == 1 or (slices == 'auto' and K > 512))
     for i, b in enumerate(batches):
         g.add_batch(layer, 'l', b.unsqueeze(0).to(dev), None)
         if i in (1, 4):
@@ -273,10 +273,10 @@ def test_hessian_calls_like_the_one_before_and_others(dev, defer, follower_at):
 
 
 @pytest.mark.parametrize('defer', [1, 3, 4, 'auto'])
-def test_hessian_deferred_launches(dev, defer):
+@pytest.mark.parametrize('K', [320, 648])
+def test_hessian_deferred_launches(dev, K, defer):
     """Folding several add_batch calls into one launch leaves H and nsamples as per-call updates do,
-    for ragged token counts and for inputs the caller overwrites right after the call."""
-    K = 320
+    for ragged token counts and for inputs the caller overwrites right after the call (token shares, staged tokens)."""
     shapes = [(1, 96), (2, 96), (1, 96), (1, 40), (1, 96), (3, 64), (1, 96), (1, 700), (1, 96)]
     g = make_gptq(hessian_defer=defer)
     layer = Layer(torch.zeros(8, K, device=dev))
@@ -1231,6 +1231,38 @@ def test_split_gemm_has_fp32_accuracy(dev):
         assert float((Us[0] - Us[1]).abs().max() / Us[0].abs().max()) < 1e-5
     finally:
         lib.lcq_set_gemm_split(L.i32(1))
+
+
+@pytest.mark.parametrize('K', [4616, 8328])
+def test_chain_with_deep_updates_of_ragged_matrices(dev, K):
+    """The deep updates of long chains on operands split ahead, on matrices that are no whole number of 256 x 256 tiles: on the
+    caller's stream, and beside the next super-panel on a second one (from K = 8192 on).  The factor is as close to the fp64
+    identity as the fp32 pipe's and agrees with it to fp32 rounding."""
+    from lightcompress_amd import _lib as L
+    lib = L.lib()
+    g = torch.Generator(device=dev).manual_seed(K)
+    X = torch.randn(K + K // 2, K, device=dev, generator=g) * torch.exp(0.7 * torch.randn(K, device=dev, generator=g))
+    H0 = X.t() @ X / K
+    Hd = H0.double()
+    Hd.diagonal().add_(0.01 * torch.diag(H0).double().mean())
+    nbytes = lib.lcq_chol_inv_upper_workspace_bytes(K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    Us, res = {}, {}
+    try:
+        for mode in (0, 1):
+            lib.lcq_set_gemm_split(mode)
+            H = H0.clone()
+            L.check(lib.lcq_chol_inv_upper(L.ptr(H), K, None, 0.01, None, 0, L.ptr(H), L.ptr(ws), nbytes, L.ptr(status), L.stream()), 'chain')
+            assert int(status.item()) == 0
+            Us[mode] = H.double()
+            E = Us[mode].t().contiguous() @ (Us[mode] @ Hd)
+            E.diagonal().sub_(1)
+            res[mode] = float(E.abs().max())
+    finally:
+        lib.lcq_set_gemm_split(1)
+    assert res[1] <= max(2 * res[0], 1e-5) and res[0] < 2e-5, res
+    assert float((Us[0] - Us[1]).abs().max() / Us[0].abs().max()) < 1e-5
 
 
 @pytest.mark.parametrize('R,Kc,N,kind', [(3072, 1024, 3072, 'plain'), (2305, 512, 4000, 'rows'), (4096, 512, 2177, 'spread'),

@@ -200,12 +200,12 @@ def test_input_written_in_place_between_two_hooks_is_not_shared_silently(dev):
     gp.subset_transform({'layers': layers})
 
 
+@pytest.mark.parametrize('K', [384, 640])
 @pytest.mark.parametrize('read_at', [0, 2, 4])
-def test_hessian_read_between_the_hooks_of_one_pass(dev, read_at):
+def test_hessian_read_between_the_hooks_of_one_pass(dev, read_at, K):
     """Reading H after the leader's hook and before the follower's folds the staged tokens; the follower, one call
     behind at that moment, is given its own Hessian first (the state before that call) and goes on alone.  Every
-    result equals separate accumulation bit for bit."""
-    K = 384
+    result equals separate accumulation bit for bit (token shares, staged tokens)."""
     Ws = {'a': (torch.randn(32, K, generator=gen(15)) * 0.02).bfloat16(), 'b': (torch.randn(48, K, generator=gen(16)) * 0.02).bfloat16()}
     xs = [(torch.randn(1, 64, K, generator=gen(8700 + i))).bfloat16().to(dev) for i in range(6)]
     out = {}

@@ -902,8 +902,8 @@ def test_mse_range_is_the_one_of_the_re_reading_kernel(dev, rows, cols, dtype, b
     (64, 4104, torch.bfloat16, 4, True)])
 def test_mse_range_search_that_ends_early(dev, rows, cols, dtype, bit, sym):
     """Once the ends of a row alone clip more than the best error, the steps that only shrink the range further are left out;
-    not where one of them would have its scale clamped at 1e-5, which widens its range again.  Rows with outliers (the search
-    ends after a few steps), lopsided rows (zero point at a bound), and rows whose range crosses 1e-5 * levels at the first,
+    not where one of them would have its range clamped at 1e-5, which widens it again.  Rows with outliers (the search
+    ends after a few steps), lopsided rows (zero point at a bound), and rows whose range crosses 1e-5 at the first,
     a middle or the last step; compared with the re-reading kernel, which runs every step (rows padded with zeros as above)."""
     g = torch.Generator(device=dev).manual_seed(rows + cols)
     w = torch.randn(rows, cols, generator=g, device=dev) * 0.02
