@@ -244,7 +244,7 @@ def bench_hessian(args, out, x=None):
     def hess(b):
         xp = L.ptr(packed[b % len(packed)])
         L.check(lib.lcq_hessian_accum_packed(L.ptr(H), K, xp, xp, L.BF16, TL, 0.5, 0.01, L.ptr(ws), ws_bytes, st), 'hessian')
-    t_h = timeit(hess, 16, 8)
+    t_h = timeit(hess, 32, 16)
     # the vendor library on the same operands, for scale: the full product X^T X as one bf16 GEMM through torch
     # (hipBLASLt; bf16 output, no accumulation into H), same token-major layout of both operands
     xl = [x[b * FOLD:(b + 1) * FOLD].reshape(TL, K) for b in range(nb // FOLD)]
@@ -252,7 +252,7 @@ def bench_hessian(args, out, x=None):
     alg_flops = 2.0 * TL * K * K
     tiles = sum(K // 256 - ti for ti in range(K // 256))              # 256x256 tiles that reach the upper triangle
     exe_flops = 2.0 * TL * tiles * 256 * 256
-    traffic, stale = traffic_bytes('hessian_packed_kernel_K14336_T32768', t_h * 1e6) if TL == 32768 else (None, None)
+    traffic, stale = traffic_bytes('hessian_packed_kernel_K14336_T8192', t_h * 1e6) if TL == 8192 else (None, None)
     out['roofline'] = {
         'kernel': f'hessian_packed_kernel<bf16> K=14336 T={TL} (+ packed_fold_kernel)', 'bound': 'mfma', 'achieved': round(exe_flops / t_h / 1e12, 2),
         'peak': 2500.0, 'unit': 'TFLOP/s', 'frac': round(exe_flops / t_h / 2.5e15, 4),

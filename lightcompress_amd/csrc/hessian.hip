@@ -373,7 +373,8 @@ __global__ __launch_bounds__(256) void tail_fold_kernel(float* __restrict__ H, i
 //  * four LDS stages of 32 tokens, one barrier per slab: at the middle of a slab every wave holds the rest of it in
 //    registers, so its stage is free for the slab four ahead.
 // The chip clocks down under this load (random tokens 1.7 GHz, zeros run 1.3 times as fast), which is what bounds it.
-// Measured (us, without the copy): K = 14336, 8192 tokens 1448 -> 1293 (1.33 PFLOP/s of the tiles computed; 1.25 on another box),
+// Measured (us, without the copy): K = 14336, 8192 tokens 1448 -> 1293 (1.33 PFLOP/s of the tiles computed; with a scale per
+// channel 1350, 1.27: the clock goes by what the operands hold),
 // K = 4096, 32768 tokens 525 -> 477, K = 8192, 16384 tokens 996 -> 901, K = 7168, 16384 tokens 743 -> 660, K = 2048, 32768 tokens
 // 143 -> 136; against hessian_kernel with the token shares or split rounds it had for the same work.
 typedef const __attribute__((address_space(3))) char* lds_ptr;
