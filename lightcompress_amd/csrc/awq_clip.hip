@@ -160,18 +160,23 @@ __global__ __launch_bounds__(256) void clamp_groups_scalar_kernel(const void* __
 //   products  v_mfma_f32_32x32x4_2b with ONE non-zero k slot per block is an outer product: block 0 gives x[t, j] w[r, j],
 //             block 1 gives x[t, j+1] w[r, j+1] for 32 tokens x 32 rows (exact in fp32), in the same registers of both blocks;
 //   rounding  one v_cvt_pk per pair (j, j+1): 16 instructions for 2048 products, all the vector pipe has to do;
-//   sums      four rounded pairs of a lane are one A operand of v_mfma_f32_16x16x32 (k = 8 values of a lane); a constant
-//             0 / 1 B operand adds each pair and sends it to a column of its own.
-// Layouts: products leave lane l with row l % 32 and tokens 8 (i / 4) + 4 (l / 32) + i % 4 in register i; the sums leave
-// sum[q][i] = token 8 q + 4 ((l >> 3) & 1) + (l & 3), row 16 ((l >> 2) & 1) + 4 (l >> 4) + i.
-// What bounds it: 64 + 4 x 16 matrix-pipe cycles per 2048 products; the 16 conversions (64 vector cycles) run under the
-// next products.  v_mfma_f32_32x32x1 and v_dot2_f32_bf16 would do the same sums, but neither overlaps with vector
-// instructions on this chip (229 against 128 cycles), and moving a quarter of the sums to the vector pipe made it 13 %
-// slower.  Measured (rows 11008 x 4096 + 11008 x 4096 + 4096 x 11008, 512 tokens, 10 steps): 92.3 -> 25.8 ms, the matrix
-// pipes busy in 78 % of the cycles; the products one after the other in the same registers 31.2, without all
-// conversions ahead of the sums 28.3.
+//   sums      16 rounded values of a lane (four columns of four tokens) are its share of the dense operand of
+//             v_smfmac_f32_16x16x64, whose other operand is sparse: two of four values.  That one holds ones where a value belongs
+//             to an output and nothing elsewhere: 1024 values meet their sums in 16 cycles, where a dense instruction takes 512.
+// Layouts: products leave lane l with row l % 32 and tokens 8 (i / 4) + 4 (l / 32) + i % 4 in register i.  Lane l supplies the
+// values k = 8 (l / 16) .. + 7 and 32 + 8 (l / 16) .. + 7 of column l % 16 of the dense operand, and the sparse one holds the values
+// k = 16 (l / 16) .. + 15 of row l % 16, two of every four.  Row 4 h + o adds what the lanes of quarter h hold of output o, and the
+// accumulator has rows 4 (l / 16) + i of column l % 16 in register i: sum[q][i] of a lane is its own product register 4 q + i.
+// What bounds it: 2 x 64 + 4 x 16 matrix-pipe cycles per 4096 products, and 32 conversions of 4 cycles each (half the rate of other
+// vector instructions) that only partly run beside them: two waves per SIMD take 302 cycles (328 with the pairs added by four
+// v_mfma_f32_16x16x32 per 2048 products, 256 matrix cycles).  v_mfma_f32_32x32x1 and v_dot2_f32_bf16 would do the same sums, but
+// neither overlaps with vector instructions on this chip, and moving a quarter of the sums to the vector pipe made it 13 % slower.
+// Measured: 4096 x 11008, 512 tokens, 10 steps, all errors: 8.57 ms with those, 7.95 so; the products one after the other in the
+// same registers, or conversions between the sums instead of ahead of them, are slower still.
 typedef __attribute__((ext_vector_type(4))) short i16x4;
 typedef __attribute__((ext_vector_type(32))) float f32x32;
+typedef __attribute__((ext_vector_type(16))) __bf16 bf16x16;
+typedef __attribute__((ext_vector_type(8))) uint32_t u32x8;
 
 __device__ __forceinline__ f32x32 outer_products(u32x2 a, u32x2 b) {
   f32x32 z;
@@ -179,15 +184,16 @@ __device__ __forceinline__ f32x32 outer_products(u32x2 a, u32x2 b) {
   for (int i = 0; i < 32; ++i) z[i] = 0.0f;
   return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(__builtin_bit_cast(i16x4, a), __builtin_bit_cast(i16x4, b), z, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 add_pairs(u32x4 pairs, u32x4 ones, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pairs), __builtin_bit_cast(bf16x8, ones), c, 0, 0, 0);
+// The sparse operand: where this lane's share holds ones, and which two of every four values they stand for.
+// Outputs 0 and 1 of a lane are in its values 0 .. 7, two and three in 8 .. 15; an even one in the first two of every four.
+struct Sums { u32x4 ones; int places; };
+__device__ __forceinline__ Sums sums_of_own_values(int lane) {
+  const int h = (lane >> 2) & 3, o = lane & 3, quarter = lane >> 4;         // row l % 16 = 4 h + o of the operand
+  const uint32_t one = quarter == (h >> 1) + (o & 2) ? 0x3f803f80u : 0u, first = (h & 1) ? 0u : one, second = (h & 1) ? one : 0u;
+  return Sums{u32x4{first, first, second, second}, (o & 1) ? 0xeeee : 0x4444};
 }
-// B operand of add_pairs: lane (h = l / 16, n = l % 16) holds k = 8 h + i of column n; pair i / 2 of quarter h goes to column 4 h + i / 2
-__device__ __forceinline__ u32x4 pair_columns(int lane) {
-  u32x4 b;
-  #pragma unroll
-  for (int d = 0; d < 4; ++d) b[d] = (lane & 15) == 4 * (lane >> 4) + d ? 0x3f803f80u : 0u;
-  return b;
+__device__ __forceinline__ f32x4 add_values(const u32x8& values, const Sums& to, f32x4 c) {
+  return __builtin_amdgcn_smfmac_f32_16x16x64_bf16(__builtin_bit_cast(bf16x8, to.ones), __builtin_bit_cast(bf16x16, values), c, to.places, 0, 0);
 }
 
 constexpr int GT = 32;                   // tokens and rows of one wave's tile
@@ -196,7 +202,7 @@ template <int GS> constexpr int gd_pitch() { return GS * 2 + 16; }     // bytes 
 // column pair are issued before the current ones are rounded: the empty asm keeps that order (without it the compiler
 // runs the two one after the other in the same registers).
 template <int GS>
-__device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint32_t mask, u32x4 ones, f32x4* sum) {
+__device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint32_t mask, const Sums& to, f32x4* sum) {
   #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   u32x4 b = *(const u32x4*)wrow, ahead = *(const u32x4*)(wrow + 16);
@@ -213,6 +219,9 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
   };
   f32x32 d[2];
   d[0] = products(0);
+  u32x8 pr[4];                                              // four columns (2 i .. 2 i + 3) of the four tokens of product register 4 q + k
+  #pragma unroll
+  for (int q = 0; q < 4; ++q) pr[q] = u32x8{0, 0, 0, 0, 0, 0, 0, 0};
   #pragma unroll
   for (int i = 0; i < GS / 2; ++i) {
     f32x32& cur = d[i & 1];
@@ -220,45 +229,46 @@ __device__ __forceinline__ void dots_tile(const u32x4* a, const char* wrow, uint
       d[(i + 1) & 1] = products(i + 1);
       asm volatile("" : "+v"(d[0]), "+v"(d[1]));
     }
-    u32x4 pr[4];
     #pragma unroll
     for (int q = 0; q < 4; ++q)
       #pragma unroll
-      for (int k = 0; k < 4; ++k) pr[q][k] = bf16_pack_rne(cur[4 * q + k], cur[16 + 4 * q + k]);
+      for (int k = 0; k < 4; ++k) pr[q][4 * (k >> 1) + 2 * (i & 1) + (k & 1)] = bf16_pack_rne(cur[4 * q + k], cur[16 + 4 * q + k]);
     asm volatile("" : "+v"(pr[0]), "+v"(pr[1]), "+v"(pr[2]), "+v"(pr[3]));
-    #pragma unroll
-    for (int q = 0; q < 4; ++q) sum[q] = add_pairs(pr[q], ones, sum[q]);
+    if (i & 1) {
+      #pragma unroll
+      for (int q = 0; q < 4; ++q) sum[q] = add_values(pr[q], to, sum[q]);
+    }
   }
 }
 
-// One row of A in add_pairs holds two weight rows (lanes m and m + 16), kept apart by the zeros of B, and 0 * infinity is NaN:
-// an infinite or NaN product (an infinite or NaN weight, a product beyond the largest bf16 number) turns the sums of its
-// partner row 16 rows away into NaN as well.  So a lane with a sum that is not finite adds its products up again one by one:
-// x: the group's columns of token 0, w(i): where the weights of the lane's row i lie in LDS.  Off the path of finite tiles,
-// which pay for the test alone.
-template <int GS, class Rows>
-__device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __restrict__ x, int64_t K, int t0, int T, const Rows& w,
-                                                              int lane, f32x4* sum) {
+// A column of the dense operand in add_values holds the values of four lanes (l % 16), kept apart by the zeros of the other one, and
+// 0 * infinity is NaN: an infinite or NaN product (an infinite or NaN weight, a product beyond the largest bf16 number) turns the sums
+// of those lanes into NaN as well.  So a lane with a sum that is not finite adds its products up again one by one:
+// x: the group's columns of token 0, w: where the weights of the lane's row lie in LDS.  Off the path of finite tiles, which pay for
+// the test alone.
+template <int GS>
+__device__ __forceinline__ void redo_sums_that_are_not_finite(const uint16_t* __restrict__ x, int64_t K, int t0, int T, const char* w, int lane,
+                                                              f32x4* sum) {
   float m = 0.0f;
   #pragma unroll
   for (int q = 0; q < 4; ++q)
     #pragma unroll
     for (int i = 0; i < 4; i += 2) m = nan_max(nan_max(m, fabsf(sum[q][i])), fabsf(sum[q][i + 1]));
   if (__builtin_expect(m < __builtin_inff(), 1)) return;
-  const int tok = t0 + 4 * ((lane >> 3) & 1) + (lane & 3);
+  const int tok = t0 + 4 * (lane >> 5);
   #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   #pragma unroll 1
   for (int j = 0; j < GS; ++j) {
-    float wv[4];
+    const float wv = u2f((uint32_t)*(const uint16_t*)(w + 2 * j) << 16);
     #pragma unroll
-    for (int i = 0; i < 4; ++i) wv[i] = u2f((uint32_t)*(const uint16_t*)(w(i) + 2 * j) << 16);
-    #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float xv = tok + 8 * q < T ? u2f((uint32_t)x[(int64_t)(tok + 8 * q) * K + j] << 16) : 0.0f;
+    for (int q = 0; q < 4; ++q)
       #pragma unroll
-      for (int i = 0; i < 4; ++i) sum[q][i] += rnd<true>(xv * wv[i]);
-    }
+      for (int i = 0; i < 4; ++i) {
+        const int t = tok + 8 * q + i;
+        const float xv = t < T ? u2f((uint32_t)x[(int64_t)t * K + j] << 16) : 0.0f;
+        sum[q][i] += rnd<true>(xv * wv);
+      }
   }
 }
 
@@ -280,10 +290,30 @@ __device__ __forceinline__ void round_sums(f32x4* v) {
       v[q][i] = o0; v[q][i + 1] = o1;
     }
 }
-// e[i] = the errors of row i of the lane over the tokens of the tile (the same in the eight lanes that share its rows); org rounded
-__device__ __forceinline__ void tile_errors(const f32x4* cur, const f32x4* org, float* e) {
+// the rounded sums of a lane as 32 bytes in two pieces (tokens 0 .. 7 and 8 .. 15 of the lane), the pieces of the 64 lanes side by side
+constexpr int ORG_HALF = 64 * 16;
+__device__ __forceinline__ void store_org(char* at, const f32x4* v) {
   #pragma unroll
-  for (int i = 0; i < 4; ++i) e[i] = 0.0f;
+  for (int p = 0; p < 2; ++p)
+    *(u32x4*)(at + p * ORG_HALF) = u32x4{bf16_pack(v[2 * p][0], v[2 * p][1]), bf16_pack(v[2 * p][2], v[2 * p][3]),
+                                         bf16_pack(v[2 * p + 1][0], v[2 * p + 1][1]), bf16_pack(v[2 * p + 1][2], v[2 * p + 1][3])};
+}
+__device__ __forceinline__ void load_org(const char* at, f32x4* v) {
+  #pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const u32x4 raw = *(const u32x4*)(at + p * ORG_HALF);
+    #pragma unroll
+    for (int d = 0; d < 4; ++d) { v[2 * p + d / 2][2 * (d & 1)] = u2f(raw[d] << 16); v[2 * p + d / 2][2 * (d & 1) + 1] = u2f(raw[d] & 0xffff0000u); }
+  }
+}
+// v of lane l + v of lane l ^ 32
+__device__ __forceinline__ float both_halves(float v) {
+  const auto s = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
+  return u2f(s[0]) + u2f(s[1]);
+}
+// the error of the lane's row over the 32 tokens of the tile; org rounded
+__device__ __forceinline__ float tile_error(const f32x4* cur, const f32x4* org) {
+  float e[2] = {0.0f, 0.0f};
   #pragma unroll
   for (int q = 0; q < 4; ++q)
     #pragma unroll
@@ -294,15 +324,9 @@ __device__ __forceinline__ void tile_errors(const f32x4* cur, const f32x4* org, 
       rnd_pair<true>(c0, c1);
       c0 *= c0; c1 *= c1;
       rnd_pair<true>(c0, c1);
-      e[i] += c0; e[i + 1] += c1;
+      e[0] += c0; e[1] += c1;
     }
-  // over the tokens of the tile: lanes that differ in bits 0, 1 and 3
-  #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    e[i] += lane_xor<1>(e[i]);
-    e[i] += lane_xor<2>(e[i]);
-    e[i] += u2f((uint32_t)__builtin_amdgcn_ds_swizzle((int)f2u(e[i]), 0x201F));      // xor 8
-  }
+  return both_halves(e[0] + e[1]);
 }
 
 __device__ __forceinline__ float shrunk(float v, int s, int n_grid) { return rnd<true>(v * (float)(1.0 - (double)s / (double)n_grid)); }
@@ -356,27 +380,21 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
   __syncthreads();
 
   const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
-  const u32x4 ones = pair_columns(lane);
+  const Sums to = sums_of_own_values(lane);
   const char* wrow = smem + (lane & 31) * PITCH_W;
-  const char* const rows_of_lane = smem + (16 * ((lane >> 2) & 1) + 4 * (lane >> 4)) * PITCH_W;
   for (int t0 = wave * GT; t0 < T; t0 += waves * GT) {
     u32x4 a[GS / 8];
     load_token<GS>(x + g * GS, K, T, t0 + (lane & 31), a);
     f32x4 org[4], cur[4];
-    dots_tile<GS>(a, wrow, mask, ones, org);
-    redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, [&](int i) { return rows_of_lane + i * PITCH_W; }, lane, org);
+    dots_tile<GS>(a, wrow, mask, to, org);
+    redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, wrow, lane, org);
     round_sums(org);
     #pragma unroll 1
     for (int s = 0; s < n_steps; ++s) {
-      dots_tile<GS>(a, wrow + (s + 1) * VERSION, mask, ones, cur);
-      redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, [&](int i) { return rows_of_lane + (s + 1) * VERSION + i * PITCH_W; }, lane, cur);
-      float e[4];
-      tile_errors(cur, org, e);
-      if ((lane & 0xb) == 0) {
-        float* es = esum + (wave * n_steps + s) * GT + 16 * ((lane >> 2) & 1) + 4 * (lane >> 4);
-        #pragma unroll
-        for (int i = 0; i < 4; ++i) es[i] += e[i];
-      }
+      dots_tile<GS>(a, wrow + (s + 1) * VERSION, mask, to, cur);
+      redo_sums_that_are_not_finite<GS>(x + g * GS, K, t0, T, wrow + (s + 1) * VERSION, lane, cur);
+      const float e = tile_error(cur, org);
+      if (lane < GT) esum[(wave * n_steps + s) * GT + lane] += e;
     }
   }
   __syncthreads();
@@ -436,8 +454,8 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
   const int rounds = (T + waves * GT - 1) / (waves * GT), pairs = n_steps * GT;
   const int G = K / GS, g = blockIdx.x % G, r0 = (blockIdx.x / G) * GT;
-  uint16_t* const orgs = (uint16_t*)(smem + (n_steps + 1) * VERSION);    // [tokens][32] bf16
-  float* const part = (float*)(orgs + rounds * waves * GT * GT);         // [waves][pairs] bounds; later [waves][pairs] exact sums
+  char* const orgs = smem + (n_steps + 1) * VERSION;                     // [tiles] rounded sums of the original weights (store_org)
+  float* const part = (float*)(orgs + rounds * waves * 2 * ORG_HALF);    // [waves][pairs] bounds; later [waves][pairs] exact sums
   float* const tab = part + waves * pairs * 2;                           // [rounds][pairs] lower, upper
   float* const bounds = tab + rounds * pairs * 2;                        // [pairs] lower, upper
   uint16_t* const list = (uint16_t*)(bounds + pairs * 2);                // (step, row) = entry / 32, entry % 32
@@ -451,30 +469,20 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
   __syncthreads();
 
   const uint32_t mask = lane < 32 ? 0xffffu : 0xffff0000u;
-  const u32x4 ones = pair_columns(lane);
+  const Sums to = sums_of_own_values(lane);
   const int h = lane >> 5, c = lane & 31;
-  const int row4 = 16 * ((lane >> 2) & 1) + 4 * (lane >> 4), tok4 = 4 * ((lane >> 3) & 1) + (lane & 3);    // of the exact sums
   for (int k = 0; k < rounds; ++k) {
     const int t0 = (k * waves + wave) * GT;
     if (t0 < T) {
       u32x4 a[GS / 8];
       load_token<GS>(xg, K, T, t0 + c, a);
-      {
-        f32x4 org[4];
-        dots_tile<GS>(a, smem + c * PITCH_W, mask, ones, org);
-        redo_sums_that_are_not_finite<GS>(xg, K, t0, T, [&](int i) { return smem + (row4 + i) * PITCH_W; }, lane, org);
-        round_sums(org);
-        #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *(u32x2*)(orgs + (t0 + 8 * q + tok4) * GT + row4) = u32x2{bf16_pack(org[q][0], org[q][1]), bf16_pack(org[q][2], org[q][3])};
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
       // v_mfma_f32_32x32x16: lane (h, c) supplies token / row c and columns 16 ks + 8 h .. + 7; register r holds token
-      // 8 (r / 4) + 4 h + r % 4 of row c
-      float o[16];
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) o[r] = u2f((uint32_t)orgs[(t0 + 8 * (r >> 2) + 4 * h + (r & 3)) * GT + c] << 16);
+      // 8 (r / 4) + 4 h + r % 4 of row c, as the exact sums do
+      f32x4 org[4];
+      dots_tile<GS>(a, smem + c * PITCH_W, mask, to, org);
+      redo_sums_that_are_not_finite<GS>(xg, K, t0, T, smem + c * PITCH_W, lane, org);
+      round_sums(org);
+      store_org(orgs + (k * waves + wave) * 2 * ORG_HALF + lane * 16, org);
       u32x4 ax[GS / 16];
       #pragma unroll
       for (int ks = 0; ks < GS / 16; ++ks)
@@ -511,13 +519,13 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
           float lo = 0.0f, hi = 0.0f;
           #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const float d = fabsf(sum[v][r] - o[r]), b = CLIP_U * ((mag[v][r] + fabsf(sum[v][r])) + d);
+            const float d = fabsf(sum[v][r] - org[r >> 2][r & 3]), b = CLIP_U * ((mag[v][r] + fabsf(sum[v][r])) + d);
             const float l = fmaxf(d - b, 0.0f), u = d + b;
             lo = __builtin_fmaf(l, l, lo);
             hi = __builtin_fmaf(u, u, hi);
           }
-          lo += __shfl_xor(lo, 32);
-          hi += __shfl_xor(hi, 32);
+          lo = both_halves(lo);
+          hi = both_halves(hi);
           if (h == 0 && s + v < n_steps) *(f32x2*)(part + 2 * ((wave * n_steps + s + v) * GT + c)) = f32x2{lo, hi};
         }
       }
@@ -607,24 +615,13 @@ __global__ __launch_bounds__(512, 2) void clip_search_pruned_kernel(const uint16
       #pragma unroll 1
       for (int p = 0; p < n; p += GT) {
         const int mine = list[p + c];
-        int entry[4];
-        #pragma unroll
-        for (int i = 0; i < 4; ++i) entry[i] = list[p + row4 + i];
-        const auto where = [&](int e) { return smem + ((e >> 5) + 1) * VERSION + (e & 31) * PITCH_W; };
+        const char* const wrow = smem + ((mine >> 5) + 1) * VERSION + (mine & 31) * PITCH_W;
         f32x4 org[4], cur[4];
-        dots_tile<GS>(a, where(mine), mask, ones, cur);
-        redo_sums_that_are_not_finite<GS>(xg, K, t0, T, [&](int i) { return where(entry[i]); }, lane, cur);
-        #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          #pragma unroll
-          for (int i = 0; i < 4; ++i) org[q][i] = u2f((uint32_t)orgs[(t0 + 8 * q + tok4) * GT + (entry[i] & 31)] << 16);
-        float e[4];
-        tile_errors(cur, org, e);
-        if ((lane & 0xb) == 0) {
-          #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (p + row4 + i < n) part[wave * pairs + entry[i]] += e[i];
-        }
+        dots_tile<GS>(a, wrow, mask, to, cur);
+        redo_sums_that_are_not_finite<GS>(xg, K, t0, T, wrow, lane, cur);
+        load_org(orgs + (k * waves + wave) * 2 * ORG_HALF + ((mine & 31) + 32 * h) * 16, org);
+        const float e = tile_error(cur, org);
+        if (h == 0 && p + c < n) part[wave * pairs + mine] += e;
       }
     }
     __syncthreads();
