@@ -189,305 +189,215 @@ __global__ __launch_bounds__(256) void build_gather_kernel(const float* __restri
   }
 }
 
-// Diagonal block: Cholesky factor L11 of a 128x128 block and its inverse, one workgroup of 8 waves.
-// A wave that is alone on its SIMD issues about one instruction per 8 cycles, and a column-by-column sweep with a
-// barrier per column executes ~150 instructions per column in every wave: 70 us per block, none of it arithmetic.
-// Here the 128 columns are 8 panels of 16, and the serial part of a panel runs without barriers in one to three waves, a row per lane:
-//   * waves 0-3 ("update waves") hold the lower triangle in registers, 8x8 per thread, dealt out cyclically (thread
-//     (ty, tx) owns rows ty + 16 ii and columns tx + 16 cc);
-//   * waves 4, 6 and 7 ("panel waves") take the current 16-column panel from LDS with one row per lane and factor it in
-//     registers: pivot and multipliers travel by v_readlane, 2 instructions per (column, later column) pair; they leave
-//     the scaled panel in LDS;
-//   * the update waves apply a finished panel first to the next panel's columns, hand those to the panel waves, and
-//     apply it to the rest of their registers while those are already factoring (a right-looking update
-//     with look-ahead); two barriers per panel;
-//   * wave 5 inverts the 16x16 diagonal block of the previous panel meanwhile (forward substitution in registers);
-//   * afterwards all 8 waves merge the inverted diagonal blocks pairwise, 16 -> 32 -> 64 -> 128,
-//     [[A,0],[B,C]]^-1 = [[A^-1,0],[-C^-1 B A^-1, C^-1]], from LDS.
-// Bound by the serial chain of one wave's instructions: 26.4 us per block (32.8 with two rows per lane in one panel wave,
-// one LDS read at a time in front of the hand-over and one per matrix instruction in the merges; 28.7 with a condition around
-// every load of the block; the same bits).
-// Row (column) r of the block lives at float `lds_slot(r)` of an LDS row.  Thread t of the 16 x 16 update grid owns rows
-// t + 16 ii, ii < 8: the first four sit at 4 t .. 4 t + 3 and the other four at 64 + 4 t .., so both 16-byte pieces of
-// a thread are contiguous with its neighbours' (no bank conflicts for 16-byte accesses), and 16 consecutive rows are 16
-// bytes apart (none for the 4-byte accesses of the panel wave and of the matrix-pipe operand reads either).
-constexpr int lds_slot(int r) { return ((r >> 4) < 4) ? 4 * (r & 15) + (r >> 4) : 64 + 4 * (r & 15) + (r >> 4) - 4; }
+// Diagonal block: Cholesky factor L11 of a 128x128 block and the inverse of L11, one workgroup of 8 waves.
+// A wave that is alone on its SIMD issues about one instruction per 8 cycles, so what counts is how many instructions the serial
+// part needs.  The 128 columns are 8 panels of 16; everything that is not the pivot chain of a panel runs on the fp32 matrix pipe:
+//   * the panel waves (4, 6, 7) take a panel from LDS with one row per lane and factor it without barriers.  A column costs one
+//     v_readlane (the pivot), a reciprocal square root, one product and at most four v_mfma_f32_4x4x1_16b: 16 blocks of 4 x 4 are
+//     64 rows x 4 columns, and with the A operand of ONE block broadcast to all of them (cbsz = 4, abid = the quad of lanes that
+//     holds the rows these columns belong to) one instruction is the rank-1 update of four columns for all rows of the wave.
+//     The rows of an identity ride along behind the panel's: they come out as the transposed inverse of its 16 x 16 block.
+//   * the update waves (1, 2, 3, 5) hold the lower triangle behind in 16 x 16 tiles, the accumulators of v_mfma_f32_16x16x4f32
+//     (wave u tile rows u and 7 - u).  They apply a finished panel first to the next panel's columns, hand those over, and do the
+//     rest of the update while the panel waves are factoring (a right-looking update with look-ahead; two barriers per panel).
+//   * They also build the inverse X block row by block row beside the panels: T_Pj = sum_k L_Pk X_kj waits in the accumulators
+//     for the inverse of panel P's block, X_Pj = -X_PP T_Pj goes to memory (and LDS, for the rows below) one panel later.  Behind
+//     the last panel only X_7j is left.
+// Contractions take k = 4 (l / 16) + i in instruction i, so an operand is one 16-byte read of a row and an accumulator is the B
+// operand of the next product as it stands.  The panels and tiles hold -A, so that updates add.
+// Bound by the serial chain of one wave's instructions: 14.3 us per block (26.4 us with updates of 8 x 8 values per thread, 240
+// v_readlane / v_fma per panel and the inverse by three levels of merges at the end).
 constexpr int LP = NB + 4;       // row pitch of the LDS matrices (16-byte aligned rows, 4-bank skew)
+constexpr int PP = 16 + 4;       // row pitch of the panel
 
 struct PotrfLds {
-  float L[8][16][LP];    // L[P][k][lds_slot(r)] = L(r, 16 P + k); zero above the diagonal inside the panel's own 16 rows
-  float X[NB][LP];       // L^-1, row-major
-  float Pn[16][LP];      // the panel on its way to the panel wave, same layout as L[P], unscaled (padded rows: the 16
-                         // rows a publishing wave writes at once fall into different banks)
-  float T[64 * 64];      // products of the inverse merges
+  float L[NB][LP];       // L row-major, below the 16 x 16 diagonal blocks
+  float XT[NB][LP];      // XT[c][r] = X(r, c), X = L^-1: the tiles on and below its diagonal
+  float Pn[NB][PP];      // - the panel on its way to the panel waves
 };
 
 __device__ __forceinline__ float rdlane(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
-// panel P: columns 16 P .. +15, rows 16 P .. 127.  Lanes 0 .. 15 of every panel wave hold the panel's own 16 rows (the multipliers
-// come from there), the other 48 lanes the rows behind them, dealt to as many waves as they need: wave `w` (0, 1, 2) takes rows
-// 16 P + 16 + 48 w ...  One row per lane in up to three waves on SIMDs of their own: two rows per lane in one wave are half as many
-// instructions again on the critical path.  Wave 0 writes the panel's own rows.
-__device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int w, int lane, bool& bad) {
-  #pragma clang fp contract(fast)   // a -= l*l as one FMA; nothing here needs op-by-op rounding
-  const int row = 16 * P + lane + (lane < 16 ? 0 : 48 * w);
-  const bool ok = row < NB;
-  const int slot = lds_slot(ok ? row : 0);
-  float a[16];
+// Panel P: columns 16 P .. +15.  Lanes 0 .. 15 of every panel wave hold the panel's own 16 rows (pivots and multipliers come from
+// there), the other 48 lanes the rows behind them and then 16 rows of the identity, dealt to as many waves as they need.
+// `least` gathers the pivots (NaN stays).
+__device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int w, int lane, float& least) {
+  #pragma clang fp contract(fast)   // the residual of the reciprocal square root as FMAs
+  const int behind = NB - 16 * P - 16;                      // rows behind the panel's own
+  const int q = lane - 16 + 48 * w;                         // this lane's row among those and the identity's
+  const bool own = lane < 16, rest = !own && q < behind, unit = !own && q >= behind && q < behind + 16;
+  const float* const from = s.Pn[own ? 16 * P + lane : rest ? 16 * P + 16 + q : 16 * P];
+  const int one = own || rest ? -1 : q - behind;            // where a row of the identity has its one
+  f32x4 n[4];
   #pragma unroll
-  for (int k = 0; k < 16; ++k) a[k] = ok ? s.Pn[k][slot] : 0.0f;
+  for (int b = 0; b < 4; ++b) n[b] = *(const f32x4*)(from + 4 * b);
+  #pragma unroll
+  for (int j = 0; j < 16; ++j) n[j >> 2][j & 3] = own || rest ? n[j >> 2][j & 3] : j == one ? -1.0f : 0.0f;
+  f32x4 l[4];
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const float piv = rdlane(a[j], j);
-    bad = bad || !(piv > 0.0f);
-    float rinv = __builtin_amdgcn_rsqf(piv);          // 1/sqrt(pivot), one Newton step to full precision
-    rinv = rinv * (1.5f - 0.5f * piv * rinv * rinv);
-    a[j] *= rinv;                                     // the diagonal entry becomes sqrt(pivot); rows above it hold zeros
-    #pragma unroll
-    for (int c = j + 1; c < 16; ++c) {
-      const float m = rdlane(a[j], c);                // L(16 P + c, 16 P + j)
-      a[c] -= a[j] * m;                               // (entries above the diagonal pick up garbage; never read, masked below)
-    }
+    const float x = n[j >> 2][j & 3], piv = -rdlane(x, j);
+    least = nan_min(least, piv);
+    const float r = __builtin_amdgcn_rsqf(piv);             // 1/sqrt(pivot), one Newton step to full precision
+    const float v = x * -(r + (0.5f * r) * (1.0f - (piv * r) * r));
+    l[j >> 2][j & 3] = v;                                   // (own rows above the diagonal hold garbage; nothing reads it)
+    // columns from j + 1 on; those of j's own four that are done pick up garbage
+    if (j < 3) n[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, v, n[0], 4, 0, 0);
+    if (j < 7) n[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, v, n[1], 4, 1, 0);
+    if (j < 11) n[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, v, n[2], 4, 2, 0);
+    if (j < 15) n[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, v, n[3], 4, 3, 0);
   }
-  if (ok && (lane >= 16 || w == 0)) {
+  if (rest || unit) {
+    float* const to = rest ? &s.L[16 * P + 16 + q][16 * P] : &s.XT[16 * P + q - behind][16 * P];
     #pragma unroll
-    for (int k = 0; k < 16; ++k) s.L[P][k][slot] = (lane >= k) ? a[k] : 0.0f;
+    for (int b = 0; b < 4; ++b) *(f32x4*)(to + 4 * b) = l[b];
   }
 }
 
-// X_QQ = L_QQ^-1 for the 16x16 diagonal block Q: lane c (mod 16) carries column c of the inverse
-__device__ __forceinline__ void potrf_diag_inv(PotrfLds& s, int Q, int lane) {
-  #pragma clang fp contract(fast)
-  const int c0 = 16 * Q, l16 = lane & 15;
-  const int sl = lds_slot(c0 + l16);
-  float t[16], x[16];
+// c + sum over 16 of the contraction: a and b as read from rows (lane l: row l % 16, k = 4 (l / 16) + i in element i)
+__device__ __forceinline__ f32x4 potrf_mac(const f32x4& a, const f32x4& b, f32x4 c) {
   #pragma unroll
-  for (int k = 0; k < 16; ++k) t[k] = s.L[Q][k][sl];          // lane j: row j of the block
-  #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    float acc = (l16 == j) ? 1.0f : 0.0f;
-    #pragma unroll
-    for (int k = 0; k < j; ++k) acc -= rdlane(t[k], j) * x[k];
-    const float d = rdlane(t[j], j);
-    float r = __builtin_amdgcn_rcpf(d);
-    r = r * (2.0f - d * r);
-    x[j] = acc * r;
-  }
-  if (lane < 16) {
-    #pragma unroll
-    for (int j = 0; j < 16; ++j) s.X[c0 + j][c0 + lane] = (lane <= j) ? x[j] : 0.0f;
-  }
+  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+  return c;
 }
 
-// a[ii][cc] -= sum_k L(row, 16 PL + k) L(col, 16 PL + k) for the register columns CC_LO .. 7 (rows ii >= cc), or for
-// the single column CC_LO (ONE).  Compile-time ranges: a run-time range costs a branch per register column and
-// panel column, and a wave here pays ~10 cycles for every instruction it issues.
-template <int PL, int CC_LO, bool ONE>
-__device__ __forceinline__ void potrf_update(const PotrfLds& s, float (&a)[8][8], int ty, int tx) {
-  #pragma clang fp contract(fast)
-  if constexpr (CC_LO < 8) {
-    constexpr int UNROLL = ONE ? 16 : 2;
-    // ONE is on the critical path (the panel waves wait for it): all of its LDS reads in flight at once
-    #pragma unroll UNROLL
-    for (int k = 0; k < 16; ++k) {
-      const f32x4 r0 = *(const f32x4*)(s.L[PL][k] + 4 * ty), r1 = *(const f32x4*)(s.L[PL][k] + 64 + 4 * ty);
-      const float lr[8] = {r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]};
-      if constexpr (ONE) {
-        const float lc = s.L[PL][k][(CC_LO < 4 ? 4 * tx + CC_LO : 64 + 4 * tx + CC_LO - 4)];
-        #pragma unroll
-        for (int ii = CC_LO; ii < 8; ++ii) a[ii][CC_LO] -= lr[ii] * lc;
-      } else {
-        const f32x4 c0 = *(const f32x4*)(s.L[PL][k] + 4 * tx), c1 = *(const f32x4*)(s.L[PL][k] + 64 + 4 * tx);
-        const float lc[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-        #pragma unroll
-        for (int cc = CC_LO; cc < 8; ++cc)
-          #pragma unroll
-          for (int ii = cc; ii < 8; ++ii) a[ii][cc] -= lr[ii] * lc[cc];
-      }
+// What an update wave holds.  Tile (i, j), transposed: lane l element e is row 16 i + l % 16, column 16 j + 4 (l / 16) + e.
+// t[0]: tile row u (tiles 0 .. 3 at most), t[1]: tile row 7 - u.
+struct PotrfTiles { f32x4 top[4], bottom[8]; };
+
+// the columns of panel J to the panel waves (J, the panel in front of it applied already)
+template <int J>
+__device__ __forceinline__ void potrf_publish(PotrfLds& s, const PotrfTiles& t, int u, int m, int g) {
+  if constexpr (J < 4) { if (u >= J) *(f32x4*)(s.Pn[16 * u + m] + 4 * g) = t.top[J]; }
+  if (7 - u >= J) *(f32x4*)(s.Pn[16 * (7 - u) + m] + 4 * g) = t.bottom[J];
+}
+
+// panel P on tile columns LO .. HI
+template <int P, int LO, int HI>
+__device__ __forceinline__ void potrf_update(const PotrfLds& s, PotrfTiles& t, int u, int m, int g) {
+  if constexpr (LO <= HI) {
+    if (7 - u < LO) return;
+    const f32x4 hi = *(const f32x4*)(s.L[16 * (7 - u) + m] + 16 * P + 4 * g);
+    const f32x4 lo = *(const f32x4*)(s.L[16 * u + m] + 16 * P + 4 * g);       // (read only where u > P)
+    #pragma unroll
+    for (int j = LO; j <= HI; ++j) {
+      if (j > 7 - u) continue;
+      const f32x4 a = *(const f32x4*)(s.L[16 * j + m] + 16 * P + 4 * g);
+      t.bottom[j] = potrf_mac(a, hi, t.bottom[j]);
+      if (j < 4 && j <= u) t.top[j & 3] = potrf_mac(a, lo, t.top[j & 3]);
     }
   }
 }
 
-// register column PC (columns tx + 16 PC) -> Pn, zero above the diagonal
-template <int PC>
-__device__ __forceinline__ void potrf_publish(PotrfLds& s, const float (&a)[8][8], int ty, int tx) {
-  float v[8];
-  #pragma unroll
-  for (int ii = 0; ii < 8; ++ii) v[ii] = (ty + 16 * ii >= tx + 16 * PC) ? a[ii][PC] : 0.0f;
-  *(f32x4*)(s.Pn[tx] + 4 * ty) = f32x4{v[0], v[1], v[2], v[3]};
-  *(f32x4*)(s.Pn[tx] + 64 + 4 * ty) = f32x4{v[4], v[5], v[6], v[7]};
-}
-
-// panel P of the sweep, all 8 waves
+// Column block j of the inverse, beside panel P: X_ij of tile row i = P - 1, whose own block has been inverted, then T of row P.
 template <int P>
-__device__ __forceinline__ void potrf_phase(PotrfLds& s, float (&a)[8][8], int wave, int lane, bool upd, int ty, int tx, bool& bad) {
-  __syncthreads();                                   // Pn holds panel P; L[P - 1] is complete
-  constexpr int BEHIND = NB - 16 * P - 16;           // rows behind the panel's own
-  if (wave == 4 || (BEHIND > 48 && wave == 6) || (BEHIND > 96 && wave == 7)) {
-    potrf_panel(s, P, wave == 4 ? 0 : wave - 5, lane, bad);
-  } else if (wave == 5) {
-    if constexpr (P > 0) potrf_diag_inv(s, P - 1, lane);
-  } else if (upd) {
-    if constexpr (P > 0) potrf_update<P - 1, P + 1, false>(s, a, ty, tx);     // panel P - 1 on everything behind panel P
-  }
-  __syncthreads();                                   // L[P] is complete
-  if constexpr (P < 7) {
-    if (upd) {
-      potrf_update<P, P + 1, true>(s, a, ty, tx);      // panel P on the next panel's columns, handed over at once
-      potrf_publish<P + 1>(s, a, ty, tx);
-    }
-  }
-}
-
-// One level of the inverse: the blocks of size S on the diagonal of X are inverted already, the block below each even
-// one follows as X21 = -X22 (L21 X11), two products on the fp32 matrix pipe with operands straight from LDS.
-// v_mfma_f32_32x32x2f32: lane l supplies A(row l % 32, k = l / 32) and B(k = l / 32, column l % 32); accumulator
-// register r holds row 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32.  v_mfma_f32_16x16x4f32: A(row l % 16,
-// k = l / 16), B(k = l / 16, column l % 16), register r holds row 4 (l / 16) + r of column l % 16.
-// One wave per 32x32 (16x16) output tile; both triangular operands are cut at tile granularity and read zeros above
-// their diagonals (X is cleared at the start).
-typedef __attribute__((ext_vector_type(16))) float potrf_f32x16;
-
-template <int S>
-__device__ __forceinline__ void potrf_merge(PotrfLds& s, int wave, int lane) {
-  if constexpr (S >= 32) {
-    constexpr int TS = S / 32, TPP = TS * TS, NT = (NB / (2 * S)) * TPP;
-    const int p = wave / TPP, t = wave % TPP, ti = t / TS, tj = t % TS;
-    const int o = 2 * S * p, lm = lane & 31, lk = lane >> 5;
-    const bool on = wave < NT;
-    if (on) {
-      potrf_f32x16 acc;
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-      const int rs = lds_slot(o + S + 32 * ti + lm);
-      for (int k0 = 32 * tj; k0 < S; k0 += 32) {         // X11(k, j) = 0 for k < j
-        float av[16], bv[16];                            // the operands of 16 instructions in flight: the chain waits for LDS once
-        #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kk = o + k0 + 2 * i + lk;
-          av[i] = s.L[kk >> 4][kk & 15][rs];
-          bv[i] = s.X[kk][o + 32 * tj + lm];
-        }
-        #pragma unroll
-        for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], acc, 0, 0, 0);
-      }
-      #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        s.T[(p * S + 32 * ti + 8 * (r >> 2) + 4 * lk + (r & 3)) * S + 32 * tj + lm] = acc[r];
-    }
-    __syncthreads();
-    if (on) {
-      potrf_f32x16 acc;
-      #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-      for (int k0 = 0; k0 < 32 * (ti + 1); k0 += 32) {   // X22(i, k) = 0 for k > i
-        float av[16], bv[16];
-        #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kk = k0 + 2 * i + lk;
-          av[i] = s.X[o + S + 32 * ti + lm][o + S + kk];
-          bv[i] = s.T[(p * S + kk) * S + 32 * tj + lm];
-        }
-        #pragma unroll
-        for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[i], acc, 0, 0, 0);
-      }
-      #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        s.X[o + S + 32 * ti + 8 * (r >> 2) + 4 * lk + (r & 3)][o + 32 * tj + lm] = -acc[r];
-    }
-    __syncthreads();
+__device__ __forceinline__ void potrf_inverse(PotrfLds& s, f32x4& T, int j, int nb, float* __restrict__ Dinv, int m, int g) {
+  constexpr int I = P - 1;
+  if (I < j) return;
+  f32x4 x;                                                  // X_II(m, 4 g + e)
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = s.XT[16 * I + 4 * g + e][16 * I + m];
+  if (I == j) {
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = (16 * I + m < nb && 16 * I + 4 * g + e < nb) ? x[e] : 0.0f;   // (the padding's diagonal)
+    *(f32x4*)(Dinv + (16 * I + m) * NB + 16 * I + 4 * g) = x;
   } else {
-    static_assert(S == 16, "block sizes 16, 32, 64");
-    const int p = wave, o = 32 * p, lm = lane & 15, lk = lane >> 4;
-    const bool on = wave < NB / 32;
-    if (on) {
-      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      const int rs = lds_slot(o + 16 + lm);
-      #pragma unroll
-      for (int k = 0; k < 16; k += 4) {
-        const int kk = o + k + lk;
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s.L[kk >> 4][kk & 15][rs], s.X[kk][o + lm], acc, 0, 0, 0);
-      }
-      #pragma unroll
-      for (int r = 0; r < 4; ++r) s.T[(p * 16 + 4 * lk + r) * 16 + lm] = acc[r];
-    }
-    __syncthreads();
-    if (on) {
-      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-      #pragma unroll
-      for (int k = 0; k < 16; k += 4) {
-        const int kk = k + lk;
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s.X[o + 16 + lm][o + 16 + kk], s.T[(p * 16 + kk) * 16 + lm], acc, 0, 0, 0);
-      }
-      #pragma unroll
-      for (int r = 0; r < 4; ++r) s.X[o + 16 + 4 * lk + r][o + lm] = -acc[r];
-    }
-    __syncthreads();
+    f32x4 v = potrf_mac(x, T, f32x4{0.0f, 0.0f, 0.0f, 0.0f});                 // rows 4 g + e, column m
+    v = -v;
+    if constexpr (P < 8) *(f32x4*)(s.XT[16 * j + m] + 16 * I + 4 * g) = v;
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) Dinv[(16 * I + 4 * g + e) * NB + 16 * j + m] = v[e];
+  }
+  if constexpr (P < 8) {
+    T = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    #pragma unroll
+    for (int k = 0; k < P; ++k)
+      if (k >= j) T = potrf_mac(*(const f32x4*)(s.L[16 * P + m] + 16 * k + 4 * g), *(const f32x4*)(s.XT[16 * j + m] + 16 * k + 4 * g), T);
   }
 }
 
-__global__ __launch_bounds__(512) void potrf_diag_kernel(float* __restrict__ Ablk, int lda, int nb,
+// what an update wave does beside panel P and behind it
+template <int P>
+__device__ __forceinline__ void potrf_phase(PotrfLds& s, PotrfTiles& t, f32x4 (&T)[2], int u, int nb, float* __restrict__ Dinv, int m, int g) {
+  __syncthreads();                                          // Pn holds panel P; L and the inverted blocks up to panel P - 1
+  if constexpr (P > 0) {
+    potrf_update<P - 1, P + 1, 7>(s, t, u, m, g);
+    potrf_inverse<P>(s, T[0], u, nb, Dinv, m, g);
+    potrf_inverse<P>(s, T[1], 7 - u, nb, Dinv, m, g);
+  }
+  __syncthreads();                                          // L of panel P is complete
+  if constexpr (P < 7) {
+    potrf_update<P, P + 1, P + 1>(s, t, u, m, g);
+    potrf_publish<P + 1>(s, t, u, m, g);
+  }
+}
+
+__global__ __launch_bounds__(512) void potrf_diag_kernel(const float* __restrict__ Ablk, int lda, int nb,
                                                          float* __restrict__ Dinv, PrepScalars* sc) {
   __shared__ __align__(16) PotrfLds s;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ty = (tid >> 4) & 15, tx = tid & 15;
-  const bool upd = tid < 256;
-  float a[8][8];
-  if (upd) {
-    // a whole block: plain loads (all in flight), the diagonal 16 x 16 squares masked afterwards; a load under a condition of its
-    // own costs five instructions more and a branch
-    if (nb == NB) {
-      const float* p = Ablk + (long long)ty * lda + tx;
-      #pragma unroll
-      for (int ii = 0; ii < 8; ++ii)
-        #pragma unroll
-        for (int cc = 0; cc <= ii; ++cc) a[ii][cc] = p[(long long)16 * ii * lda + 16 * cc];
-      #pragma unroll
-      for (int ii = 0; ii < 8; ++ii) {
-        a[ii][ii] = tx <= ty ? a[ii][ii] : 0.0f;
-        #pragma unroll
-        for (int cc = ii + 1; cc < 8; ++cc) a[ii][cc] = 0.0f;
+  if (wave == 0 || wave == 4 || wave >= 6) {
+    if (wave == 0) {                                        // the tiles above the diagonal are zeros
+      for (int r = 0; r < NB - 16; r += 2) {
+        const int row = r + (lane >> 5), c4 = (lane & 31) * 4;
+        if (c4 >= (row & ~15) + 16) *(f32x4*)(Dinv + row * NB + c4) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       }
-    } else {
+    }
+    float least = __builtin_inff();
+    const int w = wave == 0 ? 3 : wave == 4 ? 0 : wave - 5;                   // wave 0 has no rows: NB <= 3 x 48
+    for (int P = 0; P < 8; ++P) {
+      __syncthreads();
+      if (48 * w < NB - 16 * P) potrf_panel(s, P, w, lane, least);
+      __syncthreads();
+    }
+    if (wave == 4 && lane == 0 && !(least > 0.0f)) sc->status = 1;
+    return;
+  }
+  const int u = wave == 5 ? 0 : wave;
+  PotrfTiles t;
+  // a whole block: plain loads, all in flight (those above the diagonal are never used)
+  if (nb == NB && lda % 4 == 0 && ((uintptr_t)Ablk & 15) == 0) {
+    const float* const top = Ablk + (long long)(16 * u + m) * lda + 4 * g;
+    const float* const bottom = Ablk + (long long)(16 * (7 - u) + m) * lda + 4 * g;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < 4) t.top[j & 3] = *(const f32x4*)(top + 16 * j);
+      t.bottom[j] = *(const f32x4*)(bottom + 16 * j);
+    }
+  } else {
+    const auto load = [&](int i, int j, f32x4& v) {
+      const int r = 16 * i + m, c = 16 * j + 4 * g;
       #pragma unroll
-      for (int ii = 0; ii < 8; ++ii)
-        #pragma unroll
-        for (int cc = 0; cc < 8; ++cc) {
-          const int r = ty + 16 * ii, c = tx + 16 * cc;
-          a[ii][cc] = (r < nb && c <= r) ? Ablk[(long long)r * lda + c] : ((r == c) ? 1.0f : 0.0f);   // pad with identity
-        }
+      for (int e = 0; e < 4; ++e) v[e] = (r < nb && c + e <= r) ? Ablk[(long long)r * lda + c + e] : (r == c + e) ? 1.0f : 0.0f;   // pad with identity
+    };
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < 4) load(u, j, t.top[j & 3]);
+      load(7 - u, j, t.bottom[j]);
     }
   }
-  for (int e = tid; e < NB * LP / 4; e += 512) ((f32x4*)&s.X[0][0])[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (upd) {
-    potrf_publish<0>(s, a, ty, tx);
-  }
-  bool bad = false;
-  potrf_phase<0>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<1>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<2>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<3>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<4>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<5>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<6>(s, a, wave, lane, upd, ty, tx, bad);
-  potrf_phase<7>(s, a, wave, lane, upd, ty, tx, bad);
-  __syncthreads();
-  if (wave == 5) potrf_diag_inv(s, 7, lane);
-  if (wave == 4 && bad && lane == 0) sc->status = 1;
-  __syncthreads();
-  potrf_merge<16>(s, wave, lane);
-  potrf_merge<32>(s, wave, lane);
-  potrf_merge<64>(s, wave, lane);
-  for (int v = tid; v < NB * NB / 4; v += 512) {            // L^-1, row-major, zeros above the diagonal and in the padding
-    const int r = v >> 5, c4 = (v & 31) * 4;
-    f32x4 x = *(const f32x4*)(&s.X[r][c4]);
+  #pragma unroll
+  for (int j = 0; j < 8; ++j)
     #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = (r < nb && c4 + e <= r) ? x[e] : 0.0f;
-    *(f32x4*)(Dinv + r * NB + c4) = x;
-  }
+    for (int e = 0; e < 4; ++e) {
+      if (j < 4) t.top[j & 3][e] = (j < u || 4 * g + e <= m) ? -t.top[j & 3][e] : 0.0f;
+      t.bottom[j][e] = (j < 7 - u || 4 * g + e <= m) ? -t.bottom[j][e] : 0.0f;
+    }
+  potrf_publish<0>(s, t, u, m, g);
+  f32x4 T[2];
+  potrf_phase<0>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<1>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<2>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<3>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<4>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<5>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<6>(s, t, T, u, nb, Dinv, m, g);
+  potrf_phase<7>(s, t, T, u, nb, Dinv, m, g);
+  potrf_inverse<8>(s, T[0], u, nb, Dinv, m, g);
+  potrf_inverse<8>(s, T[1], 7 - u, nb, Dinv, m, g);
   // (L itself is not written back: everything after this kernel works with the inverse, the solved panels and the
   // blocks behind them; place_diag_kernel puts the inverse where the block was.)
 }

@@ -531,6 +531,34 @@ def test_prepare_weights_without_a_permutation(dev, dtype, R, K):
             assert float(out[R * K + 1]) == 7.0
 
 
+@pytest.mark.parametrize('K', [1, 15, 16, 17, 31, 48, 65, 97, 112, 113, 127, 128, 129, 131, 257])
+def test_diagonal_blocks_of_every_fill(dev, K):
+    """One to three diagonal blocks whose last is filled to either side of a 16-column panel, of the 48 rows a wave takes and of
+    the block itself, in rows that do and do not start on 16 bytes.  The matrix has a condition number below 3, so the factor of
+    its inverse is within a few K roundings of fp64's; a pivot that is not positive, or NaN, is reported wherever it stands."""
+    from lightcompress_amd import _lib as L
+    x = torch.randn(K, K, generator=gen(5200 + K), dtype=torch.float64)
+    x = x + x.t()
+    H = (torch.eye(K, dtype=torch.float64) + 0.5 * x / (torch.linalg.matrix_norm(x, 2) + 1e-9)).float()
+    nbytes = L.lib().lcq_chol_inv_upper_workspace_bytes(K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+
+    def chain(h):
+        hd, U, status = torch.triu(h).to(dev).contiguous(), torch.full((K, K), 7.0, device=dev), torch.full((1,), 9, dtype=torch.int32, device=dev)
+        L.check(L.lib().lcq_chol_inv_upper(L.ptr(hd), K, None, 0.0, None, 0, L.ptr(U), L.ptr(ws), nbytes, L.ptr(status), L.stream()), 'chain')
+        return U.cpu().double(), int(status.item())
+
+    U, status = chain(H)
+    Uo = torch.linalg.cholesky(torch.linalg.inv(H.double()), upper=True)
+    assert status == 0 and torch.equal(torch.triu(U), U)
+    assert float((U - Uo).norm() / Uo.norm()) <= 3 * 4 * K * 2.0 ** -24       # condition x (factor, inverse, two roundings each) x K u
+    for at in sorted({0, K // 3, K - 1}):
+        for v in (-1.0, float('nan')):
+            bad = H.clone()
+            bad[at, at] = v
+            assert chain(bad)[1] == 1, (at, v)
+
+
 def test_cholesky_reports_indefinite_matrix(dev):
     from lightcompress_amd import _lib as L
     K = 128
