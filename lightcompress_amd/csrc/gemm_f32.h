@@ -536,9 +536,163 @@ __global__ __launch_bounds__(256) void gemm_f32_batched_kernel(const float* A, i
                            flags, m0, n0, sA, sB);
 }
 
+// A contraction of exactly 128 (panel solves and rank-128 updates of the blocked chains, the column loop's updates inside a window):
+// C = A op(B) (ADD: C -= A op(B)), no LDS and no barrier between loads and products.  An operand of v_mfma_f32_16x16x4f32 is one element
+// of a 16-byte piece that a lane reads where it lies (lane (g, m) = (l / 16, l % 16) of instruction e supplies k = 16 s + 4 g + e), so all
+// loads of a wave are in flight before its first product and a launch is little more than a memory latency and the 64 products of a
+// wave.  B given as [n][k] takes the place of the rows of the product, whose accumulator is then four columns of one row of C; from a
+// B given as [k][n] a lane reads two neighbouring columns, one for each of two products.  Either way C is read and written in pieces of
+// 8 or 16 bytes.  A wave owns 16 x 32 of C, a workgroup WN of them side by side.  Rows and columns are clamped for reading; N is a
+// multiple of 4.  Without ADD C may be A itself (a workgroup spans all of N then; the barrier is for that).
+template <bool B_T, int WN, bool ADD>
+__global__ __launch_bounds__(64 * WN) void gemm_f32_rank128_kernel(GemmProblem p, int flags) {
+  const int m0 = 16 * blockIdx.y, lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  if ((flags & GEMM_LOWER_TILES) && 32 * WN * (int)blockIdx.x >= m0 + 16) return;
+  const int n0 = 32 * (WN * blockIdx.x + (threadIdx.x >> 6));
+  f32x4 a[8], bt[2][8];
+  f32x2 bn[8][4];
+  const float* const pa = p.A + (long long)min(m0 + m, p.M - 1) * p.lda + 4 * g;
+  #pragma unroll
+  for (int s = 0; s < 8; ++s) a[s] = *(const f32x4*)(pa + 16 * s);
+  if constexpr (B_T) {
+    #pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float* const pb = p.B + (long long)min(n0 + 16 * j + m, p.N - 1) * p.ldb + 4 * g;
+      #pragma unroll
+      for (int s = 0; s < 8; ++s) bt[j][s] = *(const f32x4*)(pb + 16 * s);
+    }
+  } else {
+    const float* const pb = p.B + (long long)(4 * g) * p.ldb + min(n0 + 2 * m, p.N - 2);
+    #pragma unroll
+    for (int s = 0; s < 8; ++s)
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) bn[s][e] = *(const f32x2*)(pb + (long long)(16 * s + e) * p.ldb);
+  }
+  // this lane's pieces of C: row m0 + m, columns n0 + 16 q + 4 g .. + 3 (B_T); rows m0 + 4 g + q, columns n0 + 2 m, + 1
+  constexpr int PIECES = B_T ? 2 : 4, WIDTH = B_T ? 4 : 2;
+  typedef __attribute__((ext_vector_type(WIDTH))) float piece;
+  const auto row_of = [&](int q) { return m0 + (B_T ? m : 4 * g + q); };
+  const auto col_of = [&](int q) { return n0 + (B_T ? 16 * q + 4 * g : 2 * m); };
+  piece old[PIECES];
+  if constexpr (ADD) {
+    #pragma unroll
+    for (int q = 0; q < PIECES; ++q) old[q] = *(const piece*)(p.C + (long long)min(row_of(q), p.M - 1) * p.ldc + min(col_of(q), p.N - WIDTH));
+  }
+  f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+  // Loads that the compiler lets slip in between the products wait for one memory latency after the other: with a B from beyond L2 14 us
+  // instead of 8.3 for 1000 x 384.  (With both operands in L2, as in the chain, that is the better order: K = 1024 205 us against 211.)
+  if constexpr (!B_T) __builtin_amdgcn_sched_barrier(0);
+  #pragma unroll
+  for (int s = 0; s < 8; ++s)
+    #pragma unroll
+    for (int e = 0; e < 4; ++e)
+      #pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (B_T) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bt[j][s][e], a[s][e], acc[j], 0, 0, 0);
+        else acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][e], bn[s][e][j], acc[j], 0, 0, 0);
+      }
+  if constexpr (!ADD) __syncthreads();
+  #pragma unroll
+  for (int q = 0; q < PIECES; ++q) {
+    piece v;
+    if constexpr (B_T) v = acc[q];
+    else v = piece{acc[0][q], acc[1][q]};
+    if constexpr (ADD) v = old[q] - v;
+    if (row_of(q) < p.M && col_of(q) < p.N) *(piece*)(p.C + (long long)row_of(q) * p.ldc + col_of(q)) = v;
+  }
+}
+
+// The same product, C -= A B with B given as [k][n], for many rows: a wave keeps 64 columns of B in registers (128 of them) and streams
+// 16 rows of A and C at a time, the next ones in flight while it multiplies: `step` waves per 64 columns, waves side by side on columns
+// side by side of the same rows.  The same sums in the same order as the kernel above: the same bits.  Bound by the fp32 matrix pipe
+// (108 of 157 TFLOP/s for 28672 x 896) beside the reading and writing of C.
+static __global__ __launch_bounds__(256, 2) void gemm_f32_rank128_stream_kernel(GemmProblem p, int step) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int groups = (p.N + 63) / 64, id = 4 * blockIdx.x + (threadIdx.x >> 6), n0 = id % groups * 64, tiles = (p.M + 15) / 16;
+  int t = id / groups;
+  if (t >= step || t >= tiles) return;
+  const int col = n0 + 4 * m, from = min(col, p.N - 4);
+  f32x4 b[8][4];                                            // columns 4 m .. of k = 16 s + 4 g + e
+  #pragma unroll
+  for (int s = 0; s < 8; ++s)
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) b[s][e] = *(const f32x4*)(p.B + (long long)(16 * s + 4 * g + e) * p.ldb + from);
+  f32x4 a[8], c[4];
+  const auto fetch = [&](int t, f32x4 (&a)[8], f32x4 (&c)[4]) {
+    const float* const pa = p.A + (long long)min(16 * t + m, p.M - 1) * p.lda + 4 * g;
+    #pragma unroll
+    for (int s = 0; s < 8; ++s) a[s] = *(const f32x4*)(pa + 16 * s);
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] = *(const f32x4*)(p.C + (long long)min(16 * t + 4 * g + r, p.M - 1) * p.ldc + from);
+  };
+  fetch(t, a, c);
+  for (; t < tiles; t += step) {
+    f32x4 an[8], cn[4], acc[4];
+    fetch(min(t + step, tiles - 1), an, cn);
+    __builtin_amdgcn_sched_barrier(0);                      // (or the loads move behind the products)
+    #pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    #pragma unroll
+    for (int s = 0; s < 8; ++s)
+      #pragma unroll
+      for (int e = 0; e < 4; ++e)
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][e], b[s][e][j], acc[j], 0, 0, 0);
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] -= f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+    // the next rows are waited for here, ahead of the stores: a wait behind them would be for the stores as well
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for (int s = 0; s < 8; ++s) { a[s] = an[s]; asm volatile("" : "+v"(a[s])); }
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(cn[r]));
+    __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * t + 4 * g + r;
+      if (row < p.M && col < p.N) *(f32x4*)(p.C + (long long)row * p.ldc + col) = c[r];
+    }
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) c[r] = cn[r];
+  }
+}
+
+// Contractions of 128 whose rows start on 16 bytes take the kernels above: solve C = A B^T in place (N = 128) and C -= A op(B).
+// Measured against the tiles through LDS below, the column loop's schedule with U and W from beyond L2 (us with the events around a launch):
+//   C -= A B, M x N     1000 x 128  1000 x 384  1000 x 896  4096 x 128  4096 x 384  4096 x 896  28672 x 128  28672 x 896
+//   through LDS            10.0        11.8        14.9        11.0        17.8        22.5        23.2        110.3
+//   one wave, 16 x 32       8.2         8.3        14.0         8.6        14.9        29.6        30.6        199.5
+//   stream, one wave/SIMD   9.1        10.1        13.6        10.3        14.6        19.7        19.3         72.6
+// (two streaming waves per SIMD: half as fast again).  The line between the two is 1024 tiles of 16 x 64, a stream's one tile per wave.
+// In the chain, whose launches are small or run beside the deep updates, one wave per workgroup is the best form (K = 1024: 208 us, two
+// waves 209, four 215, 64 x 64 tiles 222, streams 240; through LDS 237; K = 4096: 1148, 1157, 1176, 1193, 1245; 1257; K = 14336 9.7 ms
+// against 10.0), and 16 x 128 for a solve (32 x 128: 225 us for K = 1024).
+template <bool B_T>
+inline bool launch_rank128(const GemmProblem& g, float alpha, float beta, int flags, hipStream_t st) {
+  if (g.Kc != 128 || g.N % 4 != 0 || g.lda % 4 != 0 || g.ldb % 4 != 0 || g.ldc % 4 != 0 || (flags & (GEMM_K_FROM_N | GEMM_K_TO_M)) ||
+      (((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) & 15) != 0)
+    return false;
+  const long long tiles = (long long)((g.M + 15) / 16) * ((g.N + 63) / 64);
+  const unsigned gy = (unsigned)((g.M + 15) / 16);
+  if (B_T && alpha == 1.0f && beta == 0.0f && g.N == 128) {
+    gemm_f32_rank128_kernel<B_T, 4, false><<<dim3(1, gy), dim3(256), 0, st>>>(g, flags);
+  } else if (alpha == -1.0f && beta == 1.0f && (const float*)g.C != g.A) {
+    if (B_T || tiles <= 1024) {
+      gemm_f32_rank128_kernel<B_T, 1, true><<<dim3((unsigned)((g.N + 31) / 32), gy), dim3(64), 0, st>>>(g, flags);
+    } else {
+      const int groups = (g.N + 63) / 64, most = groups < 1024 ? 1024 / groups : 1;                    // waves per 64 columns
+      const unsigned rounds = (gy + most - 1) / most, used = (gy + rounds - 1) / rounds;
+      gemm_f32_rank128_stream_kernel<<<dim3((unsigned)(((long long)used * groups + 3) / 4)), dim3(256), 0, st>>>(g, (int)used);
+    }
+  } else {
+    return false;
+  }
+  return true;
+}
+
 template <bool B_T>
 inline void launch_gemm(const GemmProblem& g, float alpha, float beta, int flags, hipStream_t st) {
-  if (g.M <= 0 || g.N <= 0) return;
+  if (g.M <= 0 || g.N <= 0 || launch_rank128<B_T>(g, alpha, beta, flags, st)) return;
   const unsigned gx = (unsigned)((g.N + GT - 1) / GT), gy = (unsigned)((g.M + GT - 1) / GT);
   const bool split = g_gemm_split.load(std::memory_order_relaxed) != 0;
   // the bf16 pipe also pays for launches of at most one tile per CU when the contraction is long: a tile's time is

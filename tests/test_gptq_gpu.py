@@ -1211,6 +1211,29 @@ def test_owq_layer(dev, gran, n_out):
         assert torch.equal(fq[:, perm][:, :nq], want)
 
 
+@pytest.mark.parametrize('R', [1, 15, 16, 17, 100, 1200, 2600, 4100])
+@pytest.mark.parametrize('N', [4, 28, 32, 36, 64, 68, 132, 388, 896])
+def test_updates_of_depth_128(dev, R, N):
+    """W[:, j1:j1 + N] -= Err U[:128]: one wave per 16 x 32, streams beyond 1024 tiles of 16 x 64 (with and without a last round that
+    not every wave has), ragged rows and columns, and a start off the 16-byte boundary, which the general kernel takes.  Against fp64
+    with the bound of a sum of 129 terms in any order, 129 u of the terms' magnitudes; nothing else is touched."""
+    from lightcompress_amd import _lib as L
+    g = gen(9000 + R + N)
+    K = 128 + N + 12
+    E = torch.randn(R, 132, generator=g).to(dev)
+    U = torch.randn(K, K, generator=g).to(dev)
+    W0 = torch.randn(R + 3, K, generator=g).to(dev)
+    for j1 in (128, 132, 129):
+        W = W0.clone()
+        L.check(L.lib().lcq_gptq_trailing(L.ptr(W), L.ptr(E), 132, L.ptr(U), R, K, 0, 128, j1, j1 + N, L.stream()), 'trailing')
+        e, u = E.double()[:, :128], U.double()[:128, j1:j1 + N]
+        want, size = W0.double().clone(), W0.double().abs()[:R, j1:j1 + N] + e.abs() @ u.abs()
+        want[:R, j1:j1 + N] -= e @ u
+        assert float(((W.double() - want)[:R, j1:j1 + N].abs() / size).max()) <= 129 * 2.0 ** -24, j1
+        want[:R, j1:j1 + N] = W.double()[:R, j1:j1 + N]
+        assert torch.equal(W.double(), want), j1
+
+
 def test_split_gemm_has_fp32_accuracy(dev):
     """The large fp32 products run on the bf16 matrix pipe with three-way split operands (lcq_set_gemm_split, default
     on).  Against an fp64 product: the split path is as close as the fp32 pipe, for both operand layouts ([k][n] through
