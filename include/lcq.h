@@ -82,7 +82,7 @@ extern "C" {
                                     rounded zero points, |qmin|, qmax <= 256; cols % 8 == 0, 16-byte aligned) */
 #define LCQ_FLAG_SCALES_F16 32768  /* lcq_quant_int, not STATIC: `scales` is fp16: the row type's scale cast once more (scales.to(float16)) */
 #define LCQ_FLAG_RANGE_F16 8192    /* LCQ_FLAG_RANGE_BF16 for ranges that were fp16 */
-#define LCQ_FLAG_ROWS16 4096       /* lcq_gptq_block: 16 rows per workgroup whatever R is (the default takes 32 from 6144 rows on; same results bit for bit) */
+#define LCQ_FLAG_ROWS16 4096       /* lcq_gptq_block: 16 rows per workgroup where 32 would be taken (from 6144 rows on, forms that do not run by panels of 64 rows); same results bit for bit */
 #define LCQ_FLAG_ROW_QP 512       /* lcq_quant_fp_emu, STATIC only: `scales` holds one value per row */
 
 /* errors */

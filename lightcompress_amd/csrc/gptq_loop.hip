@@ -87,6 +87,17 @@ __device__ __forceinline__ ColQ make_colq(float s, float z, float qmin, float qm
   return q;
 }
 
+// scale and zero point of a group with this range
+__device__ __forceinline__ void group_params(const LoopArgs& a, float mn, float mx, float& s, float& z) {
+  if (a.sym) {
+    s = fmaxf(fmaxf(fabsf(mx), fabsf(mn)), 1e-5f) / a.qmax;
+    z = 0.0f;
+  } else {
+    s = fmaxf(mx - mn, 1e-5f) / (a.qmax - a.qmin);
+    z = a.nrz ? a.qmin - mn / s : fminf(fmaxf(a.qmin - rintf(mn / s), a.qmin), a.qmax);
+  }
+}
+
 // A group opens at column idx: scale and zero point from the range of W[row, idx : min(idx+g, K)] as it is in
 // memory now -- trailing updates of earlier blocks applied, this block's own updates not (gptq.py:216-222 reads
 // W, not W1).
@@ -107,13 +118,7 @@ __device__ __forceinline__ ColQ open_group(const LoopArgs& a, int idx, int lane,
   mn = team_reduce<16, false>(mn);
   mx = team_reduce<16, true>(mx);
   float s, z;
-  if (a.sym) {
-    s = fmaxf(fmaxf(fabsf(mx), fabsf(mn)), 1e-5f) / a.qmax;
-    z = 0.0f;
-  } else {
-    s = fmaxf(mx - mn, 1e-5f) / (a.qmax - a.qmin);
-    z = a.nrz ? a.qmin - mn / s : fminf(fmaxf(a.qmin - rintf(mn / s), a.qmin), a.qmax);
-  }
+  group_params(a, mn, mx, s, z);
   if (row_ok && lane == 0) {
     a.scales[row * a.G + idx / a.g] = s;
     if (!a.sym) a.zeros[row * a.G + idx / a.g] = z;
@@ -355,6 +360,289 @@ __global__ __launch_bounds__(16 * RW) void gptq_block_kernel(LoopArgs a) {
   }
 }
 
+// The same block for its most frequent forms: 128 whole columns, groups of 16, 32, 64 or 128 of them that open inside the block or
+// parameters that are given for groups of whole panels or rows, rounded zero points.  What the kernel above spends its time on are instructions: sixteen lanes share a row, so a column's quantization is
+// issued once per four rows, and its update takes eight multiply-adds.  Here a wave quantizes 64 rows, one per lane:
+//   * the chain wave (0) takes 16 columns from LDS and goes through them without a barrier.  A column is about nine instructions and at
+//     most four v_mfma_f32_4x4x1_16b: with ONE block of the A operand (four columns of a row of U) broadcast to all 16 (cbsz = 4, abid),
+//     an instruction updates four columns of 64 rows;
+//   * the update waves (1, 2, 3, 5) hold 16 rows each in 16 x 16 tiles, the accumulators of v_mfma_f32_16x16x4f32.  They apply the
+//     errors of a finished panel first to the next panel's columns and hand those over, then to the rest beside the chain of the next
+//     panel.  Two barriers per panel;
+//   * waves 4, 6 and 7 bring U to LDS; 6 and 7 then write the outputs of a finished panel.  The chain wave keeps its SIMD to itself: beside an update wave its products wait for
+//     the other's, 32 cycles each, and a panel takes up to 2400 cycles instead of 1200.
+// The ranges of all groups are known before the first column (groups are read from W as it is in memory).
+// Quotients go through the group's reciprocal as above.  Where a product is closer to a rounding boundary than its error can be,
+// |t| 2^-22 for |t| up to the code range + 1, the wave runs the panel again with true divisions: 1.5 % of the panels at 4 bits.
+// (The 2^-11 of the kernel above, for codes up to 1024, would be one of 1000 products.)
+// Bound by the chain: eight times 1330 cycles for its columns and 1000 for the handing over, behind 6500 for the ranges and U.
+// R = 64: 14.2 -> 12.8 us per block, 1000: 15.6 -> 13.7, 4096: 17.3 -> 14.9, 6144: 20.3 -> 16.1, 14336: 29.7 -> 21.3, 28672: 49.5 -> 31.7
+// (two workgroups per CU).  The chain wave bringing in the errors of the panel before by itself, 64 more matrix instructions, cost 700
+// cycles per panel instead of the 500 of the handing over.
+constexpr int PT = 20;           // row pitch of a 16 x 16 tile and of the panel: 16-byte rows, 16 rows of 4 lanes in different banks
+struct PanelLds {
+  float U[36][16][PT];           // tiles (p, j), j >= p, of Hinv1; zero on and below the diagonal
+  float Pn[64][PT];              // the panel on its way to the chain wave
+  float E[64][PT];               // -err of the finished panel
+  float Wq[64][PT], Dq[64][PT];  // its weights as they were quantized, and what they became
+  float Rd[BS], Dg[BS];          // 1 / U[i, i], U[i, i]
+  f32x4 pa[8][64];               // per panel and row: s, 1 / s, qmin - z, qmax - z
+  f32x2 pb[8][64];               // z, distance from a rounding boundary that is enough
+};
+__device__ __forceinline__ constexpr int panel_tile(int p, int j) { return 8 * p - p * (p - 1) / 2 + j - p; }
+
+// c + a b over 16 of the contraction, k = 4 (l / 16) + e in instruction e
+__device__ __forceinline__ f32x4 panel_mac(const f32x4& a, const f32x4& b, f32x4 c) {
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+  return c;
+}
+// columns 16 j .. of the rows of U that belong to panel p, as the first operand
+__device__ __forceinline__ f32x4 panel_u(const PanelLds& s, int p, int j, int m, int g) {
+  f32x4 v;
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = s.U[panel_tile(p, j)][4 * g + e][m];
+  return v;
+}
+
+// the 16 columns of a panel, in order: w -> as quantized, dq: quantized and back, e = -err.  EXACT: true divisions.  Returns the smallest distance of a product
+// from a rounding boundary.
+template <bool EXACT>
+__device__ __forceinline__ float panel_chain(const LoopArgs& a, f32x4 (&w)[4], float (&dq)[16], float (&e)[16], const float (&u)[16], const f32x4 (&nrd)[4],
+                                             const f32x4& pa, float z) {
+  float margin = 0.5f;
+  #pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float x = w[j >> 2][j & 3];
+    if (EXACT) {
+      const float code = rintf(x / pa[0]) + z;
+      dq[j] = (__builtin_amdgcn_fmed3f(code, a.qmin, a.qmax) - z) * pa[0];
+    } else {
+      const float t = x * pa[1], rt = rintf(t);
+      margin = nan_min(margin, fabsf(fabsf(t - rt) - 0.5f));
+      dq[j] = __builtin_amdgcn_fmed3f(rt, pa[2], pa[3]) * pa[0];
+    }
+    e[j] = (x - dq[j]) * nrd[j >> 2][j & 3];
+    // U is zero up to the column itself: what has been quantized stays as it was
+    if (j < 3) w[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[0], 4, 0, 0);
+    if (j < 7) w[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[1], 4, 1, 0);
+    if (j < 11) w[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[2], 4, 2, 0);
+    if (j < 15) w[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[3], 4, 3, 0);
+  }
+  return margin;
+}
+
+__global__ __launch_bounds__(512) void gptq_panel_kernel(LoopArgs a) {
+  __shared__ __align__(16) PanelLds s;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  const int id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int last = 8;
+  asm volatile("" : "+s"(last));                            // (or the loops over the panels are unrolled, and wait for instruction fetches)
+  if (id == 4 || id >= 6) {
+    // rows of panels 0, 5, 7 / 1, 4, 6 / 2, 3 of Hinv1: 12, 13 and 11 tiles, all loads in flight
+    const int p0 = id == 4 ? 0 : id - 5, p1 = 5 - p0, p2 = p0 == 2 ? 8 : 7 - p0, n0 = 8 - p0, n1 = n0 + 8 - p1;
+    const int panels = p0 | p1 << 4 | p2 << 8, starts = n0 << 4 | n1 << 8;    // (nibbles instead of selects: those became memory)
+    const int r = lane >> 2, c = 4 * (lane & 3);
+    f32x4 v[13];
+    const auto tile_of = [=](int q, int& p, int& j) {
+      const int at = 4 * ((q >= n0) + (q >= n1));
+      p = (panels >> at) & 15;
+      j = p + q - ((starts >> at) & 15);
+      return p < 8 && j < 8;
+    };
+    #pragma unroll
+    for (int q = 0; q < 13; ++q) {
+      int p, j;
+      if (!tile_of(q, p, j)) p = j = 7;
+      v[q] = *(const f32x4*)(a.U + (long long)(a.i1 + 16 * p + r) * a.K + a.i1 + 16 * j + c);
+    }
+    #pragma unroll
+    for (int q = 0; q < 13; ++q) {
+      int p, j;
+      if (!tile_of(q, p, j)) continue;
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) v[q][e] = p == j && c + e <= r ? 0.0f : v[q][e];
+      *(f32x4*)(s.U[panel_tile(p, j)][r] + c) = v[q];
+    }
+    __syncthreads();
+    if (id == 4) return;
+    // waves 6 and 7: the outputs of panel P - 1 beside the chain of panel P, two tiles of 16 rows each
+    long long at[2], to[2];
+    bool row_ok[2];
+    #pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const long long row = (long long)blockIdx.x * 64 + 32 * (id - 6) + 16 * h + m;
+      row_ok[h] = row < a.R;
+      at[h] = (row_ok[h] ? row : a.R - 1) * a.K + a.i1 + 4 * g;
+      to[h] = row * a.ldErr + 4 * g;
+    }
+    const auto fetch = [&](int Q, f32x4 (&w0)[2]) __attribute__((always_inline)) {
+      if (a.W0)
+        #pragma unroll
+        for (int h = 0; h < 2; ++h) w0[h] = *(const f32x4*)(a.W0 + at[h] + 16 * Q);
+    };
+    const auto outputs = [&](int Q, const f32x4 (&w0)[2]) __attribute__((always_inline)) {
+      const int col = 16 * Q;
+      const f32x4 rd = *(const f32x4*)(s.Rd + col + 4 * g), d = *(const f32x4*)(s.Dg + col + 4 * g);
+      #pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = 32 * (id - 6) + 16 * h + m;
+        const f32x4 wq = *(const f32x4*)(s.Wq[row] + 4 * g), dq = *(const f32x4*)(s.Dq[row] + 4 * g);
+        f32x4 out, loss;
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float diff = wq[e] - dq[e];
+          out[e] = a.W0 ? dq[e] - w0[h][e] : diff * rd[e];
+          loss[e] = (diff * diff) / (2.0f * (d[e] * d[e]));
+        }
+        if (row_ok[h]) {
+          *(f32x4*)(a.tmp + at[h] + col) = wq;
+          *(f32x4*)(a.Losses + at[h] + col) = loss;
+          *(f32x4*)(a.Err + to[h] + col) = out;
+        }
+      }
+    };
+    // W0 comes a panel or two ahead, into registers of its own for even and odd panels: a copy of them would wait for the loads, and
+    // for the stores in front of them, before the barrier
+    f32x4 even[2] = {}, odd[2] = {};
+    fetch(0, even);
+    #pragma unroll 1
+    for (int P = 0; P < last; P += 2) {
+      if (P > 0) outputs(P - 1, odd);
+      fetch(P + 1, odd);
+      __syncthreads();
+      __syncthreads();                                      // panel P is done
+      outputs(P, even);
+      if (P < 6) fetch(P + 2, even);
+      __syncthreads();
+      __syncthreads();
+    }
+    outputs(7, odd);
+    return;
+  }
+  if (id == 0) {
+    #pragma unroll
+    for (int c = lane; c < BS; c += 64) {
+      const float d = a.U[(long long)(a.i1 + c) * a.K + a.i1 + c];
+      s.Dg[c] = d;
+      s.Rd[c] = 1.0f / d;
+    }
+    __syncthreads();
+    f32x4 pa = {1.0f, 1.0f, 0.0f, 0.0f}, nrd[4];
+    f32x2 pb = {0.0f, 0.0f};
+    float u[16], dq[16], e[16];
+    const auto fetch = [&](int P) {
+      #pragma unroll
+      for (int j = 0; j < 16; ++j) u[j] = s.U[panel_tile(P, P)][j][m];
+      #pragma unroll
+      for (int b = 0; b < 4; ++b) nrd[b] = -*(const f32x4*)(s.Rd + 16 * P + 4 * b);
+      pa = s.pa[P][lane];
+      pb = s.pb[P][lane];
+    };
+    fetch(0);
+    #pragma unroll 1
+    for (int P = 0; P < last; ++P) {
+      f32x4 w[4], kept[4];
+      #pragma unroll
+      for (int b = 0; b < 4; ++b) kept[b] = w[b] = *(const f32x4*)(s.Pn[lane] + 4 * b);
+      const bool unsure = !(panel_chain<false>(a, w, dq, e, u, nrd, pa, pb[0]) > pb[1]);
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(unsure) != 0, 0)) {
+        #pragma unroll
+        for (int b = 0; b < 4; ++b) w[b] = kept[b];
+        panel_chain<true>(a, w, dq, e, u, nrd, pa, pb[0]);
+      }
+      #pragma unroll
+      for (int b = 0; b < 4; ++b) *(f32x4*)(s.E[lane] + 4 * b) = f32x4{e[4 * b], e[4 * b + 1], e[4 * b + 2], e[4 * b + 3]};
+      __syncthreads();                                      // E holds panel P
+      // beside the handing over
+      #pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        *(f32x4*)(s.Wq[lane] + 4 * b) = w[b];
+        *(f32x4*)(s.Dq[lane] + 4 * b) = f32x4{dq[4 * b], dq[4 * b + 1], dq[4 * b + 2], dq[4 * b + 3]};
+      }
+      if (P < 7) fetch(P + 1);
+      __syncthreads();                                      // Wq and Dq hold panel P, Pn panel P + 1
+    }
+    return;
+  }
+
+  const int wave = id == 5 ? 0 : id;
+  const long long row = (long long)blockIdx.x * 64 + 16 * wave + m;
+  const bool row_ok = row < a.R;
+  const long long at = (row_ok ? row : a.R - 1) * a.K + a.i1;
+  // tile j of this wave's 16 rows, transposed: lane element e is row m, column 16 j + 4 g + e
+  f32x4 t[8];
+  #pragma unroll
+  for (int j = 0; j < 8; ++j) t[j] = *(const f32x4*)(a.W + at + 16 * j + 4 * g);
+  *(f32x4*)(s.Pn[16 * wave + m] + 4 * g) = t[0];
+  {
+    // ranges of the groups: over a lane's elements, its tiles, and the four lanes of a row
+    const int gt = a.is_static ? 1 : a.g >> 4, sh = 31 - __builtin_clz(gt);   // panels per group, a power of two
+    float mn[8], mx[8], sc = 1.0f, z = 0.0f, mine[2] = {}, zero[2] = {};      // a lane's parameters are those of panels g and g + 4
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      mn[j] = nan_min(nan_min(t[j][0], t[j][1]), nan_min(t[j][2], t[j][3]));
+      mx[j] = nan_max(nan_max(t[j][0], t[j][1]), nan_max(t[j][2], t[j][3]));
+    }
+    #pragma unroll
+    for (int span = 1; span < 8; span *= 2)
+      if (span < gt)
+        #pragma unroll
+        for (int j = 0; j < 8; j += 2 * span) { mn[j] = nan_min(mn[j], mn[j + span]); mx[j] = nan_max(mx[j], mx[j + span]); }
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (a.is_static) {
+        const long long from = (row_ok ? row : a.R - 1) * a.G + (a.g > 0 ? (a.i1 + 16 * j) / a.g : 0);
+        sc = a.scales[from];
+        z = a.sym ? 0.0f : a.zeros[from];
+      } else if ((j & (gt - 1)) == 0) {
+        float lo = nan_min(mn[j], lane_xor<16>(mn[j])), hi = nan_max(mx[j], lane_xor<16>(mx[j]));
+        lo = nan_min(lo, lane_xor<32>(lo));
+        hi = nan_max(hi, lane_xor<32>(hi));
+        group_params(a, lo, hi, sc, z);
+        if (g == 0 && row_ok) {
+          const long long to = row * a.G + (a.i1 >> 4 >> sh) + (j >> sh);
+          a.scales[to] = sc;
+          if (!a.sym) a.zeros[to] = z;
+        }
+      }
+      mine[j >> 2] = g == (j & 3) ? sc : mine[j >> 2];
+      zero[j >> 2] = g == (j & 3) ? z : zero[j >> 2];
+    }
+    #pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const ColQ q = make_colq(mine[h], zero[h], a.qmin, a.qmax);
+      s.pa[4 * h + g][16 * wave + m] = f32x4{q.s, q.r, q.lo, q.hi};
+      s.pb[4 * h + g][16 * wave + m] = f32x2{q.z, q.fast ? (fmaxf(fabsf(q.lo), fabsf(q.hi)) + 1.0f) * 4.76837158e-7f : __builtin_inff()};
+    }
+  }
+  __syncthreads();                                          // U, the first panel and the parameters
+  #pragma unroll
+  for (int k = 0; k < 7; ++k) t[k] = t[k + 1];              // from here on t[0] is the panel after the one in the chain
+  f32x4 err = {0.0f, 0.0f, 0.0f, 0.0f};
+  #pragma unroll 1
+  for (int P = 0; P < last; ++P) {
+    f32x4 u[6], next = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (P < 7) next = panel_u(s, P, P + 1, m, g);
+    if (P > 0) {                                            // panel P - 1 on the tiles behind
+      #pragma unroll
+      for (int k = 0; k < 6; ++k) u[k] = panel_u(s, P - 1, min(P + 1 + k, 7), m, g);
+      #pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (k < 7 - P) t[k] = panel_mac(u[k], err, t[k]);
+    }
+    __syncthreads();                                        // E holds panel P
+    err = *(const f32x4*)(s.E[16 * wave + m] + 4 * g);
+    if (P < 7) {
+      t[0] = panel_mac(next, err, t[0]);
+      *(f32x4*)(s.Pn[16 * wave + m] + 4 * g) = t[0];
+    }
+    __syncthreads();                                        // Wq and Dq hold panel P, Pn panel P + 1
+    #pragma unroll
+    for (int k = 0; k < 6; ++k) t[k] = t[k + 1];
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -380,7 +668,16 @@ int lcq_gptq_block(float* W, float* tmp, float* Losses, float* Err, int64_t ldEr
                 reinterpret_cast<uintptr_t>(U)) & 15) == 0;
   const bool oct = !is_static && group_size % 8 == 0 && i1 % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
-  // From 6144 rows on, 32 rows per workgroup: one copy of Hinv1 in LDS (70 KB) per eight waves, so that the two
+  const bool whole = is_static ? !gidx && (group_size <= 0 || group_size % 16 == 0)
+                               : group_size == 16 || group_size == 32 || group_size == 64 || group_size == BS;
+  const bool panels = whole && !a.nrz && count == BS && i1 % BS == 0 && K % 4 == 0 && a.aligned && ldErr % 4 == 0 &&
+                      (((uintptr_t)Err | (uintptr_t)W0) & 15) == 0;
+  if (panels) {
+    gptq_panel_kernel<<<dim3((unsigned)((R + 63) / 64)), dim3(512), 0, st>>>(a);
+    LCQ_CHECK_LAUNCH();
+    return LCQ_OK;
+  }
+  // The other forms.  From 6144 rows on, 32 rows per workgroup: one copy of Hinv1 in LDS (70 KB) per eight waves, so that the two
   // workgroups a CU holds put four waves on every SIMD (R = 28672: 57 -> 48 us per block, 14336: 35 -> 29, 6144:
   // 20 -> 19; at 4096 rows, one workgroup per CU either way, the smaller workgroup is faster, 17 against 19 us).
   // The rows do not interact: the results are the same bit for bit.

@@ -1593,3 +1593,65 @@ def test_block_kernel_workgroup_shapes_agree(dev, R, mode):
     for a, b in zip(*outs):
         assert torch.equal(a, b)
     assert float(outs[0][1].sum()) > 0 and bool(torch.isfinite(outs[0][2]).all())
+
+
+@pytest.mark.parametrize('R', [1, 15, 16, 17, 63, 64, 65, 130])
+@pytest.mark.parametrize('g', [16, 32, 64, 128])
+@pytest.mark.parametrize('sym,factor', [(False, False), (True, True)])
+def test_panels_of_whole_blocks(dev, R, g, sym, factor):
+    """lcq_gptq_block on 128 whole columns with groups that open inside the block: scales and zero points are those of the ranges in
+    W, every weight is quantized by the reference's expressions from the value it has then (products near a rounding boundary, exact
+    halves, an infinity and a NaN among them), its error or Q - W0 and its loss follow bit for bit, and what it is then is
+    W - sum_k err_k U[k, :] up to the roundings of that sum (k of them on its largest magnitude).  Nothing else is written."""
+    from lightcompress_amd import _lib as L
+    K, i1 = 384, 128
+    G, qmin, qmax = K // g, (-8.0 if sym else 0.0), (7.0 if sym else 15.0)
+    U = (torch.triu(torch.randn(K, K, generator=gen(11)) * 0.05) + torch.eye(K) * 1.5).to(dev)
+    W0 = (torch.randn(R, K, generator=gen(12)) * 0.05).to(dev)
+    W = W0 + 0.01
+    W[0, i1:i1 + 128] = (torch.arange(128, device=dev) % 16 - 8) * 0.5         # a range of 7.5: scale 0.5, or halves of 0.536
+    if R > 16:
+        W[3, i1 + 40], W[16, i1 + 100] = float('inf'), float('nan')
+    tmp, Lo = torch.full_like(W, 7.0), torch.full_like(W, 7.0)
+    Err = torch.full((R, 132), 7.0, device=dev)
+    sc, ze = torch.full((R, G), 7.0, device=dev), torch.full((R, G), 7.0, device=dev)
+    before = W.clone()
+    L.check(L.lib().lcq_gptq_block(L.ptr(W), L.ptr(tmp), L.ptr(Lo), L.ptr(Err), 132, L.ptr(U), L.ptr(W0) if factor else None, R, K, K, i1,
+                                   128, g, L.f32(qmin), L.f32(qmax), L.FLAG_SYM if sym else 0, L.ptr(sc), L.ptr(ze), None, G, L.stream()),
+            'block')
+    assert torch.equal(W.nan_to_num(5.0, 6.0), before.nan_to_num(5.0, 6.0))
+    same = lambda a, b: torch.equal(a.nan_to_num(123.0, 1e30, -1e30), b.nan_to_num(123.0, 1e30, -1e30))
+    d = torch.diag(U)[i1:i1 + 128]
+    t, ranges = tmp[:, i1:i1 + 128], W[:, i1:i1 + 128].view(R, 128 // g, g)
+    mn, mx = ranges.amin(-1), ranges.amax(-1)
+    tiny = torch.tensor(1e-5, device=dev)
+    if sym:
+        s = torch.maximum(mn.abs(), mx.abs()).clamp(min=1e-5) / torch.tensor(qmax, device=dev)
+        z = torch.zeros_like(s)
+    else:
+        s = (mx - mn).clamp(min=1e-5) / torch.tensor(qmax - qmin, device=dev)
+        z = (qmin - torch.round(mn / s)).clamp(qmin, qmax)
+    plain = torch.isfinite(mn) & torch.isfinite(mx)
+    got_s, got_z = sc[:, i1 // g:(i1 + 128) // g], ze[:, i1 // g:(i1 + 128) // g]
+    assert torch.equal(got_s[plain], s[plain]) and (sym or torch.equal(got_z[plain], z[plain]))
+    assert bool((sc[:, :i1 // g] == 7).all() and (sc[:, (i1 + 128) // g:] == 7).all())
+    se, zeros = got_s.repeat_interleave(g, 1), (torch.zeros_like(got_s) if sym else got_z).repeat_interleave(g, 1)
+    dq = ((torch.round(t / se) + zeros).clamp(qmin, qmax) - zeros) * se
+    ok = torch.isfinite(t).all(1) & plain.all(1)                                # rows without the infinity or the NaN
+    assert int(ok.sum()) >= R - 2
+    diff = t - dq
+    want = dq - W0[:, i1:i1 + 128] if factor else diff * (torch.ones((), device=dev) / d)
+    assert same(Err[ok][:, :128], want[ok]) and bool((Err[:, 128:] == 7).all())
+    assert same(Lo[:, i1:i1 + 128][ok], ((diff * diff) / (2.0 * (d * d)))[ok])
+    for x in (tmp, Lo):
+        assert bool((x[:, :i1] == 7).all() and (x[:, i1 + 128:] == 7).all())
+    e = (diff * (torch.ones((), device=dev) / d)).double()
+    B = torch.triu(U[i1:i1 + 128, i1:i1 + 128], 1).double()
+    exact, size = W[:, i1:i1 + 128].double() - e @ B, W[:, i1:i1 + 128].abs().double() + e.abs() @ B.abs()
+    assert bool(((t.double() - exact).abs() <= 129 * 2.0 ** -24 * size)[ok].all())
+    # the same parameters as given ones: the same results
+    t2, L2, E2 = torch.full_like(W, 7.0), torch.full_like(W, 7.0), torch.full_like(Err, 7.0)
+    L.check(L.lib().lcq_gptq_block(L.ptr(W), L.ptr(t2), L.ptr(L2), L.ptr(E2), 132, L.ptr(U), L.ptr(W0) if factor else None, R, K, K, i1,
+                                   128, g, L.f32(qmin), L.f32(qmax), L.FLAG_STATIC | (L.FLAG_SYM if sym else 0), L.ptr(sc), L.ptr(ze), None,
+                                   G, L.stream()), 'block')
+    assert same(t2, tmp) and same(L2, Lo) and same(E2, Err)
