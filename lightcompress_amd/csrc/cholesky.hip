@@ -200,20 +200,20 @@ __global__ __launch_bounds__(256) void build_gather_kernel(const float* __restri
 //   * the update waves (1, 2, 3, 5) hold the lower triangle behind in 16 x 16 tiles, the accumulators of v_mfma_f32_16x16x4f32
 //     (wave u tile rows u and 7 - u).  They apply a finished panel first to the next panel's columns, hand those over, and do the
 //     rest of the update while the panel waves are factoring (a right-looking update with look-ahead; two barriers per panel).
-//   * They also build the inverse X block row by block row beside the panels: T_Pj = sum_k L_Pk X_kj waits in the accumulators
-//     for the inverse of panel P's block, X_Pj = -X_PP T_Pj goes to memory (and LDS, for the rows below) one panel later.  Behind
-//     the last panel only X_7j is left.
+//   * They also build the inverse beside the panels, a column block j per wave and half: X_Pj = -X_PP T_Pj goes to memory, and from the
+//     registers it is in to the rows below, T_rj += L_rP X_Pj: products that do not wait for one another.  Behind the last
+//     panel only X_7j is left.  (T of a row summed up when its turn comes, one chain of up to 28 products: 1.5 us more per block.)
 // Contractions take k = 4 (l / 16) + i in instruction i, so an operand is one 16-byte read of a row and an accumulator is the B
 // operand of the next product as it stands.  The panels and tiles hold -A, so that updates add.
-// Bound by the serial chain of one wave's instructions: 14.3 us per block (26.4 us with updates of 8 x 8 values per thread, 240
+// Bound by the serial chain of one wave's instructions: 12.5 us per block (26.4 us with updates of 8 x 8 values per thread, 240
 // v_readlane / v_fma per panel and the inverse by three levels of merges at the end).
 constexpr int LP = NB + 4;       // row pitch of the LDS matrices (16-byte aligned rows, 4-bank skew)
 constexpr int PP = 16 + 4;       // row pitch of the panel
 
 struct PotrfLds {
   float L[NB][LP];       // L row-major, below the 16 x 16 diagonal blocks
-  float XT[NB][LP];      // XT[c][r] = X(r, c), X = L^-1: the tiles on and below its diagonal
-  float Pn[NB][PP];      // - the panel on its way to the panel waves
+  float XT[8][16][PP];   // the inverted diagonal blocks, transposed: XT[i][c][r] = X(16 i + r, 16 i + c), X = L^-1
+  float Pn[NB + 16][PP]; // - the panel on its way to the panel waves, and behind it - the identity
 };
 
 __device__ __forceinline__ float rdlane(float v, int l) {
@@ -228,13 +228,10 @@ __device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int w, int lane,
   const int behind = NB - 16 * P - 16;                      // rows behind the panel's own
   const int q = lane - 16 + 48 * w;                         // this lane's row among those and the identity's
   const bool own = lane < 16, rest = !own && q < behind, unit = !own && q >= behind && q < behind + 16;
-  const float* const from = s.Pn[own ? 16 * P + lane : rest ? 16 * P + 16 + q : 16 * P];
-  const int one = own || rest ? -1 : q - behind;            // where a row of the identity has its one
+  const float* const from = s.Pn[own ? 16 * P + lane : 16 * P + 16 + q];        // (the identity follows row 127)
   f32x4 n[4];
   #pragma unroll
-  for (int b = 0; b < 4; ++b) n[b] = *(const f32x4*)(from + 4 * b);
-  #pragma unroll
-  for (int j = 0; j < 16; ++j) n[j >> 2][j & 3] = own || rest ? n[j >> 2][j & 3] : j == one ? -1.0f : 0.0f;
+  for (int b = 0; b < 4; ++b) n[b] = *(const f32x4*)((own || rest || unit ? from : s.Pn[0]) + 4 * b);
   f32x4 l[4];
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
@@ -250,7 +247,7 @@ __device__ __forceinline__ void potrf_panel(PotrfLds& s, int P, int w, int lane,
     if (j < 15) n[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, v, n[3], 4, 3, 0);
   }
   if (rest || unit) {
-    float* const to = rest ? &s.L[16 * P + 16 + q][16 * P] : &s.XT[16 * P + q - behind][16 * P];
+    float* const to = rest ? &s.L[16 * P + 16 + q][16 * P] : s.XT[P][q - behind];
     #pragma unroll
     for (int b = 0; b < 4; ++b) *(f32x4*)(to + 4 * b) = l[b];
   }
@@ -263,73 +260,70 @@ __device__ __forceinline__ f32x4 potrf_mac(const f32x4& a, const f32x4& b, f32x4
   return c;
 }
 
-// What an update wave holds.  Tile (i, j), transposed: lane l element e is row 16 i + l % 16, column 16 j + 4 (l / 16) + e.
-// t[0]: tile row u (tiles 0 .. 3 at most), t[1]: tile row 7 - u.
-struct PotrfTiles { f32x4 top[4], bottom[8]; };
+// What an update wave holds: tile rows u (`top`) and 7 - u (`bottom`), tile (i, j) transposed: lane element e is row 16 i + l % 16, column
+// 16 j + 4 (l / 16) + e; and what the rows below still lack of column blocks u and 7 - u of the inverse, T[.][r] = sum L_rk X_kj.
+struct PotrfTiles { f32x4 top[4], bottom[8], T[2][8]; };
 
-// the columns of panel J to the panel waves (J, the panel in front of it applied already)
+// the columns of panel J to the panel waves
 template <int J>
 __device__ __forceinline__ void potrf_publish(PotrfLds& s, const PotrfTiles& t, int u, int m, int g) {
   if constexpr (J < 4) { if (u >= J) *(f32x4*)(s.Pn[16 * u + m] + 4 * g) = t.top[J]; }
   if (7 - u >= J) *(f32x4*)(s.Pn[16 * (7 - u) + m] + 4 * g) = t.bottom[J];
 }
 
-// panel P on tile columns LO .. HI
-template <int P, int LO, int HI>
-__device__ __forceinline__ void potrf_update(const PotrfLds& s, PotrfTiles& t, int u, int m, int g) {
-  if constexpr (LO <= HI) {
-    if (7 - u < LO) return;
-    const f32x4 hi = *(const f32x4*)(s.L[16 * (7 - u) + m] + 16 * P + 4 * g);
-    const f32x4 lo = *(const f32x4*)(s.L[16 * u + m] + 16 * P + 4 * g);       // (read only where u > P)
-    #pragma unroll
-    for (int j = LO; j <= HI; ++j) {
-      if (j > 7 - u) continue;
-      const f32x4 a = *(const f32x4*)(s.L[16 * j + m] + 16 * P + 4 * g);
-      t.bottom[j] = potrf_mac(a, hi, t.bottom[j]);
-      if (j < 4 && j <= u) t.top[j & 3] = potrf_mac(a, lo, t.top[j & 3]);
-    }
-  }
-}
-
-// Column block j of the inverse, beside panel P: X_ij of tile row i = P - 1, whose own block has been inverted, then T of row P.
-template <int P>
-__device__ __forceinline__ void potrf_inverse(PotrfLds& s, f32x4& T, int j, int nb, float* __restrict__ Dinv, int m, int g) {
-  constexpr int I = P - 1;
+// Column block j of the inverse, beside panel I + 1: X_Ij of tile row I, whose own block has been inverted, and its part in the rows below
+// (l[r]: row r of L's panel I, as the first operand).
+template <int I>
+__device__ __forceinline__ void potrf_inverse(const PotrfLds& s, f32x4 (&T)[8], int j, const f32x4 (&x)[2], const f32x4 (&l)[8], int nb,
+                                              float* __restrict__ Dinv, int m, int g) {
   if (I < j) return;
-  f32x4 x;                                                  // X_II(m, 4 g + e)
-  #pragma unroll
-  for (int e = 0; e < 4; ++e) x[e] = s.XT[16 * I + 4 * g + e][16 * I + m];
+  f32x4 v;                                                  // X_Ij: rows 4 g + e, column m
   if (I == j) {
+    v = x[1];
     #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = (16 * I + m < nb && 16 * I + 4 * g + e < nb) ? x[e] : 0.0f;   // (the padding's diagonal)
-    *(f32x4*)(Dinv + (16 * I + m) * NB + 16 * I + 4 * g) = x;
+    for (int r = I + 1; r < 8; ++r) T[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   } else {
-    f32x4 v = potrf_mac(x, T, f32x4{0.0f, 0.0f, 0.0f, 0.0f});                 // rows 4 g + e, column m
-    v = -v;
-    if constexpr (P < 8) *(f32x4*)(s.XT[16 * j + m] + 16 * I + 4 * g) = v;
-    #pragma unroll
-    for (int e = 0; e < 4; ++e) Dinv[(16 * I + 4 * g + e) * NB + 16 * j + m] = v[e];
+    v = -potrf_mac(x[0], T[I], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
   }
-  if constexpr (P < 8) {
-    T = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  #pragma unroll
+  for (int e = 0; e < 4; ++e)                               // (the padding's diagonal is no part of the inverse)
+    Dinv[(16 * I + 4 * g + e) * NB + 16 * j + m] = 16 * I + 4 * g + e < nb ? v[e] : 0.0f;
+  #pragma unroll
+  for (int e = 0; e < 4; ++e)
     #pragma unroll
-    for (int k = 0; k < P; ++k)
-      if (k >= j) T = potrf_mac(*(const f32x4*)(s.L[16 * P + m] + 16 * k + 4 * g), *(const f32x4*)(s.XT[16 * j + m] + 16 * k + 4 * g), T);
-  }
+    for (int r = I + 1; r < 8; ++r) T[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(l[r][e], v[e], T[r], 0, 0, 0);
 }
 
-// what an update wave does beside panel P and behind it
+// what an update wave does with panel P once that is complete, but for the next panel's columns
 template <int P>
-__device__ __forceinline__ void potrf_phase(PotrfLds& s, PotrfTiles& t, f32x4 (&T)[2], int u, int nb, float* __restrict__ Dinv, int m, int g) {
-  __syncthreads();                                          // Pn holds panel P; L and the inverted blocks up to panel P - 1
-  if constexpr (P > 0) {
-    potrf_update<P - 1, P + 1, 7>(s, t, u, m, g);
-    potrf_inverse<P>(s, T[0], u, nb, Dinv, m, g);
-    potrf_inverse<P>(s, T[1], 7 - u, nb, Dinv, m, g);
+__device__ __forceinline__ void potrf_rest(const PotrfLds& s, PotrfTiles& t, int u, int nb, float* __restrict__ Dinv, int m, int g) {
+  f32x4 l[8], x[2];                                         // rows of L's panel P; X_PP(m, 4 g + e) and X_PP(4 g + e, m)
+  #pragma unroll
+  for (int r = P + 1; r < 8; ++r) l[r] = *(const f32x4*)(s.L[16 * r + m] + 16 * P + 4 * g);
+  const f32x4 hi = *(const f32x4*)(s.L[16 * (7 - u) + m] + 16 * P + 4 * g);
+  const f32x4 lo = *(const f32x4*)(s.L[16 * u + m] + 16 * P + 4 * g);         // (used only where u > P)
+  #pragma unroll
+  for (int e = 0; e < 4; ++e) x[0][e] = s.XT[P][4 * g + e][m];
+  x[1] = *(const f32x4*)(s.XT[P][m] + 4 * g);
+  #pragma unroll
+  for (int j = P + 2; j < 8; ++j) {
+    if (j <= 7 - u) t.bottom[j] = potrf_mac(l[j], hi, t.bottom[j]);
+    if (j < 4 && j <= u) t.top[j & 3] = potrf_mac(l[j], lo, t.top[j & 3]);
   }
-  __syncthreads();                                          // L of panel P is complete
+  potrf_inverse<P>(s, t.T[0], u, x, l, nb, Dinv, m, g);
+  potrf_inverse<P>(s, t.T[1], 7 - u, x, l, nb, Dinv, m, g);
+}
+
+template <int P>
+__device__ __forceinline__ void potrf_phase(PotrfLds& s, PotrfTiles& t, int u, int nb, float* __restrict__ Dinv, int m, int g) {
+  __syncthreads();                                          // Pn holds panel P
+  if constexpr (P > 0) potrf_rest<P - 1>(s, t, u, nb, Dinv, m, g);
+  __syncthreads();                                          // L of panel P and its inverted block are complete
   if constexpr (P < 7) {
-    potrf_update<P, P + 1, P + 1>(s, t, u, m, g);
+    const f32x4 a = *(const f32x4*)(s.L[16 * (P + 1) + m] + 16 * P + 4 * g);
+    const f32x4 hi = *(const f32x4*)(s.L[16 * (7 - u) + m] + 16 * P + 4 * g), lo = *(const f32x4*)(s.L[16 * u + m] + 16 * P + 4 * g);
+    if (P + 1 <= 7 - u) t.bottom[P + 1] = potrf_mac(a, hi, t.bottom[P + 1]);
+    if constexpr (P < 3) { if (P + 1 <= u) t.top[P + 1] = potrf_mac(a, lo, t.top[P + 1]); }
     potrf_publish<P + 1>(s, t, u, m, g);
   }
 }
@@ -339,6 +333,8 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(const float* __restrict
   __shared__ __align__(16) PotrfLds s;
   const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int panels = 8;
+  asm volatile("" : "+s"(panels));                          // (or the loops over the panels are unrolled, and wait for instruction fetches)
   if (wave == 0 || wave == 4 || wave >= 6) {
     if (wave == 0) {                                        // the tiles above the diagonal are zeros
       for (int r = 0; r < NB - 16; r += 2) {
@@ -346,9 +342,14 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(const float* __restrict
         if (c4 >= (row & ~15) + 16) *(f32x4*)(Dinv + row * NB + c4) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       }
     }
+    if (wave == 6) {
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) s.Pn[NB + m][4 * g + e] = 4 * g + e == m ? -1.0f : 0.0f;
+    }
     float least = __builtin_inff();
     const int w = wave == 0 ? 3 : wave == 4 ? 0 : wave - 5;                   // wave 0 has no rows: NB <= 3 x 48
-    for (int P = 0; P < 8; ++P) {
+    #pragma unroll 1
+    for (int P = 0; P < panels; ++P) {
       __syncthreads();
       if (48 * w < NB - 16 * P) potrf_panel(s, P, w, lane, least);
       __syncthreads();
@@ -356,16 +357,18 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(const float* __restrict
     if (wave == 4 && lane == 0 && !(least > 0.0f)) sc->status = 1;
     return;
   }
-  const int u = wave == 5 ? 0 : wave;
+  // the busiest first, on the SIMD that panels leave first; the two that share one are among the others (u in the order 5, 1, 2, 3:
+  // 1 us more per block)
+  const int u = wave == 3 ? 0 : wave == 1 ? 1 : wave == 5 ? 2 : 3;
   PotrfTiles t;
   // a whole block: plain loads, all in flight (those above the diagonal are never used)
   if (nb == NB && lda % 4 == 0 && ((uintptr_t)Ablk & 15) == 0) {
-    const float* const top = Ablk + (long long)(16 * u + m) * lda + 4 * g;
-    const float* const bottom = Ablk + (long long)(16 * (7 - u) + m) * lda + 4 * g;
+    const float* const pt = Ablk + (long long)(16 * u + m) * lda + 4 * g;
+    const float* const pb = Ablk + (long long)(16 * (7 - u) + m) * lda + 4 * g;
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if (j < 4) t.top[j & 3] = *(const f32x4*)(top + 16 * j);
-      t.bottom[j] = *(const f32x4*)(bottom + 16 * j);
+      if (j < 4) t.top[j & 3] = *(const f32x4*)(pt + 16 * j);
+      t.bottom[j] = *(const f32x4*)(pb + 16 * j);
     }
   } else {
     const auto load = [&](int i, int j, f32x4& v) {
@@ -387,17 +390,15 @@ __global__ __launch_bounds__(512) void potrf_diag_kernel(const float* __restrict
       t.bottom[j][e] = (j < 7 - u || 4 * g + e <= m) ? -t.bottom[j][e] : 0.0f;
     }
   potrf_publish<0>(s, t, u, m, g);
-  f32x4 T[2];
-  potrf_phase<0>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<1>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<2>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<3>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<4>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<5>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<6>(s, t, T, u, nb, Dinv, m, g);
-  potrf_phase<7>(s, t, T, u, nb, Dinv, m, g);
-  potrf_inverse<8>(s, T[0], u, nb, Dinv, m, g);
-  potrf_inverse<8>(s, T[1], 7 - u, nb, Dinv, m, g);
+  potrf_phase<0>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<1>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<2>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<3>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<4>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<5>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<6>(s, t, u, nb, Dinv, m, g);
+  potrf_phase<7>(s, t, u, nb, Dinv, m, g);
+  potrf_rest<7>(s, t, u, nb, Dinv, m, g);
   // (L itself is not written back: everything after this kernel works with the inverse, the solved panels and the
   // blocks behind them; place_diag_kernel puts the inverse where the block was.)
 }
