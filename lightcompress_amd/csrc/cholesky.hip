@@ -116,28 +116,61 @@ __global__ __launch_bounds__(256) void prepare_w_vec_kernel(const u32x4* __restr
     for (int i = 0; i < N; i += 4) out[at * (N / 4) + i / 4] = f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
   }
 }
+// Row-major data to LDS, 16 bytes per thread and eight loads in flight (one load at a time is a memory latency per 16 bytes and thread).
+template <int THREADS>
+__device__ __forceinline__ void rows_to_lds(void* to, const void* from, long long nbytes) {
+  if ((((uintptr_t)from) & 15) != 0) {
+    for (long long i = threadIdx.x; i < nbytes; i += THREADS) ((unsigned char*)to)[i] = ((const unsigned char*)from)[i];
+    return;
+  }
+  const int n16 = (int)(nbytes >> 4);
+  int i0 = threadIdx.x;
+  for (; i0 + 7 * THREADS < n16; i0 += 8 * THREADS) {
+    u32x4 v[8];
+    #pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = ((const u32x4*)from)[i0 + k * THREADS];
+    #pragma unroll
+    for (int k = 0; k < 8; ++k) ((u32x4*)to)[i0 + k * THREADS] = v[k];
+  }
+  for (; i0 < n16; i0 += 2 * THREADS) {
+    const bool two = i0 + THREADS < n16;
+    const u32x4 v = ((const u32x4*)from)[i0], w = ((const u32x4*)from)[two ? i0 + THREADS : i0];
+    ((u32x4*)to)[i0] = v;
+    if (two) ((u32x4*)to)[i0 + THREADS] = w;
+  }
+  for (long long i = ((long long)n16 << 4) + threadIdx.x; i < nbytes; i += THREADS) ((unsigned char*)to)[i] = ((const unsigned char*)from)[i];
+}
+
 // The same with a permutation: a gather inside every row.  From memory that is one 64-byte sector per element; here
-// the workgroup's rows (`rows` of them, as many as fit 64 KB) come in as they lie, 16 bytes per lane, and the gather
-// reads LDS.  The permutation is read once per workgroup and column.
+// the workgroup's rows (`rows` of them, as many as fit 64 KB) come in as they lie, and the gather reads LDS, four columns per thread
+// where K allows it.  The permutation is read once per workgroup and column.
+// HBM-bound: 14336 x 4096 bf16 91 -> 68 us, 4096 x 14336 fp32 251 -> 110 (one load in flight per thread and 4-byte stores before).
 template <int DT>
-__global__ __launch_bounds__(256) void prepare_w_gather_kernel(const void* __restrict__ w, long long R, int K, int rows,
+__global__ __launch_bounds__(512) void prepare_w_gather_kernel(const void* __restrict__ w, long long R, int K, int rows,
                                                                const long long* __restrict__ perm,
                                                                const uint8_t* __restrict__ dead, float* __restrict__ out) {
   extern __shared__ __align__(16) unsigned char staged[];
   constexpr int ES = DT == LCQ_F32 ? 4 : 2;
   const long long row0 = (long long)blockIdx.x * rows;
   const int n = (int)((R - row0 < rows) ? (R - row0) : rows);
-  const long long nbytes = (long long)n * K * ES;
-  const unsigned char* src = (const unsigned char*)w + row0 * K * ES;
-  if ((((uintptr_t)src) & 15) == 0) {
-    const long long n16 = nbytes >> 4;
-    for (long long i = threadIdx.x; i < n16; i += 256) ((u32x4*)staged)[i] = ((const u32x4*)src)[i];
-    for (long long i = (n16 << 4) + threadIdx.x; i < nbytes; i += 256) staged[i] = src[i];
-  } else {
-    for (long long i = threadIdx.x; i < nbytes; i += 256) staged[i] = src[i];
-  }
+  rows_to_lds<512>(staged, (const unsigned char*)w + row0 * K * ES, (long long)n * K * ES);
   __syncthreads();
-  for (int j = threadIdx.x; j < K; j += 256) {
+  if (K % 4 == 0 && (((uintptr_t)out) & 15) == 0) {
+    for (int j = 4 * threadIdx.x; j < K; j += 2048) {
+      int c[4];
+      bool dz[4];
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) { c[e] = (int)perm[j + e]; dz[e] = dead && dead[c[e]]; }
+      for (int r = 0; r < n; ++r) {
+        f32x4 v;
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) { const float x = load_w<DT>(staged, (long long)(r * K + c[e])); v[e] = dz[e] ? 0.0f : x; }
+        *(f32x4*)(out + (row0 + r) * K + j) = v;
+      }
+    }
+    return;
+  }
+  for (int j = threadIdx.x; j < K; j += 512) {
     const long long c = perm[j];
     const bool dz = dead && dead[c];
     for (int r = 0; r < n; ++r) {
@@ -167,19 +200,43 @@ __global__ __launch_bounds__(256) void build_kernel(const float* __restrict__ H,
 // The same from a fully symmetric H and with a permutation: row a of A draws on row perm[K-1-a] of H only, which
 // comes in as it lies (16 bytes per lane) and is gathered from LDS.  (Picking H[min][max] from memory, as build_kernel
 // does, walks down a column of H for half of the entries: one 64-byte sector per element.)
-__global__ __launch_bounds__(256) void build_gather_kernel(const float* __restrict__ H, int K, const long long* __restrict__ perm,
+// HBM-bound: K = 14336 666 -> 355 us (one load in flight, the permutation read behind the row, 4-byte stores before); 4096 23 as before.
+__global__ __launch_bounds__(512) void build_gather_kernel(const float* __restrict__ H, int K, const long long* __restrict__ perm,
                                                            const PrepScalars* __restrict__ sc, float* __restrict__ A) {
   extern __shared__ __align__(16) float hrow[];
   const int a = blockIdx.x;
-  const float* src = H + perm[K - 1 - a] * (long long)K;
-  if ((((uintptr_t)src) & 15) == 0 && (K & 3) == 0) {
-    for (int i = threadIdx.x; i < (K >> 2); i += 256) ((f32x4*)hrow)[i] = ((const f32x4*)src)[i];
-  } else {
-    for (int i = threadIdx.x; i < K; i += 256) hrow[i] = src[i];
-  }
-  __syncthreads();
   const float damp = sc->damp;
-  for (int b = threadIdx.x; b < K; b += 256) {
+  if (K % 4 == 0) {
+    // the permutation of all of a thread's columns (K <= 16384) while the row is on its way
+    int c[8][4];
+    #pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int b = 4 * threadIdx.x + 2048 * q;
+      if (b < K && b <= a)
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) c[q][e] = (int)perm[K - 1 - b - e];
+    }
+    rows_to_lds<512>(hrow, H + perm[K - 1 - a] * (long long)K, 4ll * K);
+    __syncthreads();
+    #pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int b = 4 * threadIdx.x + 2048 * q;
+      if (b < K) {
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (b <= a)
+          #pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float h = hrow[c[q][e]];                  // (columns past the diagonal too: every entry of perm is one of H)
+            v[e] = b + e < a ? h : b + e == a ? h + damp : 0.0f;
+          }
+        *(f32x4*)(A + (long long)a * K + b) = v;
+      }
+    }
+    return;
+  }
+  rows_to_lds<512>(hrow, H + perm[K - 1 - a] * (long long)K, 4ll * K);
+  __syncthreads();
+  for (int b = threadIdx.x; b < K; b += 512) {
     float v = 0.0f;
     if (b <= a) {
       v = hrow[perm[K - 1 - b]];
@@ -414,16 +471,34 @@ __global__ __launch_bounds__(256) void place_diag_kernel(float* __restrict__ A, 
   }
 }
 
-// U[i][j] = Linv[K-1-i][K-1-j].  With `Dinv` (K in whole blocks) the diagonal blocks come from there.
+// U[i][j] = Linv[K-1-i][K-1-j], zeros below the diagonal.  With `Dinv` (K in whole blocks) the diagonal blocks come from there.
+// V: four columns per thread (K a multiple of 4, U on 16 bytes): K = 14336 412 -> 187 us,
+// 4096 28 -> 16, which workgroups of 256 single elements took to start.
+template <bool V>
 __global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ Linv, int K, const float* __restrict__ Dinv,
                                                       float* __restrict__ U) {
-  const int i = blockIdx.y;
-  const int j = blockIdx.x * 256 + threadIdx.x;
+  const int i = blockIdx.y, a = K - 1 - i;
+  const int j = (blockIdx.x * 256 + threadIdx.x) * (V ? 4 : 1);
   if (j >= K) return;
-  const int a = K - 1 - i, b = K - 1 - j;
-  float v = 0.0f;
-  if (j >= i) v = (Dinv && a / NB == b / NB) ? Dinv[(long long)a * NB + b % NB] : Linv[(long long)a * K + b];
-  U[(long long)i * K + j] = v;
+  if constexpr (V) {
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (j + 3 >= i) {
+      const int b = K - 4 - j;                              // columns b .. b + 3, the last one first
+      const f32x4 x = *(const f32x4*)(Dinv && a / NB == b / NB ? Dinv + (long long)a * NB + b % NB : Linv + (long long)a * K + b);
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = j + e >= i ? x[3 - e] : 0.0f;
+    }
+    *(f32x4*)(U + (long long)i * K + j) = v;
+  } else {
+    const int b = K - 1 - j;
+    float v = 0.0f;
+    if (j >= i) v = (Dinv && a / NB == b / NB) ? Dinv[(long long)a * NB + b % NB] : Linv[(long long)a * K + b];
+    U[(long long)i * K + j] = v;
+  }
+}
+static void launch_scatter(const float* Linv, int K, const float* Dinv, float* U, hipStream_t st) {
+  if (K % 4 == 0 && ((uintptr_t)U & 15) == 0) scatter_kernel<true><<<dim3((unsigned)((K + 1023) / 1024), (unsigned)K), dim3(256), 0, st>>>(Linv, K, Dinv, U);
+  else scatter_kernel<false><<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(Linv, K, Dinv, U);
 }
 
 }  // namespace
@@ -459,9 +534,9 @@ int lcq_gptq_prepare_weights(const void* w, int dtype, int64_t R, int64_t K, con
     const int64_t g = (R + rows - 1) / rows;
     if (g > 0x7fffffff) return LCQ_EINVAL;
     const size_t lds = (size_t)rows * K * es;
-    if (dtype == LCQ_F32) prepare_w_gather_kernel<LCQ_F32><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
-    else if (dtype == LCQ_BF16) prepare_w_gather_kernel<LCQ_BF16><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
-    else prepare_w_gather_kernel<LCQ_F16><<<dim3((unsigned)g), dim3(256), lds, st>>>(w, R, (int)K, rows, p, dead, out);
+    if (dtype == LCQ_F32) prepare_w_gather_kernel<LCQ_F32><<<dim3((unsigned)g), dim3(512), lds, st>>>(w, R, (int)K, rows, p, dead, out);
+    else if (dtype == LCQ_BF16) prepare_w_gather_kernel<LCQ_BF16><<<dim3((unsigned)g), dim3(512), lds, st>>>(w, R, (int)K, rows, p, dead, out);
+    else prepare_w_gather_kernel<LCQ_F16><<<dim3((unsigned)g), dim3(512), lds, st>>>(w, R, (int)K, rows, p, dead, out);
   }
   else if (!p && K % 8 == 0 && K <= (1 << 28) && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 15) == 0 &&
            (dtype == LCQ_F32 || dtype == LCQ_BF16 || dtype == LCQ_F16)) {
@@ -525,7 +600,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   }
   if (perm && K <= 16384) {                       // a row of H fits the 64 KB of LDS a workgroup may ask for
     if (lcq_symmetrize(H, K, stream) != LCQ_OK) return LCQ_ELAUNCH;
-    build_gather_kernel<<<dim3((unsigned)K), dim3(256), (size_t)K * 4, st>>>(H, K, (const long long*)perm, sc, A);
+    build_gather_kernel<<<dim3((unsigned)K), dim3(512), (size_t)K * 4, st>>>(H, K, (const long long*)perm, sc, A);
   } else {
     build_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(H, K, (const long long*)perm, sc, A);
   }
@@ -621,7 +696,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
       else if (tm == 64) gemm_f32_batched_kernel<false, 64, true><<<grid, dim3(256), 0, st>>>(A, K, Dinv, NB, A, K, bt, 1.0f, 0.0f, 0);
       else gemm_f32_batched_kernel<false><<<grid, dim3(256), 0, st>>>(A, K, Dinv, NB, A, K, bt, 1.0f, 0.0f, 0);
     }
-    scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, Dinv, U);
+    launch_scatter(A, K, Dinv, U, st);
     if (status)
       (void)hipMemcpyAsync(status, &sc->status, sizeof(int), hipMemcpyDeviceToDevice, st);
     LCQ_CHECK_LAUNCH();
@@ -673,7 +748,7 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
     nseg = w;
   }
 
-  scatter_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(A, K, nullptr, U);
+  launch_scatter(A, K, nullptr, U, st);
   if (status)
     (void)hipMemcpyAsync(status, &sc->status, sizeof(int), hipMemcpyDeviceToDevice, st);
   LCQ_CHECK_LAUNCH();

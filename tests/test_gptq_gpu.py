@@ -531,6 +531,46 @@ def test_prepare_weights_without_a_permutation(dev, dtype, R, K):
             assert float(out[R * K + 1]) == 7.0
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('R,K', [(1, 4), (3, 6), (9, 1000), (7, 1001), (33, 2056), (5, 2048), (2, 9000), (3, 16384)])
+def test_prepare_weights_with_a_permutation(dev, dtype, R, K):
+    """The fp32 copy with its columns permuted: four columns per thread or one, whole and partial staging loops, weights off a
+    16-byte boundary, outputs off one, dead columns."""
+    from lightcompress_amd import _lib as L
+    perm = torch.randperm(K, generator=gen(K)).to(dev)
+    dead = torch.rand(K, generator=gen(K + 1)).to(dev) < 0.3
+    for woff, ooff in ((0, 0), (1, 0), (0, 1)):
+        w = torch.randn(R * K + 1, generator=gen(R + K)).to(dtype).to(dev)[woff:woff + R * K].view(R, K)
+        for d in (None, dead):
+            want = w.float()
+            if d is not None:
+                want[:, d] = 0.0
+            out = torch.full((R * K + 2,), 7.0, device=dev)
+            got = out[ooff:ooff + R * K].view(R, K)
+            L.check(L.lib().lcq_gptq_prepare_weights(L.ptr(w), L.dtype_code(dtype), R, K, L.ptr(perm),
+                                                     None if d is None else d.data_ptr(), L.ptr(got), L.stream()), 'prepare')
+            assert torch.equal(got, want[:, perm])
+            assert float(out[R * K + 1]) == 7.0
+
+
+@pytest.mark.parametrize('K', [3, 5, 128, 131, 516, 2052, 2304])
+def test_chain_with_a_permutation_is_that_of_the_permuted_matrix(dev, K):
+    """Without damping (whose mean would be summed in another order) the factor of H[perm][:, perm] is the same bits whether the chain
+    permutes or the caller does."""
+    from lightcompress_amd import _lib as L
+    x = torch.randn(2 * K, K, generator=gen(5300 + K), dtype=torch.float64)
+    H = (x.t() @ x / K + torch.eye(K, dtype=torch.float64)).float().to(dev)
+    perm = torch.randperm(K, generator=gen(K)).to(dev)
+    nbytes = L.lib().lcq_chol_inv_upper_workspace_bytes(K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    out = []
+    for h, p in ((H, perm), (H[perm][:, perm], None)):
+        hd, U = torch.triu(h).contiguous(), torch.full((K, K), 7.0, device=dev)
+        L.check(L.lib().lcq_chol_inv_upper(L.ptr(hd), K, L.ptr(p), 0.0, None, 0, L.ptr(U), L.ptr(ws), nbytes, None, L.stream()), 'chain')
+        out.append(U)
+    assert torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize('K', [1, 15, 16, 17, 31, 48, 65, 97, 112, 113, 127, 128, 129, 131, 257])
 def test_diagonal_blocks_of_every_fill(dev, K):
     """One to three diagonal blocks whose last is filled to either side of a 16-column panel, of the 48 rows a wave takes and of
