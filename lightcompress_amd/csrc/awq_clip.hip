@@ -434,7 +434,7 @@ __global__ __launch_bounds__(512, 2) void clip_search_kernel(const uint16_t* __r
 // CLIP_SMALL where underflow might count, or near the 1e9 the search starts from) have every step evaluated.
 // Measured (an MLP's Linears as above, all three without errors, 10 steps): 25.7 -> 17.9 ms; 3.7 of 10 steps are evaluated (5.6 without the
 // first step ahead of the others: 21.0 ms; a second and a third step by itself: 19.2, 20.7, a pass costs its tiles however few rows
-// it still has), the matrix pipes are busy in 58 % of the cycles (the making of the versions, estimates and decisions are not
+// it still has), the matrix pipes are busy in 45 % of the cycles (the making of the versions, estimates and decisions are not
 // overlapped by another workgroup: one fills the LDS).  One step at a time in the estimates, and decisions by a single wave: 1.6 ms
 // more.  Four waves per SIMD, tokens read as they are used so that 128 registers hold it: 23.0 against 21.0 ms, the conversions of
 // two waves already fill the vector pipe beside the products.
