@@ -406,15 +406,20 @@ __device__ __forceinline__ f32x4 panel_u(const PanelLds& s, int p, int j, int m,
 }
 
 // the 16 columns of a panel, in order: w -> as quantized, dq: quantized and back, e = -err.  EXACT: true divisions.  Returns the smallest distance of a product
-// from a rounding boundary.
+// from a rounding boundary, NaN if a product was not finite.
+// An update covers four columns, and U is zero up to the column itself: what has been quantized stays as it was while the errors are
+// finite.  Zero times an infinite or NaN error is NaN, in the finished columns of the four as well as in those behind, whose products then
+// are NaN: such panels run again, and EXACT keeps every column as it found it.
 template <bool EXACT>
 __device__ __forceinline__ float panel_chain(const LoopArgs& a, f32x4 (&w)[4], float (&dq)[16], float (&e)[16], const float (&u)[16], const f32x4 (&nrd)[4],
                                              const f32x4& pa, float z) {
   float margin = 0.5f;
+  f32x4 found[4];
   #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const float x = w[j >> 2][j & 3];
     if (EXACT) {
+      found[j >> 2][j & 3] = x;
       const float code = rintf(x / pa[0]) + z;
       dq[j] = (__builtin_amdgcn_fmed3f(code, a.qmin, a.qmax) - z) * pa[0];
     } else {
@@ -423,11 +428,14 @@ __device__ __forceinline__ float panel_chain(const LoopArgs& a, f32x4 (&w)[4], f
       dq[j] = __builtin_amdgcn_fmed3f(rt, pa[2], pa[3]) * pa[0];
     }
     e[j] = (x - dq[j]) * nrd[j >> 2][j & 3];
-    // U is zero up to the column itself: what has been quantized stays as it was
     if (j < 3) w[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[0], 4, 0, 0);
     if (j < 7) w[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[1], 4, 1, 0);
     if (j < 11) w[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[2], 4, 2, 0);
     if (j < 15) w[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(u[j], e[j], w[3], 4, 3, 0);
+  }
+  if (EXACT) {
+    #pragma unroll
+    for (int b = 0; b < 4; ++b) w[b] = found[b];
   }
   return margin;
 }

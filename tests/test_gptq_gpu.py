@@ -1695,3 +1695,37 @@ def test_panels_of_whole_blocks(dev, R, g, sym, factor):
                                    128, g, L.f32(qmin), L.f32(qmax), L.FLAG_STATIC | (L.FLAG_SYM if sym else 0), L.ptr(sc), L.ptr(ze), None,
                                    G, L.stream()), 'block')
     assert same(t2, tmp) and same(L2, Lo) and same(E2, Err)
+
+
+@pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
+@pytest.mark.parametrize('at', [0, 1, 42, 63, 64, 126, 127])
+@pytest.mark.parametrize('static', [False, True])
+def test_a_weight_that_is_not_finite_stays_behind_the_columns_in_front(dev, value, at, static):
+    """One infinite or NaN weight among 128 whole columns (lcq_gptq_block by panels): a column's record, error and loss are what they
+    were when its turn came, so the columns in front of the first error that is not finite are those of a run without that weight, bit
+    for bit, the weight's own record is the weight, and no other row knows of it.  With searched ranges of 16 columns that error may
+    be the first of the weight's group, whose scale the weight decides."""
+    from lightcompress_amd import _lib as L
+    R, K, i1, g, row = 70, 256, 128, 16, 66
+    G = K // g
+    U = (torch.triu(torch.randn(K, K, generator=gen(31)) * 0.05) + torch.eye(K) * 1.5).to(dev)
+    plain = (torch.randn(R, K, generator=gen(32)) * 0.05).to(dev)
+    hurt = plain.clone()
+    hurt[row, i1 + at] = value
+    out = []
+    for W in (plain, hurt):
+        tmp, Lo, Err = torch.zeros_like(W), torch.zeros_like(W), torch.zeros(R, 128, device=dev)
+        sc, ze = torch.full((R, G), 0.01, device=dev), torch.full((R, G), 8.0, device=dev)
+        L.check(L.lib().lcq_gptq_block(L.ptr(W), L.ptr(tmp), L.ptr(Lo), L.ptr(Err), 128, L.ptr(U), None, R, K, K, i1, 128, g, L.f32(0.0),
+                                       L.f32(15.0), L.FLAG_STATIC if static else 0, L.ptr(sc), L.ptr(ze), None, G, L.stream()), 'block')
+        out.append((tmp[:, i1:].cpu(), Lo[:, i1:].cpu(), Err.cpu()))
+    front = at if static else at // g * g
+    for a, b in zip(*out):
+        assert torch.equal(a[:row], b[:row]) and torch.equal(a[row + 1:], b[row + 1:])
+        assert torch.equal(a[row, :front], b[row, :front])
+    a, b = out[0][0][row], out[1][0][row]
+    if static:
+        assert torch.equal(b[at:at + 1].nan_to_num(5.0, 6.0, 7.0), hurt[row, i1 + at].cpu().view(1).nan_to_num(5.0, 6.0, 7.0))
+        assert not bool(torch.isfinite(b[at + 1:]).any())
+    elif front < at:
+        assert float(b[front]) == float(a[front])
