@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "launch_rules.h"
 
 namespace lcq {
 
@@ -672,22 +673,19 @@ inline bool launch_rank128(const GemmProblem& g, float alpha, float beta, int fl
   if (g.Kc != 128 || g.N % 4 != 0 || g.lda % 4 != 0 || g.ldb % 4 != 0 || g.ldc % 4 != 0 || (flags & (GEMM_K_FROM_N | GEMM_K_TO_M)) ||
       (((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) & 15) != 0)
     return false;
-  const long long tiles = (long long)((g.M + 15) / 16) * ((g.N + 63) / 64);
   const unsigned gy = (unsigned)((g.M + 15) / 16);
-  if (B_T && alpha == 1.0f && beta == 0.0f && g.N == 128) {
-    gemm_f32_rank128_kernel<B_T, 4, false><<<dim3(1, gy), dim3(256), 0, st>>>(g, flags);
-  } else if (alpha == -1.0f && beta == 1.0f && (const float*)g.C != g.A) {
-    if (B_T || tiles <= 1024) {
-      gemm_f32_rank128_kernel<B_T, 1, true><<<dim3((unsigned)((g.N + 31) / 32), gy), dim3(64), 0, st>>>(g, flags);
-    } else {
+  switch (rank128_form(B_T, g.M, g.N, alpha, beta, (const float*)g.C == g.A, (flags & GEMM_LOWER_TILES) != 0)) {
+    case Rank128::none: return false;
+    case Rank128::solve: gemm_f32_rank128_kernel<B_T, 4, false><<<dim3(1, gy), dim3(256), 0, st>>>(g, flags); return true;
+    case Rank128::waves: gemm_f32_rank128_kernel<B_T, 1, true><<<dim3((unsigned)((g.N + 31) / 32), gy), dim3(64), 0, st>>>(g, flags); return true;
+    case Rank128::stream: {
       const int groups = (g.N + 63) / 64, most = groups < 1024 ? 1024 / groups : 1;                    // waves per 64 columns
       const unsigned rounds = (gy + most - 1) / most, used = (gy + rounds - 1) / rounds;
       gemm_f32_rank128_stream_kernel<<<dim3((unsigned)(((long long)used * groups + 3) / 4)), dim3(256), 0, st>>>(g, (int)used);
+      return true;
     }
-  } else {
-    return false;
   }
-  return true;
+  return false;
 }
 
 template <bool B_T>
