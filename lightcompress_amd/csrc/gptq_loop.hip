@@ -39,6 +39,7 @@
 
 #include "gemm_f32.h"
 #include "gemm_s3p.h"
+#include "launch_rules.h"
 #include "lcq_internal.h"
 
 namespace {
@@ -676,11 +677,8 @@ int lcq_gptq_block(float* W, float* tmp, float* Losses, float* Err, int64_t ldEr
                 reinterpret_cast<uintptr_t>(U)) & 15) == 0;
   const bool oct = !is_static && group_size % 8 == 0 && i1 % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
-  const bool whole = is_static ? !gidx && (group_size <= 0 || group_size % 16 == 0)
-                               : group_size == 16 || group_size == 32 || group_size == 64 || group_size == BS;
-  const bool panels = whole && !a.nrz && count == BS && i1 % BS == 0 && K % 4 == 0 && a.aligned && ldErr % 4 == 0 &&
-                      (((uintptr_t)Err | (uintptr_t)W0) & 15) == 0;
-  if (panels) {
+  const bool on16 = a.aligned && (((uintptr_t)Err | (uintptr_t)W0) & 15) == 0;
+  if (gptq_by_panels(is_static, gidx != nullptr, !a.nrz, group_size, R, K, i1, count, ldErr, on16, qmin, qmax)) {
     gptq_panel_kernel<<<dim3((unsigned)((R + 63) / 64)), dim3(512), 0, st>>>(a);
     LCQ_CHECK_LAUNCH();
     return LCQ_OK;
