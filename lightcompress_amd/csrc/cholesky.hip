@@ -23,6 +23,7 @@
 //                  blocks: [[A,0],[B,C]]^-1 = [[A^-1,0],[-C^-1 B A^-1, C^-1]]
 //   scatter        U[i][j] = Linv[K-1-i][K-1-j], j >= i; zeros below the diagonal
 #include <mutex>
+#include <type_traits>
 #include "gemm_f32.h"
 #include "gemm_s3p.h"
 #include "lcq_internal.h"
@@ -116,29 +117,31 @@ __global__ __launch_bounds__(256) void prepare_w_vec_kernel(const u32x4* __restr
     for (int i = 0; i < N; i += 4) out[at * (N / 4) + i / 4] = f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
   }
 }
-// Row-major data to LDS, 16 bytes per thread and eight loads in flight (one load at a time is a memory latency per 16 bytes and thread).
-template <int THREADS>
-__device__ __forceinline__ void rows_to_lds(void* to, const void* from, long long nbytes) {
-  if ((((uintptr_t)from) & 15) != 0) {
-    for (long long i = threadIdx.x; i < nbytes; i += THREADS) ((unsigned char*)to)[i] = ((const unsigned char*)from)[i];
-    return;
-  }
-  const int n16 = (int)(nbytes >> 4);
+// `n` pieces to LDS, eight loads in flight per thread (one load at a time is a memory latency per piece and thread).
+template <int THREADS, class V>
+__device__ __forceinline__ void pieces_to_lds(V* to, const V* from, int n) {
   int i0 = threadIdx.x;
-  for (; i0 + 7 * THREADS < n16; i0 += 8 * THREADS) {
-    u32x4 v[8];
+  for (; i0 + 7 * THREADS < n; i0 += 8 * THREADS) {
+    V v[8];
     #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = ((const u32x4*)from)[i0 + k * THREADS];
+    for (int k = 0; k < 8; ++k) v[k] = from[i0 + k * THREADS];
     #pragma unroll
-    for (int k = 0; k < 8; ++k) ((u32x4*)to)[i0 + k * THREADS] = v[k];
+    for (int k = 0; k < 8; ++k) to[i0 + k * THREADS] = v[k];
   }
-  for (; i0 < n16; i0 += 2 * THREADS) {
-    const bool two = i0 + THREADS < n16;
-    const u32x4 v = ((const u32x4*)from)[i0], w = ((const u32x4*)from)[two ? i0 + THREADS : i0];
-    ((u32x4*)to)[i0] = v;
-    if (two) ((u32x4*)to)[i0 + THREADS] = w;
+  for (; i0 < n; i0 += 2 * THREADS) {
+    const bool two = i0 + THREADS < n;
+    const V v = from[i0], w = from[two ? i0 + THREADS : i0];
+    to[i0] = v;
+    if (two) to[i0 + THREADS] = w;
   }
-  for (long long i = ((long long)n16 << 4) + threadIdx.x; i < nbytes; i += THREADS) ((unsigned char*)to)[i] = ((const unsigned char*)from)[i];
+}
+// Row-major elements to LDS (`to` on 16 bytes): 16 bytes per thread, or element by element where they do not start on 16 bytes.
+template <int THREADS, class E>
+__device__ __forceinline__ void rows_to_lds(E* to, const E* from, int n) {
+  if ((((uintptr_t)from) & 15) != 0) { pieces_to_lds<THREADS>(to, from, n); return; }
+  constexpr int PER = 16 / (int)sizeof(E);
+  pieces_to_lds<THREADS>((u32x4*)to, (const u32x4*)from, n / PER);
+  for (int i = n / PER * PER + threadIdx.x; i < n; i += THREADS) to[i] = from[i];
 }
 
 // The same with a permutation: a gather inside every row.  From memory that is one 64-byte sector per element; here
@@ -150,10 +153,10 @@ __global__ __launch_bounds__(512) void prepare_w_gather_kernel(const void* __res
                                                                const long long* __restrict__ perm,
                                                                const uint8_t* __restrict__ dead, float* __restrict__ out) {
   extern __shared__ __align__(16) unsigned char staged[];
-  constexpr int ES = DT == LCQ_F32 ? 4 : 2;
+  typedef typename std::conditional<DT == LCQ_F32, float, uint16_t>::type Element;
   const long long row0 = (long long)blockIdx.x * rows;
   const int n = (int)((R - row0 < rows) ? (R - row0) : rows);
-  rows_to_lds<512>(staged, (const unsigned char*)w + row0 * K * ES, (long long)n * K * ES);
+  rows_to_lds<512>((Element*)staged, (const Element*)w + row0 * K, n * K);
   __syncthreads();
   if (K % 4 == 0 && (((uintptr_t)out) & 15) == 0) {
     for (int j = 4 * threadIdx.x; j < K; j += 2048) {
@@ -200,27 +203,40 @@ __global__ __launch_bounds__(256) void build_kernel(const float* __restrict__ H,
 // The same from a fully symmetric H and with a permutation: row a of A draws on row perm[K-1-a] of H only, which
 // comes in as it lies (16 bytes per lane) and is gathered from LDS.  (Picking H[min][max] from memory, as build_kernel
 // does, walks down a column of H for half of the entries: one 64-byte sector per element.)
-// HBM-bound: K = 14336 666 -> 355 us (one load in flight, the permutation read behind the row, 4-byte stores before); 4096 23 as before.
-__global__ __launch_bounds__(512) void build_gather_kernel(const float* __restrict__ H, int K, const long long* __restrict__ perm,
-                                                           const PrepScalars* __restrict__ sc, float* __restrict__ A) {
+// HBM-bound at large K: K = 14336 567 -> 298 us, 8192 121 -> 96, 4096 22.0 -> 18.5, 2048 10.3 -> 7.8, 1280 6.5 -> 6.0 (256 threads, one load in flight, the
+// permutation read behind the row and 4-byte stores before; kernel traces).
+// V: K a multiple of 4, at most 4 Q THREADS, and H on 16 bytes: a thread's pieces of the row and its columns of the permutation are all in flight (the
+// permutation first: it waits for nothing), no more threads or columns than a row has.  (512 threads for 16384 columns, whatever K: 7.6 us at 1280, 15.3 at
+// 3000, where 6.5 and 13.9 were taken before.)  Otherwise a column per thread, Q of the permutation in flight, rows that may start off 16 bytes, then
+// staged by 4: K = 2047 8.9 us (9.0 before; 15.3 staged byte by byte), 4095 24.4 (24.4; 41), 14335 406 (1040; 700).
+template <bool V, int THREADS, int Q>
+__global__ __launch_bounds__(THREADS) void build_gather_kernel(const float* __restrict__ H, int K, const long long* __restrict__ perm,
+                                                               const PrepScalars* __restrict__ sc, float* __restrict__ A) {
   extern __shared__ __align__(16) float hrow[];
   const int a = blockIdx.x;
   const float damp = sc->damp;
-  if (K % 4 == 0) {
-    // the permutation of all of a thread's columns (K <= 16384) while the row is on its way
-    int c[8][4];
+  if constexpr (V) {
+    int c[Q][4];
     #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int b = 4 * threadIdx.x + 2048 * q;
+    for (int q = 0; q < Q; ++q) {
+      const int b = 4 * (threadIdx.x + THREADS * q);
       if (b < K && b <= a)
         #pragma unroll
         for (int e = 0; e < 4; ++e) c[q][e] = (int)perm[K - 1 - b - e];
     }
-    rows_to_lds<512>(hrow, H + perm[K - 1 - a] * (long long)K, 4ll * K);
+    const float* const row = H + perm[K - 1 - a] * (long long)K;
+    f32x4 piece[Q];
+    #pragma unroll
+    for (int q = 0; q < Q; ++q) piece[q] = *(const f32x4*)(row + min(4 * (int)(threadIdx.x + THREADS * q), K - 4));
+    #pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int b = 4 * (threadIdx.x + THREADS * q);
+      if (b < K) *(f32x4*)(hrow + b) = piece[q];
+    }
     __syncthreads();
     #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int b = 4 * threadIdx.x + 2048 * q;
+    for (int q = 0; q < Q; ++q) {
+      const int b = 4 * (threadIdx.x + THREADS * q);
       if (b < K) {
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (b <= a)
@@ -232,18 +248,37 @@ __global__ __launch_bounds__(512) void build_gather_kernel(const float* __restri
         *(f32x4*)(A + (long long)a * K + b) = v;
       }
     }
-    return;
-  }
-  rows_to_lds<512>(hrow, H + perm[K - 1 - a] * (long long)K, 4ll * K);
-  __syncthreads();
-  for (int b = threadIdx.x; b < K; b += 512) {
-    float v = 0.0f;
-    if (b <= a) {
-      v = hrow[perm[K - 1 - b]];
-      if (a == b) v += damp;
+  } else {
+    rows_to_lds<THREADS>(hrow, H + perm[K - 1 - a] * (long long)K, K);
+    __syncthreads();
+    for (int b0 = threadIdx.x; b0 < K; b0 += Q * THREADS) {
+      int c[Q];
+      #pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int b = b0 + THREADS * q;
+        if (b < K && b <= a) c[q] = (int)perm[K - 1 - b];
+      }
+      #pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int b = b0 + THREADS * q;
+        if (b < K) A[(long long)a * K + b] = b > a ? 0.0f : b == a ? hrow[c[q]] + damp : hrow[c[q]];
+      }
     }
-    A[(long long)a * K + b] = v;
   }
+}
+// K <= 16384: a row of H fits the 64 KB of LDS a workgroup may ask for
+static void launch_build_gather(const float* H, int K, const long long* perm, const PrepScalars* sc, float* A, hipStream_t st) {
+  const dim3 grid((unsigned)K);
+  const size_t lds = (size_t)K * 4;
+  if (K % 4 != 0 || ((uintptr_t)H & 15) != 0) {
+    if (K <= 4096) build_gather_kernel<false, 256, 4><<<grid, dim3(256), lds, st>>>(H, K, perm, sc, A);
+    else build_gather_kernel<false, 512, 4><<<grid, dim3(512), lds, st>>>(H, K, perm, sc, A);
+  }
+  else if (K <= 1024) build_gather_kernel<true, 256, 1><<<grid, dim3(256), lds, st>>>(H, K, perm, sc, A);
+  else if (K <= 2048) build_gather_kernel<true, 256, 2><<<grid, dim3(256), lds, st>>>(H, K, perm, sc, A);
+  else if (K <= 4096) build_gather_kernel<true, 512, 2><<<grid, dim3(512), lds, st>>>(H, K, perm, sc, A);
+  else if (K <= 8192) build_gather_kernel<true, 512, 4><<<grid, dim3(512), lds, st>>>(H, K, perm, sc, A);
+  else build_gather_kernel<true, 512, 8><<<grid, dim3(512), lds, st>>>(H, K, perm, sc, A);
 }
 
 // Diagonal block: Cholesky factor L11 of a 128x128 block and the inverse of L11, one workgroup of 8 waves.
@@ -598,9 +633,9 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
     if (g > 65536) g = 65536;
     apply_dead_kernel<<<dim3((unsigned)g), dim3(256), 0, st>>>(W, R, K, dead);
   }
-  if (perm && K <= 16384) {                       // a row of H fits the 64 KB of LDS a workgroup may ask for
+  if (perm && K <= 16384) {
     if (lcq_symmetrize(H, K, stream) != LCQ_OK) return LCQ_ELAUNCH;
-    build_gather_kernel<<<dim3((unsigned)K), dim3(512), (size_t)K * 4, st>>>(H, K, (const long long*)perm, sc, A);
+    launch_build_gather(H, K, (const long long*)perm, sc, A, st);
   } else {
     build_kernel<<<dim3((unsigned)((K + 255) / 256), (unsigned)K), dim3(256), 0, st>>>(H, K, (const long long*)perm, sc, A);
   }

@@ -553,22 +553,26 @@ def test_prepare_weights_with_a_permutation(dev, dtype, R, K):
             assert float(out[R * K + 1]) == 7.0
 
 
-@pytest.mark.parametrize('K', [3, 5, 128, 131, 516, 2052, 2304])
+@pytest.mark.parametrize('K', [3, 5, 128, 131, 516, 1024, 1028, 2048, 2050, 2052, 2304, 4096, 4097, 4100, 8192, 8196])
 def test_chain_with_a_permutation_is_that_of_the_permuted_matrix(dev, K):
     """Without damping (whose mean would be summed in another order) the factor of H[perm][:, perm] is the same bits whether the chain
-    permutes or the caller does."""
+    permutes or the caller does (K and H on and off 16 bytes, every number of columns per thread and its edges)."""
     from lightcompress_amd import _lib as L
-    x = torch.randn(2 * K, K, generator=gen(5300 + K), dtype=torch.float64)
-    H = (x.t() @ x / K + torch.eye(K, dtype=torch.float64)).float().to(dev)
+    if K <= 2304:
+        x = torch.randn(2 * K, K, generator=gen(5300 + K), dtype=torch.float64)
+        H = (x.t() @ x / K + torch.eye(K, dtype=torch.float64)).float().to(dev)
+    else:
+        x = torch.randn(K, K, generator=gen(5300 + K)).to(dev) * (0.5 / K ** 0.5)
+        H = x + x.t() + 3 * torch.eye(K, device=dev)
     perm = torch.randperm(K, generator=gen(K)).to(dev)
     nbytes = L.lib().lcq_chol_inv_upper_workspace_bytes(K)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     out = []
-    for h, p in ((H, perm), (H[perm][:, perm], None)):
-        hd, U = torch.triu(h).contiguous(), torch.full((K, K), 7.0, device=dev)
+    for h, p, off in ((H, perm, 0), (H[perm][:, perm], None, 0), (H, perm, 1)):
+        hd, U = torch.empty(K * K + off, device=dev)[off:].view(K, K).copy_(torch.triu(h)), torch.full((K, K), 7.0, device=dev)
         L.check(L.lib().lcq_chol_inv_upper(L.ptr(hd), K, L.ptr(p), 0.0, None, 0, L.ptr(U), L.ptr(ws), nbytes, None, L.stream()), 'chain')
         out.append(U)
-    assert torch.equal(out[0], out[1])
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
 
 
 @pytest.mark.parametrize('K', [1, 15, 16, 17, 31, 48, 65, 97, 112, 113, 127, 128, 129, 131, 257])
