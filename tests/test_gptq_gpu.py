@@ -1608,20 +1608,24 @@ def test_switch_combinations_give_one_result(dev):
 
 
 @pytest.mark.parametrize('R', [6144, 6151, 9000])
-@pytest.mark.parametrize('mode', ['searched', 'searched_sym', 'static', 'block_factor'])
+@pytest.mark.parametrize('mode', ['group256', 'group8', 'unrounded', 'static_gidx', 'group8_block_factor'])
 def test_block_kernel_workgroup_shapes_agree(dev, R, mode):
-    """lcq_gptq_block takes 32 rows per workgroup from 6144 rows on and 16 below (the kernel every small case above
-    runs against the oracle): rows do not interact, so the two shapes must agree bit for bit on every output, also
-    with a ragged last workgroup."""
+    """lcq_gptq_block takes 32 rows per workgroup from 6144 rows on and 16 below (the kernel that the small cases of these forms run
+    against the oracle) where a block does not run by panels of 64 rows: groups longer than a block or shorter than a panel, unrounded
+    zero points, columns with a group index.  Rows do not interact, so the two shapes must agree bit for bit on every output, also with
+    a ragged last workgroup."""
     from lightcompress_amd import _lib as L
     lib = L.lib()
-    K, i1, g = 512, 256, 64
+    K, i1 = 512, 256
+    g = {'group256': 256, 'unrounded': 64, 'static_gidx': 64}.get(mode, 8)
     G = K // g
     U = (torch.triu(torch.randn(K, K, generator=gen(1)) * 0.02) + torch.eye(K) * 1.5).to(dev)
     W0 = (torch.randn(R, K, generator=gen(2)) * 0.05).to(dev)
+    gidx = torch.randint(0, G, (K,), generator=gen(5), dtype=torch.int32).to(dev) if mode == 'static_gidx' else None
     outs = []
     for extra in (L.FLAG_ROWS16, 0):
-        flags = extra | (L.FLAG_SYM if mode == 'searched_sym' else 0) | (L.FLAG_STATIC if mode == 'static' else 0)
+        flags = extra | (L.FLAG_SYM if mode == 'group8' else 0) | (L.FLAG_STATIC if gidx is not None else 0)
+        flags |= L.FLAG_NO_ROUND_ZP if mode == 'unrounded' else 0
         W = W0.clone()
         W[:, i1:] += 0.01                                   # what earlier blocks' updates would have left
         tmp, Lo = torch.zeros_like(W), torch.zeros_like(W)
@@ -1629,8 +1633,8 @@ def test_block_kernel_workgroup_shapes_agree(dev, R, mode):
         sc = (torch.rand(R, G, generator=gen(3)) * 0.01 + 0.005).to(dev)
         ze = torch.randint(0, 16, (R, G), generator=gen(4)).float().to(dev)
         L.check(lib.lcq_gptq_block(L.ptr(W), L.ptr(tmp), L.ptr(Lo), L.ptr(Err), L.i64(128), L.ptr(U),
-                                   L.ptr(W0) if mode == 'block_factor' else None, L.i64(R), L.i64(K), L.i64(K), L.i64(i1),
-                                   L.i32(128), L.i32(g), L.f32(0.0), L.f32(15.0), L.i32(flags), L.ptr(sc), L.ptr(ze), None,
+                                   L.ptr(W0) if 'block_factor' in mode else None, L.i64(R), L.i64(K), L.i64(K), L.i64(i1),
+                                   L.i32(128), L.i32(g), L.f32(0.0), L.f32(15.0), L.i32(flags), L.ptr(sc), L.ptr(ze), L.ptr(gidx),
                                    L.i64(G), L.stream()), 'lcq_gptq_block')
         torch.cuda.synchronize()
         outs.append((tmp, Lo, Err, sc, ze))
@@ -1639,17 +1643,18 @@ def test_block_kernel_workgroup_shapes_agree(dev, R, mode):
     assert float(outs[0][1].sum()) > 0 and bool(torch.isfinite(outs[0][2]).all())
 
 
-@pytest.mark.parametrize('R', [1, 15, 16, 17, 63, 64, 65, 130])
+@pytest.mark.parametrize('R', [1, 15, 16, 17, 63, 64, 65, 130, 6151])
 @pytest.mark.parametrize('g', [16, 32, 64, 128])
-@pytest.mark.parametrize('sym,factor', [(False, False), (True, True)])
-def test_panels_of_whole_blocks(dev, R, g, sym, factor):
+@pytest.mark.parametrize('bits,sym,factor', [(4, False, False), (4, True, True), (8, False, True), (8, True, False), (11, False, False)])
+def test_panels_of_whole_blocks(dev, R, g, bits, sym, factor):
     """lcq_gptq_block on 128 whole columns with groups that open inside the block: scales and zero points are those of the ranges in
-    W, every weight is quantized by the reference's expressions from the value it has then (products near a rounding boundary, exact
-    halves, an infinity and a NaN among them), its error or Q - W0 and its loss follow bit for bit, and what it is then is
-    W - sum_k err_k U[k, :] up to the roundings of that sum (k of them on its largest magnitude).  Nothing else is written."""
+    W, every weight is quantized by the reference's expressions from the value it has then (products near a rounding boundary and exact
+    halves among them; codes that run few, some or all panels again with divisions), its error or Q - W0 and its loss follow bit for
+    bit, and what it is then is W - sum_k err_k U[k, :] up to the roundings of that sum (k of them on its largest magnitude).  Nothing
+    else is written.  (Rows with an infinity or a NaN are compared between searched and given parameters only.)"""
     from lightcompress_amd import _lib as L
     K, i1 = 384, 128
-    G, qmin, qmax = K // g, (-8.0 if sym else 0.0), (7.0 if sym else 15.0)
+    G, qmin, qmax = K // g, (-2.0 ** (bits - 1) if sym else 0.0), (2.0 ** (bits - 1) - 1 if sym else 2.0 ** bits - 1)
     U = (torch.triu(torch.randn(K, K, generator=gen(11)) * 0.05) + torch.eye(K) * 1.5).to(dev)
     W0 = (torch.randn(R, K, generator=gen(12)) * 0.05).to(dev)
     W = W0 + 0.01
@@ -1668,7 +1673,6 @@ def test_panels_of_whole_blocks(dev, R, g, sym, factor):
     d = torch.diag(U)[i1:i1 + 128]
     t, ranges = tmp[:, i1:i1 + 128], W[:, i1:i1 + 128].view(R, 128 // g, g)
     mn, mx = ranges.amin(-1), ranges.amax(-1)
-    tiny = torch.tensor(1e-5, device=dev)
     if sym:
         s = torch.maximum(mn.abs(), mx.abs()).clamp(min=1e-5) / torch.tensor(qmax, device=dev)
         z = torch.zeros_like(s)
