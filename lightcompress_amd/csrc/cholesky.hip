@@ -644,8 +644,9 @@ static int chol_chain(float* H, int64_t K64, const int64_t* perm, float percdamp
   // one, but their trailing update is applied only inside the current 512-column super-panel;
   // the rest of the matrix is updated once per super-panel with a 512-deep contraction, which
   // cuts the read-modify-write traffic on the trailing matrix fourfold.
-  // The last 1024 columns are one super-panel: their rank-128 updates are at most 98 of the 64 x 128 tiles, so each still takes
-  // one tile's time (8 us), while the 512-deep update they replace ran on 10 to 36 of 256 CUs (32 us).
+  // The last 1024 columns are one super-panel: their rank-128 updates stay launches of about 5 us, while the 512-deep update that they
+  // replace runs on 10 to 36 of 256 CUs (32 us).  K = 1024: 213 us with 512 columns, 189 so; 2048: 484 and 460; 4096: 1099 and 1074.
+  // (1536 and 2048 columns: 2048 443 and 439, 4096 1057 and 1053; 14336 the same within 1 %.)
   constexpr int TAIL = 8 * NB;
   const auto super_end = [&](int o0) { return K - o0 <= TAIL ? K : o0 + NBO; };
   // Long chains: the deep update behind a super-panel is split into the columns of the NEXT super-panel (on the

@@ -514,8 +514,8 @@ __global__ __launch_bounds__(256, 2) void gemm_s3_batched_kernel(const float* A,
 extern std::atomic<int> g_gemm_split;
 
 // TM = 128, 64 or 32 rows of C per workgroup.  The short tiles are for launches that would not give every CU a
-// 128-row tile (rank-128 updates and panel solves of the blocked chains): twice the workgroups, half the serial
-// MFMA work in each.
+// 128-row tile: twice the workgroups, half the serial MFMA work in each.  (Panel solves and rank-128 updates of the blocked chains come
+// here where rows do not start on 16 bytes or the last block is not full; the others take the kernels for a depth of 128 below.)
 template <bool B_T, int TM, bool DEEP = false>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmProblem g, float alpha, float beta, int flags) {
   __shared__ float sA[TM * GPA];
@@ -539,9 +539,8 @@ __global__ __launch_bounds__(256) void gemm_f32_batched_kernel(const float* A, i
 
 // A contraction of exactly 128 (panel solves and rank-128 updates of the blocked chains, the column loop's updates inside a window):
 // C = A op(B) (ADD: C -= A op(B)), no LDS and no barrier between loads and products.  An operand of v_mfma_f32_16x16x4f32 is one element
-// of a 16-byte piece that a lane reads where it lies (lane (g, m) = (l / 16, l % 16) of instruction e supplies k = 16 s + 4 g + e), so all
-// loads of a wave are in flight before its first product and a launch is little more than a memory latency and the 64 products of a
-// wave.  B given as [n][k] takes the place of the rows of the product, whose accumulator is then four columns of one row of C; from a
+// of a 16-byte piece that a lane reads where it lies (lane (g, m) = (l / 16, l % 16) of instruction e supplies k = 16 s + 4 g + e): a
+// launch is little more than a memory latency and the 64 products of a wave.  B given as [n][k] takes the place of the rows of the product, whose accumulator is then four columns of one row of C; from a
 // B given as [k][n] a lane reads two neighbouring columns, one for each of two products.  Either way C is read and written in pieces of
 // 8 or 16 bytes.  A wave owns 16 x 32 of C, a workgroup WN of them side by side.  Rows and columns are clamped for reading; N is a
 // multiple of 4.  Without ADD C may be A itself (a workgroup spans all of N then; the barrier is for that).
@@ -580,8 +579,9 @@ __global__ __launch_bounds__(64 * WN) void gemm_f32_rank128_kernel(GemmProblem p
     for (int q = 0; q < PIECES; ++q) old[q] = *(const piece*)(p.C + (long long)min(row_of(q), p.M - 1) * p.ldc + min(col_of(q), p.N - WIDTH));
   }
   f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-  // Loads that the compiler lets slip in between the products wait for one memory latency after the other: with a B from beyond L2 14 us
-  // instead of 8.3 for 1000 x 384.  (With both operands in L2, as in the chain, that is the better order: K = 1024 205 us against 211.)
+  // All loads in flight before the first product: those that the compiler lets slip in between wait for one memory latency after the other,
+  // with a B from beyond L2 14 us instead of 8.3 for 1000 x 384.  (With both operands in L2, as in the chain with B given as [n][k], the
+  // compiler's order in 24 registers is the better one: K = 1024 205 us against 211.)
   if constexpr (!B_T) __builtin_amdgcn_sched_barrier(0);
   #pragma unroll
   for (int s = 0; s < 8; ++s)
@@ -698,7 +698,8 @@ inline void launch_gemm(const GemmProblem& g, float alpha, float beta, int flags
   if (split && (long long)gx * gy >= 64 && (long long)gx * gy <= 256 && g.Kc >= 256)
     gemm_s3_kernel<B_T><<<dim3(gx, gy), dim3(256), 0, st>>>(g, alpha, beta, flags);
   // at most 128 of the 64-row tiles: 32-row tiles instead, twice the CUs and half the serial MFMA work in each (a
-  // 64 x 128 tile with a 128-deep contraction is 3.9 us of fp32 MFMA on its CU; K = 4096 chain 2.14 -> 1.99 ms)
+  // 64 x 128 tile with a 128-deep contraction is 3.9 us of fp32 MFMA on its CU; K = 4096 chain 2.14 -> 1.99 ms when all its
+  // narrow launches were these)
   else if ((long long)gx * ((g.M + 63) / 64) <= 128 && g.Kc > 0 && g.Kc <= 4 * GK &&
            !(flags & (GEMM_K_FROM_N | GEMM_K_TO_M)))
     gemm_f32_kernel<B_T, 32, true><<<dim3(gx, (unsigned)((g.M + 31) / 32)), dim3(256), 0, st>>>(g, alpha, beta, flags);

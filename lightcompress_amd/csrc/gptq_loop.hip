@@ -361,22 +361,26 @@ __global__ __launch_bounds__(16 * RW) void gptq_block_kernel(LoopArgs a) {
   }
 }
 
-// The same block for its most frequent forms: 128 whole columns, groups of 16, 32, 64 or 128 of them that open inside the block or
-// parameters that are given for groups of whole panels or rows, rounded zero points.  What the kernel above spends its time on are instructions: sixteen lanes share a row, so a column's quantization is
-// issued once per four rows, and its update takes eight multiply-adds.  Here a wave quantizes 64 rows, one per lane:
+// The same block for its most frequent forms (gptq_by_panels): 128 whole columns, groups of 16, 32, 64 or 128 of them that open inside the
+// block or parameters that are given for groups of whole panels or rows, rounded zero points.  What the kernel above spends its time on are
+// instructions: sixteen lanes share a row, so a column's quantization is issued once per four rows, and its update takes eight
+// multiply-adds.  Here a wave quantizes 64 rows, one per lane:
 //   * the chain wave (0) takes 16 columns from LDS and goes through them without a barrier.  A column is about nine instructions and at
 //     most four v_mfma_f32_4x4x1_16b: with ONE block of the A operand (four columns of a row of U) broadcast to all 16 (cbsz = 4, abid),
 //     an instruction updates four columns of 64 rows;
 //   * the update waves (1, 2, 3, 5) hold 16 rows each in 16 x 16 tiles, the accumulators of v_mfma_f32_16x16x4f32.  They apply the
 //     errors of a finished panel first to the next panel's columns and hand those over, then to the rest beside the chain of the next
 //     panel.  Two barriers per panel;
-//   * waves 4, 6 and 7 bring U to LDS; 6 and 7 then write the outputs of a finished panel.  The chain wave keeps its SIMD to itself: beside an update wave its products wait for
-//     the other's, 32 cycles each, and a panel takes up to 2400 cycles instead of 1200.
+//   * waves 4, 6 and 7 bring U to LDS; 6 and 7 then write the outputs of a finished panel.  The chain wave keeps its SIMD to itself:
+//     beside an update wave its products wait for the other's, 32 cycles each, and a panel takes up to 2400 cycles instead of 1340.
 // The ranges of all groups are known before the first column (groups are read from W as it is in memory).
-// Quotients go through the group's reciprocal as above.  Where a product is closer to a rounding boundary than its error can be,
-// |t| 2^-22 for |t| up to the code range + 1, the wave runs the panel again with true divisions: 1.5 % of the panels at 4 bits.
+// Quotients go through the group's reciprocal as above.  Where a product is closer to a rounding boundary than twice what its error can be,
+// |t| 2^-22 for |t| up to the code range + 1, the wave runs the panel again with true divisions.  With 1024 products per panel that
+// is 1 to 2 % of the panels at 4 bits, 12 to 22 % at 8 (4096 rows: 14.8 and 16.1 us per block; 16.5 by the kernel above), 40 % at codes of
+// +-512, and beyond those, where reciprocals are not used, all of them (19.3 us; 24.3 by the kernel above, which divides then too).
 // (The 2^-11 of the kernel above, for codes up to 1024, would be one of 1000 products.)
-// Bound by the chain: eight times 1330 cycles for its columns and 1000 for the handing over, behind 6500 for the ranges and U.
+// Bound by the chain: eight times 1340 cycles for its columns and 1050 to 1650 for the handing over, behind 7200 (64 rows) to 8700 (4096) for
+// the ranges and U.
 // R = 64: 14.2 -> 12.8 us per block, 1000: 15.6 -> 13.7, 4096: 17.3 -> 14.9, 6144: 20.3 -> 16.1, 14336: 29.7 -> 21.3, 28672: 49.5 -> 31.7
 // (two workgroups per CU).  The chain wave bringing in the errors of the panel before by itself, 64 more matrix instructions, cost 700
 // cycles per panel instead of the 500 of the handing over.
